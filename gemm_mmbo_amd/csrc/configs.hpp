@@ -79,6 +79,25 @@ constexpr RingRow kX16Tiles[NUM_X16_TILES] = {
     {192, 256, 2, 2, 5},     // four wavefronts of 96 x 128
 };
 
+// Tiles of the split-by-wavefront kernel (gemm_wave.hpp), all element types.  They have no config ids: the automatic pick takes
+// them by a rule of its own (mmbo_gemm.hip).
+constexpr int NUM_WAVE_TILES = 8;
+constexpr int kWaveMaxWaves = 4;                  // wavefronts of a work-group that share k
+struct WaveRow {
+    int bm, bn;
+    int depth;        // slices in a wavefront's LDS ring
+};
+constexpr WaveRow kWaveTiles[NUM_WAVE_TILES] = {
+    {16, 16, 8},      // 16 KB of ring per wavefront
+    {16, 32, 6},      // 18 KB
+    {32, 16, 6},
+    {16, 64, 4},      // 20 KB
+    {64, 16, 4},
+    {32, 32, 4},      // 16 KB
+    {32, 64, 4},      // 24 KB
+    {64, 32, 4},
+};
+
 // Config ids (fp32 and fp16 share them): [0, kStagedConfigs) the staged kernel's (tile, split) pairs, then the ring
 // kernel's (ring tile, split) pairs, then the x16 kernel's.  split_index indexes kSplits.
 constexpr int kStagedConfigs = NUM_TILES * NUM_SPLITS;

@@ -48,6 +48,10 @@ struct GemmArgs {
     uint32_t c_prefetch;    // 1: beta != 0 and the old C may be fetched into freed LDS ring buffers ahead of the epilogue
     uint32_t c_stream;      // 1: C leaves with the non-temporal hint (x16 kernel; long k, many rounds of tiles)
     uint32_t line_rows;     // 1: A, B, their leading dimensions and batch strides are multiples of a 128-byte memory line
+    uint32_t wave_pairs;    // gemm_wave.hpp: pairs of slices each wavefront of a work-group takes
+    uint32_t no_successor;  // gemm_wave.hpp: last columns of k whose edge groups of rows have no memory behind them
+    uint32_t columns_first; // gemm_wave.hpp: tiles are walked along a tile row first
+    uint32_t reduce_parts;  // splitk_reduce_kernel: threads that share the splits of one group of sums
     uint32_t ws_narrow;     // 1: a tile's span of the split-K workspace (tile columns x m floats) fits 32-bit offsets
 };
 

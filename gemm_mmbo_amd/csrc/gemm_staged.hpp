@@ -329,35 +329,43 @@ gemm_staged_kernel(const GemmArgs args)
     write_back<T, FM, FN, false>(acc, args, row0 + wm * Cfg::TM, col0 + wn * Cfg::TN, batch, split, lane);
 }
 
-// Split-K reduction: C = alpha * sum_s ws[s] + beta * C, splits added in ascending order so the
-// result does not depend on scheduling.  The workspace is [split][batch][n][m] fp32, dense, so four consecutive
-// rows of one column are one 16-byte load per split; a thread owns such a group when m % 4 == 0 (VEC4), one
-// element otherwise.  All loads of a thread are independent and issued before the first add (the loop over the
-// splits is unrolled for the split factors the library uses); the adds keep the order.
-template <typename T, bool VEC4>
+// Split-K reduction: C = alpha * sum_s ws[s] + beta * C, splits added in a fixed order so the result does not depend on
+// scheduling.  The workspace is [split][batch][n][m] fp32 (fp64 for fp64), dense, so consecutive rows of one column are one
+// 16-byte load per split; a thread owns such a group (four rows, fp64 two) when m is a multiple of it (VEC), one element
+// otherwise.  All loads of a thread are independent and issued before the first add (the loop over the splits is
+// unrolled for the split factors the library uses); the adds keep the order.  With more than sixteen splits the outputs
+// are few and one thread's chain of loads long: args.reduce_parts threads then take equal runs of the splits and the first of
+// them adds the runs up, in order, through LDS (MANY; a kernel of its own: with the parts counted at run time the common case
+// took 1 us longer).
+template <typename T, bool VEC, bool MANY>
 __global__ void __launch_bounds__(256)
 splitk_reduce_kernel(const GemmArgs args)
 {
-    constexpr int W = VEC4 ? 4 : 1;
+    using elem = typename std::conditional<sizeof(T) == 8, double, float>::type;
+    constexpr int W = VEC ? 16 / (int)sizeof(elem) : 1;
+    typedef elem sums_t __attribute__((ext_vector_type(16 / sizeof(elem))));
+    const uint32_t parts = MANY ? args.reduce_parts : 1, per_block = 256 / parts;           // a power of two, 1 .. 8
+    const uint32_t part = MANY ? threadIdx.x / per_block : 0, mine = MANY ? threadIdx.x % per_block : threadIdx.x;
     const size_t mn = (size_t)args.m * args.n;
-    const size_t idx = ((size_t)blockIdx.x * 256 + threadIdx.x) * W;
+    const size_t idx = ((size_t)blockIdx.x * per_block + mine) * W;
     const uint32_t batch = blockIdx.z;
-    if (idx >= mn) return;
-    const uint32_t row = (uint32_t)(idx % args.m), col = (uint32_t)(idx / args.m);
+    const bool inside = idx < mn;
+    if (!MANY && !inside) return;
     const size_t stride = (size_t)args.batch * mn;                  // one split further
-    const float *w = args.ws + (size_t)batch * mn + idx;
-    float s[W];
+    const elem *w = reinterpret_cast<const elem *>(args.ws) + (size_t)batch * mn + idx;
+    elem s[W];
 #pragma unroll
-    for (int e = 0; e < W; ++e) s[e] = 0.0f;
+    for (int e = 0; e < W; ++e) s[e] = 0;
     auto add_splits = [&](auto NS, uint32_t first) {
         constexpr int ns = decltype(NS)::value;
-        float v[ns][W];
+        elem v[ns][W];
 #pragma unroll
         for (int q = 0; q < ns; ++q) {
-            const float *p = w + (size_t)(first + q) * stride;
-            if constexpr (VEC4) {
-                f32x4 t = *reinterpret_cast<const f32x4 *>(p);
-                v[q][0] = t[0]; v[q][1] = t[1]; v[q][2] = t[2]; v[q][3] = t[3];
+            const elem *p = w + (size_t)(first + q) * stride;
+            if constexpr (VEC) {
+                const sums_t t = *reinterpret_cast<const sums_t *>(p);
+#pragma unroll
+                for (int e = 0; e < W; ++e) v[q][e] = t[e];
             } else {
                 v[q][0] = *p;
             }
@@ -367,35 +375,43 @@ splitk_reduce_kernel(const GemmArgs args)
 #pragma unroll
             for (int e = 0; e < W; ++e) s[e] += v[q][e];
     };
-    uint32_t sp = 0;
-    for (; sp + 8 <= args.splits; sp += 8) add_splits(std::integral_constant<int, 8>{}, sp);
-    if (sp + 4 <= args.splits) { add_splits(std::integral_constant<int, 4>{}, sp); sp += 4; }
-    if (sp + 2 <= args.splits) { add_splits(std::integral_constant<int, 2>{}, sp); sp += 2; }
-    if (sp < args.splits) add_splits(std::integral_constant<int, 1>{}, sp);
+    const uint32_t run = MANY ? (args.splits + parts - 1) / parts : args.splits;
+    uint32_t sp = MANY ? part * run : 0;
+    const uint32_t sp_end = MANY ? (inside ? min(args.splits, sp + run) : 0) : args.splits;
+    for (; sp + 8 <= sp_end; sp += 8) add_splits(std::integral_constant<int, 8>{}, sp);
+    if (sp + 4 <= sp_end) { add_splits(std::integral_constant<int, 4>{}, sp); sp += 4; }
+    if (sp + 2 <= sp_end) { add_splits(std::integral_constant<int, 2>{}, sp); sp += 2; }
+    if (sp < sp_end) add_splits(std::integral_constant<int, 1>{}, sp);
+    if constexpr (MANY) {
+        __shared__ elem partial[256 * W];
+#pragma unroll
+        for (int e = 0; e < W; ++e) partial[threadIdx.x * W + e] = s[e];
+        __syncthreads();
+        if (part != 0 || !inside) return;
+        for (uint32_t q = 1; q < parts; ++q)
+#pragma unroll
+            for (int e = 0; e < W; ++e) s[e] += partial[(q * per_block + mine) * W + e];
+    }
 
+    const uint32_t row = (uint32_t)(idx % args.m), col = (uint32_t)(idx / args.m);
     T *p = static_cast<T *>(args.C) + (int64_t)batch * args.strideC + (size_t)col * args.ldc + row;
-    const float alpha = args.alpha, beta = args.beta;
-    if (VEC4 && args.vec_c) {
-        typedef typename std::conditional<sizeof(T) == 4, u32x4, u32x2>::type cvec;
-        union { T e[4]; cvec v; } io;
-        float o[4];
+    const elem alpha = sizeof(T) == 8 ? (elem)args.alpha_d : (elem)args.alpha, beta = sizeof(T) == 8 ? (elem)args.beta_d : (elem)args.beta;
+    auto update = [&](elem sum, T old) {
+        const elem o = alpha * sum;
+        if (beta == (elem)0) return (T)o;
+        if constexpr (sizeof(T) == 8) return (T)__builtin_fma(beta, (double)old, o);
+        else return (T)__builtin_fmaf(beta, (float)old, o);
+    };
+    if (VEC && args.vec_c) {
+        struct rows_t { T e[W]; } __attribute__((aligned(sizeof(T) * W)));
+        rows_t io;
+        if (beta != (elem)0) io = *reinterpret_cast<const rows_t *>(p);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = alpha * s[e];
-        if (beta != 0.0f) {
-            io.v = *reinterpret_cast<const cvec *>(p);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(beta, (float)io.e[e], o[e]);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) io.e[e] = (T)o[e];
-        *reinterpret_cast<cvec *>(p) = io.v;
+        for (int e = 0; e < W; ++e) io.e[e] = update(s[e], io.e[e]);
+        *reinterpret_cast<rows_t *>(p) = io;
     } else {
 #pragma unroll
-        for (int e = 0; e < W; ++e) {
-            float o = alpha * s[e];
-            if (beta != 0.0f) o = __builtin_fmaf(beta, (float)p[e], o);
-            p[e] = (T)o;
-        }
+        for (int e = 0; e < W; ++e) p[e] = update(s[e], beta != (elem)0 ? p[e] : (T)0);
     }
 }
 

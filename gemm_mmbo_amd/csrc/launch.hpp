@@ -38,6 +38,11 @@ hipError_t launch_dgemm(int transA, int transB, const GemmArgs &args, hipStream_
 template <int TILE>
 int dgemm_lds_bytes();
 
+// Split-by-wavefront kernel (gemm_wave.hpp) of wave tile row TILE (dtype 2 = fp64) with `waves` wavefronts per work-group;
+// grid = (batch, nwg0*nwg1, splits).
+template <int DTYPE, int TILE>
+hipError_t launch_wave(int transA, int transB, const GemmArgs &args, int waves, hipStream_t stream);
+
 hipError_t launch_splitk_reduce(int dtype, const GemmArgs &args, hipStream_t stream);
 
 }  // namespace mmbo

@@ -3,6 +3,7 @@
 // layer src/gemm/gemm.h (front-ends), src/gemm/constants.h (tables) and src/gemm/driver.h (launch).
 #include "../../include/mmbo_gemm.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -13,6 +14,7 @@
 #include "configs.hpp"
 #include "gemm_common.hpp"
 #include "gemm_staged.hpp"
+#include "gemm_wave.hpp"
 #include "launch.hpp"
 #include "tuned_table.hpp"
 
@@ -274,6 +276,14 @@ hipError_t dispatch_x16(int tile, int ta, int tb, const GemmArgs &a, hipStream_t
     return hipErrorInvalidValue;
 }
 
+template <int DTYPE, int TILE>
+hipError_t dispatch_wave(int tile, int ta, int tb, const GemmArgs &a, int waves, hipStream_t s)
+{
+    if (tile == TILE) return launch_wave<DTYPE, TILE>(ta, tb, a, waves, s);
+    if constexpr (TILE + 1 < NUM_WAVE_TILES) return dispatch_wave<DTYPE, TILE + 1>(tile, ta, tb, a, waves, s);
+    return hipErrorInvalidValue;
+}
+
 template <int TILE>
 hipError_t dispatch_dgemm(int tile, int ta, int tb, const GemmArgs &a, hipStream_t s)
 {
@@ -370,13 +380,21 @@ double model_time_f64(int tile, size_t m, size_t n, size_t k, int batch)
 hipError_t launch_splitk_reduce(int dtype, const GemmArgs &args, hipStream_t stream)
 {
     size_t mn = (size_t)args.m * args.n;
-    const bool vec4 = args.m % 4 == 0;                   // a thread then owns four consecutive rows of one column
-    dim3 grid((unsigned)ceil_div(vec4 ? mn / 4 : mn, 256), 1, args.batch);
-    if (dtype == MMBO_F32)
-        return vec4 ? launch_kernel(splitk_reduce_kernel<float, true>, grid, dim3(256), 0, stream, args)
-                    : launch_kernel(splitk_reduce_kernel<float, false>, grid, dim3(256), 0, stream, args);
-    return vec4 ? launch_kernel(splitk_reduce_kernel<half_t, true>, grid, dim3(256), 0, stream, args)
-                : launch_kernel(splitk_reduce_kernel<half_t, false>, grid, dim3(256), 0, stream, args);
+    const bool vec = dtype == MMBO_F64 ? args.m % 2 == 0 : args.m % 4 == 0;      // a thread then owns 16 bytes of sums of one column
+    const size_t groups = vec ? mn / (dtype == MMBO_F64 ? 2 : 4) : mn;
+    // more than sixteen splits: several threads share the splits of one group (see the kernel)
+    GemmArgs a = args;
+    a.reduce_parts = args.splits <= 16 ? 1 : args.splits <= 32 ? 4 : 8;
+    dim3 grid((unsigned)ceil_div(groups * a.reduce_parts, 256), 1, args.batch);
+    auto launch = [&](auto zero) {
+        using T = decltype(zero);
+        if (a.reduce_parts == 1)
+            return vec ? launch_kernel(splitk_reduce_kernel<T, true, false>, grid, dim3(256), 0, stream, a)
+                       : launch_kernel(splitk_reduce_kernel<T, false, false>, grid, dim3(256), 0, stream, a);
+        return vec ? launch_kernel(splitk_reduce_kernel<T, true, true>, grid, dim3(256), 0, stream, a)
+                   : launch_kernel(splitk_reduce_kernel<T, false, true>, grid, dim3(256), 0, stream, a);
+    };
+    return dtype == MMBO_F32 ? launch(0.0f) : dtype == MMBO_F64 ? launch(0.0) : launch((half_t)0.0f);
 }
 
 }  // namespace mmbo
@@ -545,7 +563,7 @@ static double model_time_x16_only(int dtype, int tile, int split, size_t m, size
 }
 
 // The cost model's pick among the staged configs (fp32/fp16), which take any shape and any alignment.
-static int select_staged(int dtype, size_t m, size_t n, size_t k, int batch)
+static int select_staged(int dtype, size_t m, size_t n, size_t k, int batch, double *us = nullptr)
 {
     int best = 0;
     double best_t = 0.0;
@@ -558,19 +576,24 @@ static int select_staged(int dtype, size_t m, size_t n, size_t k, int batch)
             if (best_t == 0.0 || t < best_t) { best_t = t; best = tile + NUM_TILES * si; }
         }
     }
+    if (us) *us = best_t / 2400.0;
     return best;
 }
 
-int mmbo_select_config(int dtype, int transA, int transB, size_t m, size_t n, size_t k, int batch)
+// The pick of mmbo_select_config and, in *us, the microseconds its model (or the tuned table's record) gives it.
+static int select_config(int dtype, int transA, int transB, size_t m, size_t n, size_t k, int batch, double *us)
 {
+    *us = 0.0;
     if (!valid_dtype(dtype)) return -MMBO_ERR_INVALID_DTYPE;
     if ((transA | transB) & ~1) return -MMBO_ERR_INVALID_OP;
     if (batch < 0) return -MMBO_ERR_INVALID_SIZE;
     if (m == 0 || n == 0 || batch == 0) return 0;
     for (const TunedRow &t : kTuned)
         if (t.dtype == dtype && t.transA == transA && t.transB == transB && t.m == m && t.n == n && t.k == k &&
-            t.batch == batch)
+            t.batch == batch) {
+            *us = 2.0 * (double)m * (double)n * (double)k * batch / t.tflops * 1e-6;
             return t.config_id;
+        }
     if (dtype == MMBO_F64) {
         int best = 0;
         double best_t = 0.0;
@@ -578,6 +601,7 @@ int mmbo_select_config(int dtype, int transA, int transB, size_t m, size_t n, si
             double t = model_time_f64(tile, m, n, k, batch);
             if (best_t == 0.0 || t < best_t) { best_t = t; best = tile; }
         }
+        *us = best_t;
         return best;
     }
     // Whole-tile kernels (deeper prefetch, no edge handling) measured faster than the staged kernel on every shape
@@ -629,9 +653,18 @@ int mmbo_select_config(int dtype, int transA, int transB, size_t m, size_t n, si
                 }
             }
         }
-        if (pick >= 0) return pick;
+        if (pick >= 0) {
+            *us = pick_t;
+            return pick;
+        }
     }
-    return select_staged(dtype, m, n, k, batch);
+    return select_staged(dtype, m, n, k, batch, us);
+}
+
+int mmbo_select_config(int dtype, int transA, int transB, size_t m, size_t n, size_t k, int batch)
+{
+    double us;
+    return select_config(dtype, transA, transB, m, n, k, batch, &us);
 }
 
 int mmbo_wg_remap(unsigned linear_id, unsigned nwg0, unsigned nwg1, unsigned wgm, unsigned num_xcd,
@@ -699,6 +732,156 @@ namespace {
 // Where the partial sums of a split-K config go.
 enum class WsSource { kLibrary, kStatic };
 
+// ---- the automatic pick between a config of the tables and the split-by-wavefront kernel ------------------------------
+
+struct WavePick {
+    int tile;           // row of kWaveTiles; < 0: none
+    int waves, split;
+    double us;          // modelled
+};
+
+// Modelled microseconds of the split-by-wavefront kernel.  A work-group costs a start, its slices -- each as long as the
+// slower of its wavefronts' MFMAs and LDS reads, of the memory lines the CU's wavefronts pull through its vector path, and of
+// the lines all CUs pull -- and its part of C; work-groups run in rounds of as many as LDS lets share a CU; the whole takes
+// at least what its bytes take from memory, and a call what the host takes to launch it.  Constants: least squares over 540
+// drawn shapes x every (tile, wavefronts, splits) that fits them; the pick is within 4 - 5 % of the fastest of them on
+// average, 39 % at worst.
+struct WaveModel {
+    double launch, start;           // us
+    double mfma_eff, clk_per_read;  // MFMA rate reached in the loop; clocks per LDS fragment read
+    double gap;                     // us per slice of a wavefront that has its SIMD to itself
+    double round_trip;              // us from a slice's request to its use, shared by the pairs in flight
+    double cu_bytes, chip_bytes;    // bytes of lines per us: one CU's path, all CUs together
+    double hbm_bytes;               // bytes per us from memory
+    double c_cu, c_wave;            // us per 1024 elements of a tile's C: through the CU, through each wavefront
+    double tail;                    // us for a partial slice through registers
+    double reduce, reduce_per_mb;   // us: second launch; per MB of partial sums
+};
+constexpr WaveModel kWaveModel[3] = {
+    {2.25, 1.08, 0.899, 7.4, 0.023, 0.372, 108.4e3, 31.9e6, 5.25e6, 0.322, 0.516, 0.376, 2.08, 0.370},      // fp32
+    {2.51, 0.65, 0.421, 0.0, 0.036, 0.233, 122.7e3, 32.8e6, 5.69e6, 0.193, 1.173, 0.731, 1.68, 0.379},      // fp16
+    {2.03, 1.15, 0.734, 8.9, 0.026, 0.471, 98.6e3, 26.0e6, 5.58e6, 0.484, 0.444, 0.246, 2.31, 0.422},      // fp64
+};
+
+struct WaveShape {
+    int dtype, transA, transB;
+    size_t m, n, k;
+    int batch;
+    size_t lda, ldb;
+    bool read_c;
+};
+
+double wave_model_us(const WaveShape &p, int tile, int waves, int split)
+{
+    const WaveModel &w = kWaveModel[p.dtype];
+    const WaveRow &row = kWaveTiles[tile];
+    const double esz = p.dtype == MMBO_F64 ? 8 : p.dtype == MMBO_F32 ? 4 : 2, sum_size = p.dtype == MMBO_F64 ? 8 : 4;
+    const size_t bk = (size_t)(64 / esz);
+    const size_t pairs = ceil_div(ceil_div(p.k, bk), 2), pairs_per_split = ceil_div(pairs, (size_t)split), splits = ceil_div(pairs, pairs_per_split);
+    const double slices = (double)std::min(2 * ceil_div(pairs_per_split, (size_t)waves), ceil_div(p.k, bk));
+    const double wgs = (double)(ceil_div(p.m, row.bm) * ceil_div(p.n, row.bn) * splits) * p.batch;
+    const double ring = row.depth * (row.bm + row.bn) * 64.0, partial = (row.bm + 16 / sum_size) * row.bn * sum_size;
+    const int per_cu = std::max(1, std::min((int)(160 * 1024 / (waves * std::max(ring, partial))), 16 / waves));
+    // bytes of 128-byte lines one slice of an operand touches: whole lines where rows start on them, more where they do not
+    auto lines = [&](size_t rows, size_t dim, bool k_contiguous, size_t ld) {
+        const double here = (double)std::min(rows, ceil_div(dim, (size_t)16) * 16);
+        const bool on_lines = (size_t)(ld * esz) % 128 == 0;
+        if (k_contiguous) return here * 64 * (on_lines ? 1.0 : 1.5);
+        const double width = here * esz, per_column = on_lines ? std::max(width, 128.0) : width + 112;
+        return per_column * 64 / esz;
+    };
+    const double line_bytes = lines(row.bm, p.m, p.transA, p.lda) + lines(row.bn, p.n, !p.transB, p.ldb);
+    const int reads_rc = p.dtype == MMBO_F32 ? 4 : 2;
+    const double reads = row.bm / 16 * (p.transA ? 1 : reads_rc) + row.bn / 16 * (p.transB ? reads_rc : 1);
+    const double clocks = (p.dtype == MMBO_F16 ? 16.0 : 128.0) * (row.bm / 16) * (row.bn / 16);
+    const double work = (clocks / w.mfma_eff + reads * w.clk_per_read) / 2400.0;
+    const size_t per16 = (size_t)(16 / esz);
+    const bool tail = p.k % bk != 0 || (!p.transA && p.m % per16 != 0) || (p.transB && p.n % per16 != 0);
+    auto round = [&](double on_cu, double on_chip) {
+        const double slice = std::max(std::max(work * std::ceil(on_cu * waves / 4.0), std::max(work + w.gap, w.round_trip * 2 / row.depth)),
+                                      std::max(line_bytes * on_cu * waves / w.cu_bytes, line_bytes * waves * on_chip / w.chip_bytes));
+        return w.start + slices * slice + row.bm * row.bn * (w.c_cu * on_cu + w.c_wave / waves) / 1024 + (tail ? w.tail : 0.0);
+    };
+    const double slots = 256.0 * per_cu, full = std::floor(wgs / slots), last = wgs - full * slots;
+    double t = full * round(per_cu, slots);
+    if (last > 0) t += round(std::ceil(last / 256), last);
+    const double bytes = p.batch * ((double)p.m * p.k + (double)p.k * p.n + (double)p.m * p.n * (p.read_c ? 2 : 1)) * esz;
+    const double memory = bytes / w.hbm_bytes + 0.5 * w.start;
+    t = std::max(t, memory) + 0.15 * std::min(t, memory) + w.launch;
+    double host = 5.1;
+    if (splits > 1) {
+        t += w.reduce + w.reduce_per_mb * p.batch * (double)p.m * p.n * sum_size * splits / 1e6;
+        host = 8.8;
+    }
+    return std::max(t, host) + 0.02 * std::min(t, host);
+}
+
+WavePick pick_wave(const WaveShape &p)
+{
+    WavePick best{-1, 0, 0, 0.0};
+    const double sum_size = p.dtype == MMBO_F64 ? 8 : 4, esz = p.dtype == MMBO_F64 ? 8 : p.dtype == MMBO_F32 ? 4 : 2;
+    const size_t slices = ceil_div(p.k, (size_t)(64 / esz));
+    if (p.k == 0) return best;
+    for (int tile = 0; tile < NUM_WAVE_TILES; ++tile) {
+        const size_t tiles = ceil_div(p.m, kWaveTiles[tile].bm) * ceil_div(p.n, kWaveTiles[tile].bn);
+        if (tiles > 65535) continue;
+        for (int waves = 1; waves <= kWaveMaxWaves; waves *= 4) {
+            if (waves > 1 && slices < (size_t)waves) continue;
+            for (int split = 1; split <= 64; split *= 2) {
+                // (splits: at least a pair of slices per wavefront, not beyond what the chip holds at one time; the partial sums
+                // of either entry point fit the static workspace, so that both run the same split)
+                if (split > 1 && (slices < (size_t)split * waves * 2 || tiles * p.batch * split > 1024 ||
+                                  (double)p.m * p.n * p.batch * split * sum_size > (double)kScratchPartialBytes))
+                    break;
+                const double us = wave_model_us(p, tile, waves, split);
+                if (best.tile < 0 || us < best.us) best = WavePick{tile, waves, split, us};
+            }
+        }
+    }
+    return best;
+}
+
+// What the automatic pick runs for a shape.  The models are walked once per shape and thread (some microseconds, as much as a
+// small call takes); a small direct-mapped table keeps the answers, which are a function of the key alone.
+struct Plan {
+    WavePick wave;      // tile < 0: config_id
+    int config_id;
+};
+
+Plan plan_for(const WaveShape &p)
+{
+    struct Key {
+        int dtype, transA, transB, batch, read_c, lines_a, lines_b;
+        size_t m, n, k;
+    };
+    struct Entry {
+        bool used;
+        Key key;
+        Plan plan;
+    };
+    constexpr int kEntries = 64;
+    static thread_local Entry cache[kEntries];
+    const size_t per_line = 128 / (p.dtype == MMBO_F64 ? 8 : p.dtype == MMBO_F32 ? 4 : 2);
+    Key key;
+    std::memset(&key, 0, sizeof(key));                   // (compared as bytes)
+    key.dtype = p.dtype; key.transA = p.transA; key.transB = p.transB; key.batch = p.batch; key.read_c = p.read_c;
+    key.lines_a = p.lda % per_line == 0; key.lines_b = p.ldb % per_line == 0;
+    key.m = p.m; key.n = p.n; key.k = p.k;
+    size_t h = p.m * 0x9E3779B97F4A7C15ull ^ p.n * 0xC2B2AE3D27D4EB4Full ^ p.k * 0x165667B19E3779F9ull ^
+               (size_t)(p.batch * 16 + p.dtype * 4 + p.transA * 2 + p.transB) * 0x27D4EB2F165667C5ull;
+    Entry &e = cache[(h >> 32) % kEntries];
+    if (e.used && std::memcmp(&e.key, &key, sizeof(key)) == 0) return e.plan;
+    Plan plan;
+    double table_us;
+    plan.config_id = select_config(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, &table_us);
+    plan.wave = pick_wave(p);
+    if (plan.wave.us >= table_us) plan.wave.tile = -1;      // (150 drawn shapes: 1.42 times faster than the tables' configs alone)
+    e.used = true;
+    e.key = key;
+    e.plan = plan;
+    return plan;
+}
+
 int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
               const void *alpha, const void *A, size_t lda, long long strideA,
               const void *B, size_t ldb, long long strideB, const void *beta, void *C,
@@ -731,8 +914,63 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
 
     const size_t esz_in = f64 ? 8 : dtype == MMBO_F32 ? 4 : 2;
     if (config_id == MMBO_CONFIG_AUTO) {
-        config_id = mmbo_select_config(dtype, transA, transB, m, n, k, batch);
-        if (config_id < 0) return -config_id;
+        // Problems that a round of tiles would not spread over the chip: one launch of the split-by-wavefront kernel, which
+        // takes any shape and alignment.
+        const Plan plan = plan_for(WaveShape{dtype, transA, transB, m, n, k, batch, lda, ldb, f64 ? beta_d != 0.0 : beta_f != 0.0f});
+        const WavePick &w = plan.wave;
+        if (w.tile >= 0) {
+            const WaveRow &row = kWaveTiles[w.tile];
+            const size_t bk = 64 / esz_in;
+            // (a pair of slices must span less than the 2 GiB of a buffer descriptor)
+            if (tile_span_ok(TileRow{row.bm, row.bn, (int)(2 * bk), 0, 0}, transA, transB, lda, ldb, esz_in)) {
+                GemmArgs a;
+                std::memset(&a, 0, sizeof(a));
+                a.A = A; a.B = B; a.C = C;
+                a.alpha = alpha_f; a.beta = beta_f;
+                a.alpha_d = alpha_d; a.beta_d = beta_d;
+                a.m = (uint32_t)m; a.n = (uint32_t)n; a.k = (uint32_t)k;
+                a.lda = (uint32_t)lda; a.ldb = (uint32_t)ldb; a.ldc = (uint32_t)ldc;
+                a.strideA = strideA; a.strideB = strideB; a.strideC = strideC;
+                a.nwg0 = (uint32_t)ceil_div(m, row.bm); a.nwg1 = (uint32_t)ceil_div(n, row.bn);
+                a.batch = (uint32_t)batch;
+                // (how tiles are laid over the XCDs: see the kernel)
+                const bool tall = a.nwg0 >= a.nwg1;
+                const size_t long_ld = tall ? lda : ldb, line = 128 / esz_in;
+                const bool whole_lines = (tall ? !transA : transB) && long_ld % line == 0 && (uintptr_t)(tall ? A : B) % 128 == 0 &&
+                                         (tall ? row.bm : row.bn) % line == 0 && (tall ? a.nwg0 : a.nwg1) % 8 == 0;
+                a.wgm = whole_lines ? 1 : 8;
+                a.nxcd = whole_lines ? 1 : 8;
+                a.columns_first = whole_lines && !tall && a.nwg0 > 1;
+                const size_t pairs = ceil_div(ceil_div(k ? k : 1, bk), 2), pairs_per_split = ceil_div(pairs, w.split);
+                a.splits = (uint32_t)ceil_div(pairs, pairs_per_split);
+                a.k_per_split = (uint32_t)(a.splits > 1 ? pairs_per_split * 2 * bk : (k ? k : 1));
+                a.wave_pairs = (uint32_t)ceil_div(pairs_per_split, w.waves);
+                const uint32_t per16 = (uint32_t)(16 / esz_in);
+                const uint32_t past_a = transA ? 0 : wave::columns_without_a_successor(a.m, per16, a.lda),
+                               past_b = transB ? wave::columns_without_a_successor(a.n, per16, a.ldb) : 0;
+                a.no_successor = past_a > past_b ? past_a : past_b;
+                a.vec_c = ((uintptr_t)C % 16 == 0) && ((ldc * esz_in) % 16 == 0) && (((size_t)strideC * esz_in) % 16 == 0);
+                hipStream_t s = static_cast<hipStream_t>(stream);
+                WsHold ws_hold;
+                if (a.splits > 1) {
+                    const size_t bytes = (size_t)a.splits * batch * m * n * (f64 ? sizeof(double) : sizeof(float));
+                    char *base = nullptr;
+                    int rc = ws_source == WsSource::kStatic ? static_scratch(&base) : workspace(s, bytes, ws_hold, &base);
+                    if (rc != MMBO_OK) return rc;
+                    a.ws = reinterpret_cast<float *>(base);
+                }
+                hipError_t e = f64 ? dispatch_wave<2, 0>(w.tile, transA, transB, a, w.waves, s)
+                                   : dtype == MMBO_F32 ? dispatch_wave<0, 0>(w.tile, transA, transB, a, w.waves, s)
+                                                       : dispatch_wave<1, 0>(w.tile, transA, transB, a, w.waves, s);
+                if (e != hipSuccess) return hip_fail(e);
+                if (a.splits > 1) {
+                    e = launch_splitk_reduce(dtype, a, s);
+                    if (e != hipSuccess) return hip_fail(e);
+                }
+                return MMBO_OK;
+            }
+        }
+        config_id = plan.config_id;
         // The pick is made from the shape alone.  The ring kernels also need 16-byte aligned A and B, every
         // direct-to-LDS kernel a tile's span of an operand below 2 GiB: where the operands at hand do not qualify, the
         // x16 config of the same tile and split (any alignment), or the staged kernel, takes the call.

@@ -24,8 +24,9 @@
  *     share one, and calls from several host threads are safe.  A workspace is allocated on the first split-K call
  *     on its stream and grown when a call needs more (this waits for that stream's earlier work);
  *   - config_id selects a row of the tile-config table, like the reference's kernelId
- *     (src/gemm/constants.h:34-47,106-135); MMBO_CONFIG_AUTO lets the per-shape table pick.  Every shape runs
- *     under MMBO_CONFIG_AUTO.  Named configs: the general kernel's (no "DTL1" in the name) take any shape and
+ *     (src/gemm/constants.h:34-47,106-135); MMBO_CONFIG_AUTO lets the library pick: a config of the table, or, for problems
+ *     too small to fill the chip with the table's tiles, a kernel without a config id whose wavefronts split k among
+ *     themselves.  Every shape runs under MMBO_CONFIG_AUTO.  Named configs: the general kernel's (no "DTL1" in the name) take any shape and
  *     alignment; of the direct-to-LDS ones ("DTL1") the "MFMA16x16" family takes m, n that end inside a tile, k that
  *     ends inside a slice and A, B at any element alignment (the reference's kernels take whole tiles only: its
  *     launcher floors the grid, src/gemm/driver.h:49-50), and reads no byte outside the operands: it fetches 16
@@ -105,9 +106,10 @@ int mmbo_gemm_strided_batched(int dtype, int transA, int transB, size_t m, size_
 int mmbo_num_configs(int dtype);
 int mmbo_config_info(int dtype, int config_id, mmbo_config_desc *out);
 
-/* The per-shape pick (reference: the exact-size -> solution table of
+/* The per-shape pick among the configs of the table (reference: the exact-size -> solution table of
  * src/gemm/ref/vega20_Cijk_Ailk_Bjlk_DB.yaml:929-1177).  Returns a config id >= 0, or a
- * negative mmbo_status on bad arguments.  Pure host logic: needs no device. */
+ * negative mmbo_status on bad arguments.  Pure host logic: needs no device.  (MMBO_CONFIG_AUTO runs this config unless
+ * the kernel without a config id is faster on the shape.) */
 int mmbo_select_config(int dtype, int transA, int transB, size_t m, size_t n, size_t k, int batch);
 
 /* Host twin of the kernels' work-group -> tile mapping: linear work-group id to (tile row, tile

@@ -1,0 +1,75 @@
+"""The split-by-wavefront kernel (csrc/gemm_wave.hpp), which the automatic pick takes for small, thin and long-k problems.
+
+GPU: shapes at the edges of its tiles (16, 32, 64 rows), of its slices (32 halves, 16 floats, 8 doubles; pairs of them;
+fewer slices than wavefronts), with row-contiguous operands that end inside a 16-byte group or are shorter than one, and
+with k long enough for GlobalSplitU beyond 16 (several threads then share the splits of one sum), against the fp64 oracle
+with the suite's own bounds.  CPU: facts about the generated code that the kernel's asm statements rely on.
+"""
+import os
+import re
+import subprocess
+
+import numpy as np
+import pytest
+
+import util as U
+
+F32, F16, F64 = U.F32, U.F16, U.F64
+NAMES = {F32: "f32", F16: "f16", F64: "f64"}
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "gemm_mmbo_amd", "csrc")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+#         m    n     k    batch  what it is there for
+SHAPES = [(1, 1, 64, 1), (1, 130, 33, 1), (7, 3, 515, 1), (3, 257, 96, 1),           # rows shorter than a 16-byte group
+          (15, 17, 31, 1), (16, 16, 32, 1), (17, 15, 64, 1), (31, 33, 128, 3), (33, 31, 129, 8),
+          (63, 65, 160, 1), (65, 63, 255, 5), (128, 96, 1, 2), (40, 56, 9, 1),
+          (20, 12, 8192, 1), (12, 700, 3001, 1), (700, 12, 3001, 1), (64, 48, 40000, 1), (5, 9, 65537, 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, F16, F64], ids=NAMES.get)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_small_thin_and_long_k_shapes(dtype, ta, tb):
+    import torch
+
+    import gemm_mmbo_amd as G
+    for i, (m, n, k, batch) in enumerate(SHAPES):
+        pad = (0, 1, 8)[i % 3]
+        ar, br = U.stored_shape(ta, m, k)[0], U.stored_shape(tb, k, n)[0]
+        p = U.Problem(dtype, ta, tb, m, n, k, -1.5, (0.0, 0.5)[i % 2], lda=ar + pad, ldb=br + pad, ldc=m + pad, batch=batch,
+                      seed=300 + i, dist="normal" if dtype == F16 else "uniform", c_fill=("nan", "uniform")[i % 2])
+        got, guard = U.run_gpu(p)
+        U.check(p, got, f"{NAMES[dtype]} {'NT'[ta]}{'NT'[tb]} {m}x{n}x{k} b{batch}")
+        assert np.all(guard == 0)
+        # the entry point that allocates nothing: the same bits
+        dA, dB, dC = (torch.from_numpy(x).cuda() for x in (p.A, p.B, p.C))
+        G.gemm_strided_batched_static_workspace(dtype, ta, tb, m, n, k, -1.5, dA, p.lda, p.sa, dB, p.ldb, p.sb, p.beta, dC, p.ldc,
+                                                p.sc, batch)
+        torch.cuda.synchronize()
+        assert np.array_equal(dC.cpu().numpy().view(U.BITS[dtype]), got.view(U.BITS[dtype]))
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_generated_code(dtype, tmp_path):
+    """The direct loads set M0 inside their asm statement without telling the compiler, which must therefore not use M0
+    itself; and nothing is spilled (a reload would wait for the direct loads in flight)."""
+    out = str(tmp_path / "wave.s")
+    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                        "-Wno-unused-command-line-argument", "--cuda-device-only", "-S", f"-DMMBO_DTYPE={dtype}", "-DMMBO_TILE=7",
+                        os.path.join(CSRC, "inst_wave.hip"), "-o", out], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    inside, own, kernels = False, [], 0
+    for line in open(out):
+        t = line.strip()
+        if t.startswith(";;#ASMSTART"):
+            inside = True
+        elif t.startswith(";;#ASMEND"):
+            inside = False
+        elif not inside and not t.startswith((";", ".")):
+            own.append(t.split(";")[0])
+        kernels += t.startswith(".amdhsa_kernel")
+    assert kernels == 4
+    assert not [t for t in own if re.search(r"\bm0\b", t)]
+    assert not [t for t in own if t.startswith("scratch_")]
