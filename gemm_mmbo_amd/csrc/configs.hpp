@@ -82,7 +82,6 @@ constexpr RingRow kX16Tiles[NUM_X16_TILES] = {
 // Tiles of the split-by-wavefront kernel (gemm_wave.hpp), all element types.  They have no config ids: the automatic pick takes
 // them by a rule of its own (mmbo_gemm.hip).
 constexpr int NUM_WAVE_TILES = 8;
-constexpr int kWaveMaxWaves = 4;                  // wavefronts of a work-group that share k
 struct WaveRow {
     int bm, bn;
     int depth;        // slices in a wavefront's LDS ring
@@ -97,6 +96,8 @@ constexpr WaveRow kWaveTiles[NUM_WAVE_TILES] = {
     {32, 64, 4},      // 24 KB
     {64, 32, 4},
 };
+// wavefronts of a work-group that share k, at most: eight where their rings fit the 160 KB of LDS
+constexpr int wave_max_waves(const WaveRow &r) { return 8 * r.depth * (r.bm + r.bn) * 64 <= 160 * 1024 ? 8 : 4; }
 
 // Config ids (fp32 and fp16 share them): [0, kStagedConfigs) the staged kernel's (tile, split) pairs, then the ring
 // kernel's (ring tile, split) pairs, then the x16 kernel's.  split_index indexes kSplits.

@@ -330,10 +330,9 @@ gemm_staged_kernel(const GemmArgs args)
 }
 
 // Split-K reduction: C = alpha * sum_s ws[s] + beta * C, splits added in a fixed order so the result does not depend on
-// scheduling.  The workspace is [split][batch][n][m] fp32 (fp64 for fp64), dense, so consecutive rows of one column are one
-// 16-byte load per split; a thread owns such a group (four rows, fp64 two) when m is a multiple of it (VEC), one element
-// otherwise.  All loads of a thread are independent and issued before the first add (the loop over the splits is
-// unrolled for the split factors the library uses); the adds keep the order.  With more than sixteen splits the outputs
+// scheduling.  The workspace is [split][batch][n][m] fp32, dense, so four consecutive rows of one column are one 16-byte load per
+// split; a thread owns such a group when m % 4 == 0 (VEC), one element otherwise.  All loads of a thread are independent and issued
+// before the first add (the loop over the splits is unrolled for the split factors the library uses); the adds keep the order.  With more than sixteen splits the outputs
 // are few and one thread's chain of loads long: args.reduce_parts threads then take equal runs of the splits and the first of
 // them adds the runs up, in order, through LDS (MANY; a kernel of its own: with the parts counted at run time the common case
 // took 1 us longer).
@@ -341,9 +340,7 @@ template <typename T, bool VEC, bool MANY>
 __global__ void __launch_bounds__(256)
 splitk_reduce_kernel(const GemmArgs args)
 {
-    using elem = typename std::conditional<sizeof(T) == 8, double, float>::type;
-    constexpr int W = VEC ? 16 / (int)sizeof(elem) : 1;
-    typedef elem sums_t __attribute__((ext_vector_type(16 / sizeof(elem))));
+    constexpr int W = VEC ? 4 : 1;
     const uint32_t parts = MANY ? args.reduce_parts : 1, per_block = 256 / parts;           // a power of two, 1 .. 8
     const uint32_t part = MANY ? threadIdx.x / per_block : 0, mine = MANY ? threadIdx.x % per_block : threadIdx.x;
     const size_t mn = (size_t)args.m * args.n;
@@ -352,18 +349,18 @@ splitk_reduce_kernel(const GemmArgs args)
     const bool inside = idx < mn;
     if (!MANY && !inside) return;
     const size_t stride = (size_t)args.batch * mn;                  // one split further
-    const elem *w = reinterpret_cast<const elem *>(args.ws) + (size_t)batch * mn + idx;
-    elem s[W];
+    const float *w = args.ws + (size_t)batch * mn + idx;
+    float s[W];
 #pragma unroll
-    for (int e = 0; e < W; ++e) s[e] = 0;
+    for (int e = 0; e < W; ++e) s[e] = 0.0f;
     auto add_splits = [&](auto NS, uint32_t first) {
         constexpr int ns = decltype(NS)::value;
-        elem v[ns][W];
+        float v[ns][W];
 #pragma unroll
         for (int q = 0; q < ns; ++q) {
-            const elem *p = w + (size_t)(first + q) * stride;
+            const float *p = w + (size_t)(first + q) * stride;
             if constexpr (VEC) {
-                const sums_t t = *reinterpret_cast<const sums_t *>(p);
+                const f32x4 t = *reinterpret_cast<const f32x4 *>(p);
 #pragma unroll
                 for (int e = 0; e < W; ++e) v[q][e] = t[e];
             } else {
@@ -383,7 +380,7 @@ splitk_reduce_kernel(const GemmArgs args)
     if (sp + 2 <= sp_end) { add_splits(std::integral_constant<int, 2>{}, sp); sp += 2; }
     if (sp < sp_end) add_splits(std::integral_constant<int, 1>{}, sp);
     if constexpr (MANY) {
-        __shared__ elem partial[256 * W];
+        __shared__ float partial[256 * W];
 #pragma unroll
         for (int e = 0; e < W; ++e) partial[threadIdx.x * W + e] = s[e];
         __syncthreads();
@@ -395,23 +392,21 @@ splitk_reduce_kernel(const GemmArgs args)
 
     const uint32_t row = (uint32_t)(idx % args.m), col = (uint32_t)(idx / args.m);
     T *p = static_cast<T *>(args.C) + (int64_t)batch * args.strideC + (size_t)col * args.ldc + row;
-    const elem alpha = sizeof(T) == 8 ? (elem)args.alpha_d : (elem)args.alpha, beta = sizeof(T) == 8 ? (elem)args.beta_d : (elem)args.beta;
-    auto update = [&](elem sum, T old) {
-        const elem o = alpha * sum;
-        if (beta == (elem)0) return (T)o;
-        if constexpr (sizeof(T) == 8) return (T)__builtin_fma(beta, (double)old, o);
-        else return (T)__builtin_fmaf(beta, (float)old, o);
+    const float alpha = args.alpha, beta = args.beta;
+    auto update = [&](float sum, T old) {
+        const float o = alpha * sum;
+        return beta == 0.0f ? (T)o : (T)__builtin_fmaf(beta, (float)old, o);
     };
     if (VEC && args.vec_c) {
         struct rows_t { T e[W]; } __attribute__((aligned(sizeof(T) * W)));
         rows_t io;
-        if (beta != (elem)0) io = *reinterpret_cast<const rows_t *>(p);
+        if (beta != 0.0f) io = *reinterpret_cast<const rows_t *>(p);
 #pragma unroll
         for (int e = 0; e < W; ++e) io.e[e] = update(s[e], io.e[e]);
         *reinterpret_cast<rows_t *>(p) = io;
     } else {
 #pragma unroll
-        for (int e = 0; e < W; ++e) p[e] = update(s[e], beta != (elem)0 ? p[e] : (T)0);
+        for (int e = 0; e < W; ++e) p[e] = update(s[e], beta != 0.0f ? p[e] : (T)0);
     }
 }
 

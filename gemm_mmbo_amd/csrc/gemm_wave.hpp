@@ -184,8 +184,8 @@ struct WaveCfg {
     }
 };
 
-template <typename T, bool TA, bool TB, int BM, int BN, int DEPTH>
-__global__ void __launch_bounds__(256)
+template <typename T, bool TA, bool TB, int BM, int BN, int DEPTH, int MAX_WAVES>
+__global__ void __launch_bounds__(MAX_WAVES * 64)
 gemm_wave_kernel(const GemmArgs args)
 {
     using namespace wave;
@@ -285,7 +285,7 @@ gemm_wave_kernel(const GemmArgs args)
 
     // Old C of the groups of rows this thread will store, requested ahead of everything else.
     T *const C = static_cast<T *>(args.C) + (int64_t)batch * args.strideC + (int64_t)col0 * args.ldc + row0;
-    const bool to_ws = args.splits > 1;
+    const bool to_ws = sizeof(T) < 8 && args.splits > 1;
     const bool read_c = !to_ws && (sizeof(T) == 8 ? args.beta_d != 0.0 : args.beta != 0.0f);
     constexpr int GPC = BM / GROUP, GROUPS = GPC * BN;                             // groups per column, per tile
     constexpr int AHEAD = GROUPS / 64 < 8 ? GROUPS / 64 : 8;                       // groups of a thread requested together
@@ -410,15 +410,14 @@ gemm_wave_kernel(const GemmArgs args)
         if (c >= n_here || r >= m_here) return;
         const sums_t s = add_up(r, c);
         const bool whole = r + GROUP <= m_here;
-        if (to_ws) {
-            elem *ws = reinterpret_cast<elem *>(args.ws) + ((size_t)split * args.batch + batch) * (size_t)args.m * args.n +
-                       (size_t)(col0 + c) * args.m + row0 + r;
+        if (to_ws) {                                             // (never fp64)
+            float *ws = args.ws + ((size_t)split * args.batch + batch) * (size_t)args.m * args.n + (size_t)(col0 + c) * args.m + row0 + r;
             if (whole) {
                 __builtin_memcpy(ws, &s, sizeof(s));
             } else {
 #pragma unroll
                 for (int e = 0; e < GROUP; ++e)
-                    if (r + e < m_here) ws[e] = s[e];
+                    if (r + e < m_here) ws[e] = (float)s[e];
             }
             return;
         }

@@ -15,21 +15,22 @@ namespace mmbo {
 namespace {
 using ElemT = typename std::conditional<MMBO_DTYPE == 0, float, typename std::conditional<MMBO_DTYPE == 1, half_t, double>::type>::type;
 constexpr WaveRow R = kWaveTiles[MMBO_TILE];
+constexpr int kMaxWaves = wave_max_waves(R);
 
 template <bool TA, bool TB>
 hipError_t launch_one(const GemmArgs &args, int waves, hipStream_t stream)
 {
     using Cfg = WaveCfg<ElemT, TA, TB, R.bm, R.bn, R.depth>;
-    auto kernel = gemm_wave_kernel<ElemT, TA, TB, R.bm, R.bn, R.depth>;
-    static_assert(Cfg::lds_bytes(kWaveMaxWaves) <= 160 * 1024, "the rings do not fit the 160 KB of LDS");
-    if (waves < 1 || waves > kWaveMaxWaves) return hipErrorInvalidValue;
+    auto kernel = gemm_wave_kernel<ElemT, TA, TB, R.bm, R.bn, R.depth, kMaxWaves>;
+    static_assert(Cfg::lds_bytes(kMaxWaves) <= 160 * 1024, "the rings do not fit the 160 KB of LDS");
+    if (waves < 1 || waves > kMaxWaves) return hipErrorInvalidValue;
     static std::atomic<bool> attr_set[64];           // zero-initialised; several host threads may race to set it: harmless
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
     if (dev >= 0 && dev < 64 && !attr_set[dev].load(std::memory_order_acquire)) {
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                Cfg::lds_bytes(kWaveMaxWaves));
+                                Cfg::lds_bytes(kMaxWaves));
         if (e != hipSuccess) return e;
         attr_set[dev].store(true, std::memory_order_release);
     }

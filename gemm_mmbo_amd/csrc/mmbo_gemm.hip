@@ -380,8 +380,8 @@ double model_time_f64(int tile, size_t m, size_t n, size_t k, int batch)
 hipError_t launch_splitk_reduce(int dtype, const GemmArgs &args, hipStream_t stream)
 {
     size_t mn = (size_t)args.m * args.n;
-    const bool vec = dtype == MMBO_F64 ? args.m % 2 == 0 : args.m % 4 == 0;      // a thread then owns 16 bytes of sums of one column
-    const size_t groups = vec ? mn / (dtype == MMBO_F64 ? 2 : 4) : mn;
+    const bool vec = args.m % 4 == 0;      // a thread then owns 16 bytes of sums of one column
+    const size_t groups = vec ? mn / 4 : mn;
     // more than sixteen splits: several threads share the splits of one group (see the kernel)
     GemmArgs a = args;
     a.reduce_parts = args.splits <= 16 ? 1 : args.splits <= 32 ? 4 : 8;
@@ -394,7 +394,7 @@ hipError_t launch_splitk_reduce(int dtype, const GemmArgs &args, hipStream_t str
         return vec ? launch_kernel(splitk_reduce_kernel<T, true, true>, grid, dim3(256), 0, stream, a)
                    : launch_kernel(splitk_reduce_kernel<T, false, true>, grid, dim3(256), 0, stream, a);
     };
-    return dtype == MMBO_F32 ? launch(0.0f) : dtype == MMBO_F64 ? launch(0.0) : launch((half_t)0.0f);
+    return dtype == MMBO_F32 ? launch(0.0f) : launch((half_t)0.0f);           // (fp64 calls never split k over work-groups)
 }
 
 }  // namespace mmbo
@@ -760,7 +760,7 @@ struct WaveModel {
 constexpr WaveModel kWaveModel[3] = {
     {2.25, 1.08, 0.899, 7.4, 0.023, 0.372, 108.4e3, 31.9e6, 5.25e6, 0.322, 0.516, 0.376, 2.08, 0.370},      // fp32
     {2.51, 0.65, 0.421, 0.0, 0.036, 0.233, 122.7e3, 32.8e6, 5.69e6, 0.193, 1.173, 0.731, 1.68, 0.379},      // fp16
-    {2.03, 1.15, 0.734, 8.9, 0.026, 0.471, 98.6e3, 26.0e6, 5.58e6, 0.484, 0.444, 0.246, 2.31, 0.422},      // fp64
+    {2.03, 1.15, 0.734, 8.9, 0.026, 0.471, 98.6e3, 26.0e6, 5.58e6, 0.484, 0.444, 0.246, 0.0, 0.0},        // fp64 (never a second launch)
 };
 
 struct WaveShape {
@@ -816,22 +816,26 @@ double wave_model_us(const WaveShape &p, int tile, int waves, int split)
     return std::max(t, host) + 0.02 * std::min(t, host);
 }
 
-WavePick pick_wave(const WaveShape &p)
+// may_split: k may also be split over work-groups (GlobalSplitU: a workspace and a second launch).  Only where the pick of
+// mmbo_select_config splits as well: a caller reads from that pick whether a call uses a workspace -- whether two calls of the
+// entry point that allocates nothing may overlap, whether a call needs memory of its own before it can be captured.
+WavePick pick_wave(const WaveShape &p, bool may_split)
 {
     WavePick best{-1, 0, 0, 0.0};
-    const double sum_size = p.dtype == MMBO_F64 ? 8 : 4, esz = p.dtype == MMBO_F64 ? 8 : p.dtype == MMBO_F32 ? 4 : 2;
+    const double esz = p.dtype == MMBO_F64 ? 8 : p.dtype == MMBO_F32 ? 4 : 2;
     const size_t slices = ceil_div(p.k, (size_t)(64 / esz));
     if (p.k == 0) return best;
     for (int tile = 0; tile < NUM_WAVE_TILES; ++tile) {
         const size_t tiles = ceil_div(p.m, kWaveTiles[tile].bm) * ceil_div(p.n, kWaveTiles[tile].bn);
         if (tiles > 65535) continue;
-        for (int waves = 1; waves <= kWaveMaxWaves; waves *= 4) {
+        for (int waves : {1, 4, 8}) {
             if (waves > 1 && slices < (size_t)waves) continue;
-            for (int split = 1; split <= 64; split *= 2) {
+            if (waves > wave_max_waves(kWaveTiles[tile])) continue;
+            for (int split = 1; split <= (may_split ? 64 : 1); split *= 2) {
                 // (splits: at least a pair of slices per wavefront, not beyond what the chip holds at one time; the partial sums
                 // of either entry point fit the static workspace, so that both run the same split)
                 if (split > 1 && (slices < (size_t)split * waves * 2 || tiles * p.batch * split > 1024 ||
-                                  (double)p.m * p.n * p.batch * split * sum_size > (double)kScratchPartialBytes))
+                                  (double)p.m * p.n * p.batch * split * sizeof(float) > (double)kScratchPartialBytes))
                     break;
                 const double us = wave_model_us(p, tile, waves, split);
                 if (best.tile < 0 || us < best.us) best = WavePick{tile, waves, split, us};
@@ -874,7 +878,7 @@ Plan plan_for(const WaveShape &p)
     Plan plan;
     double table_us;
     plan.config_id = select_config(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, &table_us);
-    plan.wave = pick_wave(p);
+    plan.wave = pick_wave(p, p.dtype != MMBO_F64 && config_ref(plan.config_id).split > 1);
     if (plan.wave.us >= table_us) plan.wave.tile = -1;      // (150 drawn shapes: 1.42 times faster than the tables' configs alone)
     e.used = true;
     e.key = key;
@@ -953,7 +957,7 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
                 hipStream_t s = static_cast<hipStream_t>(stream);
                 WsHold ws_hold;
                 if (a.splits > 1) {
-                    const size_t bytes = (size_t)a.splits * batch * m * n * (f64 ? sizeof(double) : sizeof(float));
+                    const size_t bytes = (size_t)a.splits * batch * m * n * sizeof(float);
                     char *base = nullptr;
                     int rc = ws_source == WsSource::kStatic ? static_scratch(&base) : workspace(s, bytes, ws_hold, &base);
                     if (rc != MMBO_OK) return rc;

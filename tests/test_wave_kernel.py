@@ -50,6 +50,30 @@ def test_small_thin_and_long_k_shapes(dtype, ta, tb):
         assert np.array_equal(dC.cpu().numpy().view(U.BITS[dtype]), got.view(U.BITS[dtype]))
 
 
+@pytest.mark.gpu
+def test_only_calls_whose_pick_splits_k_take_a_workspace():
+    """mmbo_select_config tells a caller whether a call uses a workspace (before a capture, or beside another call of the entry
+    point that allocates nothing): with GlobalSplitU 1, and so for every fp64 call, none may be taken."""
+    import torch
+
+    import gemm_mmbo_amd as G
+    split = 0
+    for dtype in (F32, F16, F64):
+        t = {F32: torch.float32, F16: torch.float16, F64: torch.float64}[dtype]
+        for (ta, tb, m, n, k) in ((0, 0, 64, 489, 4640), (1, 0, 336, 448, 11520), (0, 1, 32, 48, 30000), (0, 0, 700, 12, 3001),
+                                  (0, 0, 40, 9000, 700), (1, 1, 100, 300, 2100), (0, 0, 500, 400, 600)):
+            dA, dB, dC = (torch.zeros(c, device="cuda", dtype=t) for c in (m * k, k * n, m * n))
+            torch.cuda.synchronize()
+            G.release_workspace()
+            G.gemm(dtype, ta, tb, m, n, k, 1.0, dA, k if ta else m, dB, n if tb else k, 0.0, dC, m)
+            torch.cuda.synchronize()
+            splits = G.config_info(dtype, G.select_config(dtype, ta, tb, m, n, k, 1))["split_k"] > 1
+            split += splits
+            assert splits or G.workspace_info()[0] == 0, (NAMES[dtype], ta, tb, m, n, k)
+    assert split > 0
+    G.release_workspace()
+
+
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
 @pytest.mark.parametrize("dtype", [0, 1, 2])
 def test_generated_code(dtype, tmp_path):
