@@ -140,33 +140,20 @@ __device__ inline void dgemm_write_back(const f64x4 (&acc)[FM][FN], const GemmAr
         }
 }
 
-// OLD_C_EARLY: the variant for beta != 0 that requests the wave tile's old C under the last stage's MFMAs (wave tiles of at
-// most four blocks).  A kernel of its own, picked by the host: the 32 registers per lane it holds the old C in take the
-// work-groups per CU from five to four, which calls without C to read would pay for nothing (1024^3, beta = 0: -1 %).
-template <bool TA, bool TB, int BM, int BN, int BK, int WM, int WN, bool OLD_C_EARLY = false>
-// Eight wavefronts with wave tiles of at most eight blocks (64 accumulator registers, two loader chunks per
-// operand) are held to 128 registers per lane so that two work-groups share a CU (the second argument is
-// wavefronts per SIMD); the others get 256.
-__global__ void __launch_bounds__(WM * WN * 64, (WM * WN >= 8 && (BM / WM / 16) * (BN / WN / 16) <= 8) ? 4 : 2)
-dgemm_kernel(const GemmArgs args)
+// One tile of C by one work-group.
+template <bool TA, bool TB, int BM, int BN, int BK, int WM, int WN, bool OLD_C_EARLY>
+__device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t col0, uint32_t batch, char *lds)
 {
     using Cfg = DgemmCfg<TA, TB, BM, BN, BK, WM, WN>;
     using TileA = typename Cfg::TileA;
     using TileB = typename Cfg::TileB;
     constexpr int FM = Cfg::FM, FN = Cfg::FN, ESZ = 8, NKK = BK / 4;
 
-    extern __shared__ __attribute__((aligned(16))) char lds[];
-
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM, wn = wave / WM;
 
-    uint32_t wg0, wg1, tile_id, batch, nxcd;
-    work_of_block(args, blockIdx.x, blockIdx.z, tile_id, batch, nxcd);
-    wg_remap(tile_id, args.nwg0, args.nwg1, args.wgm, nxcd, wg0, wg1);
-
-    const uint32_t row0 = wg0 * BM, col0 = wg1 * BN;
     const int rows_a = (int)min((uint32_t)BM, args.m - row0);
     const int rows_b = (int)min((uint32_t)BN, args.n - col0);
     const uint32_t k_len = args.k;
@@ -294,6 +281,39 @@ dgemm_kernel(const GemmArgs args)
         }
     }
     dgemm_write_back<FM, FN>(acc, args, row0 + wm * Cfg::TM, col0 + wn * Cfg::TN, batch, lane);
+}
+
+// OLD_C_EARLY: the variant for beta != 0 that requests the wave tile's old C under the last stage's MFMAs (wave tiles of at
+// most four blocks).  A kernel of its own, picked by the host: the 32 registers per lane it holds the old C in take the
+// work-groups per CU from five to four, which calls without C to read would pay for nothing (1024^3, beta = 0: -1 %).
+template <bool TA, bool TB, int BM, int BN, int BK, int WM, int WN, bool OLD_C_EARLY = false>
+// Eight wavefronts with wave tiles of at most eight blocks (64 accumulator registers, two loader chunks per
+// operand) are held to 128 registers per lane so that two work-groups share a CU (the second argument is
+// wavefronts per SIMD); the others get 256.
+__global__ void __launch_bounds__(WM * WN * 64, (WM * WN >= 8 && (BM / WM / 16) * (BN / WN / 16) <= 8) ? 4 : 2)
+dgemm_kernel(const GemmArgs args)
+{
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+
+    uint32_t wg0, wg1, tile_id, batch, nxcd;
+    if constexpr (dgemm_quarters(BM, BN)) {
+        const uint32_t whole = args.nwg0 * args.nwg1 - args.quartered;
+        if (blockIdx.x >= whole) {
+            // The tiles that would leave CUs idle in a last, partial round: four work-groups each (the rule is the host's,
+            // quartered_tiles).  The order of every sum over k is the tile's, so the result has the same bits.
+            // (A tile's quarters are `quartered` work-groups apart: on one XCD where that is a multiple of 8.)
+            const uint32_t id = blockIdx.x - whole, q = id / args.quartered;
+            wg_remap(whole + id - q * args.quartered, args.nwg0, args.nwg1, args.wgm, args.nxcd, wg0, wg1);
+            const uint32_t row0 = __builtin_amdgcn_readfirstlane(wg0 * BM + (q & 1) * (BM / 2));
+            const uint32_t col0 = __builtin_amdgcn_readfirstlane(wg1 * BN + (q >> 1) * (BN / 2));
+            if (row0 >= args.m || col0 >= args.n) return;                  // (all of the work-group)
+            dgemm_tile<TA, TB, BM / 2, BN / 2, BK, WM, WN, OLD_C_EARLY>(args, row0, col0, blockIdx.z, lds);
+            return;
+        }
+    }
+    work_of_block(args, blockIdx.x, blockIdx.z, tile_id, batch, nxcd);
+    wg_remap(tile_id, args.nwg0, args.nwg1, args.wgm, nxcd, wg0, wg1);
+    dgemm_tile<TA, TB, BM, BN, BK, WM, WN, OLD_C_EARLY>(args, wg0 * BM, wg1 * BN, batch, lds);
 }
 
 }  // namespace mmbo

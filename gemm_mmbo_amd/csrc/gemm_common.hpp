@@ -52,8 +52,12 @@ struct GemmArgs {
     uint32_t no_successor;  // gemm_wave.hpp: last columns of k whose edge groups of rows have no memory behind them
     uint32_t columns_first; // gemm_wave.hpp: tiles are walked along a tile row first
     uint32_t reduce_parts;  // splitk_reduce_kernel: threads that share the splits of one group of sums
+    uint32_t quartered;     // dgemm.hpp: this many last tiles of the walk are shared by four work-groups each, a quarter of the tile to each
     uint32_t ws_narrow;     // 1: a tile's span of the split-K workspace (tile columns x m floats) fits 32-bit offsets
 };
+
+// fp64 tiles that may go out as quarters (GemmArgs::quartered)
+constexpr bool dgemm_quarters(int bm, int bn) { return bm == 64 && bn == 64; }
 
 // Linear work-group id -> (tile row, tile column).
 //

@@ -33,7 +33,7 @@ hipError_t launch_one(const GemmArgs &args, hipStream_t stream)
         if (e != hipSuccess) return e;
         attr_set[dev].store(true, std::memory_order_release);
     }
-    dim3 grid(args.nwg0 * args.nwg1, 1, args.batch);
+    dim3 grid(args.nwg0 * args.nwg1 + 3 * args.quartered, 1, args.batch);
     return launch_kernel(kernel, grid, dim3(Cfg::NT), Cfg::LDS_BYTES, stream, args);
 }
 

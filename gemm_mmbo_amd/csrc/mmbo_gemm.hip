@@ -354,10 +354,25 @@ double model_time(int dtype, int tile, int split, size_t m, size_t n, size_t k, 
     return t;
 }
 
+// fp64: how many 64 x 64 tiles at the end of the walk go out as quarters: those behind the last whole round of the 256 CUs.
+// 1152 x 2048 is 576 tiles, 2.25 to a CU: whole, they take as long as 3 rounds; the last 64 as 256 quarters, 2.25.  A quarter
+// takes 0.3 of a tile's time (its operand traffic halves, its flops quarter), so up to three quarters to a CU, 192 tiles,
+// are worth it, however many whole rounds precede them (aligned operands, us: rest 64 of 2 rounds 66.4 -> 52.8, 100 of 2
+// 104.7 -> 88.4, 44 of 6 189.6 -> 167.5, 191 of 4 49.2 -> 48.0).  Fewer tiles than CUs are the 32 x 32 tile's.
+constexpr int kQuarterTile = 3;
+static_assert(kTilesF64[kQuarterTile].bm == 32 && kTilesF64[kQuarterTile].bn == 32, "a 64 x 64 tile's quarter");
+size_t quartered_tiles(int tile, size_t tiles, int batch)
+{
+    if (!dgemm_quarters(kTilesF64[tile].bm, kTilesF64[tile].bn) || batch != 1) return 0;
+    const size_t rest = tiles % 256;
+    return tiles >= 256 && rest <= 192 ? rest : 0;
+}
+
 // fp64: microseconds.  Work-groups run in rounds of (CUs x work-groups per CU); a tile costs a fixed overhead
 // (first stage, C update, dispatch of its successor: measured per tile and CU with K swept from 96 to 1536 on the
 // HPL shape's M and N) plus its K at the tile's in-loop efficiency (from 8192^3), both shared by the work-groups
-// resident on the CU; the last, partial round runs with fewer of them.
+// resident on the CU; the last, partial round runs with fewer of them, or as quarters that cost what the 32 x 32 tile does
+// (36 drawn shapes that end so: within 4 % of the measured time where the operands are aligned).
 double model_time_f64(int tile, size_t m, size_t n, size_t k, int batch)
 {
     //                                    128x128/4w 256x128/8w 64x64  32x32  128x128/8w 128x64
@@ -367,7 +382,12 @@ double model_time_f64(int tile, size_t m, size_t n, size_t k, int batch)
     const TileRow &r = kTilesF64[tile];
     const double cus = 256.0, flop_per_us_cu = 78.6e6 / 256.0, launch = 5.0;
     const double tiles = (double)ceil_div(m, r.bm) * (double)ceil_div(n, r.bn) * batch;
-    const double per_tile = overhead_us[tile] + 2.0 * r.bm * r.bn * (double)(k ? k : 1) / flop_per_us_cu / in_loop_eff[tile];
+    auto tile_us = [&](int t) {
+        return overhead_us[t] + 2.0 * kTilesF64[t].bm * kTilesF64[t].bn * (double)(k ? k : 1) / flop_per_us_cu / in_loop_eff[t];
+    };
+    const double per_tile = tile_us(tile);
+    if (const size_t rest = quartered_tiles(tile, (size_t)tiles, batch))
+        return launch + std::floor(tiles / cus) * per_tile + std::ceil(4.0 * (double)rest / cus) * tile_us(kQuarterTile);
     const double slots = cus * resident[tile];
     const double full = std::floor(tiles / slots), last = tiles - full * slots;
     double t = launch + full * per_tile * resident[tile];
@@ -878,6 +898,15 @@ Plan plan_for(const WaveShape &p)
     Plan plan;
     double table_us;
     plan.config_id = select_config(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, &table_us);
+    // fp64 calls that read C, at most two whole rounds of tiles with quarters behind them and a short k: all work-groups of such
+    // a call are resident at one time and update C at one time; 32 x 32 tiles, of which a CU runs some behind others, overlap a
+    // part of that (us, quarters against 32 x 32 tiles: 1152 x 2048 x 384 with ldc 44160 37.2 / 36.2, 896 x 1728 x 208 18.7 / 18.3, 2880 x
+    // 448 x 352 23.2 / 22.9; with k = 512 and 592 38.2 / 40.0 and 52.8 / 56.4, with four rounds and k = 124 32.0 / 33.1).
+    if (p.dtype == MMBO_F64 && plan.config_id >= 0 && p.read_c && p.k < 448) {
+        const TileRow &r = kTilesF64[plan.config_id];
+        const size_t tiles = ceil_div(p.m, r.bm) * ceil_div(p.n, r.bn);
+        if (tiles < 3 * 256 && quartered_tiles(plan.config_id, tiles, p.batch) > 0) plan.config_id = kQuarterTile;
+    }
     plan.wave = pick_wave(p, p.dtype != MMBO_F64 && config_ref(plan.config_id).split > 1);
     if (plan.wave.us >= table_us) plan.wave.tile = -1;      // (150 drawn shapes: 1.42 times faster than the tables' configs alone)
     e.used = true;
@@ -1065,6 +1094,7 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
         return ((uintptr_t)p % 128 == 0) && ((ld * esz) % 128 == 0) && (batch == 1 || ((size_t)stride * esz) % 128 == 0);
     };
     a.line_rows = on_lines(A, lda, strideA) && on_lines(B, ldb, strideB);
+    a.quartered = f64 ? (uint32_t)quartered_tiles(cref.tile, nwg0 * nwg1, batch) : 0;
     a.ws_narrow = (size_t)r.bn * m * 4 < 0x7FFFFF00ull;
     a.vec_c = aligned16(C, ldc, strideC) && (!cref.x16 || (size_t)r.bn * ldc * esz < 0x7FFFFF00ull);
     // beta != 0 on the x16 kernel's fp16 path: the old C of a tile is fetched into LDS under the tile's last slices (one
