@@ -20,6 +20,9 @@
 
 namespace mmbo {
 
+// Pairs of doubles wherever they lie: a 16-byte access needs no more than an element's alignment on this chip.
+typedef f64x2 __attribute__((aligned(8))) f64x2_any;
+
 // tile row (within a 16-row block) that MFMA row r = 4*e + g of the A operand carries
 __host__ __device__ constexpr int dgemm_row_of(int r) { return 8 * (r >> 3) + 2 * (r & 3) + ((r >> 2) & 1); }
 
@@ -65,8 +68,7 @@ __device__ inline void dgemm_write_back(const f64x4 (&acc)[FM][FN], const GemmAr
     const double alpha = args.alpha_d, beta = args.beta_d;
     const int g = lane >> 4, cl = lane & 15;
     double *C = static_cast<double *>(args.C) + (int64_t)batch * args.strideC;
-    const bool vec_c = args.vec_c != 0;
-    if (vec_c && wrow0 + FM * 16 <= m && wcol0 + FN * 16 <= n) {
+    if (wrow0 + FM * 16 <= m && wcol0 + FN * 16 <= n) {
         // Whole wave tile in range.  The compiler may not move a load of C above an earlier store to C, so a
         // block-by-block update pays one full memory latency per block; here the old values of HB blocks are
         // requested together before the first of them is needed.
@@ -85,16 +87,16 @@ __device__ inline void dgemm_write_back(const f64x4 (&acc)[FM][FN], const GemmAr
                         continue;
                     }
                     const double *p = p0 + (size_t)((b0 + b) / FM) * 16 * ldc + ((b0 + b) % FM) * 16;
-                    c[b][0] = *reinterpret_cast<const f64x2 *>(p);
-                    c[b][1] = *reinterpret_cast<const f64x2 *>(p + 8);
+                    c[b][0] = *reinterpret_cast<const f64x2_any *>(p);
+                    c[b][1] = *reinterpret_cast<const f64x2_any *>(p + 8);
                 }
 #pragma unroll
                 for (int b = 0; b < HB; ++b) {
                     const f64x4 &a = acc[(b0 + b) % FM][(b0 + b) / FM];
                     double *p = p0 + (size_t)((b0 + b) / FM) * 16 * ldc + ((b0 + b) % FM) * 16;
-                    *reinterpret_cast<f64x2 *>(p) = f64x2{__builtin_fma(beta, c[b][0][0], alpha * a[0]),
+                    *reinterpret_cast<f64x2_any *>(p) = f64x2{__builtin_fma(beta, c[b][0][0], alpha * a[0]),
                                                           __builtin_fma(beta, c[b][0][1], alpha * a[1])};
-                    *reinterpret_cast<f64x2 *>(p + 8) = f64x2{__builtin_fma(beta, c[b][1][0], alpha * a[2]),
+                    *reinterpret_cast<f64x2_any *>(p + 8) = f64x2{__builtin_fma(beta, c[b][1][0], alpha * a[2]),
                                                               __builtin_fma(beta, c[b][1][1], alpha * a[3])};
                 }
             }
@@ -103,8 +105,8 @@ __device__ inline void dgemm_write_back(const f64x4 (&acc)[FM][FN], const GemmAr
             for (int b = 0; b < NB; ++b) {
                 const f64x4 &a = acc[b % FM][b / FM];
                 double *p = p0 + (size_t)(b / FM) * 16 * ldc + (b % FM) * 16;
-                *reinterpret_cast<f64x2 *>(p) = f64x2{alpha * a[0], alpha * a[1]};
-                *reinterpret_cast<f64x2 *>(p + 8) = f64x2{alpha * a[2], alpha * a[3]};
+                *reinterpret_cast<f64x2_any *>(p) = f64x2{alpha * a[0], alpha * a[1]};
+                *reinterpret_cast<f64x2_any *>(p + 8) = f64x2{alpha * a[2], alpha * a[3]};
             }
         }
         return;
@@ -121,13 +123,13 @@ __device__ inline void dgemm_write_back(const f64x4 (&acc)[FM][FN], const GemmAr
                 if (row >= m) continue;
                 double *p = C + (size_t)col * ldc + row;
                 double v0 = alpha * acc[i][j][2 * h], v1 = alpha * acc[i][j][2 * h + 1];
-                if (vec_c && row + 2 <= m) {
+                if (row + 2 <= m) {
                     if (beta != 0.0) {
-                        f64x2 c = *reinterpret_cast<const f64x2 *>(p);
+                        f64x2 c = *reinterpret_cast<const f64x2_any *>(p);
                         v0 = __builtin_fma(beta, c[0], v0);
                         v1 = __builtin_fma(beta, c[1], v1);
                     }
-                    *reinterpret_cast<f64x2 *>(p) = f64x2{v0, v1};
+                    *reinterpret_cast<f64x2_any *>(p) = f64x2{v0, v1};
                 } else {
                     if (beta != 0.0) v0 = __builtin_fma(beta, p[0], v0);
                     p[0] = v0;
@@ -171,23 +173,27 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
 
     uint32_t offA[TileA::NCH], offB[TileB::NCH];
 #pragma unroll
-    for (int c = 0; c < TileA::NCH; ++c) offA[c] = TileA::goff(tid, c, lda);
+    for (int c = 0; c < TileA::NCH; ++c) offA[c] = TileA::goff(tid, c, lda, rows_a);
 #pragma unroll
-    for (int c = 0; c < TileB::NCH; ++c) offB[c] = TileB::goff(tid, c, ldb);
+    for (int c = 0; c < TileB::NCH; ++c) offB[c] = TileB::goff(tid, c, ldb, rows_b);
 
-    const bool fast = rows_a == BM && rows_b == BN && args.vec_a && args.vec_b;
+    // Whole stages are read without a test per chunk, aligned or not.  Rows past the matrix repeat its last row, or pair of rows
+    // (their products are never stored); only an odd count of contiguous rows has a pair with one half outside.
+    // Against the predicated loader for every edge tile and for all tiles of operands with a column off 16 bytes, us (64 x 64
+    // tiles): TT 2542 x 644 x 896 86 -> 60, TT 4041 x 1524 x 110 51 -> 38, TN 5397 x 610 x 643 114 -> 91, NN 4046 x 566 x 426 50 -> 41.
+    const bool fast = (TA || rows_a == BM || rows_a % 2 == 0) && (!TB || rows_b == BN || rows_b % 2 == 0);
 
     u32x4 ra[TileA::NCH], rb[TileB::NCH];
     auto load_stage = [&](int it) {
         const char *pa = gA + (int64_t)it * stepA;
         const char *pb = gB + (int64_t)it * stepB;
         if (fast && it < n_full) {
-            TileA::load_fast(ra, pa, offA);
-            TileB::load_fast(rb, pb, offB);
+            TileA::load_whole(ra, pa, offA);
+            TileB::load_whole(rb, pb, offB);
         } else {
             int kvalid = it < n_full ? BK : k_tail;
-            TileA::load_slow(ra, pa, offA, tid, lda, rows_a, kvalid, args.vec_a != 0);
-            TileB::load_slow(rb, pb, offB, tid, ldb, rows_b, kvalid, args.vec_b != 0);
+            TileA::load_slow(ra, pa, offA, tid, lda, rows_a, kvalid, false);
+            TileB::load_slow(rb, pb, offB, tid, ldb, rows_b, kvalid, false);
         }
     };
 
@@ -225,11 +231,10 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
     };
     int it = 0;
     if (fast) {
-        // interior tiles of aligned operands, while the next stage is a whole one: no test inside the loop, the
-        // predicated loader stays out of its body
+        // while the next stage is a whole one: no test inside the loop, the predicated loader stays out of its body
         for (; it + 1 < n_full; ++it) {
-            TileA::load_fast(ra, gA + (int64_t)(it + 1) * stepA, offA);
-            TileB::load_fast(rb, gB + (int64_t)(it + 1) * stepB, offB);
+            TileA::load_whole(ra, gA + (int64_t)(it + 1) * stepA, offA);
+            TileB::load_whole(rb, gB + (int64_t)(it + 1) * stepB, offB);
             multiply_stage(lds + cur * Cfg::STAGE_BYTES);
             char *nx = lds + (cur ^ 1) * Cfg::STAGE_BYTES;
             TileA::store_lds(ra, nx, tid);
@@ -250,14 +255,14 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
         if (more) load_stage(it + 1);
         if constexpr (EARLY_C) {
             const uint32_t wrow0 = row0 + wm * Cfg::TM, wcol0 = col0 + wn * Cfg::TN;
-            if (!more && args.beta_d != 0.0 && args.vec_c && wrow0 + FM * 16 <= args.m && wcol0 + FN * 16 <= args.n) {
+            if (!more && args.beta_d != 0.0 && wrow0 + FM * 16 <= args.m && wcol0 + FN * 16 <= args.n) {
                 const double *p0 = static_cast<const double *>(args.C) + (int64_t)batch * args.strideC +
                                    (size_t)(wcol0 + (lane & 15)) * args.ldc + wrow0 + 2 * (lane >> 4);
 #pragma unroll
                 for (int b = 0; b < FM * FN; ++b) {
                     const double *p = p0 + (size_t)(b / FM) * 16 * args.ldc + (b % FM) * 16;
-                    old_c[b][0] = *reinterpret_cast<const f64x2 *>(p);
-                    old_c[b][1] = *reinterpret_cast<const f64x2 *>(p + 8);
+                    old_c[b][0] = *reinterpret_cast<const f64x2_any *>(p);
+                    old_c[b][1] = *reinterpret_cast<const f64x2_any *>(p + 8);
                 }
                 have_old_c = true;
             }

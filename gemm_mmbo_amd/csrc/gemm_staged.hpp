@@ -46,9 +46,23 @@ struct OperandTile {
     {
         return ((uint32_t)outer(tid, c) * ld + (uint32_t)inner(tid) * VEC) * ESZ;
     }
+    // the same with the rows past `rows` (>= 1) moved to the last one (KC) or the last chunk with a row of the matrix (else)
+    __device__ static inline uint32_t goff(int tid, int c, uint32_t ld, int rows)
+    {
+        const int o = KC ? min(outer(tid, c), rows - 1) : outer(tid, c), in = KC ? inner(tid) : min(inner(tid), (rows - 1) / VEC);
+        return ((uint32_t)o * ld + (uint32_t)in * VEC) * ESZ;
+    }
     __device__ static inline uint32_t lds_woff(int tid, int c)
     {
         return (uint32_t)(outer(tid, c) * LDS_LD + inner(tid) * VEC) * ESZ;
+    }
+
+    typedef u32x4 __attribute__((aligned(2))) u32x4_unaligned;
+    // Whole stage of operands at any element alignment: 128-bit loads without a test.
+    __device__ static inline void load_whole(u32x4 (&regs)[NCH], const char *g, const uint32_t (&off)[NCH])
+    {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) regs[c] = *reinterpret_cast<const u32x4_unaligned *>(g + off[c]);
     }
 
     // Interior, aligned stage: plain 128-bit loads.
@@ -62,7 +76,6 @@ struct OperandTile {
     // use one 128-bit load, aligned or not (gfx950 under ROCm runs with unaligned global access enabled: a leading
     // dimension like 1023 costs split cache-line accesses, not eight 2-byte loads per chunk); only chunks that
     // straddle the matrix edge or the end of K go element by element.
-    typedef u32x4 __attribute__((aligned(2))) u32x4_unaligned;
     __device__ static inline void load_slow(u32x4 (&regs)[NCH], const char *g, const uint32_t (&off)[NCH],
                                             int tid, uint32_t /* ld: the offsets already contain it */, int rows, int kvalid, bool vec)
     {
