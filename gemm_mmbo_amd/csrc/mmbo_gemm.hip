@@ -372,7 +372,7 @@ size_t quartered_tiles(int tile, size_t tiles, int batch)
 // (first stage, C update, dispatch of its successor: measured per tile and CU with K swept from 96 to 1536 on the
 // HPL shape's M and N) plus its K at the tile's in-loop efficiency (from 8192^3), both shared by the work-groups
 // resident on the CU; the last, partial round runs with fewer of them, or as quarters that cost what the 32 x 32 tile does
-// (36 drawn shapes that end so: within 4 % of the measured time where the operands are aligned).
+// (36 drawn shapes that end so: within 12 % of the measured time, 16 % where C is read).
 double model_time_f64(int tile, size_t m, size_t n, size_t k, int batch)
 {
     //                                    128x128/4w 256x128/8w 64x64  32x32  128x128/8w 128x64
