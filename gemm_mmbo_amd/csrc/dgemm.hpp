@@ -177,23 +177,34 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
 #pragma unroll
     for (int c = 0; c < TileB::NCH; ++c) offB[c] = TileB::goff(tid, c, ldb, rows_b);
 
+    u32x4 ra[TileA::NCH], rb[TileB::NCH];
     // Whole stages are read without a test per chunk, aligned or not.  Rows past the matrix repeat its last row, or pair of rows
-    // (their products are never stored); only an odd count of contiguous rows has a pair with one half outside.
+    // (their products are never stored); an odd count of contiguous rows ends in a pair fetched one row lower (one row alone
+    // has none).
     // Against the predicated loader for every edge tile and for all tiles of operands with a column off 16 bytes, us (64 x 64
     // tiles): TT 2542 x 644 x 896 86 -> 60, TT 4041 x 1524 x 110 51 -> 38, TN 5397 x 610 x 643 114 -> 91, NN 4046 x 566 x 426 50 -> 41.
-    const bool fast = (TA || rows_a == BM || rows_a % 2 == 0) && (!TB || rows_b == BN || rows_b % 2 == 0);
+    // With odd edges on the predicated loader, their work-groups ran on long after the others: NT 1121 x 1088 x 1692 142 -> 93 us.
+    const bool fast = (TA || rows_a > 1) && (!TB || rows_b > 1);
+    const bool odd_a = fast && !TA && rows_a % 2 != 0, odd_b = fast && TB && rows_b % 2 != 0;
+    const bool fix_a = TileA::past_odd_end(tid, rows_a), fix_b = TileB::past_odd_end(tid, rows_b);
+    if (!odd_a && fix_a) { for (int c = 0; c < TileA::NCH; ++c) offA[c] += ESZ; }       // (one row alone: the plain offsets)
+    if (!odd_b && fix_b) { for (int c = 0; c < TileB::NCH; ++c) offB[c] += ESZ; }
+    auto place_odd = [&]() {
+        if (odd_a) { if (fix_a) TileA::odd_pair(ra); }
+        if (odd_b) { if (fix_b) TileB::odd_pair(rb); }
+    };
 
-    u32x4 ra[TileA::NCH], rb[TileB::NCH];
     auto load_stage = [&](int it) {
         const char *pa = gA + (int64_t)it * stepA;
         const char *pb = gB + (int64_t)it * stepB;
         if (fast && it < n_full) {
             TileA::load_whole(ra, pa, offA);
             TileB::load_whole(rb, pb, offB);
+            place_odd();
         } else {
             int kvalid = it < n_full ? BK : k_tail;
-            TileA::load_slow(ra, pa, offA, tid, lda, rows_a, kvalid, false);
-            TileB::load_slow(rb, pb, offB, tid, ldb, rows_b, kvalid, false);
+            TileA::load_slow(ra, pa + (odd_a && fix_a ? ESZ : 0), offA, tid, lda, rows_a, kvalid, false);
+            TileB::load_slow(rb, pb + (odd_b && fix_b ? ESZ : 0), offB, tid, ldb, rows_b, kvalid, false);
         }
     };
 
@@ -236,6 +247,7 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
             TileA::load_whole(ra, gA + (int64_t)(it + 1) * stepA, offA);
             TileB::load_whole(rb, gB + (int64_t)(it + 1) * stepB, offB);
             multiply_stage(lds + cur * Cfg::STAGE_BYTES);
+            place_odd();
             char *nx = lds + (cur ^ 1) * Cfg::STAGE_BYTES;
             TileA::store_lds(ra, nx, tid);
             TileB::store_lds(rb, nx + TileA::LDS_BYTES, tid);
@@ -294,8 +306,8 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
 template <bool TA, bool TB, int BM, int BN, int BK, int WM, int WN, bool OLD_C_EARLY = false>
 // Eight wavefronts with wave tiles of at most eight blocks (64 accumulator registers, two loader chunks per
 // operand) are held to 128 registers per lane so that two work-groups share a CU (the second argument is
-// wavefronts per SIMD); the others get 256.
-__global__ void __launch_bounds__(WM * WN * 64, (WM * WN >= 8 && (BM / WM / 16) * (BN / WN / 16) <= 8) ? 4 : 2)
+// wavefronts per SIMD), OLD_C_EARLY's four wavefronts so that four do; the others get 256.
+__global__ void __launch_bounds__(WM * WN * 64, (WM * WN >= 8 && (BM / WM / 16) * (BN / WN / 16) <= 8) || (OLD_C_EARLY && (BM / WM / 16) * (BN / WN / 16) <= 4) ? 4 : 2)
 dgemm_kernel(const GemmArgs args)
 {
     extern __shared__ __attribute__((aligned(16))) char lds[];
