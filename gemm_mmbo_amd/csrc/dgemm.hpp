@@ -2,8 +2,8 @@
 // (src/gemm/gemm.h:4-5,47-48 naive_dgemm / dgemm_NT; the HPL trailing update of src/gemm/run.sh:2-5).
 //
 // Same structure as the staged fp32/fp16 kernel (global loads into registers one stage ahead, padded
-// double-buffered LDS tile, one barrier per stage; edges, K tail and unaligned operands through the predicated
-// loader), with 16 x 16 MFMA blocks: an fp64 MFMA takes 64 clocks for 2,048 flops, so one 64-bit LDS read per
+// double-buffered LDS tile, one barrier per stage; whole stages of k without a test, at any edge and alignment, a partial one
+// through the predicated loader), with 16 x 16 MFMA blocks: an fp64 MFMA takes 64 clocks for 2,048 flops, so one 64-bit LDS read per
 // operand per MFMA and a single-stage prefetch keep the pipes fed.
 //
 // Register layout of v_mfma_f64_16x16x4_f64 (checked on the device): operand lane l supplies row (column)
@@ -159,8 +159,18 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
     const int rows_a = (int)min((uint32_t)BM, args.m - row0);
     const int rows_b = (int)min((uint32_t)BN, args.n - col0);
     const uint32_t k_len = args.k;
-    const int n_full = (int)(k_len / BK);
-    const int k_tail = (int)(k_len % BK);
+    // Whole stages are read without a test per chunk, aligned or not.  Rows past the matrix repeat its last row, or the chunk that
+    // holds it; where an odd count of contiguous rows ends inside that chunk, its second half is what follows in memory -- a
+    // padding row, the next column -- and its products, as those of the repeated rows, are never stored.  Only the operand's last
+    // column has nothing behind it: of a tile with such an end the last stage goes chunk by chunk.
+    // Against the predicated loader for every edge tile and for all tiles of operands with a column off 16 bytes, us (64 x 64
+    // tiles): TT 2542 x 644 x 896 86 -> 60, TT 4041 x 1524 x 110 51 -> 38, TN 5397 x 610 x 643 114 -> 91, NN 4046 x 566 x 426 50 -> 41.
+    // With odd edges on the predicated loader, their work-groups ran on long after the others: NT 1121 x 1088 x 1692 142 -> 86 us; with
+    // a correction of their last pairs inside the stage loop, every tile's LDS stores waited behind the last MFMA: NT 1152 x 2048 x 384
+    // with C read 39.7 -> 37.3 us without it, NT 44160 x 2048 x 384 1,193 -> 1,158.
+    const bool odd_end = (!TA && rows_a % 2 != 0) || (TB && rows_b % 2 != 0);
+    const int n_full = (int)((k_len - (odd_end && k_len > 0 ? 1 : 0)) / BK);
+    const int k_tail = (int)(k_len - (uint32_t)n_full * BK);
     const int n_iter = n_full + (k_tail ? 1 : 0);
 
     const uint32_t lda = args.lda, ldb = args.ldb;
@@ -178,33 +188,15 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
     for (int c = 0; c < TileB::NCH; ++c) offB[c] = TileB::goff(tid, c, ldb, rows_b);
 
     u32x4 ra[TileA::NCH], rb[TileB::NCH];
-    // Whole stages are read without a test per chunk, aligned or not.  Rows past the matrix repeat its last row, or pair of rows
-    // (their products are never stored); an odd count of contiguous rows ends in a pair fetched one row lower (one row alone
-    // has none).
-    // Against the predicated loader for every edge tile and for all tiles of operands with a column off 16 bytes, us (64 x 64
-    // tiles): TT 2542 x 644 x 896 86 -> 60, TT 4041 x 1524 x 110 51 -> 38, TN 5397 x 610 x 643 114 -> 91, NN 4046 x 566 x 426 50 -> 41.
-    // With odd edges on the predicated loader, their work-groups ran on long after the others: NT 1121 x 1088 x 1692 142 -> 93 us.
-    const bool fast = (TA || rows_a > 1) && (!TB || rows_b > 1);
-    const bool odd_a = fast && !TA && rows_a % 2 != 0, odd_b = fast && TB && rows_b % 2 != 0;
-    const bool fix_a = TileA::past_odd_end(tid, rows_a), fix_b = TileB::past_odd_end(tid, rows_b);
-    if (!odd_a && fix_a) { for (int c = 0; c < TileA::NCH; ++c) offA[c] += ESZ; }       // (one row alone: the plain offsets)
-    if (!odd_b && fix_b) { for (int c = 0; c < TileB::NCH; ++c) offB[c] += ESZ; }
-    auto place_odd = [&]() {
-        if (odd_a) { if (fix_a) TileA::odd_pair(ra); }
-        if (odd_b) { if (fix_b) TileB::odd_pair(rb); }
-    };
-
     auto load_stage = [&](int it) {
         const char *pa = gA + (int64_t)it * stepA;
         const char *pb = gB + (int64_t)it * stepB;
-        if (fast && it < n_full) {
+        if (it < n_full) {
             TileA::load_whole(ra, pa, offA);
             TileB::load_whole(rb, pb, offB);
-            place_odd();
         } else {
-            int kvalid = it < n_full ? BK : k_tail;
-            TileA::load_slow(ra, pa + (odd_a && fix_a ? ESZ : 0), offA, tid, lda, rows_a, kvalid, false);
-            TileB::load_slow(rb, pb + (odd_b && fix_b ? ESZ : 0), offB, tid, ldb, rows_b, kvalid, false);
+            TileA::load_slow(ra, pa, offA, tid, lda, rows_a, k_tail, false);
+            TileB::load_slow(rb, pb, offB, tid, ldb, rows_b, k_tail, false);
         }
     };
 
@@ -241,19 +233,16 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
         }
     };
     int it = 0;
-    if (fast) {
-        // while the next stage is a whole one: no test inside the loop, the predicated loader stays out of its body
-        for (; it + 1 < n_full; ++it) {
-            TileA::load_whole(ra, gA + (int64_t)(it + 1) * stepA, offA);
-            TileB::load_whole(rb, gB + (int64_t)(it + 1) * stepB, offB);
-            multiply_stage(lds + cur * Cfg::STAGE_BYTES);
-            place_odd();
-            char *nx = lds + (cur ^ 1) * Cfg::STAGE_BYTES;
-            TileA::store_lds(ra, nx, tid);
-            TileB::store_lds(rb, nx + TileA::LDS_BYTES, tid);
-            __syncthreads();
-            cur ^= 1;
-        }
+    // while the next stage is a whole one: no test inside the loop, the predicated loader stays out of its body
+    for (; it + 1 < n_full; ++it) {
+        TileA::load_whole(ra, gA + (int64_t)(it + 1) * stepA, offA);
+        TileB::load_whole(rb, gB + (int64_t)(it + 1) * stepB, offB);
+        multiply_stage(lds + cur * Cfg::STAGE_BYTES);
+        char *nx = lds + (cur ^ 1) * Cfg::STAGE_BYTES;
+        TileA::store_lds(ra, nx, tid);
+        TileB::store_lds(rb, nx + TileA::LDS_BYTES, tid);
+        __syncthreads();
+        cur ^= 1;
     }
     // Old C under the last stage's MFMAs (OLD_C_EARLY): requested at the top of the last stage -- no load follows it, so
     // nothing in the loop waits for it -- and the epilogue finds it in registers instead of starting with one memory

@@ -46,22 +46,11 @@ struct OperandTile {
     {
         return ((uint32_t)outer(tid, c) * ld + (uint32_t)inner(tid) * VEC) * ESZ;
     }
-    // An odd count of contiguous fp64 rows: this thread's pair has its second half, or both, outside.  goff(.., rows) then points at the
-    // last pair inside, one row lower, and odd_pair moves its second half to the first.
-    __device__ static inline bool past_odd_end(int tid, int rows) { return !KC && VEC == 2 && rows % 2 != 0 && inner(tid) * VEC >= rows - 1; }
-    __device__ static inline void odd_pair(u32x4 (&regs)[NCH])
-    {
-#pragma unroll
-        for (int c = 0; c < NCH; ++c) {
-            regs[c][0] = regs[c][2];
-            regs[c][1] = regs[c][3];
-        }
-    }
-    // goff with the rows past `rows` (>= 1, and >= 2 for the pairs above) moved to the last one (KC) or the last chunk inside (else)
+    // goff with the rows past `rows` (>= 1) moved to the last one (KC) or to the chunk that holds the last one (else)
     __device__ static inline uint32_t goff(int tid, int c, uint32_t ld, int rows)
     {
         const int o = KC ? min(outer(tid, c), rows - 1) : outer(tid, c), in = KC ? inner(tid) : min(inner(tid), (rows - 1) / VEC);
-        return ((uint32_t)o * ld + (uint32_t)in * VEC - (past_odd_end(tid, rows) ? 1u : 0u)) * ESZ;
+        return ((uint32_t)o * ld + (uint32_t)in * VEC) * ESZ;
     }
     __device__ static inline uint32_t lds_woff(int tid, int c)
     {

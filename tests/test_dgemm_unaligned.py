@@ -1,6 +1,6 @@
 """fp64 operands at every alignment on the loader that tests no chunk: even and odd row counts past the last whole tile, odd leading
 dimensions and pointers, whole and partial stages of k.  NaN in the rows between the matrix and its leading dimension: what
-a repeated row or pair of rows brings in may not come from there, nor reach a stored element."""
+a repeated row brings in, or the second half of a pair that an odd count of rows ends in, may not reach a stored element."""
 import numpy as np
 import pytest
 
@@ -16,6 +16,10 @@ pytestmark = pytest.mark.gpu
     (256, 128, 32, 1, (0, 0, 0), 1.0),         # whole tiles of odd leading dimensions
     (258, 129, 17, 3, (1, 1, 1), 0.5),         # off 16 bytes everywhere
     (2, 1, 64, 5, (1, 0, 1), 1.0),             # one pair of rows, one column
+    (131, 67, 48, 0, (0, 0, 0), 1.0),          # odd edges, whole stages only: the last one holds the column with nothing behind it
+    (129, 33, 32, 2, (0, 1, 0), 0.5),          # ... with a padding row behind each column but the last
+    (1, 1, 49, 0, (0, 0, 0), 1.0),             # one row: every pair takes in the next column
+    (1, 3, 16, 0, (1, 1, 1), 0.0),             # ... one stage, whose last column goes element by element
 ])
 def test_every_config_unaligned(ta, tb, m, n, k, pad, offsets, beta):
     import gemm_mmbo_amd as G
