@@ -370,6 +370,9 @@ gemm_wave_kernel(const GemmArgs args)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                         // (the ring slot's last reads are done)
         TileA::fill(gA + slices * stepA, lda, m_here, k_here, my_ring, lane);
         TileB::fill(gB + slices * stepB, ldb, n_here, k_here, my_ring + TileA::BYTES, lane);
+        // (what a lane reads is what others of its wavefront wrote: in order for the hardware, but not something the compiler
+        // can tell, which sees one thread's addresses)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         multiply_slice(my_ring);
     }
 

@@ -74,26 +74,82 @@ def test_only_calls_whose_pick_splits_k_take_a_workspace():
     G.release_workspace()
 
 
-@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
-@pytest.mark.parametrize("dtype", [0, 1, 2])
-def test_generated_code(dtype, tmp_path):
-    """The direct loads set M0 inside their asm statement without telling the compiler, which must therefore not use M0
-    itself; and nothing is spilled (a reload would wait for the direct loads in flight)."""
-    out = str(tmp_path / "wave.s")
-    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-                        "-Wno-unused-command-line-argument", "--cuda-device-only", "-S", f"-DMMBO_DTYPE={dtype}", "-DMMBO_TILE=7",
-                        os.path.join(CSRC, "inst_wave.hip"), "-o", out], capture_output=True, text=True)
-    assert r.returncode == 0, r.stderr[-2000:]
-    inside, own, kernels = False, [], 0
-    for line in open(out):
+NUM_TILES = 8
+
+
+@pytest.fixture(scope="module")
+def asm_files(tmp_path_factory):
+    """The generated code of every (element type, tile) the library ships."""
+    from concurrent.futures import ThreadPoolExecutor
+    outdir = tmp_path_factory.mktemp("wave")
+
+    def compile_one(unit):
+        dtype, tile = unit
+        out = str(outdir / f"wave_{dtype}_{tile}.s")
+        r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                            "-packed-fp32-ops", "-Wno-unused-command-line-argument", "--cuda-device-only", "-S",
+                            f"-DMMBO_DTYPE={dtype}", f"-DMMBO_TILE={tile}", os.path.join(CSRC, "inst_wave.hip"), "-o", out],
+                           capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return out
+    with ThreadPoolExecutor(max_workers=8) as ex:
+        return list(ex.map(compile_one, [(d, t) for d in (0, 1, 2) for t in range(NUM_TILES)]))
+
+
+def _lines(path):
+    """(inside an asm statement?, instruction or label) of one file."""
+    inside = False
+    for line in open(path):
         t = line.strip()
         if t.startswith(";;#ASMSTART"):
             inside = True
         elif t.startswith(";;#ASMEND"):
             inside = False
-        elif not inside and not t.startswith((";", ".")):
-            own.append(t.split(";")[0])
-        kernels += t.startswith(".amdhsa_kernel")
-    assert kernels == 4
-    assert not [t for t in own if re.search(r"\bm0\b", t)]
-    assert not [t for t in own if t.startswith("scratch_")]
+        elif t and (not t.startswith((";", ".")) or t.startswith(".LBB")):
+            yield inside, t.split(";")[0].strip()
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+def test_generated_code(asm_files):
+    """The direct loads set M0 inside their asm statement without telling the compiler, which must therefore not use M0
+    itself; and nothing is spilled (a reload would wait for the direct loads in flight)."""
+    for path in asm_files:
+        own = [t for inside, t in _lines(path) if not inside]
+        assert open(path).read().count(".amdhsa_kernel") == 4, path
+        assert not [t for t in own if re.search(r"\bm0\b", t)], path
+        assert not [t for t in own if t.startswith("scratch_")], path
+
+
+def _reads_that_may_overtake(lines):
+    """LDS reads that some path reaches from an LDS write without a barrier or an asm wait (which the compiler moves no access
+    across) on the way."""
+    label = {t[:-1]: i for i, (_, t) in enumerate(lines) if t.endswith(":")}
+    bad, seen = set(), set()
+    todo = [i + 1 for i, (_, t) in enumerate(lines) if t.startswith("ds_write")]
+    while todo:
+        i = todo.pop()
+        while i < len(lines) and i not in seen:
+            seen.add(i)
+            inside, t = lines[i]
+            if t.startswith(("s_barrier", "s_endpgm")) or (inside and "lgkmcnt(0)" in t):
+                break
+            if t.startswith("ds_read"):
+                bad.add(t)
+            if t.startswith(("s_branch", "s_cbranch")):
+                todo.append(label[t.split()[-1]])
+                if t.startswith("s_branch"):
+                    break
+            i += 1
+    return bad
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
+def test_slices_filled_through_registers_are_read_behind_a_wait(asm_files):
+    """A partial slice is written to LDS by all lanes and read by other lanes: the reads stay behind the writes only if the
+    compiler is told so."""
+    planted = [(False, "ds_write_b128 v0, v[1:4]"), (False, "s_waitcnt lgkmcnt(0)"), (False, "ds_read_b128 v[4:7], v0")]
+    assert _reads_that_may_overtake(planted) and not _reads_that_may_overtake([planted[0], (True, planted[1][1]), planted[2]])
+    for path in asm_files:
+        lines = list(_lines(path))
+        assert any(t.startswith("ds_write_b128") for _, t in lines)
+        assert not _reads_that_may_overtake(lines), path
