@@ -49,8 +49,9 @@ struct OperandTile {
     // goff with the rows past `rows` (>= 1) moved to the last one (KC) or to the chunk that holds the last one (else)
     __device__ static inline uint32_t goff(int tid, int c, uint32_t ld, int rows)
     {
-        const int o = KC ? min(outer(tid, c), rows - 1) : outer(tid, c), in = KC ? inner(tid) : min(inner(tid), (rows - 1) / VEC);
-        return ((uint32_t)o * ld + (uint32_t)in * VEC) * ESZ;
+        const uint32_t last = (uint32_t)rows - 1;
+        const uint32_t o = KC ? min((uint32_t)outer(tid, c), last) : outer(tid, c), in = KC ? inner(tid) : min((uint32_t)inner(tid), last / VEC);
+        return (o * ld + in * VEC) * ESZ;
     }
     __device__ static inline uint32_t lds_woff(int tid, int c)
     {
