@@ -357,22 +357,40 @@ double model_time(int dtype, int tile, int split, size_t m, size_t n, size_t k, 
 // fp64: how many 64 x 64 tiles at the end of the walk go out as quarters: those behind the last whole round of the 256 CUs.
 // 1152 x 2048 is 576 tiles, 2.25 to a CU: whole, they take as long as 3 rounds; the last 64 as 256 quarters, 2.25.  A quarter
 // takes 0.3 of a tile's time (its operand traffic halves, its flops quarter), so up to three quarters to a CU, 192 tiles,
-// are worth it, however many whole rounds precede them (aligned operands, us: rest 64 of 2 rounds 66.4 -> 52.8, 100 of 2
-// 104.7 -> 88.4, 44 of 6 189.6 -> 167.5, 191 of 4 49.2 -> 48.0).  Fewer tiles than CUs are the 32 x 32 tile's.
+// are worth it, however many whole rounds precede them (aligned operands, us: 100 of 2 104.7 -> 88.4, 44 of 6 189.6 -> 167.5, 191 of
+// 4 49.2 -> 48.0), but not three of them behind several rounds of a short k, where 0.9 of a tile's time is none to gain (145 of 5, TN 3648 x
+// 1600 x 272 whole 62.0, quarters 64.1).  Fewer tiles than CUs are the 32 x 32 tile's.
 constexpr int kQuarterTile = 3;
 static_assert(kTilesF64[kQuarterTile].bm == 32 && kTilesF64[kQuarterTile].bn == 32, "a 64 x 64 tile's quarter");
-size_t quartered_tiles(int tile, size_t tiles, int batch)
+size_t quartered_tiles(int tile, size_t tiles, int batch, size_t k)
 {
     if (!dgemm_quarters(kTilesF64[tile].bm, kTilesF64[tile].bn) || batch != 1) return 0;
     const size_t rest = tiles % 256;
+    if (rest > 128 && tiles >= 2 * 256 && tiles < 7 * 256 && k < 320) return 0;
     return tiles >= 256 && rest <= 192 ? rest : 0;
+}
+
+// fp64: does a grid of 64 x 64 tiles that ends in quarters stay with them, or do 32 x 32 tiles throughout take the call?  The model below
+// compares rounds, but not how far the work-groups of a CU overlap: with one or two whole rounds all of them are resident at one
+// time, start together and update C together, and 32 x 32 tiles, of which a CU runs some behind others, are as fast or faster,
+// unless the end is long (three quarters to a CU behind one round) or k is; behind three to six rounds it is k alone.  Behind more
+// the overlap is there.  Measured on 490 drawn shapes, quarters against 32 x 32 tiles, us: one round 5120 x 256 x 496 29.2 / 27.2, 1792 x 832 x 541 35.4 / 33.9, with three quarters 2048 x 832 x 848 55.4 / 61.9; two rounds
+// 1152 x 2048 x 384 36.7 / 35.4, x 592 52.9 / 51.3, 2112 x 1024 x 752 60.5 / 64.7, with three quarters 960 x 2752 x 624 68.4 / 63.4; more
+// 2432 x 2176 x 256 59.4 / 56.3, 4736 x 768 x 304 43.5 / 42.1, 2304 x 2048 x 384 64.6 / 66.4, 3584 x 1280 x 3342 1.5 % faster,
+// 26208 x 2033 x 152 387 / 416.  The pick is then within 0.8 % of the faster of the two on average, 4 % at worst on aligned operands.
+bool quarters_pay(size_t tiles, size_t k)
+{
+    const size_t whole = tiles / 256, quarters = ceil_div(tiles % 256, 64);
+    if (whole == 1) return quarters == 3 && k >= 400;
+    if (whole == 2) return quarters < 3 && k >= 640;
+    return whole >= 7 || k >= 320;
 }
 
 // fp64: microseconds.  Work-groups run in rounds of (CUs x work-groups per CU); a tile costs a fixed overhead
 // (first stage, C update, dispatch of its successor: measured per tile and CU with K swept from 96 to 1536 on the
 // HPL shape's M and N) plus its K at the tile's in-loop efficiency (from 8192^3), both shared by the work-groups
 // resident on the CU; the last, partial round runs with fewer of them, or as quarters that cost what the 32 x 32 tile does
-// (36 drawn shapes that end so: within 12 % of the measured time, 16 % where C is read).
+// (drawn shapes that end so: within 12 % of the measured time, 16 % where C is read).
 double model_time_f64(int tile, size_t m, size_t n, size_t k, int batch)
 {
     //                                    128x128/4w 256x128/8w 64x64  32x32  128x128/8w 128x64
@@ -386,7 +404,7 @@ double model_time_f64(int tile, size_t m, size_t n, size_t k, int batch)
         return overhead_us[t] + 2.0 * kTilesF64[t].bm * kTilesF64[t].bn * (double)(k ? k : 1) / flop_per_us_cu / in_loop_eff[t];
     };
     const double per_tile = tile_us(tile);
-    if (const size_t rest = quartered_tiles(tile, (size_t)tiles, batch))
+    if (const size_t rest = quartered_tiles(tile, (size_t)tiles, batch, k))
         return launch + std::floor(tiles / cus) * per_tile + std::ceil(4.0 * (double)rest / cus) * tile_us(kQuarterTile);
     const double slots = cus * resident[tile];
     const double full = std::floor(tiles / slots), last = tiles - full * slots;
@@ -620,6 +638,11 @@ static int select_config(int dtype, int transA, int transB, size_t m, size_t n, 
         for (int tile = 0; tile < NUM_F64_TILES; ++tile) {
             double t = model_time_f64(tile, m, n, k, batch);
             if (best_t == 0.0 || t < best_t) { best_t = t; best = tile; }
+        }
+        const size_t tiles = ceil_div(m, kTilesF64[best].bm) * ceil_div(n, kTilesF64[best].bn);
+        if (quartered_tiles(best, tiles, batch, k) > 0 && !quarters_pay(tiles, k)) {
+            best = kQuarterTile;
+            best_t = model_time_f64(best, m, n, k, batch);
         }
         *us = best_t;
         return best;
@@ -898,15 +921,6 @@ Plan plan_for(const WaveShape &p)
     Plan plan;
     double table_us;
     plan.config_id = select_config(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, &table_us);
-    // fp64 calls that read C, at most two whole rounds of tiles with quarters behind them and a short k: all work-groups of such
-    // a call are resident at one time and update C at one time; 32 x 32 tiles, of which a CU runs some behind others, overlap a
-    // part of that (us, quarters against 32 x 32 tiles: 1152 x 2048 x 384 with ldc 44160 37.2 / 36.2, 896 x 1728 x 208 18.7 / 18.3, 2880 x
-    // 448 x 352 23.2 / 22.9; with k = 512 and 592 38.2 / 40.0 and 52.8 / 56.4, with four rounds and k = 124 32.0 / 33.1).
-    if (p.dtype == MMBO_F64 && plan.config_id >= 0 && p.read_c && p.k < 448) {
-        const TileRow &r = kTilesF64[plan.config_id];
-        const size_t tiles = ceil_div(p.m, r.bm) * ceil_div(p.n, r.bn);
-        if (tiles < 3 * 256 && quartered_tiles(plan.config_id, tiles, p.batch) > 0) plan.config_id = kQuarterTile;
-    }
     plan.wave = pick_wave(p, p.dtype != MMBO_F64 && config_ref(plan.config_id).split > 1);
     // (by 8 % at least: nearer than that the models do not tell the two apart.  110 drawn shapes, against the tables' configs alone:
     // 1.367 times faster in the geometric mean, two slower by over 2 %; without the margin 1.361 and seven.)
@@ -1096,7 +1110,7 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
         return ((uintptr_t)p % 128 == 0) && ((ld * esz) % 128 == 0) && (batch == 1 || ((size_t)stride * esz) % 128 == 0);
     };
     a.line_rows = on_lines(A, lda, strideA) && on_lines(B, ldb, strideB);
-    a.quartered = f64 ? (uint32_t)quartered_tiles(cref.tile, nwg0 * nwg1, batch) : 0;
+    a.quartered = f64 ? (uint32_t)quartered_tiles(cref.tile, nwg0 * nwg1, batch, k) : 0;
     a.ws_narrow = (size_t)r.bn * m * 4 < 0x7FFFFF00ull;
     a.vec_c = aligned16(C, ldc, strideC) && (!cref.x16 || (size_t)r.bn * ldc * esz < 0x7FFFFF00ull);
     // beta != 0 on the x16 kernel's fp16 path: the old C of a tile is fetched into LDS under the tile's last slices (one
