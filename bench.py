@@ -111,13 +111,12 @@ def time_gemm(G, torch, dtype, m, n, k, steps, warmup, seed):
     calib = torch.add(A, 0)
     del calib
     stream = torch.cuda.current_stream()
-    cid = G.select_config(dtype, 0, 0, m, n, k, 1)
 
     def step():
-        G.gemm(dtype, G.OP_N, G.OP_N, m, n, k, 1.0, A, m, B, k, 0.0, C, m, cid, stream)
+        G.gemm(dtype, G.OP_N, G.OP_N, m, n, k, 1.0, A, m, B, k, 0.0, C, m, G.CONFIG_AUTO, stream)
 
     t = timed_launches(torch, stream, step, steps, warmup)
-    return t, G.config_info(dtype, cid), (A, B, C)
+    return t, G.auto_info(dtype, 0, 0, m, n, k), (A, B, C)
 
 
 def spot_check(G, dtype, m, n, k, A, B, C):
@@ -152,13 +151,12 @@ def dgemm_legs(G, torch, steps, warmup):
         B = torch.rand(k * n, device="cuda", generator=gen, dtype=torch.float64)
         C0 = torch.rand(m * n, device="cuda", generator=gen, dtype=torch.float64)
         C = C0.clone()
-        cid = G.select_config(G.F64, ta, tb, m, n, k, 1)
         nsteps = max(10, steps // 2) if tag == "8192" else max(10, steps)
-        ms = timed_launches(torch, stream, lambda: G.gemm(G.F64, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, m, cid, stream),
+        ms = timed_launches(torch, stream, lambda: G.gemm(G.F64, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, m, G.CONFIG_AUTO, stream),
                             nsteps, max(2, warmup // 4), settle=False)["median_ms"]
         # parity on a band of 64 rows of one fresh application (beta = 1 accumulates over the timed launches)
         C.copy_(C0)
-        G.gemm(G.F64, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, m, cid, stream)
+        G.gemm(G.F64, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, m, G.CONFIG_AUTO, stream)
         torch.cuda.synchronize()
         r0 = 4000
         hA, hB, hC0, hC = A.cpu().numpy(), B.cpu().numpy(), C0.cpu().numpy(), C.cpu().numpy()
@@ -168,7 +166,7 @@ def dgemm_legs(G, torch, steps, warmup):
         out[f"fp64_{tag}_tflops"] = round(tf, 2)
         out[f"fp64_{tag}_ms_per_step"] = round(ms, 4)
         out[f"fp64_{tag}_frac_of_peak"] = round(tf / PEAK_TFLOPS["f64"], 4)
-        out[f"fp64_{tag}_tile_config"] = G.config_info(G.F64, cid)["name"]
+        out[f"fp64_{tag}_tile_config"] = G.auto_info(G.F64, ta, tb, m, n, k, reads_c=beta != 0)["name"]
         out[f"fp64_{tag}_max_rel_err"] = float(f"{rel:.3e}")
         out[f"fp64_{tag}_rel_err_limit"] = float(f"{U.tol(U.F64, k):.3e}")
         if tag == "hpl":
@@ -182,7 +180,7 @@ def dgemm_legs(G, torch, steps, warmup):
 
 def skinny_legs(G, torch, steps, warmup):
     """The two HBM-bound shapes of the benchmark set (NN, alpha = 1, beta = 0, U[-1,1] inputs) in both element types:
-    time per GEMM (split-K main kernel + reduction) from events on the launch stream, algorithmic bytes / time against
+    time per GEMM (automatic pick) from events on the launch stream, algorithmic bytes / time against
     the 8 TB/s HBM peak.  Parity of these shapes at full size is in tests/test_gemm_gpu.py."""
     stream = torch.cuda.current_stream()
     gen = torch.Generator(device="cuda")
@@ -193,9 +191,8 @@ def skinny_legs(G, torch, steps, warmup):
             A = (torch.rand(m * k, device="cuda", generator=gen) * 2 - 1).to(tdt)
             B = (torch.rand(k * n, device="cuda", generator=gen) * 2 - 1).to(tdt)
             C = torch.empty(m * n, device="cuda", dtype=tdt)
-            cid = G.select_config(dtype, 0, 0, m, n, k, 1)
             # small kernels: ten groups of at least twenty back-to-back launches each, median over the groups
-            us = timed_launches(torch, stream, lambda: G.gemm(dtype, 0, 0, m, n, k, 1.0, A, m, B, k, 0.0, C, m, cid, stream),
+            us = timed_launches(torch, stream, lambda: G.gemm(dtype, 0, 0, m, n, k, 1.0, A, m, B, k, 0.0, C, m, G.CONFIG_AUTO, stream),
                                 max(steps, 200), max(warmup, 20), groups=10, settle_min_ms=30.0, settle_max_ms=200.0)["median_ms"] * 1e3
             nbytes = (m * k + k * n + m * n) * esz
             # a plain streaming kernel with the same bytes read and written, on this box, launched the same way
@@ -204,7 +201,7 @@ def skinny_legs(G, torch, steps, warmup):
                                             "frac_of_hbm_peak": round(nbytes / us * 1e-3 / 8000.0, 4),
                                             "stream_kernel_same_bytes_us": round(stream_us, 2),
                                             "tflops": round(2.0 * m * n * k / us * 1e-6, 1),
-                                            "tile_config": G.config_info(dtype, cid)["name"]}
+                                            "tile_config": G.auto_info(dtype, 0, 0, m, n, k)["name"]}
     return out
 
 
@@ -223,7 +220,6 @@ def ragged_legs(G, torch, steps, warmup):
         B = (torch.rand(k * n, device="cuda", generator=gen) * 2 - 1).to(tdt)
         C = torch.empty(m * n, device="cuda", dtype=tdt)
         lda, ldb = (k if ta else m), (n if tb else k)
-        cid = G.select_config(dtype, ta, tb, m, n, k, 1)
 
         def run():
             G.gemm(dtype, ta, tb, m, n, k, 1.0, A, lda, B, ldb, 0.0, C, m, G.CONFIG_AUTO, stream)
@@ -231,7 +227,7 @@ def ragged_legs(G, torch, steps, warmup):
         tf = 2.0 * m * n * k / us * 1e-6
         out[f"{dname}_{'NT'[ta]}{'NT'[tb]}_{m}x{n}x{k}"] = {"us": round(us, 1), "tflops": round(tf, 1),
                                                             "frac_of_peak": round(tf / PEAK_TFLOPS["f16" if dtype == G.F16 else "f32"], 4),
-                                                            "tile_config": G.config_info(dtype, cid)["name"]}
+                                                            "tile_config": G.auto_info(dtype, ta, tb, m, n, k)["name"]}
         del A, B, C
     return out
 
@@ -255,7 +251,6 @@ def config_legs(G, torch, steps, warmup):
         B = ((torch.rand(k * n * batch, device="cuda", generator=gen) * 2 - 1) * scale).to(tdt)
         C = (torch.rand(m * n * batch, device="cuda", generator=gen) * 2 - 1).to(tdt)
         lda, ldb = (k if ta else m), (n if tb else k)
-        cid = G.select_config(dtype, ta, tb, m, n, k, batch)
 
         def run():
             G.gemm_strided_batched(dtype, ta, tb, m, n, k, alpha, A, lda, m * k, B, ldb, k * n, beta, C, m, m * n, batch,
@@ -267,7 +262,7 @@ def config_legs(G, torch, steps, warmup):
         gbps = batch * (m * k + k * n + m * n * (2 if beta != 0 else 1)) * esz / us * 1e-3
         out[key] = {"us": round(us, 1), "tflops": round(tf, 1),
                     "frac_of_peak": round(tf / PEAK_TFLOPS["f16" if dtype == G.F16 else "f32"], 4),
-                    "algorithmic_GBps": round(gbps, 1), "tile_config": G.config_info(dtype, cid)["name"]}
+                    "algorithmic_GBps": round(gbps, 1), "tile_config": G.auto_info(dtype, ta, tb, m, n, k, batch, reads_c=beta != 0)["name"]}
         if batch > 1:
             # the memory-bound one: a plain streaming kernel with the same bytes read (A, B, old C) and written, on this box
             out[key]["stream_kernel_same_bytes_us"] = round(
@@ -337,8 +332,7 @@ def main():
         B1 = torch.ones(k * n, device="cuda", dtype=torch.float16)
         C1 = torch.empty(m * n, device="cuda", dtype=torch.float16)
         st = torch.cuda.current_stream()
-        cid1 = G.select_config(G.F16, 0, 0, m, n, k, 1)
-        t1 = timed_launches(torch, st, lambda: G.gemm(G.F16, G.OP_N, G.OP_N, m, n, k, 1.0, A1, m, B1, k, 0.0, C1, m, cid1, st),
+        t1 = timed_launches(torch, st, lambda: G.gemm(G.F16, G.OP_N, G.OP_N, m, n, k, 1.0, A1, m, B1, k, 0.0, C1, m, G.CONFIG_AUTO, st),
                             40, 10, settle=True)
         ones_tflops = flops / t1["median_ms"] * 1e-9
         assert float(C1[12345]) == float(k)          # 8192 ones: exact in fp16

@@ -19,7 +19,7 @@ LIB_PATH = os.path.join(_HERE, "csrc", "libmmbo_gemm.so")
 
 EXPORTS = (
     "mmbo_gemm", "mmbo_gemm_strided_batched", "mmbo_gemm_strided_batched_static_workspace", "mmbo_static_workspace_bytes",
-    "mmbo_num_configs", "mmbo_config_info", "mmbo_select_config",
+    "mmbo_num_configs", "mmbo_config_info", "mmbo_select_config", "mmbo_auto_info",
     "mmbo_wg_remap", "mmbo_chip_block_remap", "mmbo_batch_xcd_remap", "mmbo_release_workspace", "mmbo_release_stream_workspace", "mmbo_workspace_info",
     "mmbo_probe_mfma_ceiling", "mmbo_probe_stream", "mmbo_status_string", "mmbo_last_hip_error", "mmbo_version",
 )
@@ -76,6 +76,8 @@ def lib():
         L.mmbo_config_info.restype = ci
         L.mmbo_select_config.argtypes = [ci, ci, ci, sz, sz, sz, ci]
         L.mmbo_select_config.restype = ci
+        L.mmbo_auto_info.argtypes = [ci, ci, ci, sz, sz, sz, sz, sz, sz, ci, ci, ctypes.POINTER(ci), ctypes.POINTER(ConfigDesc)]
+        L.mmbo_auto_info.restype = ci
         L.mmbo_wg_remap.argtypes = [cu, cu, cu, cu, cu, ctypes.POINTER(cu), ctypes.POINTER(cu)]
         L.mmbo_wg_remap.restype = ci
         L.mmbo_chip_block_remap.argtypes = [cu, cu, cu, ctypes.POINTER(cu), ctypes.POINTER(cu)]
@@ -179,6 +181,15 @@ def select_config(dtype, transA, transB, m, n, k, batch=1):
     if c < 0:
         _check(-c)
     return c
+
+
+def auto_info(dtype, transA, transB, m, n, k, batch=1, lda=None, ldb=None, ldc=None, reads_c=False):
+    """What CONFIG_AUTO runs for a call (leading dimensions: packed unless given): the fields of config_info() and "config_id", which is
+    CONFIG_AUTO for the kernel without a config id."""
+    cid, d = ctypes.c_int(0), ConfigDesc()
+    _check(lib().mmbo_auto_info(dtype, transA, transB, m, n, k, lda or max(k if transA else m, 1), ldb or max(n if transB else k, 1),
+                                ldc or max(m, 1), 1 if reads_c else 0, batch, ctypes.byref(cid), ctypes.byref(d)))
+    return dict(d.as_dict(), config_id=cid.value)
 
 
 def wg_remap(linear_id, nwg0, nwg1, wgm=8, num_xcd=8):

@@ -931,24 +931,135 @@ Plan plan_for(const WaveShape &p)
     return plan;
 }
 
-int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
-              const void *alpha, const void *A, size_t lda, long long strideA,
-              const void *B, size_t ldb, long long strideB, const void *beta, void *C,
-              size_t ldc, long long strideC, int batch, int config_id, void *stream, WsSource ws_source)
+// What MMBO_CONFIG_AUTO runs: the split-by-wavefront kernel, which takes any shape and alignment, or a config.
+struct Route {
+    bool wave;
+    WavePick pick;
+    int config_id;
+};
+
+inline size_t element_size(int dtype) { return dtype == MMBO_F64 ? 8 : dtype == MMBO_F32 ? 4 : 2; }
+
+// aligned16: A, B, their leading dimensions and batch strides are whole 16-byte groups.
+int route_for(const WaveShape &p, bool aligned16, WsSource ws_source, Route &r)
+{
+    const size_t esz = element_size(p.dtype);
+    const Plan plan = plan_for(p);
+    r.pick = plan.wave;
+    // (a pair of slices must span less than the 2 GiB of a buffer descriptor)
+    r.wave = plan.wave.tile >= 0 &&
+             tile_span_ok(TileRow{kWaveTiles[plan.wave.tile].bm, kWaveTiles[plan.wave.tile].bn, (int)(2 * 64 / esz), 0, 0}, p.transA, p.transB,
+                          p.lda, p.ldb, esz);
+    int id = r.config_id = plan.config_id;
+    if (r.wave) return MMBO_OK;
+    const bool f64 = p.dtype == MMBO_F64;
+    // The pick is made from the shape alone.  The ring kernels also need 16-byte aligned A and B, every
+    // direct-to-LDS kernel a tile's span of an operand below 2 GiB: where the operands at hand do not qualify, the
+    // x16 config of the same tile and split (any alignment), or the staged kernel, takes the call.
+    if (!f64 && !aligned16) {
+        const ConfigRef c = config_ref(id);
+        if (c.ring && !c.x16) {
+            static const int x16_of_ring[NUM_RING_TILES] = {0, 2, 3, 4};
+            int si = 0;
+            while (si + 1 < NUM_SPLITS && kSplits[si] != c.split) ++si;
+            const int tile = x16_of_ring[c.tile];
+            id = ring_shape_ok(p.dtype, tile, c.split, p.transA, p.transB, p.m, p.n, p.k, true)
+                     ? x16_config_id(tile, si) : select_staged(p.dtype, p.m, p.n, p.k, p.batch);
+        }
+    }
+    // The entry point that allocates nothing holds kScratchPartialBytes of partial sums: where the pick's GlobalSplitU
+    // needs more, the same tile runs with the largest split that fits (down to none), so that every shape still
+    // runs under MMBO_CONFIG_AUTO.  (A config the caller names is taken as named, or refused.)
+    if (!f64 && ws_source == WsSource::kStatic) {
+        const ConfigRef c = config_ref(id);
+        int si = split_index(c.split);
+        auto fits = [&](int sidx) {
+            if (kSplits[sidx] == 1) return true;
+            if ((double)kSplits[sidx] * p.batch * (double)p.m * (double)p.n * sizeof(float) > (double)kScratchPartialBytes) return false;
+            return !c.ring || ring_shape_ok(p.dtype, c.tile, kSplits[sidx], p.transA, p.transB, p.m, p.n, p.k, c.x16);
+        };
+        while (si > 0 && !fits(si)) --si;
+        id = c.x16 ? x16_config_id(c.tile, si) : c.ring ? ring_config_id(c.tile, si) : staged_config_id(c.tile, si);
+    }
+    if (!tile_span_ok(config_tile(p.dtype, id), p.transA, p.transB, p.lda, p.ldb, esz)) {
+        // enormous leading dimensions: the first staged tile (no split-K) whose span fits, large tiles first
+        const int ntiles = f64 ? NUM_F64_TILES : NUM_TILES;
+        id = -1;
+        for (int tile = 0; tile < ntiles && id < 0; ++tile)
+            if (tile_span_ok(config_tile(p.dtype, tile), p.transA, p.transB, p.lda, p.ldb, esz)) id = tile;
+        if (id < 0) return MMBO_ERR_INVALID_SIZE;
+    }
+    r.config_id = id;
+    return MMBO_OK;
+}
+
+// The split-by-wavefront kernel with the given pick on checked arguments; `a` holds the operands, sizes, strides and scalars.
+int run_wave(const WaveShape &p, const WavePick &w, GemmArgs &a, hipStream_t s, WsSource ws_source)
+{
+    const WaveRow &row = kWaveTiles[w.tile];
+    const size_t esz = element_size(p.dtype), bk = 64 / esz;
+    a.nwg0 = (uint32_t)ceil_div(p.m, row.bm); a.nwg1 = (uint32_t)ceil_div(p.n, row.bn);
+    // (how tiles are laid over the XCDs: see the kernel)
+    const bool tall = a.nwg0 >= a.nwg1;
+    const size_t long_ld = tall ? p.lda : p.ldb, line = 128 / esz;
+    const bool whole_lines = (tall ? !p.transA : p.transB) && long_ld % line == 0 && (uintptr_t)(tall ? a.A : a.B) % 128 == 0 &&
+                             (tall ? row.bm : row.bn) % line == 0 && (tall ? a.nwg0 : a.nwg1) % 8 == 0;
+    a.wgm = whole_lines ? 1 : 8;
+    a.nxcd = whole_lines ? 1 : 8;
+    a.columns_first = whole_lines && !tall && a.nwg0 > 1;
+    const size_t pairs = ceil_div(ceil_div(p.k ? p.k : 1, bk), 2), pairs_per_split = ceil_div(pairs, (size_t)w.split);
+    a.splits = (uint32_t)ceil_div(pairs, pairs_per_split);
+    a.k_per_split = (uint32_t)(a.splits > 1 ? pairs_per_split * 2 * bk : (p.k ? p.k : 1));
+    a.wave_pairs = (uint32_t)ceil_div(pairs_per_split, (size_t)w.waves);
+    const uint32_t per16 = (uint32_t)(16 / esz);
+    const uint32_t past_a = p.transA ? 0 : wave::columns_without_a_successor(a.m, per16, a.lda),
+                   past_b = p.transB ? wave::columns_without_a_successor(a.n, per16, a.ldb) : 0;
+    a.no_successor = past_a > past_b ? past_a : past_b;
+    a.vec_c = ((uintptr_t)a.C % 16 == 0) && ((a.ldc * esz) % 16 == 0) && (((size_t)a.strideC * esz) % 16 == 0);
+    WsHold ws_hold;
+    if (a.splits > 1) {
+        const size_t bytes = (size_t)a.splits * p.batch * p.m * p.n * sizeof(float);
+        char *base = nullptr;
+        int rc = ws_source == WsSource::kStatic ? static_scratch(&base) : workspace(s, bytes, ws_hold, &base);
+        if (rc != MMBO_OK) return rc;
+        a.ws = reinterpret_cast<float *>(base);
+    }
+    hipError_t e = p.dtype == MMBO_F64 ? dispatch_wave<2, 0>(w.tile, p.transA, p.transB, a, w.waves, s)
+                   : p.dtype == MMBO_F32 ? dispatch_wave<0, 0>(w.tile, p.transA, p.transB, a, w.waves, s)
+                                         : dispatch_wave<1, 0>(w.tile, p.transA, p.transB, a, w.waves, s);
+    if (e != hipSuccess) return hip_fail(e);
+    if (a.splits > 1) {
+        e = launch_splitk_reduce(p.dtype, a, s);
+        if (e != hipSuccess) return hip_fail(e);
+    }
+    return MMBO_OK;
+}
+
+// What both entry points and the queries check of a problem before anything else.
+int check_problem(int dtype, int transA, int transB, size_t m, size_t n, size_t k, size_t lda, size_t ldb, size_t ldc, int batch)
 {
     if (!valid_dtype(dtype)) return MMBO_ERR_INVALID_DTYPE;
     if ((transA & ~1) || (transB & ~1)) return MMBO_ERR_INVALID_OP;
-    if (!alpha || !beta) return MMBO_ERR_NULL_POINTER;
     const size_t kMaxDim = 0x7FFFFFFFull;
     if (m > kMaxDim || n > kMaxDim || k > kMaxDim || lda > kMaxDim || ldb > kMaxDim || ldc > kMaxDim)
         return MMBO_ERR_INVALID_SIZE;
     if (batch < 0 || batch > 65535) return MMBO_ERR_INVALID_SIZE;
     // BLAS rule: a leading dimension is at least 1 and at least the operand's stored row count
-    {
-        size_t need_a = transA ? k : m, need_b = transB ? n : k;
-        if (lda < (need_a ? need_a : 1) || ldb < (need_b ? need_b : 1) || ldc < (m ? m : 1))
-            return MMBO_ERR_INVALID_SIZE;
-    }
+    const size_t need_a = transA ? k : m, need_b = transB ? n : k;
+    if (lda < (need_a ? need_a : 1) || ldb < (need_b ? need_b : 1) || ldc < (m ? m : 1)) return MMBO_ERR_INVALID_SIZE;
+    return MMBO_OK;
+}
+
+int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
+              const void *alpha, const void *A, size_t lda, long long strideA,
+              const void *B, size_t ldb, long long strideB, const void *beta, void *C,
+              size_t ldc, long long strideC, int batch, int config_id, void *stream, WsSource ws_source,
+              const WavePick *named_wave = nullptr)
+{
+    if (!valid_dtype(dtype)) return MMBO_ERR_INVALID_DTYPE;
+    if ((transA & ~1) || (transB & ~1)) return MMBO_ERR_INVALID_OP;
+    if (!alpha || !beta) return MMBO_ERR_NULL_POINTER;
+    if (int rc = check_problem(dtype, transA, transB, m, n, k, lda, ldb, ldc, batch)) return rc;
     if (strideA < 0 || strideB < 0 || strideC < 0) return MMBO_ERR_INVALID_SIZE;
     if (config_id != MMBO_CONFIG_AUTO && (config_id < 0 || config_id >= mmbo_num_configs(dtype)))
         return MMBO_ERR_INVALID_CONFIG;
@@ -961,109 +1072,32 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     const double beta_d = f64 ? *static_cast<const double *>(beta) : (double)*static_cast<const float *>(beta);
     const float alpha_f = (float)alpha_d, beta_f = (float)beta_d;
 
-    const size_t esz_in = f64 ? 8 : dtype == MMBO_F32 ? 4 : 2;
+    const size_t esz = element_size(dtype);
+    GemmArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.A = A; a.B = B; a.C = C; a.ws = nullptr;
+    a.alpha = alpha_f; a.beta = beta_f;
+    a.alpha_d = alpha_d; a.beta_d = beta_d;
+    a.m = (uint32_t)m; a.n = (uint32_t)n; a.k = (uint32_t)k;
+    a.lda = (uint32_t)lda; a.ldb = (uint32_t)ldb; a.ldc = (uint32_t)ldc;
+    a.strideA = strideA; a.strideB = strideB; a.strideC = strideC;
+    a.batch = (uint32_t)batch;
+    auto aligned16 = [&](const void *p, size_t ld, long long stride) {
+        return ((uintptr_t)p % 16 == 0) && ((ld * esz) % 16 == 0) && (((size_t)stride * esz) % 16 == 0);
+    };
+    a.vec_a = aligned16(A, lda, strideA);
+    a.vec_b = aligned16(B, ldb, strideB);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+
     if (config_id == MMBO_CONFIG_AUTO) {
-        // Problems that a round of tiles would not spread over the chip: one launch of the split-by-wavefront kernel, which
-        // takes any shape and alignment.
-        const Plan plan = plan_for(WaveShape{dtype, transA, transB, m, n, k, batch, lda, ldb, f64 ? beta_d != 0.0 : beta_f != 0.0f});
-        const WavePick &w = plan.wave;
-        if (w.tile >= 0) {
-            const WaveRow &row = kWaveTiles[w.tile];
-            const size_t bk = 64 / esz_in;
-            // (a pair of slices must span less than the 2 GiB of a buffer descriptor)
-            if (tile_span_ok(TileRow{row.bm, row.bn, (int)(2 * bk), 0, 0}, transA, transB, lda, ldb, esz_in)) {
-                GemmArgs a;
-                std::memset(&a, 0, sizeof(a));
-                a.A = A; a.B = B; a.C = C;
-                a.alpha = alpha_f; a.beta = beta_f;
-                a.alpha_d = alpha_d; a.beta_d = beta_d;
-                a.m = (uint32_t)m; a.n = (uint32_t)n; a.k = (uint32_t)k;
-                a.lda = (uint32_t)lda; a.ldb = (uint32_t)ldb; a.ldc = (uint32_t)ldc;
-                a.strideA = strideA; a.strideB = strideB; a.strideC = strideC;
-                a.nwg0 = (uint32_t)ceil_div(m, row.bm); a.nwg1 = (uint32_t)ceil_div(n, row.bn);
-                a.batch = (uint32_t)batch;
-                // (how tiles are laid over the XCDs: see the kernel)
-                const bool tall = a.nwg0 >= a.nwg1;
-                const size_t long_ld = tall ? lda : ldb, line = 128 / esz_in;
-                const bool whole_lines = (tall ? !transA : transB) && long_ld % line == 0 && (uintptr_t)(tall ? A : B) % 128 == 0 &&
-                                         (tall ? row.bm : row.bn) % line == 0 && (tall ? a.nwg0 : a.nwg1) % 8 == 0;
-                a.wgm = whole_lines ? 1 : 8;
-                a.nxcd = whole_lines ? 1 : 8;
-                a.columns_first = whole_lines && !tall && a.nwg0 > 1;
-                const size_t pairs = ceil_div(ceil_div(k ? k : 1, bk), 2), pairs_per_split = ceil_div(pairs, w.split);
-                a.splits = (uint32_t)ceil_div(pairs, pairs_per_split);
-                a.k_per_split = (uint32_t)(a.splits > 1 ? pairs_per_split * 2 * bk : (k ? k : 1));
-                a.wave_pairs = (uint32_t)ceil_div(pairs_per_split, w.waves);
-                const uint32_t per16 = (uint32_t)(16 / esz_in);
-                const uint32_t past_a = transA ? 0 : wave::columns_without_a_successor(a.m, per16, a.lda),
-                               past_b = transB ? wave::columns_without_a_successor(a.n, per16, a.ldb) : 0;
-                a.no_successor = past_a > past_b ? past_a : past_b;
-                a.vec_c = ((uintptr_t)C % 16 == 0) && ((ldc * esz_in) % 16 == 0) && (((size_t)strideC * esz_in) % 16 == 0);
-                hipStream_t s = static_cast<hipStream_t>(stream);
-                WsHold ws_hold;
-                if (a.splits > 1) {
-                    const size_t bytes = (size_t)a.splits * batch * m * n * sizeof(float);
-                    char *base = nullptr;
-                    int rc = ws_source == WsSource::kStatic ? static_scratch(&base) : workspace(s, bytes, ws_hold, &base);
-                    if (rc != MMBO_OK) return rc;
-                    a.ws = reinterpret_cast<float *>(base);
-                }
-                hipError_t e = f64 ? dispatch_wave<2, 0>(w.tile, transA, transB, a, w.waves, s)
-                                   : dtype == MMBO_F32 ? dispatch_wave<0, 0>(w.tile, transA, transB, a, w.waves, s)
-                                                       : dispatch_wave<1, 0>(w.tile, transA, transB, a, w.waves, s);
-                if (e != hipSuccess) return hip_fail(e);
-                if (a.splits > 1) {
-                    e = launch_splitk_reduce(dtype, a, s);
-                    if (e != hipSuccess) return hip_fail(e);
-                }
-                return MMBO_OK;
-            }
-        }
-        config_id = plan.config_id;
-        // The pick is made from the shape alone.  The ring kernels also need 16-byte aligned A and B, every
-        // direct-to-LDS kernel a tile's span of an operand below 2 GiB: where the operands at hand do not qualify, the
-        // x16 config of the same tile and split (any alignment), or the staged kernel, takes the call.
-        if (!f64) {
-            const ConfigRef c = config_ref(config_id);
-            if (c.ring && !c.x16) {
-                auto al16 = [&](const void *p, size_t ld, long long stride) {
-                    return ((uintptr_t)p % 16 == 0) && ((ld * esz_in) % 16 == 0) && (((size_t)stride * esz_in) % 16 == 0);
-                };
-                if (!al16(A, lda, strideA) || !al16(B, ldb, strideB)) {
-                    static const int x16_of_ring[NUM_RING_TILES] = {0, 2, 3, 4};
-                    int si = 0;
-                    while (si + 1 < NUM_SPLITS && kSplits[si] != c.split) ++si;
-                    const int tile = x16_of_ring[c.tile];
-                    config_id = ring_shape_ok(dtype, tile, c.split, transA, transB, m, n, k, true)
-                                    ? x16_config_id(tile, si) : select_staged(dtype, m, n, k, batch);
-                }
-            }
-        }
-        // The entry point that allocates nothing holds kScratchPartialBytes of partial sums: where the pick's GlobalSplitU
-        // needs more, the same tile runs with the largest split that fits (down to none), so that every shape still
-        // runs under MMBO_CONFIG_AUTO.  (A config the caller names is taken as named, or refused.)
-        if (!f64 && ws_source == WsSource::kStatic) {
-            const ConfigRef c = config_ref(config_id);
-            int si = split_index(c.split);
-            auto fits = [&](int sidx) {
-                if (kSplits[sidx] == 1) return true;
-                if ((double)kSplits[sidx] * batch * (double)m * (double)n * sizeof(float) > (double)kScratchPartialBytes) return false;
-                return !c.ring || ring_shape_ok(dtype, c.tile, kSplits[sidx], transA, transB, m, n, k, c.x16);
-            };
-            while (si > 0 && !fits(si)) --si;
-            config_id = c.x16 ? x16_config_id(c.tile, si) : c.ring ? ring_config_id(c.tile, si) : staged_config_id(c.tile, si);
-        }
-        if (!tile_span_ok(config_tile(dtype, config_id), transA, transB, lda, ldb, esz_in)) {
-            // enormous leading dimensions: the first staged tile (no split-K) whose span fits, large tiles first
-            const int ntiles = f64 ? NUM_F64_TILES : NUM_TILES;
-            config_id = -1;
-            for (int tile = 0; tile < ntiles && config_id < 0; ++tile)
-                if (tile_span_ok(config_tile(dtype, tile), transA, transB, lda, ldb, esz_in)) config_id = tile;
-            if (config_id < 0) return MMBO_ERR_INVALID_SIZE;
-        }
+        const WaveShape p{dtype, transA, transB, m, n, k, batch, lda, ldb, f64 ? beta_d != 0.0 : beta_f != 0.0f};
+        if (named_wave) return run_wave(p, *named_wave, a, s, ws_source);
+        Route r;
+        if (int rc = route_for(p, a.vec_a && a.vec_b, ws_source, r)) return rc;
+        if (r.wave) return run_wave(p, r.pick, a, s, ws_source);
+        config_id = r.config_id;
     }
     const ConfigRef cref = f64 ? ConfigRef{false, config_id, 1, false} : config_ref(config_id);
-    const size_t esz = f64 ? 8 : dtype == MMBO_F32 ? 4 : 2;
     int split = cref.split;
     const RingRow &rr = cref.x16 ? kX16Tiles[cref.tile] : kRingTiles[cref.ring ? cref.tile : 0];
     TileRow r = f64 ? kTilesF64[config_id] : cref.ring ? TileRow{rr.bm, rr.bn, ring_bk(dtype), 0, 0} : tile_row(dtype, cref.tile);
@@ -1081,29 +1115,15 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     split = (int)ceil_div(k ? k : 1, k_per_split);        // the last split takes what is left, a partial slice included
     if ((size_t)batch * split > 65535) return MMBO_ERR_INVALID_SIZE;
 
-    GemmArgs a;
-    std::memset(&a, 0, sizeof(a));
-    a.A = A; a.B = B; a.C = C; a.ws = nullptr;
-    a.alpha = alpha_f; a.beta = beta_f;
-    a.alpha_d = alpha_d; a.beta_d = beta_d;
-    a.m = (uint32_t)m; a.n = (uint32_t)n; a.k = (uint32_t)k;
-    a.lda = (uint32_t)lda; a.ldb = (uint32_t)ldb; a.ldc = (uint32_t)ldc;
-    a.strideA = strideA; a.strideB = strideB; a.strideC = strideC;
     a.nwg0 = (uint32_t)nwg0; a.nwg1 = (uint32_t)nwg1;
     a.wgm = 8;
     a.nxcd = 8;
     a.splits = (uint32_t)split;
     a.k_per_split = (uint32_t)(split > 1 ? k_per_split : (k ? k : 1));
-    a.batch = (uint32_t)batch;
     // (tiles that run one work-group per CU: 256 x 256 and 192 x 192)
     a.chip_block = cref.x16 && rr.depth * (rr.bm + rr.bn) * 64 > 80 * 1024 && nwg0 >= 16 && nwg1 >= 16;
     // batches of problems of at most 32 tiles (an XCD's CUs hold them at one time): each problem on one XCD
     a.batch_xcd = split == 1 && batch >= a.nxcd && batch % a.nxcd == 0 && nwg0 * nwg1 <= 32;
-    auto aligned16 = [&](const void *p, size_t ld, long long stride) {
-        return ((uintptr_t)p % 16 == 0) && ((ld * esz) % 16 == 0) && (((size_t)stride * esz) % 16 == 0);
-    };
-    a.vec_a = aligned16(A, lda, strideA);
-    a.vec_b = aligned16(B, ldb, strideB);
     // (the x16 kernel's whole-tile epilogue addresses C as a buffer with 32-bit offsets: where a tile's span of C, its columns x
     // ldc, does not fit them, C goes out element by element instead)
     auto on_lines = [&](const void *p, size_t ld, long long stride) {
@@ -1122,7 +1142,6 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     // +0.3 %); with fewer rounds or a short k plain stores win (fp16 6144^3 +1.6 %, 44160 x 2048 x 384 +2.7 %, 64 x 512^3 +14 %)
     a.c_stream = cref.x16 && rr.depth * (rr.bm + rr.bn) * 64 > 80 * 1024 && (size_t)nwg0 * nwg1 >= 4 * 256 && k >= 4096;
 
-    hipStream_t s = static_cast<hipStream_t>(stream);
     if (cref.ring && !cref.x16 && (!a.vec_a || !a.vec_b)) return MMBO_ERR_INVALID_CONFIG;
     // Split-K: the partial sums go to the stream's own workspace (or the static one), and both launches that use it (the
     // GEMM and the reduction, which adds the splits in ascending order) are queued before the hold on that workspace
@@ -1160,6 +1179,58 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
 }  // namespace
 
 extern "C" {
+
+int mmbo_auto_info(int dtype, int transA, int transB, size_t m, size_t n, size_t k, size_t lda, size_t ldb, size_t ldc, int reads_c,
+                   int batch, int *config_id, mmbo_config_desc *out)
+{
+    if (!config_id || !out) return MMBO_ERR_NULL_POINTER;
+    if (int rc = check_problem(dtype, transA, transB, m, n, k, lda, ldb, ldc, batch)) return rc;
+    Route r{false, {}, 0};
+    if (m != 0 && n != 0 && batch != 0) {
+        const size_t esz = element_size(dtype);
+        const bool aligned16 = (lda * esz) % 16 == 0 && (ldb * esz) % 16 == 0;
+        if (int rc = route_for(WaveShape{dtype, transA, transB, m, n, k, batch, lda, ldb, reads_c != 0}, aligned16, WsSource::kLibrary, r)) return rc;
+    }
+    if (!r.wave) {
+        *config_id = r.config_id;
+        return mmbo_config_info(dtype, r.config_id, out);
+    }
+    const WaveRow &row = kWaveTiles[r.pick.tile];
+    std::memset(out, 0, sizeof(*out));
+    const int bk = (int)(64 / element_size(dtype));
+    std::snprintf(out->name, sizeof(out->name), "MT%03dx%03dx%02d_WT%03dx%03d_W%d_GSU%02d_LSU%02d_DTL1_WAVE%d", row.bm, row.bn, bk, row.bm,
+                  row.bn, r.pick.waves, r.pick.split, r.pick.waves, row.depth);
+    out->macro_tile_m = out->wave_tile_m = row.bm;
+    out->macro_tile_n = out->wave_tile_n = row.bn;
+    out->depth_u = bk;
+    out->threads = r.pick.waves * 64;
+    out->split_k = r.pick.split;
+    const int sum_size = dtype == MMBO_F64 ? 8 : 4, ring = row.depth * (row.bm + row.bn) * 64, partial = (row.bm + 16 / sum_size) * row.bn * sum_size;
+    out->lds_bytes = r.pick.waves * std::max(ring, partial);
+    *config_id = MMBO_CONFIG_AUTO;
+    return MMBO_OK;
+}
+
+// Not part of the interface: mmbo_gemm_strided_batched on a given row of kWaveTiles, with given wavefronts per work-group and
+// GlobalSplitU, whatever the pick is -- the tests reach every instantiation of the kernel through it.
+int mmbo_internal_wave_gemm(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
+                            const void *alpha, const void *A, size_t lda, long long strideA,
+                            const void *B, size_t ldb, long long strideB, const void *beta, void *C,
+                            size_t ldc, long long strideC, int batch, int tile, int waves, int split, void *stream)
+{
+    if (tile < 0 || tile >= NUM_WAVE_TILES || (waves != 1 && waves != 4 && waves != 8) || waves > wave_max_waves(kWaveTiles[tile]) || split < 1 ||
+        split > 64 || (dtype == MMBO_F64 && split > 1))
+        return MMBO_ERR_INVALID_CONFIG;
+    if (int rc = check_problem(dtype, transA, transB, m, n, k, lda, ldb, ldc, batch)) return rc;
+    const size_t esz = element_size(dtype);
+    const WaveRow &row = kWaveTiles[tile];
+    if (k == 0 || ceil_div(m, row.bm) * ceil_div(n, row.bn) > 65535 ||
+        !tile_span_ok(TileRow{row.bm, row.bn, (int)(2 * 64 / esz), 0, 0}, transA, transB, lda, ldb, esz))
+        return MMBO_ERR_INVALID_SIZE;
+    const WavePick pick{tile, waves, split, 0.0};
+    return gemm_impl(dtype, transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch,
+                     MMBO_CONFIG_AUTO, stream, WsSource::kLibrary, &pick);
+}
 
 int mmbo_gemm_strided_batched(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
                               const void *alpha, const void *A, size_t lda, long long strideA,

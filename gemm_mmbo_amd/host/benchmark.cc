@@ -97,12 +97,11 @@ int main(int argc, char **argv)
     const char *tn = ta ? "T" : "N", *tbn = tb ? "T" : "N", *dn = dtype == MMBO_F16 ? "hgemm" : dtype == MMBO_F64 ? "dgemm" : "sgemm";
     const double flops = 2.0 * (double)M * N * K * batch;
     if (type == 0) {
-        int id = mmbo_select_config(dtype, ta, tb, M, N, K, batch);
-        if (id < 0) MMBO_CHECK(-id);
+        int id = MMBO_CONFIG_AUTO;
         float t = 0.0f;
-        MMBO_CHECK(time_config(id, &t));
+        MMBO_CHECK(time_config(MMBO_CONFIG_AUTO, &t));
         mmbo_config_desc d;
-        MMBO_CHECK(mmbo_config_info(dtype, id, &d));
+        MMBO_CHECK(mmbo_auto_info(dtype, ta, tb, M, N, K, lda, ldb, ldc, beta_d != 0.0, batch, &id, &d));
         double tf = 1e-12 * flops / t;
         std::printf("%s(%s%s): kernel, m, n, k, lda, ldb, time, tflops, efficiency = %d (%s), %zu, %zu, %zu, %zu, %zu, %.6f, %.3f, %.2f%%\n",
                     dn, tn, tbn, id, d.name, M, N, K, lda, ldb, t, tf, tf / peak_tflops(dtype) * 100.0);

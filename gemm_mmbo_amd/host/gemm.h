@@ -9,7 +9,7 @@
 // transposes this library has: naive_sgemm / naive_hgemm (NN, like the reference's hand-written NN kernel,
 // table id 11) and {s,h,d}gemm_{NN,NT,TN,TT}.  Same argument order and meaning:
 // A, B, C are device pointers, alpha and beta host pointers, kernelId a row of the tile-config table
-// (MMBO_CONFIG_AUTO = -1 lets the per-shape table pick).  Unlike the reference they return a status
+// (MMBO_CONFIG_AUTO = -1 lets the library pick).  Unlike the reference they return a status
 // (0 = ok) instead of exiting, and launch on the null stream without reloading a code object per call.
 #ifndef MMBO_HOST_GEMM_H
 #define MMBO_HOST_GEMM_H

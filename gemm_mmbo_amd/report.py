@@ -94,10 +94,11 @@ def run_shape(G, torch, shape, reps, inner, config, check, seed=1):
     C0 = (torch.rand(ldc * n * batch, device="cuda", generator=gen, dtype=torch.float64) * 2 - 1).to(tdt)
     C = C0.clone()
     stream = torch.cuda.current_stream()
-    cid = G.select_config(dtype, ita, itb, m, n, k, batch) if config is None else config
-    name = G.config_info(dtype, cid)["name"]
+    ran = G.auto_info(dtype, ita, itb, m, n, k, batch, lda, ldb, ldc, beta != 0) if config is None else G.config_info(dtype, config)
+    cid, name = ran.get("config_id", config), ran["name"]          # (CONFIG_AUTO: the kernel without a config id)
+    named = G.CONFIG_AUTO if config is None else config
 
-    def launch(dt=dtype, a=A, b=B, c=C, cfg=cid):
+    def launch(dt=dtype, a=A, b=B, c=C, cfg=named):
         G.gemm_strided_batched(dt, ita, itb, m, n, k, alpha, a, lda, m * k, b, ldb, k * n, beta, c, ldc, ldc * n, batch, cfg,
                                stream)
 

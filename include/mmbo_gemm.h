@@ -112,6 +112,14 @@ int mmbo_config_info(int dtype, int config_id, mmbo_config_desc *out);
  * the kernel without a config id is faster on the shape.) */
 int mmbo_select_config(int dtype, int transA, int transB, size_t m, size_t n, size_t k, int batch);
 
+/* What a call with MMBO_CONFIG_AUTO runs, for reports and tests: *config_id is a config of the table, described in *out as
+ * mmbo_config_info does, or MMBO_CONFIG_AUTO for the kernel without a config id, whose tile, threads, GlobalSplitU and
+ * wavefronts that share k ("LSU" in the name, as in the reference's solution names) *out then describes.  reads_c: beta is
+ * not zero.  A, B, C and the batch strides count as 16-byte aligned and the workspace as the library's own.  Pure host logic: needs
+ * no device. */
+int mmbo_auto_info(int dtype, int transA, int transB, size_t m, size_t n, size_t k, size_t lda, size_t ldb, size_t ldc, int reads_c,
+                   int batch, int *config_id, mmbo_config_desc *out);
+
 /* Host twin of the kernels' work-group -> tile mapping: linear work-group id to (tile row, tile
  * column).  With num_xcd = 1 and linear_id = wg0 + wg1*nwg0 this is the reference's
  * WorkGroupMapping remap (src/gemm/ref/Kernels.cpp:204-236, src/gemm/ref/map.cpp:11-38);

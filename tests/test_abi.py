@@ -278,3 +278,29 @@ def test_fp64_grids_that_end_in_quarters_are_picked_where_they_were_faster(m, n,
     """Shapes whose 64 x 64 tiles are no whole number of rounds, on which one of the two tiles was measured 2 - 11 % faster."""
     for ta, tb in ((0, 0), (0, 1), (1, 0), (1, 1)):
         assert G.select_config(G.F64, ta, tb, m, n, k) == config
+
+
+def test_auto_info_describes_what_the_automatic_pick_runs():
+    """A config of the table as config_info describes it, or the kernel without a config id; the same argument checks as a call's."""
+    for dtype, ta, tb, m, n, k in ((G.F16, 0, 0, 8192, 8192, 8192), (G.F32, 0, 1, 4096, 4096, 4096), (G.F64, 0, 1, 44160, 2048, 384),
+                                   (G.F64, 0, 1, 1152, 2048, 384)):
+        for reads_c in (False, True):
+            got = G.auto_info(dtype, ta, tb, m, n, k, reads_c=reads_c)
+            assert got["config_id"] == G.select_config(dtype, ta, tb, m, n, k)
+            assert {f: v for f, v in got.items() if f != "config_id"} == G.config_info(dtype, got["config_id"])
+    # sixteen rows against a large matrix: wavefronts that split k among themselves
+    for dtype, bk in ((G.F16, 32), (G.F32, 16), (G.F64, 8)):
+        got = G.auto_info(dtype, 0, 0, 16, 4096, 4096)
+        waves = got["threads"] // 64
+        assert got["config_id"] == G.CONFIG_AUTO and got["macro_tile_m"] == got["wave_tile_m"] == 16 and got["depth_u"] == bk
+        assert f"_GSU{got['split_k']:02d}_LSU{waves:02d}_" in got["name"] and 0 < got["lds_bytes"] <= 160 * 1024
+    # operands off 16 bytes: a ring pick goes to the x16 config of the same tile
+    ring = G.auto_info(G.F32, 0, 0, 1024, 1024, 512)
+    x16 = G.auto_info(G.F32, 0, 0, 1024, 1024, 512, lda=1025)
+    assert "_ACC" not in ring["name"] and "_ACC" in x16["name"] and ring["macro_tile_m"] == x16["macro_tile_m"]
+    assert G.auto_info(G.F32, 0, 0, 0, 5, 5)["config_id"] == 0
+    for bad, status in ((dict(dtype=7), 1), (dict(transA=2), 2), (dict(lda=15), 3), (dict(ldc=15), 3), (dict(batch=-1), 3)):
+        args = dict(dict(dtype=G.F32, transA=0, transB=0, m=16, n=16, k=16), **bad)
+        with pytest.raises(G.MmboError) as e:
+            G.auto_info(**args)
+        assert e.value.status == status

@@ -74,6 +74,21 @@ def test_only_calls_whose_pick_splits_k_take_a_workspace():
     G.release_workspace()
 
 
+@pytest.mark.gpu
+def test_reports_time_the_automatic_pick():
+    """The report driver and the benchmark main without a config id run MMBO_CONFIG_AUTO and print what it ran."""
+    import json
+    import sys
+    r = subprocess.run([sys.executable, "-m", "gemm_mmbo_amd.report", "shapes", "h,N,N,16,4096,4096", "--reps", "3"], cwd=ROOT,
+                       capture_output=True, text=True, timeout=200)
+    assert r.returncode == 0, r.stderr[-2000:]
+    rec = [json.loads(l) for l in r.stdout.splitlines() if l.startswith("{")][0]
+    assert "_WAVE" in rec["config"] and rec["config_id"] == -1 and rec["max_rel_err"] <= U.tol(F16, 4096)
+    r = subprocess.run([os.path.join(ROOT, "gemm_mmbo_amd/host/benchmark"), "0", "16", "4096", "4096", "16", "4096", "16", "N", "N", "h", "1", "1", "0"],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "_WAVE" in r.stdout, r.stdout + r.stderr
+
+
 NUM_TILES = 8
 
 
