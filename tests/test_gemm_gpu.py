@@ -898,11 +898,14 @@ def test_automatic_pick_never_fails_on_its_own_choice():
         _run_and_check(p, cid, label=f"x16 by name with unaligned operand {offs}", offsets=offs)
     # a leading dimension so large that the rows of A^T under the picked tile span more than 2 GiB (only the first k rows of
     # each stored column are used): the pick itself is refused by name, the automatic path moves to a tile that fits
-    m, n, k = 64, 16384, 100
+    m, n, k = 128, 32768, 100
     pick = G.select_config(F32, 1, 0, m, n, k)
     tm = G.config_info(F32, pick)["macro_tile_m"]
     assert tm >= 64                                             # a smaller tile exists to fall back to
-    lda = 2 ** 31 // (tm * 4) + 4096                            # tm rows of A^T span just over 2 GiB (A: 2.1 GB at tm = 64)
+    lda = 2 ** 31 // (tm * 4) + 4096                            # tm rows of A^T span just over 2 GiB (A: 2.1 GB at tm = 128)
+    assert G.auto_info(F32, 1, 0, m, n, k)["config_id"] == pick
+    fallback = G.auto_info(F32, 1, 0, m, n, k, lda=lda)
+    assert fallback["config_id"] >= 0 and fallback["macro_tile_m"] < tm
     rng = np.random.default_rng(91)
     hA = rng.uniform(-1, 1, (m, k)).astype(np.float32)          # row i = the k values of column i of the stored k x m matrix
     hB = rng.uniform(-1, 1, (n, k)).astype(np.float32)          # B stored k x n, column j = hB[j]

@@ -1,10 +1,13 @@
 """The split-by-wavefront kernel (csrc/gemm_wave.hpp), which the automatic pick takes for small, thin and long-k problems.
 
-GPU: shapes at the edges of its tiles (16, 32, 64 rows), of its slices (32 halves, 16 floats, 8 doubles; pairs of them;
-fewer slices than wavefronts), with row-contiguous operands that end inside a 16-byte group or are shorter than one, and
-with k long enough for GlobalSplitU beyond 16 (several threads then share the splits of one sum), against the fp64 oracle
-with the suite's own bounds.  CPU: facts about the generated code that the kernel's asm statements rely on.
+GPU: every (element type, tile, transposes) the library ships, named through an entry point of the tests' own, with one, four and
+eight wavefronts, with and without GlobalSplitU, at sizes around the tile, around the ring's depth of slices (odd and even runs, a
+partial slice), at every alignment, with NaN in the padding rows; the walks of the grid that only whole memory lines
+take; and small, thin and long-k shapes through the automatic pick (rows shorter than a 16-byte group, fewer slices than wavefronts,
+GlobalSplitU beyond 16, where several threads share the splits of one sum).  All against the fp64 oracle with the suite's own
+bounds.  CPU: facts about the generated code that the kernel's asm statements rely on.
 """
+import ctypes
 import os
 import re
 import subprocess
@@ -34,12 +37,14 @@ def test_small_thin_and_long_k_shapes(dtype, ta, tb):
     import torch
 
     import gemm_mmbo_amd as G
+    taken = 0
     for i, (m, n, k, batch) in enumerate(SHAPES):
         pad = (0, 1, 8)[i % 3]
         ar, br = U.stored_shape(ta, m, k)[0], U.stored_shape(tb, k, n)[0]
         p = U.Problem(dtype, ta, tb, m, n, k, -1.5, (0.0, 0.5)[i % 2], lda=ar + pad, ldb=br + pad, ldc=m + pad, batch=batch,
                       seed=300 + i, dist="normal" if dtype == F16 else "uniform", c_fill=("nan", "uniform")[i % 2])
         got, guard = U.run_gpu(p)
+        taken += G.auto_info(dtype, ta, tb, m, n, k, batch, p.lda, p.ldb, p.ldc, p.beta != 0)["config_id"] == -1
         U.check(p, got, f"{NAMES[dtype]} {'NT'[ta]}{'NT'[tb]} {m}x{n}x{k} b{batch}")
         assert np.all(guard == 0)
         # the entry point that allocates nothing: the same bits
@@ -48,6 +53,118 @@ def test_small_thin_and_long_k_shapes(dtype, ta, tb):
                                                 p.sc, batch)
         torch.cuda.synchronize()
         assert np.array_equal(dC.cpu().numpy().view(U.BITS[dtype]), got.view(U.BITS[dtype]))
+    assert 2 * taken >= len(SHAPES)               # (the others run a config: the shapes are the same for every type)
+
+
+#        rows, columns, slices in the ring
+TILES = [(16, 16, 8), (16, 32, 6), (32, 16, 6), (16, 64, 4), (64, 16, 4), (32, 32, 4), (32, 64, 4), (64, 32, 4)]
+BK = {F32: 16, F16: 32, F64: 8}
+
+
+def _wave_gemm(p, tile, waves, split, offset_elems=(0, 0, 0)):
+    """The problem on one instantiation of the kernel; returns C and the words behind it, or None where there is none."""
+    import torch
+
+    import gemm_mmbo_amd as G
+    L = G.lib()
+    f = L.mmbo_internal_wave_gemm
+    f.restype = ctypes.c_int
+    f.argtypes = L.mmbo_gemm_strided_batched.argtypes[:-2] + [ctypes.c_int] * 3 + [ctypes.c_void_p]
+    dev = []
+    for h, off in zip((p.A, p.B, p.C), offset_elems):
+        t = torch.zeros(h.size + off + 8, dtype={F32: torch.float32, F16: torch.float16, F64: torch.float64}[p.dtype], device="cuda")
+        t[off:off + h.size].copy_(torch.from_numpy(h))
+        dev.append((t, t.data_ptr() + off * U.ESZ[p.dtype]))
+    scalar = ctypes.c_double if p.dtype == F64 else ctypes.c_float
+    alpha, beta = scalar(p.alpha), scalar(p.beta)
+    rc = f(p.dtype, p.ta, p.tb, p.m, p.n, p.k, ctypes.byref(alpha), dev[0][1], p.lda, p.sa, dev[1][1], p.ldb, p.sb, ctypes.byref(beta),
+           dev[2][1], p.ldc, p.sc, p.batch, tile, waves, split, None)
+    if rc == 5:                                  # no such instantiation
+        return None
+    assert rc == 0, rc
+    torch.cuda.synchronize()
+    out = dev[2][0].cpu().numpy()
+    return out[offset_elems[2]:offset_elems[2] + p.C.size], out[offset_elems[2] + p.C.size:]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [F32, F16, F64], ids=NAMES.get)
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_every_instantiation(dtype, tile):
+    bm, bn, depth = TILES[tile]
+    bk, ran = BK[dtype], 0
+    for ta, tb in ((0, 0), (0, 1), (1, 0), (1, 1)):
+        for waves in (1, 4, 8):
+            for split in (1, 5):
+                if split > 1 and dtype == F64:
+                    continue
+                # (m, n, k, padding rows, offsets, batch): edges, an odd run of slices and a partial one; whole tiles, a full ring
+                # and one pair more; edges packed tightly, where the last columns have nothing behind them, over a batch
+                cases = [(bm - 1, bn + 1, (depth + 1) * bk * waves * split + 3, 1 + tile % 3, (1, 1, 1), 1),
+                         (2 * bm, bn, (depth + 2) * bk * waves * split, 0, (0, 0, 0), 1),
+                         (bm + 1, 2 * bn - 1, bk * waves * split + bk, 0, (0, 1, 0), 3)]
+                for i, (m, n, k, pad, offsets, batch) in enumerate(cases):
+                    beta = (0.5, 0.0, 1.0)[i]
+                    p = U.Problem(dtype, ta, tb, m, n, k, -1.5, beta, lda=(k if ta else m) + pad, ldb=(n if tb else k) + pad, ldc=m + pad,
+                                  batch=batch, seed=40 * tile + i, dist="normal" if dtype == F16 else "uniform",
+                                  c_fill="uniform" if beta else "nan")
+                    for operand, ld, rows in ((p.A, p.lda, k if ta else m), (p.B, p.ldb, n if tb else k)):
+                        operand.reshape(-1, ld)[:, rows:] = np.nan
+                    got = _wave_gemm(p, tile, waves, split, offsets)
+                    if got is None:
+                        continue
+                    ran += 1
+                    U.check(p, got[0], f"{NAMES[dtype]} tile {tile} {'NT'[ta]}{'NT'[tb]} w{waves} s{split} {m}x{n}x{k}")
+                    assert np.all(got[1] == 0), "wrote past the end of C"
+    waves = 3 if 8 * depth * (bm + bn) * 64 <= 160 * 1024 else 2
+    assert ran == (0 if dtype == F64 and tile in F64_LEFT_OUT else 4 * 3 * waves * (1 if dtype == F64 else 2))
+
+
+F64_LEFT_OUT = ()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tile,ta,tb,m,n,k,lda,ldb", [
+    (F32, 5, 0, 1, 576, 1792, 105, 640, 1856),       # longer side of whole lines across: tile rows first
+    (F16, 6, 0, 1, 65, 1024, 96, 128, 1024),         # ... two tile rows, the second nearly empty
+    (F32, 7, 0, 0, 2048, 70, 80, 2048, 81),          # longer side down: the dispatcher's order
+    (F64, 0, 0, 0, 256, 16, 40, 256, 40),            # ... one tile column
+    (F32, 5, 1, 1, 100, 70, 64, 64, 71),             # regrouped by XCD
+])
+def test_walks_of_the_grid(dtype, tile, ta, tb, m, n, k, lda, ldb):
+    p = U.Problem(dtype, ta, tb, m, n, k, 1.0, 0.5, lda=lda, ldb=ldb, ldc=m + 3, seed=tile + m, dist="normal" if dtype == F16 else "uniform")
+    got, guard = _wave_gemm(p, tile, 4, 1)
+    U.check(p, got, f"{NAMES[dtype]} tile {tile}")
+    assert np.all(guard == 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_operands_whose_slices_span_two_gigabytes_take_a_config(ta, tb):
+    """A pair of slices must fit a buffer descriptor: the automatic pick leaves the kernel where the leading dimension is too large."""
+    import torch
+
+    import gemm_mmbo_amd as G
+    m, n, k, ld = 64, 64, 20, 2 ** 31 // (32 * 4) + 64
+    lda, ldb = (k if ta else ld), (ld if tb else k)
+    assert G.auto_info(F32, ta, tb, m, n, k)["config_id"] == -1
+    huge = (lda == ld) or (ldb == ld)
+    assert (G.auto_info(F32, ta, tb, m, n, k, lda=lda, ldb=ldb)["config_id"] >= 0) == huge
+    rng = np.random.default_rng(5)
+    hA, hB = rng.uniform(-1, 1, (k, m)).astype(np.float32), rng.uniform(-1, 1, (k, n)).astype(np.float32)
+
+    def stored(h, rows_contiguous, ld):                       # h: k x rows
+        h = h if rows_contiguous else h.T.copy()
+        t = torch.zeros((h.shape[0] - 1) * ld + h.shape[1], dtype=torch.float32, device="cuda")
+        for i in range(h.shape[0]):
+            t[i * ld:i * ld + h.shape[1]] = torch.from_numpy(h[i])
+        return t
+    dA, dB = stored(hA, not ta, lda), stored(hB, bool(tb), ldb)
+    dC = torch.full((m * n,), float("nan"), dtype=torch.float32, device="cuda")
+    G.gemm(F32, ta, tb, m, n, k, 1.0, dA, lda, dB, ldb, 0.0, dC, m)
+    torch.cuda.synchronize()
+    want = hA.T.astype(np.float64) @ hB.astype(np.float64)
+    assert np.max(np.abs(dC.cpu().numpy().reshape((m, n), order="F") - want)) <= U.tol(F32, k) * max(np.max(np.abs(want)), 1.0)
 
 
 @pytest.mark.gpu
@@ -89,9 +206,6 @@ def test_reports_time_the_automatic_pick():
     assert r.returncode == 0 and "_WAVE" in r.stdout, r.stdout + r.stderr
 
 
-NUM_TILES = 8
-
-
 @pytest.fixture(scope="module")
 def asm_files(tmp_path_factory):
     """The generated code of every (element type, tile) the library ships."""
@@ -108,7 +222,7 @@ def asm_files(tmp_path_factory):
         assert r.returncode == 0, r.stderr[-2000:]
         return out
     with ThreadPoolExecutor(max_workers=8) as ex:
-        return list(ex.map(compile_one, [(d, t) for d in (0, 1, 2) for t in range(NUM_TILES)]))
+        return list(ex.map(compile_one, [(d, t) for d in (0, 1, 2) for t in range(len(TILES))]))
 
 
 def _lines(path):
