@@ -3,7 +3,7 @@
 //
 // Same structure as the staged fp32/fp16 kernel (global loads into registers one stage ahead, padded
 // double-buffered LDS tile, one barrier per stage; whole stages of k without a test, at any edge and alignment, a partial one
-// through the predicated loader), with 16 x 16 MFMA blocks: an fp64 MFMA takes 64 clocks for 2,048 flops, so one 64-bit LDS read per
+// element by element), with 16 x 16 MFMA blocks: an fp64 MFMA takes 64 clocks for 2,048 flops, so one 64-bit LDS read per
 // operand per MFMA and a single-stage prefetch keep the pipes fed.
 //
 // Register layout of v_mfma_f64_16x16x4_f64 (checked on the device): operand lane l supplies row (column)
@@ -162,7 +162,7 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
     // Whole stages are read without a test per chunk, aligned or not.  Rows past the matrix repeat its last row, or the chunk that
     // holds it; where an odd count of contiguous rows ends inside that chunk, its second half is what follows in memory -- a
     // padding row, the next column -- and its products, as those of the repeated rows, are never stored.  Only the operand's last
-    // column has nothing behind it: of a tile with such an end the last stage goes chunk by chunk.
+    // column has nothing behind it: of a tile with such an end the last stage goes element by element.
     // Against the predicated loader for every edge tile and for all tiles of operands with a column off 16 bytes, us (64 x 64
     // tiles): TT 2542 x 644 x 896 86 -> 60, TT 4041 x 1524 x 110 51 -> 38, TN 5397 x 610 x 643 114 -> 91, NN 4046 x 566 x 426 50 -> 41.
     // With odd edges on the predicated loader, their work-groups ran on long after the others: NT 1121 x 1088 x 1692 142 -> 86 us; with
@@ -188,16 +188,16 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
     for (int c = 0; c < TileB::NCH; ++c) offB[c] = TileB::goff(tid, c, ldb, rows_b);
 
     u32x4 ra[TileA::NCH], rb[TileB::NCH];
-    auto load_stage = [&](int it) {
-        const char *pa = gA + (int64_t)it * stepA;
-        const char *pb = gB + (int64_t)it * stepB;
-        if (it < n_full) {
-            TileA::load_whole(ra, pa, offA);
-            TileB::load_whole(rb, pb, offB);
-        } else {
-            TileA::load_slow(ra, pa, offA, tid, lda, rows_a, k_tail, false);
-            TileB::load_slow(rb, pb, offB, tid, ldb, rows_b, k_tail, false);
-        }
+    // The stage behind the whole ones: requested, and, once it is there, zeroed past the end of k.  (Without a branch: the predicated
+    // loader's branches made the second operand's loads wait for the first's.  NN 69 x 128 x 477 x 60 21.9 -> 20.3 us, TT 128 x 512 x 57 x 120
+    // 26.6 -> 25.2.)
+    auto load_tail = [&]() {
+        TileA::load_partial(ra, gA + (int64_t)n_full * stepA, tid, lda, rows_a, k_tail);
+        TileB::load_partial(rb, gB + (int64_t)n_full * stepB, tid, ldb, rows_b, k_tail);
+    };
+    auto clear_tail = [&]() {
+        TileA::clear_past(ra, tid, k_tail);
+        TileB::clear_past(rb, tid, k_tail);
     };
 
     f64x4 acc[FM][FN];
@@ -210,37 +210,68 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
     const uint32_t fb_off = dfrag_lane_off<!TB, TileB::LDS_LD>(lane, wn * Cfg::TN, false) + TileA::LDS_BYTES;
 
     if (n_iter > 0) {
-        load_stage(0);
+        if (n_full > 0) {
+            TileA::load_whole(ra, gA, offA);
+            TileB::load_whole(rb, gB, offB);
+        } else {
+            load_tail();
+            clear_tail();
+        }
         TileA::store_lds(ra, lds, tid);
         TileB::store_lds(rb, lds + TileA::LDS_BYTES, tid);
     }
     __syncthreads();
 
     int cur = 0;
-    auto multiply_stage = [&](const char *st) {
+    // groups of four k: fragments, MFMAs
+    auto read_groups = [&](auto &fa, auto &fb, const char *st, int k0) {
 #pragma unroll
-        for (int kk = 0; kk < NKK; ++kk) {
-            double fa[FM], fb[FN];
+        for (int kk = 0; kk < (int)(sizeof(fa) / sizeof(fa[0])); ++kk) {
 #pragma unroll
-            for (int i = 0; i < FM; ++i) fa[i] = dread_frag<TA, TileA::LDS_LD>(st, fa_off, i, kk);
+            for (int i = 0; i < FM; ++i) fa[kk][i] = dread_frag<TA, TileA::LDS_LD>(st, fa_off, i, k0 + kk);
 #pragma unroll
-            for (int j = 0; j < FN; ++j) fb[j] = dread_frag<!TB, TileB::LDS_LD>(st, fb_off, j, kk);
+            for (int j = 0; j < FN; ++j) fb[kk][j] = dread_frag<!TB, TileB::LDS_LD>(st, fb_off, j, k0 + kk);
+        }
+    };
+    auto multiply_groups = [&](const auto &fa, const auto &fb) {
+#pragma unroll
+        for (int kk = 0; kk < (int)(sizeof(fa) / sizeof(fa[0])); ++kk)
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
                 for (int j = 0; j < FN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i], fb[j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[kk][i], fb[kk][j], acc[i][j], 0, 0, 0);
+    };
+    // A stage, with `store` (the next one, from registers to LDS) ahead of its last MFMAs, which run while the stores land and past the
+    // barrier.  The order is written down and fenced (below: nothing but address arithmetic crosses; larger wave tiles: nothing): left
+    // to the compiler it differed from kernel to kernel with the code around it.  us, NT with C read, fenced against the best of those:
+    // 44160 x 2048 x 384 1,097 -> 1,068, 2304 x 2048 x 384 64.9 -> 61.3, 1152 x 2048 x 384 35.3 -> 34.7, 16 x 512 x 512 x 64 17.0 -> 16.2.
+    constexpr int LATE = FM * FN == 1 ? 2 : 1;
+    auto multiply_stage = [&](const char *st, auto &&store) {
+#pragma unroll
+        for (int kk = 0; kk < NKK - LATE; ++kk) {
+            double fa[1][FM], fb[1][FN];
+            read_groups(fa, fb, st, kk);
+            multiply_groups(fa, fb);
         }
+        double fa[LATE][FM], fb[LATE][FN];
+        read_groups(fa, fb, st, NKK - LATE);
+        store();
+        if constexpr (FM * FN == 1) __builtin_amdgcn_sched_barrier(0x6);
+        else __builtin_amdgcn_sched_barrier(0);
+        multiply_groups(fa, fb);
     };
     int it = 0;
-    // while the next stage is a whole one: no test inside the loop, the predicated loader stays out of its body
+    // while the next stage is a whole one: no test inside the loop
     for (; it + 1 < n_full; ++it) {
         TileA::load_whole(ra, gA + (int64_t)(it + 1) * stepA, offA);
         TileB::load_whole(rb, gB + (int64_t)(it + 1) * stepB, offB);
-        multiply_stage(lds + cur * Cfg::STAGE_BYTES);
-        char *nx = lds + (cur ^ 1) * Cfg::STAGE_BYTES;
-        TileA::store_lds(ra, nx, tid);
-        TileB::store_lds(rb, nx + TileA::LDS_BYTES, tid);
+        __builtin_amdgcn_sched_barrier(0x6);
+        multiply_stage(lds + cur * Cfg::STAGE_BYTES, [&]() {
+            char *nx = lds + (cur ^ 1) * Cfg::STAGE_BYTES;
+            TileA::store_lds(ra, nx, tid);
+            TileB::store_lds(rb, nx + TileA::LDS_BYTES, tid);
+        });
         __syncthreads();
         cur ^= 1;
     }
@@ -251,12 +282,21 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
     constexpr bool EARLY_C = OLD_C_EARLY && FM * FN <= 4;
     [[maybe_unused]] f64x2 old_c[EARLY_C ? FM * FN : 1][2];
     [[maybe_unused]] bool have_old_c = false;
-    for (; it < n_iter; ++it) {
-        const bool more = it + 1 < n_iter;
-        if (more) load_stage(it + 1);
+    if (n_full > 0 && k_tail > 0) {
+        load_tail();
+        multiply_stage(lds + cur * Cfg::STAGE_BYTES, [&]() {
+            clear_tail();
+            char *nx = lds + (cur ^ 1) * Cfg::STAGE_BYTES;
+            TileA::store_lds(ra, nx, tid);
+            TileB::store_lds(rb, nx + TileA::LDS_BYTES, tid);
+        });
+        __syncthreads();
+        cur ^= 1;
+    }
+    if (n_iter > 0) {
         if constexpr (EARLY_C) {
             const uint32_t wrow0 = row0 + wm * Cfg::TM, wcol0 = col0 + wn * Cfg::TN;
-            if (!more && args.beta_d != 0.0 && wrow0 + FM * 16 <= args.m && wcol0 + FN * 16 <= args.n) {
+            if (args.beta_d != 0.0 && wrow0 + FM * 16 <= args.m && wcol0 + FN * 16 <= args.n) {
                 const double *p0 = static_cast<const double *>(args.C) + (int64_t)batch * args.strideC +
                                    (size_t)(wcol0 + (lane & 15)) * args.ldc + wrow0 + 2 * (lane >> 4);
 #pragma unroll
@@ -268,16 +308,7 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
                 have_old_c = true;
             }
         }
-
-        multiply_stage(lds + cur * Cfg::STAGE_BYTES);
-
-        if (more) {
-            char *nx = lds + (cur ^ 1) * Cfg::STAGE_BYTES;
-            TileA::store_lds(ra, nx, tid);
-            TileB::store_lds(rb, nx + TileA::LDS_BYTES, tid);
-        }
-        __syncthreads();
-        cur ^= 1;
+        multiply_stage(lds + cur * Cfg::STAGE_BYTES, []() {});
     }
 
     if constexpr (EARLY_C) {

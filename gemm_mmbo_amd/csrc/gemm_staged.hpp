@@ -104,6 +104,33 @@ struct OperandTile {
         }
     }
 
+    // A partial stage without a branch (8-byte elements): each element by itself, rows and k past the matrix moved to the last ones, so
+    // that nothing outside is read; clear_past then zeroes what lies past k.  `g` is the stage's origin, kvalid >= 1.
+    __device__ static inline void load_partial(u32x4 (&regs)[NCH], const char *g, int tid, uint32_t ld, int rows, int kvalid)
+    {
+        static_assert(ESZ != 8 || VEC == 2, "two elements per chunk");
+        const uint32_t last_row = (uint32_t)rows - 1, last_k = (uint32_t)kvalid - 1;
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            u32x2 e[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t o = outer(tid, c), in = inner(tid) * 2 + h;
+                const uint32_t row = min(KC ? o : in, last_row), k = min(KC ? in : o, last_k);
+                e[h] = *reinterpret_cast<const u32x2 *>(g + (KC ? row * ld + k : k * ld + row) * ESZ);
+            }
+            regs[c] = u32x4{e[0][0], e[0][1], e[1][0], e[1][1]};
+        }
+    }
+    __device__ static inline void clear_past(u32x4 (&regs)[NCH], int tid, int kvalid)
+    {
+#pragma unroll
+        for (int c = 0; c < NCH; ++c)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if ((KC ? inner(tid) * 2 + h : outer(tid, c)) >= kvalid) regs[c][2 * h] = regs[c][2 * h + 1] = 0;
+    }
+
     __device__ static inline void store_lds(const u32x4 (&regs)[NCH], char *lds, int tid)
     {
 #pragma unroll

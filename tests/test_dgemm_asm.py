@@ -1,6 +1,7 @@
 """What the fp64 kernel's speed rests on in the generated code (no GPU needed): in the loop over whole stages the operands of the
 next stage go from registers to LDS under the MFMAs of this one, so nothing between the loads and the LDS stores may depend
-on the tile, and part of the stage's MFMAs must be left when the stores are issued."""
+on the tile, and part of the stage's MFMAs must be left when the stores are issued; the loads of a partial stage are in flight
+together."""
 import os
 import subprocess
 
@@ -37,6 +38,23 @@ def _stores_after_every_mfma(loop):
     return mfma[-1] < store
 
 
+# 8-byte loads a thread makes for a partial stage of both operands: rows x 16 of k / threads, for each row of the config table
+PARTIAL_LOADS = [(128 + 128) * 16 // 256, (256 + 128) * 16 // 512, (64 + 64) * 16 // 256, (32 + 32) * 16 // 256, (128 + 128) * 16 // 512,
+                 (128 + 64) * 16 // 256]
+
+
+def _most_8_byte_loads_in_flight(body):
+    """The longest run of 8-byte loads without a wait for loads, a branch or a label among them."""
+    most = run = 0
+    for t in body:
+        if t.startswith("global_load_dwordx2"):
+            run += 1
+            most = max(most, run)
+        elif t.endswith(":") or t.startswith(("s_cbranch", "s_branch")) or (t.startswith("s_waitcnt") and "vmcnt" in t):
+            run = 0
+    return most
+
+
 def test_loop_finder_on_planted_code():
     loop = [".LBB0_1:", "global_load_dwordx4 v[0:3], v4, s[0:1]", "v_mfma_f64_16x16x4_f64 a", "ds_write_b128 v9, v[0:3]",
             "v_mfma_f64_16x16x4_f64 b", "s_barrier", "s_cbranch_scc1 .LBB0_1"]
@@ -60,3 +78,4 @@ def test_lds_stores_run_under_the_mfmas(tile, tmp_path):
         for loop in loops:
             assert not [t for t in loop if t.startswith(("v_cndmask", "scratch_"))], name
             assert not _stores_after_every_mfma(loop), name
+        assert _most_8_byte_loads_in_flight(body) >= PARTIAL_LOADS[tile], name
