@@ -371,19 +371,19 @@ size_t quartered_tiles(int tile, size_t tiles, int batch, size_t k)
 }
 
 // fp64: does a grid of 64 x 64 tiles that ends in quarters stay with them, or do 32 x 32 tiles throughout take the call?  The model below
-// compares rounds, but not how far the work-groups of a CU overlap: with one or two whole rounds all of them are resident at one
-// time, start together and update C together, and 32 x 32 tiles, of which a CU runs some behind others, are as fast or faster,
-// unless the end is long (three quarters to a CU behind one round) or k is; behind three to six rounds it is k alone.  Behind more
-// the overlap is there.  Measured on 490 drawn shapes, quarters against 32 x 32 tiles, us: one round 5120 x 256 x 496 29.2 / 27.2, 1792 x 832 x 541 35.4 / 33.9, with three quarters 2048 x 832 x 848 55.4 / 61.9; two rounds
-// 1152 x 2048 x 384 36.7 / 35.4, x 592 52.9 / 51.3, 2112 x 1024 x 752 60.5 / 64.7, with three quarters 960 x 2752 x 624 68.4 / 63.4; more
-// 2432 x 2176 x 256 59.4 / 56.3, 4736 x 768 x 304 43.5 / 42.1, 2304 x 2048 x 384 64.6 / 66.4, 3584 x 1280 x 3342 1.5 % faster,
-// 26208 x 2033 x 152 387 / 416.  The pick is then within 0.8 % of the faster of the two on average, 4 % at worst on aligned operands.
+// compares rounds, but not how far the work-groups of a CU overlap: with few whole rounds all of them are resident at one time,
+// start together and update C together, and 32 x 32 tiles, of which a CU runs some behind others, are as fast or faster on a short
+// k or where the quarters fill a round badly.  Measured on 420 drawn shapes, quarters against 32 x 32 tiles, us (NT, C read): one round
+// 5120 x 256 x 496 (one quarter to a CU) 26.6 / 26.9, but 27.2 / 26.6 with C not read, 1792 x 832 x 541 (two) 32.0 / 33.3, 2048 x 832 x 848 (three)
+// 53.0 / 62.4, 896 x 1728 x 208 15.9 / 15.8; two rounds 1152 x 2048 x 384 (one) 34.7 / 34.8, 2112 x 1024 x 752 59.4 / 62.5, 960 x 2752 x 624 (three) 67.5 / 63.3;
+// three 2432 x 1472 x 272 40.4 / 38.3, four 2304 x 2048 x 384 61.0 / 64.7, five 2432 x 2176 x 256 49.3 / 51.7.  The pick is then within 0.6 % of the
+// faster of the two on average, 4 % at worst on aligned operands.
 bool quarters_pay(size_t tiles, size_t k)
 {
     const size_t whole = tiles / 256, quarters = ceil_div(tiles % 256, 64);
-    if (whole == 1) return quarters == 3 && k >= 400;
-    if (whole == 2) return quarters < 3 && k >= 640;
-    return whole >= 7 || k >= 320;
+    if (whole == 1) return quarters >= 2 && k >= 256;
+    if (whole == 2) return quarters < 3 && k >= 256;
+    return whole >= 5 || k >= 320;
 }
 
 // fp64: microseconds.  Work-groups run in rounds of (CUs x work-groups per CU); a tile costs a fixed overhead

@@ -268,14 +268,14 @@ def test_sizes_between_rounds_of_the_cus_get_the_192_tiles():
 
 
 @pytest.mark.parametrize("m,n,k,config", [
-    # one whole round of 64 x 64 tiles: quarters behind it only as three to a CU, on a long k
-    (5120, 256, 496, 3), (1792, 832, 541, 3), (1088, 1664, 384, 3), (2048, 832, 848, 2),
-    # two: as one or two, on a longer one
-    (1152, 2048, 384, 3), (1152, 2048, 592, 3), (2112, 1024, 752, 2), (960, 2752, 624, 3),
-    # more: by k, and always behind seven
-    (2432, 2176, 256, 3), (4736, 768, 304, 3), (2304, 2048, 384, 2), (26208, 2033, 152, 2), (31552, 1536, 240, 2)])
+    # one whole round of 64 x 64 tiles: quarters behind it only as two or three to a CU, on a long k
+    (5120, 256, 496, 3), (1792, 832, 541, 2), (1088, 1664, 384, 2), (2048, 832, 848, 2), (896, 1728, 208, 3),
+    # two: as one or two
+    (1152, 2048, 592, 2), (2112, 1024, 752, 2), (960, 2752, 624, 3),
+    # three and four: by k; more: always
+    (4736, 768, 304, 3), (2304, 2048, 384, 2), (2432, 2176, 256, 2), (26208, 2033, 152, 2), (31552, 1536, 240, 2)])
 def test_fp64_grids_that_end_in_quarters_are_picked_where_they_were_faster(m, n, k, config):
-    """Shapes whose 64 x 64 tiles are no whole number of rounds, on which one of the two tiles was measured 2 - 11 % faster."""
+    """Shapes whose 64 x 64 tiles are no whole number of rounds, on which one of the two tiles was measured faster, by up to 23 %."""
     for ta, tb in ((0, 0), (0, 1), (1, 0), (1, 1)):
         assert G.select_config(G.F64, ta, tb, m, n, k) == config
 
