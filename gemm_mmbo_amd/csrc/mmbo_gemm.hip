@@ -812,7 +812,12 @@ struct WaveShape {
     int batch;
     size_t lda, ldb;
     bool read_c;
+    bool wide_c;        // C is read, and its columns (256 rows or more) lie at least four times their own length apart
 };
+WaveShape wave_shape(int dtype, int transA, int transB, size_t m, size_t n, size_t k, int batch, size_t lda, size_t ldb, size_t ldc, bool read_c)
+{
+    return {dtype, transA, transB, m, n, k, batch, lda, ldb, read_c, read_c && m >= 256 && ldc >= 4 * m};
+}
 
 double wave_model_us(const WaveShape &p, int tile, int waves, int split)
 {
@@ -898,7 +903,7 @@ struct Plan {
 Plan plan_for(const WaveShape &p)
 {
     struct Key {
-        int dtype, transA, transB, batch, read_c, lines_a, lines_b;
+        int dtype, transA, transB, batch, read_c, wide_c, lines_a, lines_b;
         size_t m, n, k;
     };
     struct Entry {
@@ -911,7 +916,7 @@ Plan plan_for(const WaveShape &p)
     const size_t per_line = 128 / (p.dtype == MMBO_F64 ? 8 : p.dtype == MMBO_F32 ? 4 : 2);
     Key key;
     std::memset(&key, 0, sizeof(key));                   // (compared as bytes)
-    key.dtype = p.dtype; key.transA = p.transA; key.transB = p.transB; key.batch = p.batch; key.read_c = p.read_c;
+    key.dtype = p.dtype; key.transA = p.transA; key.transB = p.transB; key.batch = p.batch; key.read_c = p.read_c; key.wide_c = p.wide_c;
     key.lines_a = p.lda % per_line == 0; key.lines_b = p.ldb % per_line == 0;
     key.m = p.m; key.n = p.n; key.k = p.k;
     size_t h = p.m * 0x9E3779B97F4A7C15ull ^ p.n * 0xC2B2AE3D27D4EB4Full ^ p.k * 0x165667B19E3779F9ull ^
@@ -922,9 +927,16 @@ Plan plan_for(const WaveShape &p)
     double table_us;
     plan.config_id = select_config(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, &table_us);
     plan.wave = pick_wave(p, p.dtype != MMBO_F64 && config_ref(plan.config_id).split > 1);
-    // (by 8 % at least: nearer than that the models do not tell the two apart.  110 drawn shapes, against the tables' configs alone:
-    // 1.367 times faster in the geometric mean, two slower by over 2 %; without the margin 1.361 and seven.)
-    if (plan.wave.us >= 0.92 * table_us) plan.wave.tile = -1;
+    // By 8 % at least: nearer than that the models do not tell the two apart (110 drawn shapes, against the tables' configs alone:
+    // 1.367 times faster in the geometric mean, two slower by over 2 %; without the margin 1.361 and seven).  Updates of a C inside a
+    // much larger matrix: by 17 %.  Neither model knows where the columns of C lie; of 13 such shapes modelled up to 1.2 times faster seven
+    // were slower (fp16 NT 512 x 797 x 96, ldc 44160, 5.1 -> 6.4 us), of 15 beyond that none.
+    // The ring kernel's 64 x 64 tile without a split, picked for a few microseconds of work, takes 2.65 us less than its model says (55 drawn
+    // shapes, 2.1 - 3.0), which matters only here: by 2.0 us, as this kernel takes 0.6 less on its smallest calls and 5 % less on the others.  us
+    // here / there: fp16 TT 1024 x 640 x 512 6.4 / 5.1, TT 4 x 576 x 320 x 512 8.4 / 5.7, TN 768 x 128 x 640 4.4 / 5.5, fp32 NN 448 x 768 x 304 7.0 / 8.1.
+    double bar = (p.wide_c ? 0.83 : 0.92) * table_us;
+    if (p.dtype != MMBO_F64 && plan.config_id == ring_config_id(3, 0)) bar = std::min(bar, table_us - 2.0);
+    if (plan.wave.us >= bar) plan.wave.tile = -1;
     e.used = true;
     e.key = key;
     e.plan = plan;
@@ -1090,7 +1102,7 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     hipStream_t s = static_cast<hipStream_t>(stream);
 
     if (config_id == MMBO_CONFIG_AUTO) {
-        const WaveShape p{dtype, transA, transB, m, n, k, batch, lda, ldb, f64 ? beta_d != 0.0 : beta_f != 0.0f};
+        const WaveShape p = wave_shape(dtype, transA, transB, m, n, k, batch, lda, ldb, ldc, f64 ? beta_d != 0.0 : beta_f != 0.0f);
         if (named_wave) return run_wave(p, *named_wave, a, s, ws_source);
         Route r;
         if (int rc = route_for(p, a.vec_a && a.vec_b, ws_source, r)) return rc;
@@ -1189,7 +1201,7 @@ int mmbo_auto_info(int dtype, int transA, int transB, size_t m, size_t n, size_t
     if (m != 0 && n != 0 && batch != 0) {
         const size_t esz = element_size(dtype);
         const bool aligned16 = (lda * esz) % 16 == 0 && (ldb * esz) % 16 == 0;
-        if (int rc = route_for(WaveShape{dtype, transA, transB, m, n, k, batch, lda, ldb, reads_c != 0}, aligned16, WsSource::kLibrary, r)) return rc;
+        if (int rc = route_for(wave_shape(dtype, transA, transB, m, n, k, batch, lda, ldb, ldc, reads_c != 0), aligned16, WsSource::kLibrary, r)) return rc;
     }
     if (!r.wave) {
         *config_id = r.config_id;

@@ -304,3 +304,23 @@ def test_auto_info_describes_what_the_automatic_pick_runs():
         with pytest.raises(G.MmboError) as e:
             G.auto_info(**args)
         assert e.value.status == status
+
+
+def test_pick_between_the_table_and_the_kernel_without_a_config_id_where_measured():
+    """Calls on which a config of the table was measured 10 - 25 % faster than the split-by-wavefront kernel, and their neighbours."""
+    def auto(*args, **kw):
+        return G.auto_info(*args, **kw)["config_id"]
+    # the ring kernel's 64 x 64 tile on a few microseconds of work, and where it is not the faster one
+    assert auto(G.F16, 1, 1, 1024, 640, 512) >= 0
+    assert auto(G.F16, 1, 1, 576, 320, 512, batch=4, reads_c=True) >= 0
+    assert auto(G.F16, 1, 0, 768, 128, 640) == G.CONFIG_AUTO
+    assert auto(G.F32, 0, 0, 448, 768, 304) == G.CONFIG_AUTO
+    assert auto(G.F32, 0, 1, 128, 256, 64, batch=32) >= 0
+    assert auto(G.F32, 0, 1, 1472, 576, 128, ldc=44160, reads_c=True) >= 0
+    # updates of a C inside a much larger matrix
+    for m, n, k in ((512, 797, 96), (496, 615, 384), (792, 620, 384)):
+        assert auto(G.F16, 0, 1, m, n, k, lda=m + 8, ldb=n + 8, ldc=44160, reads_c=True) >= 0
+    # ... where the gain is large, and where C lies packed or is not read
+    assert auto(G.F32, 0, 1, 64, 489, 4640, ldc=44160, reads_c=True) == G.CONFIG_AUTO
+    assert auto(G.F16, 1, 1, 2, 6144, 4792, lda=4856, ldb=6208, ldc=66, reads_c=True) == G.CONFIG_AUTO
+    assert auto(G.F16, 0, 1, 512, 797, 96, lda=520, ldb=805, ldc=44160) == G.CONFIG_AUTO
