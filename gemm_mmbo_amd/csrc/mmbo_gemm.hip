@@ -77,10 +77,16 @@ constexpr int kMaxDevices = 64;
 //   - Each slot has its own lock, held by a call from the lookup until both launches that use the buffer (the GEMM and
 //     the reduction) are queued: two host threads on one stream cannot interleave their launches, and growing a buffer
 //     (wait for that stream, free, allocate) stalls only callers of that same stream.
+//   - A buffer is never smaller than kWaveSumsBytes, what the split-by-wavefront kernel's splits take at most.
 //   - A new stream that finds the table full retires the least recently used slot nobody holds: the table lock is given
 //     up, the device is synchronised (the slot's stream may no longer exist, so it cannot be waited for by handle) and
 //     the buffer freed.  mmbo_release_stream_workspace retires one stream's slot at the caller's request.
 constexpr size_t kMaxWsSlots = 8;
+// (work-groups of that kernel, splits included, that the automatic pick takes at most) x (sums of its largest tile)
+constexpr size_t kMaxSplitWaveGroups = 1024;
+constexpr size_t kWaveSumsBytes = kMaxSplitWaveGroups * 32 * 64 * sizeof(float);
+constexpr bool wave_sums_fit(int i = 0) { return i == NUM_WAVE_TILES || (kMaxSplitWaveGroups * kWaveTiles[i].bm * kWaveTiles[i].bn * sizeof(float) <= kWaveSumsBytes && wave_sums_fit(i + 1)); }
+static_assert(wave_sums_fit(), "the partial sums of the largest tile");
 struct WsSlot {
     hipStream_t stream = nullptr;
     char *base = nullptr;
@@ -163,7 +169,7 @@ int workspace(hipStream_t stream, size_t bytes, WsHold &hold, char **out)
                 slot->base = nullptr;
                 slot->bytes = 0;
             }
-            size_t want = bytes + bytes / 4;
+            size_t want = std::max(bytes + bytes / 4, kWaveSumsBytes);
             void *p = nullptr;
             if (hipMalloc(&p, want) != hipSuccess) {
                 (void)hipGetLastError();
@@ -881,9 +887,8 @@ WavePick pick_wave(const WaveShape &p, bool may_split)
             if (waves > wave_max_waves(kWaveTiles[tile])) continue;
             for (int split = 1; split <= (may_split ? 64 : 1); split *= 2) {
                 // (splits: at least a pair of slices per wavefront, not beyond what the chip holds at one time; the partial sums
-                // of either entry point fit the static workspace, so that both run the same split)
-                if (split > 1 && (slices < (size_t)split * waves * 2 || tiles * p.batch * split > 1024 ||
-                                  (double)p.m * p.n * p.batch * split * sizeof(float) > (double)kScratchPartialBytes))
+                // then fit the static workspace, so that both entry points run the same split)
+                if (split > 1 && (slices < (size_t)split * waves * 2 || tiles * p.batch * split > kMaxSplitWaveGroups))
                     break;
                 const double us = wave_model_us(p, tile, waves, split);
                 if (best.tile < 0 || us < best.us) best = WavePick{tile, waves, split, us};
@@ -895,9 +900,15 @@ WavePick pick_wave(const WaveShape &p, bool may_split)
 
 // What the automatic pick runs for a shape.  The models are walked once per shape and thread (some microseconds, as much as a
 // small call takes); a small direct-mapped table keeps the answers, which are a function of the key alone.
+// Whether a call needs a workspace, and how large a one at most, follows from the shape alone, not from beta or leading dimensions:
+// a program runs a shape once and then captures a call of that shape that may differ in those, which cannot allocate.  So a
+// shape whose pick of mmbo_select_config splits k is first planned with packed operands and without C.  Where that plan needs no
+// workspace, no call of the shape does; where it needs one, every call of the shape holds one as large.
 struct Plan {
     WavePick wave;      // tile < 0: config_id
     int config_id;
+    bool workspace;     // may partial sums go through memory?
+    size_t reserve;     // bytes of workspace that a call sees to although it may need less itself
 };
 
 Plan plan_for(const WaveShape &p)
@@ -926,7 +937,7 @@ Plan plan_for(const WaveShape &p)
     Plan plan;
     double table_us;
     plan.config_id = select_config(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, &table_us);
-    plan.wave = pick_wave(p, p.dtype != MMBO_F64 && config_ref(plan.config_id).split > 1);
+    const int table_split = p.dtype == MMBO_F64 ? 1 : config_ref(plan.config_id).split;
     // By 8 % at least: nearer than that the models do not tell the two apart (110 drawn shapes, against the tables' configs alone:
     // 1.367 times faster in the geometric mean, two slower by over 2 %; without the margin 1.361 and seven).  Updates of a C inside a
     // much larger matrix: by 17 %.  Neither model knows where the columns of C lie; of 13 such shapes modelled up to 1.2 times faster seven
@@ -934,9 +945,30 @@ Plan plan_for(const WaveShape &p)
     // The ring kernel's 64 x 64 tile without a split, picked for a few microseconds of work, takes 2.65 us less than its model says (55 drawn
     // shapes, 2.1 - 3.0), which matters only here: by 2.0 us, as this kernel takes 0.6 less on its smallest calls and 5 % less on the others.  us
     // here / there: fp16 TT 1024 x 640 x 512 6.4 / 5.1, TT 4 x 576 x 320 x 512 8.4 / 5.7, TN 768 x 128 x 640 4.4 / 5.5, fp32 NN 448 x 768 x 304 7.0 / 8.1.
-    double bar = (p.wide_c ? 0.83 : 0.92) * table_us;
-    if (p.dtype != MMBO_F64 && plan.config_id == ring_config_id(3, 0)) bar = std::min(bar, table_us - 2.0);
-    if (plan.wave.us >= bar) plan.wave.tile = -1;
+    auto choose = [&](const WaveShape &q, bool may_split) {
+        WavePick w = pick_wave(q, may_split);
+        double bar = (q.wide_c ? 0.83 : 0.92) * table_us;
+        if (q.dtype != MMBO_F64 && plan.config_id == ring_config_id(3, 0)) bar = std::min(bar, table_us - 2.0);
+        if (w.us >= bar) w.tile = -1;
+        return w;
+    };
+    plan.workspace = false;
+    plan.reserve = 0;
+    if (table_split == 1) {
+        plan.wave = choose(p, false);
+    } else {
+        const WavePick packed = choose(wave_shape(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, p.transA ? p.k : p.m,
+                                                  p.transB ? p.n : p.k, p.m, false), true);
+        const double table_bytes = (double)table_split * p.batch * p.m * p.n * sizeof(float);
+        plan.workspace = packed.tile < 0 || packed.split > 1;
+        if (!plan.workspace) {
+            plan.wave = pick_wave(p, false);
+        } else {
+            plan.wave = choose(p, true);
+            if (packed.tile >= 0 && plan.wave.tile < 0 && table_bytes > (double)kWaveSumsBytes) plan.wave = pick_wave(p, true);
+            plan.reserve = packed.tile < 0 ? (size_t)std::min(table_bytes, 1e18) : kWaveSumsBytes;
+        }
+    }
     e.used = true;
     e.key = key;
     e.plan = plan;
@@ -948,6 +980,7 @@ struct Route {
     bool wave;
     WavePick pick;
     int config_id;
+    size_t reserve;     // of Plan
 };
 
 inline size_t element_size(int dtype) { return dtype == MMBO_F64 ? 8 : dtype == MMBO_F32 ? 4 : 2; }
@@ -958,6 +991,7 @@ int route_for(const WaveShape &p, bool aligned16, WsSource ws_source, Route &r)
     const size_t esz = element_size(p.dtype);
     const Plan plan = plan_for(p);
     r.pick = plan.wave;
+    r.reserve = plan.reserve;
     // (a pair of slices must span less than the 2 GiB of a buffer descriptor)
     r.wave = plan.wave.tile >= 0 &&
              tile_span_ok(TileRow{kWaveTiles[plan.wave.tile].bm, kWaveTiles[plan.wave.tile].bn, (int)(2 * 64 / esz), 0, 0}, p.transA, p.transB,
@@ -981,12 +1015,14 @@ int route_for(const WaveShape &p, bool aligned16, WsSource ws_source, Route &r)
     }
     // The entry point that allocates nothing holds kScratchPartialBytes of partial sums: where the pick's GlobalSplitU
     // needs more, the same tile runs with the largest split that fits (down to none), so that every shape still
-    // runs under MMBO_CONFIG_AUTO.  (A config the caller names is taken as named, or refused.)
-    if (!f64 && ws_source == WsSource::kStatic) {
+    // runs under MMBO_CONFIG_AUTO.  (A config the caller names is taken as named, or refused.)  A shape planned without a workspace
+    // whose leading dimensions are too large for that plan runs without a split.
+    if (!f64 && (ws_source == WsSource::kStatic || !plan.workspace)) {
         const ConfigRef c = config_ref(id);
         int si = split_index(c.split);
         auto fits = [&](int sidx) {
             if (kSplits[sidx] == 1) return true;
+            if (!plan.workspace) return false;
             if ((double)kSplits[sidx] * p.batch * (double)p.m * (double)p.n * sizeof(float) > (double)kScratchPartialBytes) return false;
             return !c.ring || ring_shape_ok(p.dtype, c.tile, kSplits[sidx], p.transA, p.transB, p.m, p.n, p.k, c.x16);
         };
@@ -1006,7 +1042,7 @@ int route_for(const WaveShape &p, bool aligned16, WsSource ws_source, Route &r)
 }
 
 // The split-by-wavefront kernel with the given pick on checked arguments; `a` holds the operands, sizes, strides and scalars.
-int run_wave(const WaveShape &p, const WavePick &w, GemmArgs &a, hipStream_t s, WsSource ws_source)
+int run_wave(const WaveShape &p, const WavePick &w, GemmArgs &a, hipStream_t s, WsSource ws_source, size_t reserve)
 {
     const WaveRow &row = kWaveTiles[w.tile];
     const size_t esz = element_size(p.dtype), bk = 64 / esz;
@@ -1029,11 +1065,17 @@ int run_wave(const WaveShape &p, const WavePick &w, GemmArgs &a, hipStream_t s, 
     a.no_successor = past_a > past_b ? past_a : past_b;
     a.vec_c = ((uintptr_t)a.C % 16 == 0) && ((a.ldc * esz) % 16 == 0) && (((size_t)a.strideC * esz) % 16 == 0);
     WsHold ws_hold;
-    if (a.splits > 1) {
-        const size_t bytes = (size_t)a.splits * p.batch * p.m * p.n * sizeof(float);
+    const size_t needed = a.splits > 1 ? (size_t)a.splits * p.batch * p.m * p.n * sizeof(float) : 0;
+    size_t bytes = needed;
+    if (ws_source == WsSource::kLibrary && reserve > (needed > 0 ? kWaveSumsBytes : 0)) {
+        // (a call under capture takes what is there: it cannot allocate, nor must it where it needs nothing)
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) bytes = std::max(bytes, reserve);
+    }
+    if (bytes > 0) {
         char *base = nullptr;
         int rc = ws_source == WsSource::kStatic ? static_scratch(&base) : workspace(s, bytes, ws_hold, &base);
-        if (rc != MMBO_OK) return rc;
+        if (rc != MMBO_OK && needed > 0) return rc;
         a.ws = reinterpret_cast<float *>(base);
     }
     hipError_t e = p.dtype == MMBO_F64 ? dispatch_wave<2, 0>(w.tile, p.transA, p.transB, a, w.waves, s)
@@ -1103,10 +1145,10 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
 
     if (config_id == MMBO_CONFIG_AUTO) {
         const WaveShape p = wave_shape(dtype, transA, transB, m, n, k, batch, lda, ldb, ldc, f64 ? beta_d != 0.0 : beta_f != 0.0f);
-        if (named_wave) return run_wave(p, *named_wave, a, s, ws_source);
+        if (named_wave) return run_wave(p, *named_wave, a, s, ws_source, 0);
         Route r;
         if (int rc = route_for(p, a.vec_a && a.vec_b, ws_source, r)) return rc;
-        if (r.wave) return run_wave(p, r.pick, a, s, ws_source);
+        if (r.wave) return run_wave(p, r.pick, a, s, ws_source, r.reserve);
         config_id = r.config_id;
     }
     const ConfigRef cref = f64 ? ConfigRef{false, config_id, 1, false} : config_ref(config_id);
@@ -1197,7 +1239,7 @@ int mmbo_auto_info(int dtype, int transA, int transB, size_t m, size_t n, size_t
 {
     if (!config_id || !out) return MMBO_ERR_NULL_POINTER;
     if (int rc = check_problem(dtype, transA, transB, m, n, k, lda, ldb, ldc, batch)) return rc;
-    Route r{false, {}, 0};
+    Route r{false, {}, 0, 0};
     if (m != 0 && n != 0 && batch != 0) {
         const size_t esz = element_size(dtype);
         const bool aligned16 = (lda * esz) % 16 == 0 && (ldb * esz) % 16 == 0;

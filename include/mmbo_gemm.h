@@ -22,7 +22,10 @@
  *     reference uses, src/gemm/common.h:12); the caller synchronises.  Configs with GlobalSplitU > 1 keep their
  *     partial sums in a workspace the library owns, one per (device, stream): GEMMs on different streams never
  *     share one, and calls from several host threads are safe.  A workspace is allocated on the first split-K call
- *     on its stream and grown when a call needs more (this waits for that stream's earlier work);
+ *     on its stream, of 8 MiB or more, and grown when a call needs more (this waits for that stream's earlier work).  Under
+ *     MMBO_CONFIG_AUTO whether a call needs one, and how large a one at most, follows from types, transposes, sizes and batch alone:
+ *     a call of a shape whose pick of mmbo_select_config has GlobalSplitU 1 needs none, and one call of any other shape, with any
+ *     beta and leading dimensions, leaves enough behind for all calls of that shape on its stream (before a stream capture, say);
  *   - config_id selects a row of the tile-config table, like the reference's kernelId
  *     (src/gemm/constants.h:34-47,106-135); MMBO_CONFIG_AUTO lets the library pick: a config of the table, or, for problems
  *     too small to fill the chip with the table's tiles, a kernel without a config id whose wavefronts split k among
@@ -150,8 +153,8 @@ int mmbo_batch_xcd_remap(unsigned linear_id, unsigned tiles, unsigned batch, uns
  * The difference: the partial sums of a config with GlobalSplitU > 1 live in an array that is part
  * of the library's device image (mmbo_static_workspace_bytes() bytes of partial sums, 32 MiB, held by every GPU the
  * library runs on until the process ends) instead of in memory from hipMalloc, and the call makes no hipMalloc, hipFree
- * or other allocating call.  A call whose partial sums (GlobalSplitU x batch x m x n x 4 bytes; mmbo_config_info of
- * mmbo_select_config's pick gives GlobalSplitU) do not fit is refused with MMBO_ERR_WORKSPACE and launches nothing
+ * or other allocating call.  A call whose partial sums (GlobalSplitU x batch x m x n x 4 bytes; mmbo_config_info
+ * gives a config's GlobalSplitU) do not fit is refused with MMBO_ERR_WORKSPACE and launches nothing
  * when the caller named the config; under MMBO_CONFIG_AUTO the picked tile then runs with the largest GlobalSplitU
  * whose partial sums fit (down to none), so every shape runs under MMBO_CONFIG_AUTO here as well;
  * configs without split-K need no workspace and always run.  All calls on one GPU share that GPU's array: two such

@@ -191,6 +191,89 @@ def test_only_calls_whose_pick_splits_k_take_a_workspace():
     G.release_workspace()
 
 
+#            dtype ta tb  m    n      k       whose plans differ with beta or with padded leading dimensions
+REPLANNED = [(F16, 0, 0, 520, 608, 3968), (F32, 0, 1, 128, 10200, 2176), (F32, 0, 0, 32, 4863, 10379), (F16, 0, 0, 192, 2298, 8384),
+             (F32, 0, 1, 1856, 32, 10384), (F32, 1, 0, 32, 5454, 9120), (F16, 0, 1, 64, 48, 40000)]
+
+
+def _variants(ta, tb, m, n, k):
+    """(lda, ldb, beta) of calls of one shape: packed without C first."""
+    a, b = (k if ta else m), (n if tb else k)
+    return [(a, b, 0.0), (a, b, 1.0), (a + 1, b + 1, 0.0), (a + 8, b + 8, 1.0), (-(-a // 64) * 64, -(-b // 64) * 64, 1.0)]
+
+
+def test_whether_k_is_split_over_work_groups_follows_from_the_shape():
+    """No call of a shape whose packed call without C needs no workspace needs one, and none needs more than that call leaves behind (at
+    least 8 MiB where it needs one)."""
+    import random
+
+    import gemm_mmbo_amd as G
+
+    def need(dtype, ta, tb, m, n, k, lda, ldb, beta):
+        info = G.auto_info(dtype, ta, tb, m, n, k, 1, lda, ldb, None, beta != 0.0)
+        return (info["split_k"] * m * n * 4 if info["split_k"] > 1 else 0), info["config_id"]
+    rng, seen = random.Random(4), 0
+    shapes = list(REPLANNED)
+    while len(shapes) < 1500:
+        thin, wide, k = int(2 ** rng.uniform(3, 9)), int(2 ** rng.uniform(3, 13)), int(2 ** rng.uniform(9, 16))
+        shapes.append((rng.choice((F32, F16)), rng.randint(0, 1), rng.randint(0, 1)) + rng.choice(((thin, wide, k), (wide, thin, k))))
+    for shape in shapes:
+        ta, tb, m, n, k = shape[1:]
+        packed, *others = [need(*shape, *v) for v in _variants(ta, tb, m, n, k)]
+        for bytes_needed, _ in others:
+            assert bytes_needed <= (max(packed[0], 8 << 20) if packed[0] else 0), shape
+        # a call that names the pick of mmbo_select_config leaves enough behind as well
+        split = G.config_info(shape[0], G.select_config(*shape))["split_k"]
+        assert packed[0] <= (max(split * m * n * 4, 8 << 20) if split > 1 else 0), shape
+        seen += len({o[0] for o in [packed] + others}) > 1
+    assert seen > 0                                   # (plans do differ between the calls of a shape)
+
+
+@pytest.mark.gpu
+def test_one_call_of_a_shape_leaves_the_workspace_of_all():
+    """Run once, then captured with another beta or other leading dimensions: nothing is allocated, and each replay of the graph gives
+    the bits of the eager call."""
+    import torch
+
+    import gemm_mmbo_amd as G
+    stream = torch.cuda.Stream()
+    for shape in REPLANNED:
+        dtype, ta, tb, m, n, k = shape
+        t = {F32: torch.float32, F16: torch.float16}[dtype]
+        variants = _variants(ta, tb, m, n, k)
+        with torch.cuda.stream(stream):
+            gen = torch.Generator(device="cuda")
+            gen.manual_seed(7)
+            dA = torch.rand(max(v[0] for v in variants) * (m if ta else k), device="cuda", generator=gen).mul_(0.1).to(t)
+            dB = torch.rand(max(v[1] for v in variants) * (k if tb else n), device="cuda", generator=gen).mul_(0.1).to(t)
+            C0 = torch.rand(m * n, device="cuda", generator=gen).to(t)
+            dC = C0.clone()
+
+            def call(lda, ldb, beta):
+                G.gemm(dtype, ta, tb, m, n, k, 1.0, dA, lda, dB, ldb, beta, dC, m, -1, stream)
+            torch.cuda.synchronize()
+            for first in (variants[0], variants[3]):
+                G.release_workspace()
+                call(*first)
+                torch.cuda.synchronize()
+                held = G.workspace_info()
+                for v in variants:
+                    dC.copy_(C0)
+                    call(*v)
+                    torch.cuda.synchronize()
+                    want = dC.clone()
+                    graph = torch.cuda.CUDAGraph()
+                    with torch.cuda.graph(graph, stream=stream):
+                        call(*v)
+                    for _ in range(3):
+                        dC.copy_(C0)
+                        graph.replay()
+                        torch.cuda.synchronize()
+                        assert torch.equal(dC.view(torch.uint8), want.view(torch.uint8)), (shape, v)
+                    assert G.workspace_info() == held, (shape, v)
+    G.release_workspace()
+
+
 @pytest.mark.gpu
 def test_reports_time_the_automatic_pick():
     """The report driver and the benchmark main without a config id run MMBO_CONFIG_AUTO and print what it ran."""
