@@ -825,6 +825,17 @@ WaveShape wave_shape(int dtype, int transA, int transB, size_t m, size_t n, size
     return {dtype, transA, transB, m, n, k, batch, lda, ldb, read_c, read_c && m >= 256 && ldc >= 4 * m};
 }
 
+// us that one slice takes a SIMD: its MFMAs and LDS reads
+double wave_slice_work_us(const WaveShape &p, int tile)
+{
+    const WaveModel &w = kWaveModel[p.dtype];
+    const WaveRow &row = kWaveTiles[tile];
+    const int reads_rc = p.dtype == MMBO_F32 ? 4 : 2;
+    const double reads = row.bm / 16 * (p.transA ? 1 : reads_rc) + row.bn / 16 * (p.transB ? reads_rc : 1);
+    const double clocks = (p.dtype == MMBO_F16 ? 16.0 : 128.0) * (row.bm / 16) * (row.bn / 16);
+    return (clocks / w.mfma_eff + reads * w.clk_per_read) / 2400.0;
+}
+
 double wave_model_us(const WaveShape &p, int tile, int waves, int split)
 {
     const WaveModel &w = kWaveModel[p.dtype];
@@ -845,10 +856,7 @@ double wave_model_us(const WaveShape &p, int tile, int waves, int split)
         return per_column * 64 / esz;
     };
     const double line_bytes = lines(row.bm, p.m, p.transA, p.lda) + lines(row.bn, p.n, !p.transB, p.ldb);
-    const int reads_rc = p.dtype == MMBO_F32 ? 4 : 2;
-    const double reads = row.bm / 16 * (p.transA ? 1 : reads_rc) + row.bn / 16 * (p.transB ? reads_rc : 1);
-    const double clocks = (p.dtype == MMBO_F16 ? 16.0 : 128.0) * (row.bm / 16) * (row.bn / 16);
-    const double work = (clocks / w.mfma_eff + reads * w.clk_per_read) / 2400.0;
+    const double work = wave_slice_work_us(p, tile);
     const size_t per16 = (size_t)(16 / esz);
     const bool tail = p.k % bk != 0 || (!p.transA && p.m % per16 != 0) || (p.transB && p.n % per16 != 0);
     auto round = [&](double on_cu, double on_chip) {
@@ -873,15 +881,18 @@ double wave_model_us(const WaveShape &p, int tile, int waves, int split)
 // may_split: k may also be split over work-groups (GlobalSplitU: a workspace and a second launch).  Only where the pick of
 // mmbo_select_config splits as well: a caller reads from that pick whether a call uses a workspace -- whether two calls of the
 // entry point that allocates nothing may overlap, whether a call needs memory of its own before it can be captured.
-WavePick pick_wave(const WaveShape &p, bool may_split)
+// Only a pick below `limit` microseconds.
+WavePick pick_wave(const WaveShape &p, bool may_split, double limit = 1e300)
 {
-    WavePick best{-1, 0, 0, 0.0};
+    WavePick best{-1, 0, 0, limit};
     const double esz = p.dtype == MMBO_F64 ? 8 : p.dtype == MMBO_F32 ? 4 : 2;
     const size_t slices = ceil_div(p.k, (size_t)(64 / esz));
     if (p.k == 0) return best;
     for (int tile = 0; tile < NUM_WAVE_TILES; ++tile) {
         const size_t tiles = ceil_div(p.m, kWaveTiles[tile].bm) * ceil_div(p.n, kWaveTiles[tile].bn);
         if (tiles > 65535) continue;
+        // (the slices' work alone, spread over all SIMDs, however k is split: most tiles, and most large calls, need no more than this)
+        if ((kWaveModel[p.dtype].launch + (double)slices * tiles * p.batch * wave_slice_work_us(p, tile) / 1024.0) * 0.999999 >= best.us) continue;
         for (int waves : {1, 4, 8}) {
             if (waves > 1 && slices < (size_t)waves) continue;
             if (waves > wave_max_waves(kWaveTiles[tile])) continue;
@@ -891,15 +902,15 @@ WavePick pick_wave(const WaveShape &p, bool may_split)
                 if (split > 1 && (slices < (size_t)split * waves * 2 || tiles * p.batch * split > kMaxSplitWaveGroups))
                     break;
                 const double us = wave_model_us(p, tile, waves, split);
-                if (best.tile < 0 || us < best.us) best = WavePick{tile, waves, split, us};
+                if (us < best.us) best = WavePick{tile, waves, split, us};
             }
         }
     }
     return best;
 }
 
-// What the automatic pick runs for a shape.  The models are walked once per shape and thread (some microseconds, as much as a
-// small call takes); a small direct-mapped table keeps the answers, which are a function of the key alone.
+// What the automatic pick runs for a shape.  The models are walked once per shape and thread (a microsecond or two, a part of what a
+// small call takes); a small table of four ways keeps the answers, which are a function of the key alone.
 // Whether a call needs a workspace, and how large a one at most, follows from the shape alone, not from beta or leading dimensions:
 // a program runs a shape once and then captures a call of that shape that may differ in those, which cannot allocate.  So a
 // shape whose pick of mmbo_select_config splits k is first planned with packed operands and without C.  Where that plan needs no
@@ -910,6 +921,8 @@ struct Plan {
     bool workspace;     // may partial sums go through memory?
     size_t reserve;     // bytes of workspace that a call sees to although it may need less itself
 };
+
+thread_local size_t g_plans_made = 0;
 
 Plan plan_for(const WaveShape &p)
 {
@@ -922,8 +935,12 @@ Plan plan_for(const WaveShape &p)
         Key key;
         Plan plan;
     };
-    constexpr int kEntries = 64;
-    static thread_local Entry cache[kEntries];
+    constexpr int kSets = 32, kWays = 4;
+    struct Set {
+        Entry way[kWays];
+        unsigned next;              // the way that goes next: the oldest
+    };
+    static thread_local Set cache[kSets];
     const size_t per_line = 128 / (p.dtype == MMBO_F64 ? 8 : p.dtype == MMBO_F32 ? 4 : 2);
     Key key;
     std::memset(&key, 0, sizeof(key));                   // (compared as bytes)
@@ -932,8 +949,10 @@ Plan plan_for(const WaveShape &p)
     key.m = p.m; key.n = p.n; key.k = p.k;
     size_t h = p.m * 0x9E3779B97F4A7C15ull ^ p.n * 0xC2B2AE3D27D4EB4Full ^ p.k * 0x165667B19E3779F9ull ^
                (size_t)(p.batch * 16 + p.dtype * 4 + p.transA * 2 + p.transB) * 0x27D4EB2F165667C5ull;
-    Entry &e = cache[(h >> 32) % kEntries];
-    if (e.used && std::memcmp(&e.key, &key, sizeof(key)) == 0) return e.plan;
+    Set &set = cache[(h >> 32) % kSets];
+    for (const Entry &e : set.way)
+        if (e.used && std::memcmp(&e.key, &key, sizeof(key)) == 0) return e.plan;
+    ++g_plans_made;
     Plan plan;
     double table_us;
     plan.config_id = select_config(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, &table_us);
@@ -946,11 +965,9 @@ Plan plan_for(const WaveShape &p)
     // shapes, 2.1 - 3.0), which matters only here: by 2.0 us, as this kernel takes 0.6 less on its smallest calls and 5 % less on the others.  us
     // here / there: fp16 TT 1024 x 640 x 512 6.4 / 5.1, TT 4 x 576 x 320 x 512 8.4 / 5.7, TN 768 x 128 x 640 4.4 / 5.5, fp32 NN 448 x 768 x 304 7.0 / 8.1.
     auto choose = [&](const WaveShape &q, bool may_split) {
-        WavePick w = pick_wave(q, may_split);
         double bar = (q.wide_c ? 0.83 : 0.92) * table_us;
         if (q.dtype != MMBO_F64 && plan.config_id == ring_config_id(3, 0)) bar = std::min(bar, table_us - 2.0);
-        if (w.us >= bar) w.tile = -1;
-        return w;
+        return pick_wave(q, may_split, bar);             // (none at `bar` or beyond)
     };
     plan.workspace = false;
     plan.reserve = 0;
@@ -969,9 +986,8 @@ Plan plan_for(const WaveShape &p)
             plan.reserve = packed.tile < 0 ? (size_t)std::min(table_bytes, 1e18) : kWaveSumsBytes;
         }
     }
-    e.used = true;
-    e.key = key;
-    e.plan = plan;
+    set.way[set.next] = Entry{true, key, plan};
+    set.next = (set.next + 1) % kWays;
     return plan;
 }
 
@@ -1264,6 +1280,9 @@ int mmbo_auto_info(int dtype, int transA, int transB, size_t m, size_t n, size_t
     *config_id = MMBO_CONFIG_AUTO;
     return MMBO_OK;
 }
+
+// Not part of the interface: how often this thread has walked the models for the automatic pick.
+size_t mmbo_internal_plans_made(void) { return g_plans_made; }
 
 // Not part of the interface: mmbo_gemm_strided_batched on a given row of kWaveTiles, with given wavefronts per work-group and
 // GlobalSplitU, whatever the pick is -- the tests reach every instantiation of the kernel through it.

@@ -324,3 +324,19 @@ def test_pick_between_the_table_and_the_kernel_without_a_config_id_where_measure
     assert auto(G.F32, 0, 1, 64, 489, 4640, ldc=44160, reads_c=True) == G.CONFIG_AUTO
     assert auto(G.F16, 1, 1, 2, 6144, 4792, lda=4856, ldb=6208, ldc=66, reads_c=True) == G.CONFIG_AUTO
     assert auto(G.F16, 0, 1, 512, 797, 96, lda=520, ldb=805, ldc=44160) == G.CONFIG_AUTO
+
+
+def test_shapes_in_turn_are_planned_once():
+    """A program that goes round a few dozen shapes, or calls one with and without C, does not pay for a plan on each call."""
+    made = G.lib().mmbo_internal_plans_made
+    made.restype = ctypes.c_size_t
+    shapes = [(dtype, ta, 0, m, n, 40 + 8 * m) for dtype in (G.F32, G.F16, G.F64) for ta in (0, 1) for m, n in ((17, 90), (64, 64), (300, 35), (130, 1000))]
+    for reads_c in (False, True):
+        for s in shapes:
+            G.auto_info(*s, reads_c=reads_c)
+    before = made()
+    for _ in range(3):
+        for s in shapes:
+            for reads_c in (False, True):
+                G.auto_info(*s, reads_c=reads_c)
+    assert made() - before <= 12                 # (of 144: a set of the table may hold more shapes than it has ways)
