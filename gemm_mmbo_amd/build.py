@@ -19,7 +19,7 @@ NUM_TILES = 6  # keep in step with csrc/configs.hpp
 NUM_RING_TILES = 4
 NUM_F64_TILES = 6
 NUM_X16_TILES = 8
-NUM_WAVE_TILES = 8
+NUM_WAVE_TILES = {0: 8, 1: 8, 2: 6}  # by element type (fp32, fp16, fp64)
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -73,7 +73,7 @@ def _units():
         for tile in range(NUM_X16_TILES):
             units.append(("inst_x16.hip", f"inst_x16_{dtype}_{tile}.o", [f"-DMMBO_DTYPE={dtype}", f"-DMMBO_TILE={tile}"]))
     for dtype in (0, 1, 2):
-        for tile in range(NUM_WAVE_TILES):
+        for tile in range(NUM_WAVE_TILES[dtype]):
             units.append(("inst_wave.hip", f"inst_wave_{dtype}_{tile}.o", [f"-DMMBO_DTYPE={dtype}", f"-DMMBO_TILE={tile}"]))
     for tile in range(NUM_F64_TILES):
         units.append(("inst_dgemm.hip", f"inst_dgemm_{tile}.o", [f"-DMMBO_TILE={tile}"]))

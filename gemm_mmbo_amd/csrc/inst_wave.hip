@@ -14,6 +14,7 @@ namespace mmbo {
 
 namespace {
 using ElemT = typename std::conditional<MMBO_DTYPE == 0, float, typename std::conditional<MMBO_DTYPE == 1, half_t, double>::type>::type;
+static_assert(MMBO_TILE < wave_tiles(MMBO_DTYPE), "a tile this type has");
 constexpr WaveRow R = kWaveTiles[MMBO_TILE];
 constexpr int kMaxWaves = wave_max_waves(R);
 

@@ -286,7 +286,7 @@ template <int DTYPE, int TILE>
 hipError_t dispatch_wave(int tile, int ta, int tb, const GemmArgs &a, int waves, hipStream_t s)
 {
     if (tile == TILE) return launch_wave<DTYPE, TILE>(ta, tb, a, waves, s);
-    if constexpr (TILE + 1 < NUM_WAVE_TILES) return dispatch_wave<DTYPE, TILE + 1>(tile, ta, tb, a, waves, s);
+    if constexpr (TILE + 1 < wave_tiles(DTYPE)) return dispatch_wave<DTYPE, TILE + 1>(tile, ta, tb, a, waves, s);
     return hipErrorInvalidValue;
 }
 
@@ -888,7 +888,7 @@ WavePick pick_wave(const WaveShape &p, bool may_split, double limit = 1e300)
     const double esz = p.dtype == MMBO_F64 ? 8 : p.dtype == MMBO_F32 ? 4 : 2;
     const size_t slices = ceil_div(p.k, (size_t)(64 / esz));
     if (p.k == 0) return best;
-    for (int tile = 0; tile < NUM_WAVE_TILES; ++tile) {
+    for (int tile = 0; tile < wave_tiles(p.dtype); ++tile) {
         const size_t tiles = ceil_div(p.m, kWaveTiles[tile].bm) * ceil_div(p.n, kWaveTiles[tile].bn);
         if (tiles > 65535) continue;
         // (the slices' work alone, spread over all SIMDs, however k is split: most tiles, and most large calls, need no more than this)
@@ -1214,7 +1214,7 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
 
     if (cref.ring && !cref.x16 && (!a.vec_a || !a.vec_b)) return MMBO_ERR_INVALID_CONFIG;
     // Split-K: the partial sums go to the stream's own workspace (or the static one), and both launches that use it (the
-    // GEMM and the reduction, which adds the splits in ascending order) are queued before the hold on that workspace
+    // GEMM and the reduction, which adds the splits in a fixed order) are queued before the hold on that workspace
     // is given up.
     WsHold ws_hold;
     if (split > 1) {
@@ -1291,7 +1291,8 @@ int mmbo_internal_wave_gemm(int dtype, int transA, int transB, size_t m, size_t 
                             const void *B, size_t ldb, long long strideB, const void *beta, void *C,
                             size_t ldc, long long strideC, int batch, int tile, int waves, int split, void *stream)
 {
-    if (tile < 0 || tile >= NUM_WAVE_TILES || (waves != 1 && waves != 4 && waves != 8) || waves > wave_max_waves(kWaveTiles[tile]) || split < 1 ||
+    if (!valid_dtype(dtype)) return MMBO_ERR_INVALID_DTYPE;
+    if (tile < 0 || tile >= wave_tiles(dtype) || (waves != 1 && waves != 4 && waves != 8) || waves > wave_max_waves(kWaveTiles[tile]) || split < 1 ||
         split > 64 || (dtype == MMBO_F64 && split > 1))
         return MMBO_ERR_INVALID_CONFIG;
     if (int rc = check_problem(dtype, transA, transB, m, n, k, lda, ldb, ldc, batch)) return rc;
