@@ -44,7 +44,7 @@ import time
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PEAK_TFLOPS = {"h": 2500.0, "s": 157.3, "d": 78.6}
 ESZ = {"h": 2, "s": 4, "d": 8}
-LIB_KERNEL = re.compile(r"mmbo(::|\d+)?.*(gemm_x16_kernel|gemm_ring_kernel|gemm_staged_kernel|dgemm_kernel|splitk_reduce_kernel)")
+LIB_KERNEL = re.compile(r"mmbo(::|\d+)?.*(gemm_x16_kernel|gemm_ring_kernel|gemm_staged_kernel|gemm_wave_kernel|dgemm_kernel|splitk_reduce_kernel)")
 LONG_KERNEL_NS = 200e3          # below this GRBM_GUI_ACTIVE is not a clock measurement
 
 SQ_COUNTERS = ["SQ_VALU_MFMA_BUSY_CYCLES", "SQ_BUSY_CYCLES", "SQ_WAVE_CYCLES", "SQ_INSTS_VALU_MFMA_MOPS_F16",
@@ -63,6 +63,8 @@ SKINNY = ["h,N,N,4096,128,4096", "s,N,N,4096,128,4096", "h,N,N,128,4096,8192", "
 CONFIGS = ["s,N,N,1024,1024,1024", "s,N,T,4096,4096,4096,1,1.5,0.5", "s,T,N,4096,4096,4096,1,1.5,0.5",
            "h,T,N,512,512,512,64,1,1", "d,N,T,44160,2048,384,1,-1,1,44160"]
 MIDSIZE = ["h,N,N,2048,2048,2048", "h,N,N,3000,3000,3000", "h,N,N,4096,4096,4096"]
+SMALL_THIN = ["h,N,N,16,4096,4096", "s,N,N,96,72,150,5", "d,N,N,64,489,4640", "h,N,T,32,59,55680"]
+FP64_UPDATES = ["d,N,T,2304,2048,384,1,-1,1,44160", "d,N,T,1152,2048,384,1,-1,1,44160", "d,N,T,1121,1088,1692"]
 
 CASES = {
     "gemm_x16_f16_8192": {
@@ -81,6 +83,14 @@ CASES = {
         "title": "Benchmark configurations 1, 2, 5 and the reference's fp64 HPL shape (src/gemm/run.sh:2-5), automatic pick",
         "program": ["-m", "gemm_mmbo_amd.report", "shapes"] + CONFIGS + ["--no-check", "--reps", "10", "--ceilings"],
         "passes": ["trace", "sq"], "specs": CONFIGS},
+    "small_thin": {
+        "title": "Small, thin and long-k GEMMs that the split-by-wavefront kernel takes, automatic pick",
+        "program": ["-m", "gemm_mmbo_amd.report", "shapes"] + SMALL_THIN + ["--no-check", "--reps", "10"],
+        "passes": ["trace", "sq", "fetch", "write"], "specs": SMALL_THIN},
+    "fp64_updates": {
+        "title": "fp64 grids that are no whole number of rounds of 64x64 tiles: two updates of a large C, and odd edges, automatic pick",
+        "program": ["-m", "gemm_mmbo_amd.report", "shapes"] + FP64_UPDATES + ["--no-check", "--reps", "10", "--ceilings"],
+        "passes": ["trace", "sq", "fetch", "write"], "specs": FP64_UPDATES},
     "midsize_fp16": {
         "title": "HGEMM NN at sizes whose tile counts do not fill a whole number of rounds of 256 CUs, automatic pick",
         "program": ["-m", "gemm_mmbo_amd.report", "shapes"] + MIDSIZE + ["--no-check", "--reps", "10", "--ceilings"],

@@ -101,3 +101,16 @@ def test_command_line_front_end_and_fixture_generator(tmp_path):
     assert subprocess.run([sys.executable, str(tmp_path / "gen.py")], capture_output=True).returncode == 0
     for path, data in before.items():
         assert open(os.path.join(str(tmp_path / "regen"), os.path.relpath(path, FIX)), "rb").read() == data, path
+
+
+def test_every_kernel_of_the_library_counts_as_one_of_its_own():
+    """The summaries cut a trace by call: a kernel the pattern does not know would shift all that follow."""
+    csrc = os.path.join(ROOT, "gemm_mmbo_amd", "csrc")
+    kernels = set()
+    for f in os.listdir(csrc):
+        if f.endswith((".hpp", ".hip")) and f != "probe.hip":
+            kernels.update(re.findall(r"__global__[^;{]*?\b(\w+_kernel)\(const GemmArgs", open(os.path.join(csrc, f)).read(), flags=re.S))
+    assert len(kernels) >= 6
+    for k in kernels:
+        assert P.LIB_KERNEL.search(f"void mmbo::{k}<float, false, false>(mmbo::GemmArgs)"), k
+        assert P.LIB_KERNEL.search(f"_ZN4mmbo{len(k)}{k}IDF16_Lb0EEEvNS_8GemmArgsE"), k
