@@ -164,8 +164,8 @@ __device__ inline void dgemm_tile(const GemmArgs &args, uint32_t row0, uint32_t 
     // padding row, the next column -- and its products, as those of the repeated rows, are never stored.  Only the operand's last
     // column has nothing behind it: of a tile with such an end the last stage goes element by element.
     // Against the predicated loader for every edge tile and for all tiles of operands with a column off 16 bytes, us (64 x 64
-    // tiles): TT 2542 x 644 x 896 86 -> 60, TT 4041 x 1524 x 110 51 -> 38, TN 5397 x 610 x 643 114 -> 91, NN 4046 x 566 x 426 50 -> 41.
-    // With odd edges on the predicated loader, their work-groups ran on long after the others: NT 1121 x 1088 x 1692 142 -> 86 us; with
+    // tiles): TT 2542 x 644 x 896 86 -> 61, TT 4041 x 1524 x 110 51 -> 37, TN 5397 x 610 x 643 114 -> 91, NN 4046 x 566 x 426 50 -> 41.
+    // With odd edges on the predicated loader, their work-groups ran on long after the others: NT 1121 x 1088 x 1692 142 -> 81 us; with
     // a correction of their last pairs inside the stage loop, every tile's LDS stores waited behind the last MFMA: NT 1152 x 2048 x 384
     // with C read 40.1 -> 38.6 us without it, NT 44160 x 2048 x 384 1,186 -> 1,154.
     const uint32_t odd_end = ((TA ? 0u : (uint32_t)rows_a) | (TB ? (uint32_t)rows_b : 0u)) & 1u;
