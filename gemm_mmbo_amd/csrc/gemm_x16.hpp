@@ -836,12 +836,12 @@ gemm_x16_kernel(const GemmArgs args)
     // when beta != 0 (reference: src/gemm/ref/Kernels.cpp:87); with GlobalSplitU > 1 the raw sums go to the fp32
     // workspace [split][batch][n][m] and the reduction kernel applies alpha and beta.
     const uint32_t wrow0 = row0 + wm * Cfg::TM + 4 * (lane >> 4), wcol0 = col0 + wn * Cfg::TN + (lane & 15);
-    if (m_here < (uint32_t)BM || n_here < (uint32_t)BN) {
+    const bool edge = m_here < (uint32_t)BM || n_here < (uint32_t)BN;
+    if (edge || (args.splits == 1 && !args.c_narrow)) {
         // Edge tile (reference: the un-shift and the guarded store, src/gemm/ref/Kernels.cpp:1007-1121).  Tile row r is
         // row r of C, except in the last 16-byte group of a row-contiguous A (Tile::rc_group_off): there tile rows
         // gsm+shm .. gsm+EPC-1 are rows gsm .. m_here-1, and tile rows gsm .. gsm+shm-1 repeat rows that the group
-        // before already produced.  Columns likewise under a row-contiguous B.  Every element is tested against the
-        // tile's extent; four rows go out as one vector where all four exist unshifted and C allows it.
+        // before already produced.  Columns likewise under a row-contiguous B.
         // (a k-contiguous operand has no shift: gs = the extent, sh = 0, and the tests below reduce to r < extent)
         // The extents and the lane number pass through an empty asm: everything below is derived from them here, after
         // the slice loop.  Otherwise the compiler computes the per-block tests up front and, with the register file full
@@ -850,54 +850,137 @@ gemm_x16_kernel(const GemmArgs args)
         asm volatile("" : "+s"(e_m), "+s"(e_n), "+v"(e_lane));
         const uint32_t gsm = TA ? e_m : (e_m - 1) / EPC * EPC, shm = TA ? 0u : gsm + EPC - e_m;
         const uint32_t gsn = !TB ? e_n : (e_n - 1) / EPC * EPC, shn = !TB ? 0u : gsn + EPC - e_n;
-        const uint32_t vec_rows = shm == 0 ? e_m : gsm;                     // tile rows below this are in place
         const float alpha = args.alpha, beta = args.beta;
         const bool to_ws = args.splits > 1;
-        float *ws = args.ws + ((size_t)split * args.batch + batch) * (size_t)args.m * args.n;
         T *C = static_cast<T *>(args.C) + (int64_t)batch * args.strideC;
-        const bool vec_c = args.vec_c != 0;
-        typedef typename std::conditional<ESZ == 2, u32x2, u32x4>::type cvec;
-        const uint32_t lrow0 = wm * Cfg::TM + 4 * (e_lane >> 4), lcol0 = wn * Cfg::TN + (e_lane & 15);
-        static_for<FM * FN>([&](auto IJ) {
-            constexpr int j = decltype(IJ)::value / FM, i = decltype(IJ)::value % FM, base = (i * FN + j) * 4;
-            const uint32_t lr = lrow0 + i * 16, lc = lcol0 + j * 16;
-            float v[4] = {acc_read<base>(), acc_read<base + 1>(), acc_read<base + 2>(), acc_read<base + 3>()};
-            // the column of C this lane's tile column stands for, if any
-            const bool col_ok = lc < gsn || (lc >= gsn + shn && lc - shn < e_n);
-            const uint32_t col = col0 + (lc < gsn ? lc : lc - shn);
-            if (col_ok) {
-                if (!to_ws && vec_c && lr + 3 < vec_rows) {
-                    T *p = C + (size_t)col * args.ldc + row0 + lr;
-                    union { T e[4]; cvec v; } io;
-                    if (beta != 0.0f) {
-                        io.v = *reinterpret_cast<const cvec *>(p);
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) io.e[r] = (T)__builtin_fmaf(beta, (float)io.e[r], alpha * v[r]);
+        const uint32_t lcol0 = wn * Cfg::TN + (e_lane & 15);
+        // the column of C a lane's tile column stands for, relative to the tile's first, if any
+        auto column_exists = [&](uint32_t lc) { return lc < gsn || (lc >= gsn + shn && lc - shn < e_n); };
+        auto column = [&](uint32_t lc) { return lc < gsn ? lc : lc - shn; };
+        if (to_ws || !args.c_narrow) {
+            // Partial sums, or a C whose tiles span more than the 32-bit offsets of a buffer access: four rows of sums as one
+            // vector where all four exist unshifted, everything else element by element.
+            const uint32_t vec_rows = shm == 0 ? e_m : gsm, lrow0 = wm * Cfg::TM + 4 * (e_lane >> 4);
+            float *ws = args.ws + ((size_t)split * args.batch + batch) * (size_t)args.m * args.n;
+            static_for<FM * FN>([&](auto IJ) {
+                constexpr int j = decltype(IJ)::value / FM, i = decltype(IJ)::value % FM, base = (i * FN + j) * 4;
+                const uint32_t lr = lrow0 + i * 16, lc = lcol0 + j * 16;
+                const f32x4 v = {acc_read<base>(), acc_read<base + 1>(), acc_read<base + 2>(), acc_read<base + 3>()};
+                if (column_exists(lc)) {
+                    const uint32_t col = col0 + column(lc);
+                    if (to_ws && lr + 3 < vec_rows) {
+                        __builtin_memcpy(ws + (size_t)col * args.m + row0 + lr, &v, sizeof(v));       // (dword-aligned)
                     } else {
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) io.e[r] = (T)(alpha * v[r]);
-                    }
-                    *reinterpret_cast<cvec *>(p) = io.v;
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const uint32_t tr = lr + r;
-                        const bool row_ok = tr < gsm || (tr >= gsm + shm && tr - shm < e_m);
-                        const uint32_t row = row0 + (tr < gsm ? tr : tr - shm);
-                        if (row_ok) {
-                            if (to_ws) {
-                                ws[(size_t)col * args.m + row] = v[r];
-                            } else {
-                                T *p = C + (size_t)col * args.ldc + row;
-                                float o = alpha * v[r];
-                                if (beta != 0.0f) o = __builtin_fmaf(beta, (float)*p, o);
-                                *p = (T)o;
+                        for (int r = 0; r < 4; ++r) {
+                            const uint32_t tr = lr + r;
+                            const bool row_ok = tr < gsm || (tr >= gsm + shm && tr - shm < e_m);
+                            const uint32_t row = row0 + (tr < gsm ? tr : tr - shm);
+                            if (row_ok) {
+                                if (to_ws) {
+                                    ws[(size_t)col * args.m + row] = v[r];
+                                } else {
+                                    T *p = C + (size_t)col * args.ldc + row;
+                                    float o = alpha * v[r];
+                                    if (beta != 0.0f) o = __builtin_fmaf(beta, (float)*p, o);
+                                    *p = (T)o;
+                                }
                             }
                         }
                     }
                 }
+                __builtin_amdgcn_sched_barrier(0);          // one block at a time: keeps the address arithmetic of 64 blocks from piling up
+            });
+            continue;
+        }
+        // A lane stores 16 bytes per unit: four rows of one block (fp32) or, of two vertically adjacent blocks that have been
+        // through the lane exchange described below, eight rows (fp16).  Either way these are exactly one 16-byte group
+        // of rows of the operand, so a lane's rows are all in place, or they are the one group that the edge cuts, or there
+        // are none.  The cut group's rows go one by one (the rows it repeats are another lane's to update).  Bound by the round
+        // trip of the old C, which is therefore requested for the whole wave tile (fp32: for up to 16 blocks) before the first value
+        // of it is used, and by the number of store requests.  Block after block with a round trip each, four rows
+        // to a store, fp16 beta = 1, us: 19101 x 723 x 186 91.4 -> 38.7, 640 x 1308 x 640 12.0 -> 9.1; beta = 0 1170 x 1152 x 523 11.6 -> 10.8.
+        // Plain stores, as the columns of such a C rarely start on 16-byte boundaries (device scope 47.6 and 8.8).
+        constexpr bool PAIRS = ESZ == 2;
+        static_assert(!PAIRS || FM % 2 == 0, "fp16 blocks go out in vertical pairs");
+        constexpr int FR = PAIRS ? FM / 2 : FM, UNIT_ROWS = PAIRS ? 32 : 16;          // units down a wave tile, rows of each
+        const uint32_t g4 = e_lane >> 4;
+        const uint32_t lrow0 = wm * Cfg::TM + (PAIRS && (g4 & 1) ? 4 * g4 + 12 : 4 * g4);
+        const uint32_t whole_end = e_m / EPC * EPC, cut = e_m % EPC;                // rows in whole groups, rows of the cut one
+        const uint32_t e_first = TA ? 0u : EPC - cut, e_end = TA ? cut : EPC;        // which of the cut group's elements exist
+        const __amdgpu_buffer_rsrc_t tile_c = __builtin_amdgcn_make_buffer_rsrc(
+            reinterpret_cast<void *>(uniform_address(C + (size_t)col0 * args.ldc + row0)), 0, 0x7fffffff, 0x00020000);
+        // the cut group's first element (under a shift it lies before the group's place, and with less than one group of rows
+        // before the tile: as a pointer, since a buffer's offsets do not reach back)
+        T *const cut_c = C + (size_t)col0 * args.ldc + row0 + whole_end - (TA ? 0u : EPC - cut);
+        union group_t { T e[EPC]; u32x4 v; };
+        // (fp16: at most 32 units, 128 registers; fp32: up to 16 at a time)
+        constexpr int UNITS = FR * FN, COLS = PAIRS ? FN : (FN % 4 == 0 && 4 * FR <= 16) ? 4 : (FN % 2 == 0 && 2 * FR <= 16) ? 2 : 1, CHUNK = COLS * FR;
+        const bool read_c = beta != 0.0f;
+        static_for<UNITS / CHUNK>([&](auto CC) {
+        group_t old_c[CHUNK];
+        if (read_c) {
+            static_for<CHUNK>([&](auto Q) {
+                constexpr int q = decltype(Q)::value, u = decltype(CC)::value * CHUNK + q, j = u / FR, i = u % FR;
+                const uint32_t lr = lrow0 + i * UNIT_ROWS, lc = lcol0 + j * 16;
+                old_c[q].v = u32x4{0u, 0u, 0u, 0u};
+                if (column_exists(lc)) {
+                    if (lr + EPC <= whole_end) {
+                        old_c[q].v = __builtin_amdgcn_raw_buffer_load_b128(tile_c, (column(lc) * args.ldc + lr) * ESZ, 0, 0);
+                    } else if (lr == whole_end && cut != 0) {
+                        const T *p = cut_c + (size_t)column(lc) * args.ldc;
+#pragma unroll
+                        for (uint32_t e = 0; e < EPC; ++e)
+                            if (e >= e_first && e < e_end) old_c[q].e[e] = p[e];
+                    }
+                }
+            });
+        }
+        static_for<CHUNK>([&](auto Q) {
+            constexpr int q = decltype(Q)::value, u = decltype(CC)::value * CHUNK + q, j = u / FR, i = u % FR;
+            const uint32_t lr = lrow0 + i * UNIT_ROWS, lc = lcol0 + j * 16;
+            group_t out;
+            if constexpr (PAIRS) {
+                constexpr int b0 = (2 * i * FN + j) * 4, b1 = ((2 * i + 1) * FN + j) * 4;
+                float x[4] = {alpha * acc_read<b0>(), alpha * acc_read<b0 + 1>(), alpha * acc_read<b0 + 2>(), alpha * acc_read<b0 + 3>()};
+                float y[4] = {alpha * acc_read<b1>(), alpha * acc_read<b1 + 1>(), alpha * acc_read<b1 + 2>(), alpha * acc_read<b1 + 3>()};
+                if (read_c) {
+                    const u32x4 c = old_c[q].v;
+                    auto o0 = __builtin_amdgcn_permlane16_swap(c[0], c[2], false, false);
+                    auto o1 = __builtin_amdgcn_permlane16_swap(c[1], c[3], false, false);
+                    union { T e[4]; uint32_t u[2]; } xo, yo;
+                    xo.u[0] = o0[0]; xo.u[1] = o1[0];
+                    yo.u[0] = o0[1]; yo.u[1] = o1[1];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        x[r] = __builtin_fmaf(beta, (float)xo.e[r], x[r]);
+                        y[r] = __builtin_fmaf(beta, (float)yo.e[r], y[r]);
+                    }
+                }
+                union { T e[4]; uint32_t u[2]; } xs, ys;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) { xs.e[r] = (T)x[r]; ys.e[r] = (T)y[r]; }
+                auto s0 = __builtin_amdgcn_permlane16_swap(xs.u[0], ys.u[0], false, false);
+                auto s1 = __builtin_amdgcn_permlane16_swap(xs.u[1], ys.u[1], false, false);
+                out.v = u32x4{(uint32_t)s0[0], (uint32_t)s1[0], (uint32_t)s0[1], (uint32_t)s1[1]};
+            } else {
+                constexpr int base = (i * FN + j) * 4;
+                float v[4] = {alpha * acc_read<base>(), alpha * acc_read<base + 1>(), alpha * acc_read<base + 2>(), alpha * acc_read<base + 3>()};
+#pragma unroll
+                for (int r = 0; r < 4; ++r) out.e[r] = read_c ? (T)__builtin_fmaf(beta, (float)old_c[q].e[r], v[r]) : (T)v[r];
             }
-            __builtin_amdgcn_sched_barrier(0);          // one block at a time: keeps the address arithmetic of 64 blocks from piling up
+            if (column_exists(lc)) {
+                if (lr + EPC <= whole_end) {
+                    __builtin_amdgcn_raw_buffer_store_b128(out.v, tile_c, (column(lc) * args.ldc + lr) * ESZ, 0, 0);
+                } else if (lr == whole_end && cut != 0) {
+                    T *p = cut_c + (size_t)column(lc) * args.ldc;
+#pragma unroll
+                    for (uint32_t e = 0; e < EPC; ++e)
+                        if (e >= e_first && e < e_end) p[e] = out.e[e];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);              // one unit at a time: keeps the address arithmetic of all of them from piling up
+        });
         });
         continue;
     }
@@ -935,8 +1018,10 @@ gemm_x16_kernel(const GemmArgs args)
     const float alpha = args.alpha, beta = args.beta;
     const uint32_t ldc = args.ldc;
     T *C = static_cast<T *>(args.C) + (int64_t)batch * args.strideC;
-    const bool vec_c = args.vec_c != 0;
-    typedef typename std::conditional<ESZ == 2, u32x2, u32x4>::type cvec;       // four consecutive rows of one column
+    // (the columns of C may start anywhere: the vector types promise no more than an element's alignment, which is all the hardware's
+    // accesses need.  Element by element, 2188 x 2672 x 2112 fp16 TN beta = 1 took 66.9 us, now 37.2)
+    typedef typename std::conditional<ESZ == 2, u32x2, u32x4>::type cvec __attribute__((aligned(2)));       // four consecutive rows of one column
+    typedef u32x4 __attribute__((aligned(2))) pair_vec;
     // fp16: a lane's four rows are 8 bytes, a column of one block 32 bytes -- a quarter of a cache line per request.  Two
     // vertically adjacent blocks therefore travel together: v_permlane16_swap hands the lanes of the even 16-lane rows their
     // lower neighbour's four rows of the upper block and the odd rows their upper neighbour's of the lower block, so every
@@ -945,15 +1030,15 @@ gemm_x16_kernel(const GemmArgs args)
     // Two results at a time go through the packed conversion (round to nearest even, like the scalar cast).
     constexpr bool PAIRED_C = ESZ == 2 && FM % 2 == 0;
     const uint32_t pair_row0 = row0 + wm * Cfg::TM + (((lane >> 4) & 1) ? 4 * (lane >> 4) + 12 : 4 * (lane >> 4));
-    // The whole-tile store sequences below address C as a buffer whose origin is the tile's first element (the host lets
-    // vec_c stand only where a tile's span of C, BN x ldc elements, fits the 32-bit offsets of a buffer access): the lane's
+    // The whole-tile store sequences below address C as a buffer whose origin is the tile's first element (args.c_narrow:
+    // a tile's span of C, BN x ldc elements, fits the 32-bit offsets of a buffer access): the lane's
     // part of an address is worked out once, a block adds its column (one vector addition per block column) and, as an
     // immediate, its row.  (The column as the instruction's scalar offset would save that addition, but the compiler then
     // leaves out the wait states between a 16-byte store and the next write to its data registers -- it takes them to be
     // needed only without a scalar offset -- and with the accumulator reads of the next block right behind the store
     // a few lanes stored the next block's value: seen on the 8-wave fp32 tile.)
-    // Two cache policies, one copy of each store sequence per policy, chosen once:
-    // * device scope (sc1) by default: the stores go through the XCD's L2 to memory as they are made.  Left in the L2 as
+    // Three cache policies, one copy of each store sequence per policy, chosen once:
+    // * device scope (sc1) where the columns of C start on 16-byte boundaries: the stores go through the XCD's L2 to memory as they are made.  Left in the L2 as
     //   ordinary stores are, C is written back when the kernel ends, and where the epilogue is on the critical path (one
     //   round of tiles, short k) that is time added at the end: 64 x 512^3 fp16 26.6 -> 25.7 us, 2048^3 21.6 -> 20.9;
     // * non-temporal where the host asks for it (args.c_stream: a long slice loop and four or more rounds of tiles per CU):
@@ -962,7 +1047,9 @@ gemm_x16_kernel(const GemmArgs args)
     //   the epilogue itself takes 1 us longer, the next tile's loop 3-6 us less).  Not everywhere: with this hint the two
     //   64-byte halves of a line travel to memory separately (64 x 512^3 fp16: 7.4 us to issue a wavefront's 32 stores
     //   against 3.5).
-    const bool c_stream = args.c_stream != 0;
+    // * plain where they do not: pieces that start inside a 16-byte group share memory lines with their neighbours, which an L2
+    //   that keeps them merges (fp16 beta = 1, both policies with the same vectors, us: NT 13020 x 1557 x 128 48.4 -> 36.0, TN 2188 x 2672 x
+    //   2112 43.1 -> 37.2; 16-byte aligned columns are the other way round: NT 7424 x 1536 x 358 sc1 20.4, plain 22.0).
     const T *c_origin = C + (size_t)col0 * ldc + row0;
     // (the descriptor is put together inside each copy, from an address that has just passed through readfirstlane: built once
     // up here it reached some of the copies in vector registers, and every store became a loop over the distinct descriptors)
@@ -974,20 +1061,21 @@ gemm_x16_kernel(const GemmArgs args)
     const uint32_t c_lane = ((wn * Cfg::TN + (lane & 15)) * ldc + wm * Cfg::TM + 4 * (lane >> 4)) * ESZ;
     const uint32_t c_lane_pair = ((wn * Cfg::TN + (lane & 15)) * ldc + (pair_row0 - row0)) * ESZ;
     auto store_c = [](auto STREAM, auto value, __amdgpu_buffer_rsrc_t tile_c, uint32_t lane_and_row, uint32_t column) {
-        constexpr int policy = decltype(STREAM)::value ? 2 : 16;            // nt : sc1
+        constexpr int policy = decltype(STREAM)::value;
         if constexpr (sizeof(value) == 16) __builtin_amdgcn_raw_buffer_store_b128(value, tile_c, lane_and_row, column, policy);
         else __builtin_amdgcn_raw_buffer_store_b64(value, tile_c, lane_and_row, column, policy);
     };
     auto per_policy = [&](auto &&body) {
-        if (c_stream) body(std::true_type{});
-        else body(std::false_type{});
+        if (args.c_stream) body(std::integral_constant<int, 2>{});                  // nt
+        else if (args.vec_c) body(std::integral_constant<int, 16>{});                // sc1
+        else body(std::integral_constant<int, 0>{});                                 // plain
     };
     auto two = [](float a, float b) -> uint32_t {
         typedef float f32x2 __attribute__((ext_vector_type(2)));
         typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
         return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), f16x2));
     };
-    if (vec_c && beta != 0.0f) {
+    if (beta != 0.0f) {
         if constexpr (PAIRED_C) {
             // the whole wave tile of old C is requested before its first value is used (see below) -- or was requested
             // under the last four slices and is waiting in the ring buffers those slices left (c_ahead)
@@ -1018,7 +1106,7 @@ gemm_x16_kernel(const GemmArgs args)
             if (!from_lds)
             static_for<FM * FN / 2>([&](auto IJ) {
                 constexpr int j = decltype(IJ)::value / (FM / 2), i = 2 * (decltype(IJ)::value % (FM / 2));
-                cold[decltype(IJ)::value] = *reinterpret_cast<const u32x4 *>(C + (size_t)(wcol0 + j * 16) * ldc + pair_row0 + i * 16);
+                cold[decltype(IJ)::value] = *reinterpret_cast<const pair_vec *>(C + (size_t)(wcol0 + j * 16) * ldc + pair_row0 + i * 16);
             });
             per_policy([&](auto STREAM) {
             const __amdgpu_buffer_rsrc_t tile_c = c_buffer();
@@ -1074,7 +1162,7 @@ gemm_x16_kernel(const GemmArgs args)
     // beta == 0: C is never read.  The aligned and the element-wise variant are separate straight-line sequences: with
     // the choice made per block the epilogue was bound by instruction issue (64 blocks x ~20 instructions with two
     // branches each took 7 us of a 220 us tile at 8192^3, whatever the number of work-groups writing at the time).
-    if (vec_c && PAIRED_C) {
+    if constexpr (PAIRED_C) {
         // alpha == 1 gets a copy of the sequence without the multiplications: with the packed conversions that makes 4 (12)
         // instructions per eight results where scalar casts took 16.
         auto store_all = [&](auto UNIT_ALPHA, auto STREAM, __amdgpu_buffer_rsrc_t tile_c) {
@@ -1098,7 +1186,7 @@ gemm_x16_kernel(const GemmArgs args)
             if (alpha == 1.0f) store_all(std::true_type{}, STREAM, tile_c);
             else store_all(std::false_type{}, STREAM, tile_c);
         });
-    } else if (vec_c) {
+    } else {
         per_policy([&](auto STREAM) {
             const __amdgpu_buffer_rsrc_t tile_c = c_buffer();
         static_for<FM * FN>([&](auto IJ) {
@@ -1110,18 +1198,6 @@ gemm_x16_kernel(const GemmArgs args)
             io.e[3] = (T)(alpha * acc_read<base + 3>());
             store_c(STREAM, io.v, tile_c, c_lane + j * c_block_col + i * 16 * ESZ, 0u);
         });
-        });
-    } else {
-        static_for<FM * FN>([&](auto IJ) {
-            constexpr int j = decltype(IJ)::value / FM, i = decltype(IJ)::value % FM, base = (i * FN + j) * 4;
-            T *p = C + (size_t)(wcol0 + j * 16) * ldc + wrow0 + i * 16;
-            float v[4] = {alpha * acc_read<base>(), alpha * acc_read<base + 1>(), alpha * acc_read<base + 2>(), alpha * acc_read<base + 3>()};
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float o = v[r];
-                if (beta != 0.0f) o = __builtin_fmaf(beta, (float)p[r], o);
-                p[r] = (T)o;
-            }
         });
     }
     }   // tiles of this work-group

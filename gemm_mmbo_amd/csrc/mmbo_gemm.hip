@@ -1202,11 +1202,11 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     a.line_rows = on_lines(A, lda, strideA) && on_lines(B, ldb, strideB);
     a.quartered = f64 ? (uint32_t)quartered_tiles(cref.tile, nwg0 * nwg1, batch, k) : 0;
     a.ws_narrow = (size_t)r.bn * m * 4 < 0x7FFFFF00ull;
-    a.vec_c = aligned16(C, ldc, strideC) && (!cref.x16 || (size_t)r.bn * ldc * esz < 0x7FFFFF00ull);
-    // beta != 0 on the x16 kernel's fp16 path: the old C of a tile is fetched into LDS under the tile's last slices (one
-    // tile's span of C, tile columns x ldc, must then fit the 32-bit offsets of a buffer load)
-    a.c_prefetch = cref.x16 && dtype == MMBO_F16 && beta_f != 0.0f && split == 1 && a.vec_c &&
-                   (size_t)r.bn * ldc * esz < 0x7FFFFF00ull;
+    a.vec_c = aligned16(C, ldc, strideC);
+    a.c_narrow = (size_t)r.bn * ldc * esz < 0x7FFFFF00ull;
+    // beta != 0 on the x16 kernel's fp16 path: the old C of a tile is fetched into LDS under the tile's last slices (through
+    // buffer loads, at any alignment)
+    a.c_prefetch = cref.x16 && dtype == MMBO_F16 && beta_f != 0.0f && split == 1 && a.c_narrow;
     // C with the non-temporal hint: only where resident work-groups walk at least four rounds of tiles (256 CUs) with a long
     // slice loop -- there the operand panels the next tiles share are worth more in the L2 than a fast epilogue (8192^3:
     // +0.3 %); with fewer rounds or a short k plain stores win (fp16 6144^3 +1.6 %, 44160 x 2048 x 384 +2.7 %, 64 x 512^3 +14 %)
