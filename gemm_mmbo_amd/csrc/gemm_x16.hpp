@@ -837,7 +837,7 @@ gemm_x16_kernel(const GemmArgs args)
     // workspace [split][batch][n][m] and the reduction kernel applies alpha and beta.
     const uint32_t wrow0 = row0 + wm * Cfg::TM + 4 * (lane >> 4), wcol0 = col0 + wn * Cfg::TN + (lane & 15);
     const bool edge = m_here < (uint32_t)BM || n_here < (uint32_t)BN;
-    if (edge || (args.splits == 1 && !args.c_narrow)) {
+    if (edge || (args.splits == 1 && (!args.c_narrow || (ESZ == 2 && args.c_odd)))) {
         // Edge tile (reference: the un-shift and the guarded store, src/gemm/ref/Kernels.cpp:1007-1121).  Tile row r is
         // row r of C, except in the last 16-byte group of a row-contiguous A (Tile::rc_group_off): there tile rows
         // gsm+shm .. gsm+EPC-1 are rows gsm .. m_here-1, and tile rows gsm .. gsm+shm-1 repeat rows that the group
@@ -896,56 +896,118 @@ gemm_x16_kernel(const GemmArgs args)
         // A lane stores 16 bytes per unit: four rows of one block (fp32) or, of two vertically adjacent blocks that have been
         // through the lane exchange described below, eight rows (fp16).  Either way these are exactly one 16-byte group
         // of rows of the operand, so a lane's rows are all in place, or they are the one group that the edge cuts, or there
-        // are none.  The cut group's rows go one by one (the rows it repeats are another lane's to update).  Bound by the round
-        // trip of the old C, which is therefore requested for the whole wave tile (fp32: for up to 16 blocks) before the first value
-        // of it is used, and by the number of store requests.  Block after block with a round trip each, four rows
-        // to a store, fp16 beta = 1, us: 19101 x 723 x 186 91.4 -> 38.7, 640 x 1308 x 640 12.0 -> 9.1; beta = 0 1170 x 1152 x 523 11.6 -> 10.8.
-        // Plain stores, as the columns of such a C rarely start on 16-byte boundaries (device scope 47.6 and 8.8).
+        // are none.  Bound by the round trip of the old C, which is therefore requested for up to 16 units before the first value
+        // of it is used, by the number of requests, and by the fetch of its own instructions.  Block after block with a round trip
+        // each, four rows to a store and the cut group's rows one by one, fp16 NT beta = 1, us: 19101 x 723 x 186 91.4 -> 38.7, 710 x
+        // 1408 x 105 13.2 -> 8.5; 1783 x 1408 x 1600 beta = 0.5 22.1 -> 17.0; beta = 0 1170 x 1152 x 523 11.6 -> 10.8.  Plain stores, as the columns
+        // of such a C rarely start on 16-byte boundaries (the first of these with device scope: 47.6).
+        //   The cut group: its old C is the 16 bytes that end at its last row, its new rows go out in pieces of 4, 2 and 1 (the
+        // rows in front of them are another lane's to update).
+        //   fp16, columns of C that start on an odd element (args.c_odd): a 16-byte access off a dword boundary takes the CU's
+        // vector path several times as long as one off a 16-byte boundary (1792 x 1408 x 1600, ldc 1792 / 1793 / 1794, us:
+        // beta = 0 15.5 / 17.9 / 15.3, beta = 0.5 15.0 / 20.9 / 15.9).  In such a column a lane reads the eight rows from one before
+        // its own, writes the eight from one after, and the row that is missing comes from, or belongs to, the next group down
+        // the column: another lane of the same unit or the next unit's, so units are walked upwards.  At the end of the wave tile
+        // the odd rows travel alone.  ldc 1793 of the same calls: 16.3 and 18.8; 8192 x 2048 x 256, ldc 8193, 27.6 -> 20.6 and 37.5 -> 29.8.
         constexpr bool PAIRS = ESZ == 2;
         static_assert(!PAIRS || FM % 2 == 0, "fp16 blocks go out in vertical pairs");
         constexpr int FR = PAIRS ? FM / 2 : FM, UNIT_ROWS = PAIRS ? 32 : 16;          // units down a wave tile, rows of each
         const uint32_t g4 = e_lane >> 4;
         const uint32_t lrow0 = wm * Cfg::TM + (PAIRS && (g4 & 1) ? 4 * g4 + 12 : 4 * g4);
         const uint32_t whole_end = e_m / EPC * EPC, cut = e_m % EPC;                // rows in whole groups, rows of the cut one
-        const uint32_t e_first = TA ? 0u : EPC - cut, e_end = TA ? cut : EPC;        // which of the cut group's elements exist
-        const __amdgpu_buffer_rsrc_t tile_c = __builtin_amdgcn_make_buffer_rsrc(
-            reinterpret_cast<void *>(uniform_address(C + (size_t)col0 * args.ldc + row0)), 0, 0x7fffffff, 0x00020000);
-        // the cut group's first element (under a shift it lies before the group's place, and with less than one group of rows
-        // before the tile: as a pointer, since a buffer's offsets do not reach back)
-        T *const cut_c = C + (size_t)col0 * args.ldc + row0 + whole_end - (TA ? 0u : EPC - cut);
+        const bool any_odd = PAIRS && args.c_odd != 0, read_c = beta != 0.0f;
+        const T *const c_tile = C + (size_t)col0 * args.ldc + row0;
+        // (the buffer starts eight elements before the tile: the reads above reach back one row, and up to EPC - 1)
+        constexpr uint32_t BEFORE = 8;
+        const __amdgpu_buffer_rsrc_t tile_c =
+            __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(uniform_address(c_tile - BEFORE)), 0, 0x7fffffff, 0x00020000);
+        const uint32_t tile_odd = (uint32_t)((uintptr_t)c_tile / ESZ);
+        // fp16: the lane with the group below this one (the same unit's, or the first lane row of the next unit), and the last whole
+        // group of the wave tile
+        const uint32_t next_lane = ((g4 == 0 ? 32u : g4 == 1 ? 48u : g4 == 2 ? 16u : 0u) + (e_lane & 15)) * 4;
+        const uint32_t bottom = min(whole_end, (uint32_t)((wm + 1) * Cfg::TM)) - EPC;
+        auto below = [&](uint32_t first, uint32_t &saved) {          // the first dword of the group below; lower units come first
+            const uint32_t got = __builtin_amdgcn_ds_bpermute(next_lane, first), here = g4 == 3 ? saved : got;
+            saved = got;
+            return here;
+        };
+        auto one_row_on = [](u32x4 v, uint32_t first_below) {        // rows r .. r + 7 -> r + 1 .. r + 8
+            return u32x4{__builtin_amdgcn_alignbyte(v[1], v[0], 2), __builtin_amdgcn_alignbyte(v[2], v[1], 2),
+                         __builtin_amdgcn_alignbyte(v[3], v[2], 2), __builtin_amdgcn_alignbyte(first_below, v[3], 2)};
+        };
+        auto cut_to_front = [&](u32x4 v) {                           // the last `cut` elements of a group -> the first
+            const uint32_t bytes = (EPC - cut) * ESZ;
+            if (bytes & 8) v = u32x4{v[2], v[3], 0u, 0u};
+            if (bytes & 4) v = u32x4{v[1], v[2], v[3], 0u};
+            if (bytes & 2) v = one_row_on(v, 0u);
+            return v;
+        };
         union group_t { T e[EPC]; u32x4 v; };
-        // (fp16: at most 32 units, 128 registers; fp32: up to 16 at a time)
-        constexpr int UNITS = FR * FN, COLS = PAIRS ? FN : (FN % 4 == 0 && 4 * FR <= 16) ? 4 : (FN % 2 == 0 && 2 * FR <= 16) ? 2 : 1, CHUNK = COLS * FR;
-        const bool read_c = beta != 0.0f;
+        // (up to 16 units, 64 registers, at a time: with 32 on the 128 x 128 wave tile the compiler ran out of registers)
+        constexpr int UNITS = FR * FN, COLS = PAIRS ? (UNITS > 16 ? FN / 2 : FN) : (FN % 4 == 0 && 4 * FR <= 16) ? 4 : (FN % 2 == 0 && 2 * FR <= 16) ? 2 : 1, CHUNK = COLS * FR;
+        // (a copy of the walk for each: its instructions come cold, once per tile; in one, 1792 x 1405 x 1600 NT beta = 0.5 took 18.6 us
+        // instead of 16.5)
+        auto walk = [&](auto ODD_COLUMNS) {
+        constexpr bool ODD = decltype(ODD_COLUMNS)::value;
         static_for<UNITS / CHUNK>([&](auto CC) {
+        constexpr int j0 = decltype(CC)::value * COLS;
         group_t old_c[CHUNK];
+        [[maybe_unused]] uint32_t old_last[COLS];                         // odd columns: the last row of the bottom group
         if (read_c) {
-            static_for<CHUNK>([&](auto Q) {
-                constexpr int q = decltype(Q)::value, u = decltype(CC)::value * CHUNK + q, j = u / FR, i = u % FR;
-                const uint32_t lr = lrow0 + i * UNIT_ROWS, lc = lcol0 + j * 16;
-                old_c[q].v = u32x4{0u, 0u, 0u, 0u};
-                if (column_exists(lc)) {
-                    if (lr + EPC <= whole_end) {
-                        old_c[q].v = __builtin_amdgcn_raw_buffer_load_b128(tile_c, (column(lc) * args.ldc + lr) * ESZ, 0, 0);
-                    } else if (lr == whole_end && cut != 0) {
-                        const T *p = cut_c + (size_t)column(lc) * args.ldc;
+            static_for<COLS>([&](auto J) {
+                constexpr int jj = decltype(J)::value, j = j0 + jj;
+                const uint32_t lc = lcol0 + j * 16, col_off = column(lc) * args.ldc + BEFORE;
+                [[maybe_unused]] const uint32_t odd = ODD ? (tile_odd + column(lc) * args.ldc) & 1 : 0u;
+                static_for<FR>([&](auto I) {
+                    constexpr int i = decltype(I)::value, q = jj * FR + i;
+                    const uint32_t lr = lrow0 + i * UNIT_ROWS;
+                    old_c[q].v = u32x4{0u, 0u, 0u, 0u};
+                    if (column_exists(lc)) {
+                        if (lr + EPC <= whole_end) {
+                            old_c[q].v = __builtin_amdgcn_raw_buffer_load_b128(tile_c, (col_off + lr - odd) * ESZ, 0, 0);
+                        } else if (lr == whole_end && cut != 0) {
+                            if (row0 + e_m >= EPC) {
+                                old_c[q].v = __builtin_amdgcn_raw_buffer_load_b128(tile_c, (col_off + e_m - EPC) * ESZ, 0, 0);
+                            } else if constexpr (TA && i == 0) {                 // fewer rows than a group in all
 #pragma unroll
-                        for (uint32_t e = 0; e < EPC; ++e)
-                            if (e >= e_first && e < e_end) old_c[q].e[e] = p[e];
+                                for (uint32_t e = 0; e < EPC; ++e)
+                                    if (e < cut) old_c[q].e[e] = c_tile[(size_t)column(lc) * args.ldc + e];
+                            }
+                        }
                     }
+                });
+                if constexpr (ODD) {
+                    old_last[jj] = 0;
+                    if (odd && column_exists(lc) && whole_end != 0 && bottom >= lrow0 && ((bottom - lrow0) & (UNIT_ROWS - 1)) == 0)
+                        old_last[jj] = __builtin_amdgcn_raw_buffer_load_b16(tile_c, (col_off + bottom + EPC - 1) * ESZ, 0, 0);
                 }
             });
         }
-        static_for<CHUNK>([&](auto Q) {
-            constexpr int q = decltype(Q)::value, u = decltype(CC)::value * CHUNK + q, j = u / FR, i = u % FR;
-            const uint32_t lr = lrow0 + i * UNIT_ROWS, lc = lcol0 + j * 16;
+        static_for<COLS>([&](auto J) {
+        constexpr int jj = decltype(J)::value, j = j0 + jj;
+        const uint32_t lc = lcol0 + j * 16, col_off = column(lc) * args.ldc + BEFORE;
+        const bool col_ok = column_exists(lc);
+        [[maybe_unused]] const uint32_t odd = ODD ? (tile_odd + column(lc) * args.ldc) & 1 : 0u;
+        [[maybe_unused]] uint32_t old_saved = 0, new_saved = 0;
+        static_for<FR>([&](auto I) {
+            constexpr int i = FR - 1 - decltype(I)::value, q = jj * FR + i;
+            const uint32_t lr = lrow0 + i * UNIT_ROWS;
+            const bool whole = lr + EPC <= whole_end, is_cut = lr == whole_end && cut != 0;
+            [[maybe_unused]] const bool last = lr == bottom;
             group_t out;
             if constexpr (PAIRS) {
                 constexpr int b0 = (2 * i * FN + j) * 4, b1 = ((2 * i + 1) * FN + j) * 4;
                 float x[4] = {alpha * acc_read<b0>(), alpha * acc_read<b0 + 1>(), alpha * acc_read<b0 + 2>(), alpha * acc_read<b0 + 3>()};
                 float y[4] = {alpha * acc_read<b1>(), alpha * acc_read<b1 + 1>(), alpha * acc_read<b1 + 2>(), alpha * acc_read<b1 + 3>()};
                 if (read_c) {
-                    const u32x4 c = old_c[q].v;
+                    u32x4 c = old_c[q].v;
+                    if constexpr (ODD) {
+                        uint32_t first_below = below(c[0], old_saved);
+                        if (last) first_below = old_last[jj];
+                        const u32x4 d = one_row_on(c, first_below);
+                        if (odd && whole) c = d;
+                    }
+                    if (TA && is_cut && row0 + e_m >= EPC) c = cut_to_front(c);
                     auto o0 = __builtin_amdgcn_permlane16_swap(c[0], c[2], false, false);
                     auto o1 = __builtin_amdgcn_permlane16_swap(c[1], c[3], false, false);
                     union { T e[4]; uint32_t u[2]; } xo, yo;
@@ -966,22 +1028,62 @@ gemm_x16_kernel(const GemmArgs args)
             } else {
                 constexpr int base = (i * FN + j) * 4;
                 float v[4] = {alpha * acc_read<base>(), alpha * acc_read<base + 1>(), alpha * acc_read<base + 2>(), alpha * acc_read<base + 3>()};
+                group_t c;
+                if (read_c) {
+                    c = old_c[q];
+                    if (TA && is_cut && row0 + e_m >= EPC) c.v = cut_to_front(c.v);
+                }
 #pragma unroll
-                for (int r = 0; r < 4; ++r) out.e[r] = read_c ? (T)__builtin_fmaf(beta, (float)old_c[q].e[r], v[r]) : (T)v[r];
+                for (int r = 0; r < 4; ++r) out.e[r] = read_c ? (T)__builtin_fmaf(beta, (float)c.e[r], v[r]) : (T)v[r];
             }
-            if (column_exists(lc)) {
-                if (lr + EPC <= whole_end) {
-                    __builtin_amdgcn_raw_buffer_store_b128(out.v, tile_c, (column(lc) * args.ldc + lr) * ESZ, 0, 0);
-                } else if (lr == whole_end && cut != 0) {
-                    T *p = cut_c + (size_t)column(lc) * args.ldc;
-#pragma unroll
-                    for (uint32_t e = 0; e < EPC; ++e)
-                        if (e >= e_first && e < e_end) p[e] = out.e[e];
+            u32x4 rows = out.v;                                      // what this lane writes, from row lr (lr + 1 in an odd column) on
+            if constexpr (ODD) {
+                const u32x4 d = one_row_on(rows, below(rows[0], new_saved));
+                if (odd && whole) rows = d;
+            }
+            if (col_ok) {
+                const uint32_t at = (col_off + lr + odd) * ESZ;
+                if (whole && !(ODD && odd && last)) {
+                    __builtin_amdgcn_raw_buffer_store_b128(rows, tile_c, at, 0, 0);
+                } else if (is_cut) {
+                    // (dword-sized pieces at any element: the sizes are the cut's binary digits)
+                    u32x4 v = TA ? out.v : cut_to_front(out.v);
+                    uint32_t p = (col_off + lr) * ESZ;
+                    if (ESZ == 2 && (cut & 4)) {
+                        __builtin_amdgcn_raw_buffer_store_b64(u32x2{v[0], v[1]}, tile_c, p, 0, 0);
+                        v = u32x4{v[2], v[3], 0u, 0u};
+                        p += 8;
+                    }
+                    if (cut & 2) {
+                        if constexpr (ESZ == 2) __builtin_amdgcn_raw_buffer_store_b32(v[0], tile_c, p, 0, 0);
+                        else __builtin_amdgcn_raw_buffer_store_b64(u32x2{v[0], v[1]}, tile_c, p, 0, 0);
+                        v[0] = ESZ == 2 ? v[1] : v[2];
+                        p += 2 * ESZ;
+                    }
+                    if (cut & 1) {
+                        if constexpr (ESZ == 2) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)v[0], tile_c, p, 0, 0);
+                        else __builtin_amdgcn_raw_buffer_store_b32(v[0], tile_c, p, 0, 0);
+                    }
+                }
+                if constexpr (ODD) {
+                    if (odd && whole && last) {
+                        __builtin_amdgcn_raw_buffer_store_b96(u32x3{rows[0], rows[1], rows[2]}, tile_c, at, 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(out.v[3] >> 16), tile_c, at + 12, 0, 0);
+                    }
+                    if (i == 0 && odd && whole && g4 == 0) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)out.v[0], tile_c, at - ESZ, 0, 0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);              // one unit at a time: keeps the address arithmetic of all of them from piling up
         });
         });
+        });
+        };
+        if constexpr (PAIRS) {
+            if (any_odd) walk(std::true_type{});
+            else walk(std::false_type{});
+        } else {
+            walk(std::false_type{});
+        }
         continue;
     }
     if (args.splits > 1) {

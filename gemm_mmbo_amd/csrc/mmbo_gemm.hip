@@ -1204,9 +1204,11 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     a.ws_narrow = (size_t)r.bn * m * 4 < 0x7FFFFF00ull;
     a.vec_c = aligned16(C, ldc, strideC);
     a.c_narrow = (size_t)r.bn * ldc * esz < 0x7FFFFF00ull;
+    // fp16: columns on odd elements leave by the epilogue that never makes a wide access off a dword boundary
+    a.c_odd = dtype == MMBO_F16 && (uintptr_t)C % 4 == 0 && (ldc % 2 != 0 || (batch > 1 && strideC % 2 != 0));
     // beta != 0 on the x16 kernel's fp16 path: the old C of a tile is fetched into LDS under the tile's last slices (through
     // buffer loads, at any alignment)
-    a.c_prefetch = cref.x16 && dtype == MMBO_F16 && beta_f != 0.0f && split == 1 && a.c_narrow;
+    a.c_prefetch = cref.x16 && dtype == MMBO_F16 && beta_f != 0.0f && split == 1 && a.c_narrow && !a.c_odd;
     // C with the non-temporal hint: only where resident work-groups walk at least four rounds of tiles (256 CUs) with a long
     // slice loop -- there the operand panels the next tiles share are worth more in the L2 than a fast epilogue (8192^3:
     // +0.3 %); with fewer rounds or a short k plain stores win (fp16 6144^3 +1.6 %, 44160 x 2048 x 384 +2.7 %, 64 x 512^3 +14 %)

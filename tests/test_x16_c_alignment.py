@@ -1,5 +1,5 @@
 """The 16x16-block ring kernel's epilogue where the columns of C start at any element: whole tiles and edge tiles, with the old C fetched
-under the last slices (fp16), requested ahead, or not read, in every transpose, against the fp64 oracle with the suite's own bounds."""
+under the last slices (fp16), requested ahead, or not read, columns on odd elements, in every transpose, against the fp64 oracle with the suite's own bounds."""
 import numpy as np
 import pytest
 
@@ -30,9 +30,11 @@ def test_columns_of_c_at_any_element(dtype, ta, tb):
         #        m          n       slices  ldc - m  offset of C
         cases = [(bm, bn, 8, 1, 1), (2 * bm, bn, 3, g // 2, 0), (bm, 2 * bn, 9, 0, g - 1),             # whole tiles
                  (bm + g, bn + 1, 8, 3, 1), (bm + g - 1, bn + g, 3, 0, 0),                            # the cut group one row long, all but one
-                 (2 * bm - 1, bn + 3, 2, 1, 0), (g, bn - 1, 8, 1, 3)]
+                 (2 * bm - 1, bn + 3, 2, 1, 0), (g, bn - 1, 8, 1, 3),
+                 # columns on odd elements of a C that starts on a dword: every length of the cut group, whole tiles, over a batch
+                 (2 * bm, bn + 1, 3, 1, 0)] + [(bm // 2 + 2 * g + r, bn - 2, 2, 1 - (g + r) % 2, 0) for r in range(g)] + [(g + 1, g + 2, 2, 0, 0)]
         for q, (m, n, slices, more, offset) in enumerate(cases):
-            alpha, beta, batch = (1.0, -1.5)[(i + q) % 2], (0.0, 0.5, 1.0)[(i + q) % 3], 1 + (q == 3)
+            alpha, beta, batch = (1.0, -1.5)[(i + q) % 2], (0.0, 0.5, 1.0)[(i + q) % 3], 1 + (q in (3, 7))
             p = U.Problem(dtype, ta, tb, m, n, bk * slices, alpha, beta, ldc=m + more, batch=batch, seed=60 * i + q,
                           dist="normal" if dtype == F16 else "uniform", c_fill="uniform" if beta else "nan")
             got, guard = U.run_gpu(p, cid, (0, 0, offset))
