@@ -398,13 +398,17 @@ gemm_wave_kernel(const GemmArgs args)
     auto add_up = [&](uint32_t r, uint32_t c) {
         const char *p = lds + (c * LDR + r) * sizeof(elem);
         auto of = [&](int w) { return *reinterpret_cast<const sums_t *>(p + w * Cfg::PARTIAL_BYTES); };
+        // All reads ahead of the additions, whose order stays: a loop over `waves` is one LDS round trip per wavefront (the
+        // compiler unrolls it by eight and takes these seven in what is left over).  fp16 16 x 4096 x 4096: 8.45 -> 8.20 us.
         sums_t s = of(0);
-        int w = 1;
-        if (waves == 4) {                                        // (reads ahead of the additions, whose order stays)
+        if (waves > 1) {                                         // 4 or 8
             const sums_t s1 = of(1), s2 = of(2), s3 = of(3);
-            return ((s + s1) + s2) + s3;
+            if (MAX_WAVES == 8 && waves == 8) {
+                const sums_t s4 = of(4), s5 = of(5), s6 = of(6), s7 = of(7);
+                return ((((((s + s1) + s2) + s3) + s4) + s5) + s6) + s7;
+            }
+            s = ((s + s1) + s2) + s3;
         }
-        for (; w < waves; ++w) s += of(w);
         return s;
     };
     const elem alpha = sizeof(T) == 8 ? (elem)args.alpha_d : (elem)args.alpha, beta = sizeof(T) == 8 ? (elem)args.beta_d : (elem)args.beta;
