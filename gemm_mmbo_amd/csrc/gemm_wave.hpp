@@ -25,6 +25,19 @@ namespace mmbo {
 
 namespace wave {
 
+// 16 bytes without their first `count` elements (0 .. all of them), zeros behind the others
+template <int ESZ>
+__device__ inline u32x4 drop_elements(const u32x4 &x, uint32_t count)
+{
+    uint64_t lo = (uint64_t)x[1] << 32 | x[0], hi = (uint64_t)x[3] << 32 | x[2];
+    const uint32_t bits = count * ESZ * 8, r = bits & 63;
+    if (bits >= 64) lo = hi, hi = 0;
+    if (bits >= 128) lo = 0;
+    lo = lo >> r | (hi << 1) << (63 - r);
+    hi >>= r;
+    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+
 // One operand's part of one slice: R rows x 64 bytes of k, fetched and read by one wavefront.
 template <typename T, bool KC, int R>
 struct Tile {
@@ -64,38 +77,60 @@ struct Tile {
     }
 
     // The same slots through registers: k_here (<= the slice) columns of k exist, `valid` rows; only elements that exist are
-    // read, the others are zero.
-    __device__ static inline void fill(const char *g, uint32_t ld, uint32_t valid, uint32_t k_here, char *dst, int lane)
+    // read, the others are zero.  `before`: how many elements of the contiguous dimension lie in front of this slice
+    // (k-contiguous: the k before it, else the rows).  A group that the end of that dimension cuts comes as the 16 bytes that end
+    // there, shifted: element by element it was up to seven memory round trips one behind the other, each waited for before the
+    // next (fp16 halves share registers).  fp16 TN, us: 33 x 4096 x 4093 17.7 -> 15.1, 40 x 2048 x 1001 with beta 6.1 -> 5.8.
+    __device__ static inline void fetch(u32x4 (&x)[LOADS], const char *g, uint32_t ld, uint32_t valid, uint32_t k_here, uint32_t before, int lane)
     {
+        const uint32_t here = KC ? k_here : valid;                    // elements of the contiguous dimension from this slice's origin on
+        if (__builtin_amdgcn_readfirstlane(before + here) < EPC) {    // the whole operand is shorter than 16 bytes in it
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                uint32_t line, first;
+                slot(lane, i, line, first);
+                union { T e[EPC]; u32x4 v; } u;
+                const T *const p = reinterpret_cast<const T *>(g) + (size_t)(min(line, (KC ? valid : k_here) - 1) * ld);
+#pragma unroll
+                for (uint32_t e = 0; e < EPC; ++e) u.e[e] = p[min(first + e, here - 1)];
+                const uint32_t kept = !KC && line >= k_here ? 0 : here - min(first, here);
+#pragma unroll
+                for (uint32_t e = 0; e < EPC; ++e)
+                    if (e >= kept) u.e[e] = (T)0;
+                x[i] = u.v;
+            }
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {                             // (lines that do not exist repeat the last)
+            uint32_t line, first;
+            slot(lane, i, line, first);
+            const int from = min((int)first, (int)here - (int)EPC);
+            __builtin_memcpy(&x[i], g + (size_t)(min(line, (KC ? valid : k_here) - 1) * ld) * ESZ + (int64_t)from * ESZ, 16);   // (element alignment is enough)
+        }
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
-            union { T e[EPC]; u32x4 v; } u;
-            u.v = u32x4{0u, 0u, 0u, 0u};
-            if constexpr (KC) {
-                const uint32_t row = i * 16 + (lane >> 2), k0 = ((lane & 3) ^ ((row >> 1) & 3)) * EPC;
-                const char *p = g + (size_t)(min(row, valid - 1) * ld) * ESZ + k0 * ESZ;
-                if (k0 + EPC <= k_here) {
-                    __builtin_memcpy(&u, p, 16);                      // (element alignment is enough for a 16-byte access)
-                } else {
-#pragma unroll
-                    for (uint32_t e = 0; e < EPC; ++e)
-                        if (k0 + e < k_here) u.e[e] = reinterpret_cast<const T *>(p)[e];
-                }
-            } else {
-                const uint32_t k = i * KPI + lane / CPR, r0 = ((lane % CPR) ^ rc_mask(k)) * EPC;
-                if (k < k_here) {
-                    const char *p = g + (size_t)(k * ld) * ESZ + r0 * ESZ;
-                    if (r0 + EPC <= valid) {
-                        __builtin_memcpy(&u, p, 16);
-                    } else {
-#pragma unroll
-                        for (uint32_t e = 0; e < EPC; ++e)
-                            if (r0 + e < valid) u.e[e] = reinterpret_cast<const T *>(p)[e];
-                    }
-                }
-            }
-            *reinterpret_cast<u32x4 *>(dst + i * 1024 + lane * 16) = u.v;
+            uint32_t line, first;
+            slot(lane, i, line, first);
+            const int past = (int)first - min((int)first, (int)here - (int)EPC);
+            x[i] = drop_elements<ESZ>(x[i], past >= (int)EPC || (!KC && line >= k_here) ? EPC : (uint32_t)past);
         }
+    }
+    // line (row of a k-contiguous tile, else k) and first element of LDS slot i * 64 + lane
+    __device__ static inline void slot(int lane, int i, uint32_t &line, uint32_t &first)
+    {
+        if constexpr (KC) {
+            line = i * 16 + (lane >> 2);
+            first = ((lane & 3) ^ ((line >> 1) & 3)) * EPC;
+        } else {
+            line = i * KPI + lane / CPR;
+            first = ((lane % CPR) ^ rc_mask(line)) * EPC;
+        }
+    }
+    __device__ static inline void put(const u32x4 (&x)[LOADS], char *dst, int lane)
+    {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) *reinterpret_cast<u32x4 *>(dst + i * 1024 + lane * 16) = x[i];
     }
 
     // Fragments of the F blocks for one slice.  fp16: lane l holds row l % 16, k = 8 * (l / 16) + 0..7 (one 16x16x32 MFMA).
@@ -368,8 +403,11 @@ gemm_wave_kernel(const GemmArgs args)
         const int64_t slices = (k0 - k_begin) / BK;
         const uint32_t k_here = min((uint32_t)BK, k_end - k0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                         // (the ring slot's last reads are done)
-        TileA::fill(gA + slices * stepA, lda, m_here, k_here, my_ring, lane);
-        TileB::fill(gB + slices * stepB, ldb, n_here, k_here, my_ring + TileA::BYTES, lane);
+        u32x4 xa[TileA::LOADS], xb[TileB::LOADS];
+        TileA::fetch(xa, gA + slices * stepA, lda, m_here, k_here, TA ? k0 : row0, lane);
+        TileB::fetch(xb, gB + slices * stepB, ldb, n_here, k_here, TB ? col0 : k0, lane);
+        TileA::put(xa, my_ring, lane);
+        TileB::put(xb, my_ring + TileA::BYTES, lane);
         // (what a lane reads is what others of its wavefront wrote: in order for the hardware, but not something the compiler
         // can tell, which sees one thread's addresses)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");

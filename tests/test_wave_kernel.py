@@ -122,6 +122,34 @@ def test_every_instantiation(dtype, tile):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype,tile", SHIPPED, ids=lambda v: str(v))
+def test_groups_that_an_edge_cuts(dtype, tile):
+    """16-byte groups cut by the end of k, of a row-contiguous operand, or of a column of C that is read come as the 16 bytes that end there:
+    every length of the cut group, operands shorter than one group, NaN in the padding behind."""
+    bm, bn, _ = TILES[tile]
+    bk, per16 = BK[dtype], 16 // U.ESZ[dtype]
+    q = 0
+    for ta, tb in ((0, 0), (0, 1), (1, 0), (1, 1)):
+        for cut in range(1, per16 + 1):
+            waves, pad = (1, 4, 8)[q % 3], (0, 1, 3)[q % 3]
+            if waves > 1 and 8 * TILES[tile][2] * (bm + bn) * 64 > 160 * 1024:
+                waves = 4
+            cases = [(bm + cut, bn + 1, 2 * bk * waves + cut, 1), (cut, 2 * bn - 1, bk + per16 + cut, 2), (bm - cut, cut, cut, 3),
+                     (bm + 1, bn + cut, 4 * bk * waves + 2 * bk - cut, 1)]
+            for i, (m, n, k, batch) in enumerate(cases):
+                beta = (0.5, 1.0, -1.0, 0.0)[i]
+                p = U.Problem(dtype, ta, tb, m, n, k, (1.0, -1.5)[i % 2], beta, lda=(k if ta else m) + pad, ldb=(n if tb else k) + pad, ldc=m + pad,
+                              batch=batch, seed=10 * q + i, dist="normal" if dtype == F16 else "uniform", c_fill="uniform" if beta else "nan")
+                for operand, ld, rows in ((p.A, p.lda, k if ta else m), (p.B, p.ldb, n if tb else k)):
+                    operand.reshape(-1, ld)[:, rows:] = np.nan
+                got = _wave_gemm(p, tile, waves, 1, (q % 2, i % 2, (q + i) % 2))
+                assert got is not None
+                U.check(p, got[0], f"{NAMES[dtype]} tile {tile} {'NT'[ta]}{'NT'[tb]} w{waves} {m}x{n}x{k} pad {pad}")
+                assert np.all(got[1] == 0), "wrote past the end of C"
+            q += 1
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype,tile,ta,tb,m,n,k,lda,ldb", [
     (F32, 5, 0, 1, 576, 1792, 105, 640, 1856),       # longer side of whole lines across: tile rows first
     (F16, 6, 0, 1, 65, 1024, 96, 128, 1024),         # ... two tile rows, the second nearly empty
