@@ -80,7 +80,7 @@ struct Tile {
     // read, the others are zero.  `before`: how many elements of the contiguous dimension lie in front of this slice
     // (k-contiguous: the k before it, else the rows).  A group that the end of that dimension cuts comes as the 16 bytes that end
     // there, shifted: element by element it was up to seven memory round trips one behind the other, each waited for before the
-    // next (fp16 halves share registers).  fp16 TN, us: 33 x 4096 x 4093 17.7 -> 15.1, 40 x 2048 x 1001 with beta 6.1 -> 5.8.
+    // next (fp16 halves share registers).  fp16 TN, us: 33 x 4096 x 4093 17.7 -> 15.1, 40 x 2048 x 1001 with beta 6.1 -> 5.8.  fp16 TN, us: 33 x 4096 x 4093 17.7 -> 15.1, 40 x 2048 x 1001 with beta 6.1 -> 5.8.
     __device__ static inline void fetch(u32x4 (&x)[LOADS], const char *g, uint32_t ld, uint32_t valid, uint32_t k_here, uint32_t before, int lane)
     {
         const uint32_t here = KC ? k_here : valid;                    // elements of the contiguous dimension from this slice's origin on
@@ -325,21 +325,41 @@ gemm_wave_kernel(const GemmArgs args)
     constexpr int GPC = BM / GROUP, GROUPS = GPC * BN;                             // groups per column, per tile
     constexpr int AHEAD = GROUPS / 64 < 8 ? GROUPS / 64 : 8;                       // groups of a thread requested together
     struct rows_t { T e[GROUP]; };
-    rows_t old_c[AHEAD];
+    // (kept as they come, in whole registers: halves taken apart on arrival made every group wait for its own load, the first ones
+    // ahead of the ring's first request.  A group that the edge cuts is the GROUP rows that end there, shifted where it is used -- the rows
+    // in front of it may belong to another work-group, and are dropped.  fp16 with beta, us: TN 32 x 9356 x 1808 11.9 -> 11.3,
+    // TT 619 x 523 x 389 on the device 6.6 -> 5.9.)
+    typedef uint32_t raw_t __attribute__((ext_vector_type(GROUP * ESZ / 4)));
+    raw_t old_c[AHEAD];
+    static_assert(GROUPS % 64 == 0, "a wavefront's groups of one request are all in the tile or all behind it");
     auto request_c = [&](uint32_t first) {
+        if (args.m >= (uint32_t)GROUP) {
 #pragma unroll
-        for (int a = 0; a < AHEAD; ++a) {
-            const uint32_t g = first + a * threads, r = (g % GPC) * GROUP, c = g / GPC;
-            if (g < GROUPS && c < n_here) {
-                const T *p = C + (size_t)c * args.ldc + r;
-                if (r + GROUP <= m_here) {
-                    __builtin_memcpy(&old_c[a], p, sizeof(rows_t));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < GROUP; ++e)
-                        if (r + e < m_here) old_c[a].e[e] = p[e];
-                }
+            for (int a = 0; a < AHEAD; ++a) {
+                const uint32_t g = first + a * threads;                            // (columns that do not exist repeat one that does)
+                if (__builtin_amdgcn_readfirstlane(g) >= GROUPS) continue;         // (no wavefront is half behind the tile: it only queues for nothing)
+                const int r = min((int)((g % GPC) * GROUP), (int)m_here - GROUP);
+                __builtin_memcpy(&old_c[a], C + (int64_t)((size_t)min(g / GPC, n_here - 1) * args.ldc) + r, sizeof(raw_t));
             }
+        } else {
+#pragma unroll
+            for (int a = 0; a < AHEAD; ++a) {
+                const uint32_t g = first + a * threads, r = (g % GPC) * GROUP, c = min(g / GPC, n_here - 1);
+                if (__builtin_amdgcn_readfirstlane(g) >= GROUPS) continue;
+                rows_t o;
+#pragma unroll
+                for (int e = 0; e < GROUP; ++e) o.e[e] = C[(size_t)c * args.ldc + min(r + e, m_here - 1)];
+                old_c[a] = __builtin_bit_cast(raw_t, o);
+            }
+        }
+    };
+    auto old_rows = [&](const raw_t &x, uint32_t r) {
+        const int past = args.m >= (uint32_t)GROUP ? (int)r - min((int)r, (int)m_here - GROUP) : 0;          // < GROUP where r is a row
+        if constexpr (sizeof(raw_t) == 8) {
+            const uint64_t v = __builtin_bit_cast(uint64_t, x) >> ((past & 3) * 16);
+            return __builtin_bit_cast(rows_t, v);
+        } else {
+            return __builtin_bit_cast(rows_t, drop_elements<ESZ>(x, past));
         }
     };
     if (read_c) request_c(tid);
@@ -437,7 +457,7 @@ gemm_wave_kernel(const GemmArgs args)
         const char *p = lds + (c * LDR + r) * sizeof(elem);
         auto of = [&](int w) { return *reinterpret_cast<const sums_t *>(p + w * Cfg::PARTIAL_BYTES); };
         // All reads ahead of the additions, whose order stays: a loop over `waves` is one LDS round trip per wavefront (the
-        // compiler unrolls it by eight and takes these seven in what is left over).  fp16 16 x 4096 x 4096: 8.45 -> 8.20 us.
+        // compiler unrolls it by eight and takes these seven in what is left over).  fp16 16 x 4096 x 4096: 8.45 -> 8.20 us.  fp16 16 x 4096 x 4096: 8.45 -> 8.20 us.
         sums_t s = of(0);
         if (waves > 1) {                                         // 4 or 8
             const sums_t s1 = of(1), s2 = of(2), s3 = of(3);
@@ -450,7 +470,7 @@ gemm_wave_kernel(const GemmArgs args)
         return s;
     };
     const elem alpha = sizeof(T) == 8 ? (elem)args.alpha_d : (elem)args.alpha, beta = sizeof(T) == 8 ? (elem)args.beta_d : (elem)args.beta;
-    auto finish = [&](uint32_t g, rows_t o) {
+    auto finish = [&](uint32_t g, const raw_t &old) {
         const uint32_t r = (g % GPC) * GROUP, c = g / GPC;
         if (c >= n_here || r >= m_here) return;
         const sums_t s = add_up(r, c);
@@ -467,6 +487,7 @@ gemm_wave_kernel(const GemmArgs args)
             return;
         }
         T *p = C + (size_t)c * args.ldc + r;
+        rows_t o = read_c ? old_rows(old, r) : rows_t{};
 #pragma unroll
         for (int e = 0; e < GROUP; ++e) {
             elem v = alpha * s[e];
