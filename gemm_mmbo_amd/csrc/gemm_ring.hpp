@@ -26,6 +26,19 @@ namespace mmbo {
 
 namespace ring {
 
+// 16 bytes without their first `count` elements (0 .. all of them), zeros behind the others
+template <int ESZ>
+__device__ inline u32x4 drop_elements(const u32x4 &x, uint32_t count)
+{
+    uint64_t lo = (uint64_t)x[1] << 32 | x[0], hi = (uint64_t)x[3] << 32 | x[2];
+    const uint32_t bits = count * ESZ * 8, r = bits & 63;
+    if (bits >= 64) lo = hi, hi = 0;
+    if (bits >= 128) lo = 0;
+    lo = lo >> r | (hi << 1) << (63 - r);
+    hi >>= r;
+    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+
 template <typename T> struct Slice;
 template <> struct Slice<half_t> { static constexpr int BK = 32; };
 template <> struct Slice<float>  { static constexpr int BK = 16; };

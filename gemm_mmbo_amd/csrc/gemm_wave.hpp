@@ -25,19 +25,6 @@ namespace mmbo {
 
 namespace wave {
 
-// 16 bytes without their first `count` elements (0 .. all of them), zeros behind the others
-template <int ESZ>
-__device__ inline u32x4 drop_elements(const u32x4 &x, uint32_t count)
-{
-    uint64_t lo = (uint64_t)x[1] << 32 | x[0], hi = (uint64_t)x[3] << 32 | x[2];
-    const uint32_t bits = count * ESZ * 8, r = bits & 63;
-    if (bits >= 64) lo = hi, hi = 0;
-    if (bits >= 128) lo = 0;
-    lo = lo >> r | (hi << 1) << (63 - r);
-    hi >>= r;
-    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
-}
-
 // One operand's part of one slice: R rows x 64 bytes of k, fetched and read by one wavefront.
 template <typename T, bool KC, int R>
 struct Tile {
@@ -113,7 +100,7 @@ struct Tile {
             uint32_t line, first;
             slot(lane, i, line, first);
             const int past = (int)first - min((int)first, (int)here - (int)EPC);
-            x[i] = drop_elements<ESZ>(x[i], past >= (int)EPC || (!KC && line >= k_here) ? EPC : (uint32_t)past);
+            x[i] = ring::drop_elements<ESZ>(x[i], past >= (int)EPC || (!KC && line >= k_here) ? EPC : (uint32_t)past);
         }
     }
     // line (row of a k-contiguous tile, else k) and first element of LDS slot i * 64 + lane
@@ -359,7 +346,7 @@ gemm_wave_kernel(const GemmArgs args)
             const uint64_t v = __builtin_bit_cast(uint64_t, x) >> ((past & 3) * 16);
             return __builtin_bit_cast(rows_t, v);
         } else {
-            return __builtin_bit_cast(rows_t, drop_elements<ESZ>(x, past));
+            return __builtin_bit_cast(rows_t, ring::drop_elements<ESZ>(x, past));
         }
     };
     if (read_c) request_c(tid);
