@@ -15,8 +15,9 @@
 // Ragged problems: a k-contiguous operand repeats its last row for the rows past the edge.  A row-contiguous one reads
 // whole 16-byte groups of rows; a group that straddles the edge takes in what follows in memory -- padding rows, the next
 // column -- whose products land in rows and columns of the tile that are never stored.  Only the last few columns of
-// the operand have nothing behind them: those (and a last partial slice) go through registers, element by element.  So
-// any m, n, k, leading dimension and element alignment is taken, and no byte outside the operands is read.
+// the operand have nothing behind them: those (and a last partial slice) go through registers, a group that an edge cuts as
+// the 16 bytes that end there.  So any m, n, k, leading dimension and element alignment is taken, and no byte outside the
+// operands is read.
 #pragma once
 
 #include "gemm_ring.hpp"
@@ -64,10 +65,13 @@ struct Tile {
     }
 
     // The same slots through registers: k_here (<= the slice) columns of k exist, `valid` rows; only elements that exist are
-    // read, the others are zero.  `before`: how many elements of the contiguous dimension lie in front of this slice
-    // (k-contiguous: the k before it, else the rows).  A group that the end of that dimension cuts comes as the 16 bytes that end
-    // there, shifted: element by element it was up to seven memory round trips one behind the other, each waited for before the
-    // next (fp16 halves share registers).  fp16 TN, us: 33 x 4096 x 4093 17.7 -> 15.1, 40 x 2048 x 1001 with beta 6.1 -> 5.8.  fp16 TN, us: 33 x 4096 x 4093 17.7 -> 15.1, 40 x 2048 x 1001 with beta 6.1 -> 5.8.
+    // read, those past k are zero (rows past the edge only feed rows of the tile that are never stored).  `before`: how many
+    // elements of the contiguous dimension lie in front of this slice (k-contiguous: the k before it, else the rows).  A group
+    // that the end of that dimension cuts comes as the 16 bytes that end there, shifted: element by element it was up to seven
+    // memory round trips one behind the other, each waited for before the next (fp16 halves share registers).  fp16 TN, us: 33 x
+    // 4096 x 4093 17.7 -> 15.1, 40 x 2048 x 1001 with beta 6.1 -> 5.8.  What does not exist is not requested, and nothing is
+    // shifted where no group is cut (every line repeated and every group shifted, us: fp32 NT 480 x 1280 x 111 6.74 -> 6.41, 640 x 414 x
+    // 1009 12.67 -> 12.53, fp16 NN 2269 x 25 x 744 4.80 -> 4.63, with beta 4.99 -> 4.86).
     __device__ static inline void fetch(u32x4 (&x)[LOADS], const char *g, uint32_t ld, uint32_t valid, uint32_t k_here, uint32_t before, int lane)
     {
         const uint32_t here = KC ? k_here : valid;                    // elements of the contiguous dimension from this slice's origin on
@@ -88,19 +92,22 @@ struct Tile {
             }
             return;
         }
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) {                             // (lines that do not exist repeat the last)
-            uint32_t line, first;
-            slot(lane, i, line, first);
-            const int from = min((int)first, (int)here - (int)EPC);
-            __builtin_memcpy(&x[i], g + (size_t)(min(line, (KC ? valid : k_here) - 1) * ld) * ESZ + (int64_t)from * ESZ, 16);   // (element alignment is enough)
-        }
+        // (as a buffer from 16 bytes in front of the slice on: a request behind its 2 GiB returns zeros without going to memory)
+        const __amdgpu_buffer_rsrc_t slice = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(ring::uniform_address(g - 16)), 0, 0x7fffffff, 0x00020000);
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
             uint32_t line, first;
             slot(lane, i, line, first);
-            const int past = (int)first - min((int)first, (int)here - (int)EPC);
-            x[i] = ring::drop_elements<ESZ>(x[i], past >= (int)EPC || (!KC && line >= k_here) ? EPC : (uint32_t)past);
+            const uint32_t at = 16 + (KC ? min(line, valid - 1) : line) * ld * ESZ + min((int)first, (int)here - (int)EPC) * ESZ;
+            x[i] = __builtin_amdgcn_raw_buffer_load_b128(slice, (KC ? first : line) >= k_here ? 0x80000000u : at, 0, 0);   // (element alignment is enough)
+        }
+        if (__builtin_amdgcn_readfirstlane(here) % EPC != 0) {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                uint32_t line, first;
+                slot(lane, i, line, first);
+                x[i] = ring::drop_elements<ESZ>(x[i], (int)first - min((int)first, (int)here - (int)EPC));
+            }
         }
     }
     // line (row of a k-contiguous tile, else k) and first element of LDS slot i * 64 + lane
@@ -324,7 +331,7 @@ gemm_wave_kernel(const GemmArgs args)
 #pragma unroll
             for (int a = 0; a < AHEAD; ++a) {
                 const uint32_t g = first + a * threads;                            // (columns that do not exist repeat one that does)
-                if (__builtin_amdgcn_readfirstlane(g) >= GROUPS) continue;         // (no wavefront is half behind the tile: it only queues for nothing)
+                if (__builtin_amdgcn_readfirstlane(g) >= n_here * GPC) continue;    // (a wavefront with none of the columns only queues for nothing)
                 const int r = min((int)((g % GPC) * GROUP), (int)m_here - GROUP);
                 __builtin_memcpy(&old_c[a], C + (int64_t)((size_t)min(g / GPC, n_here - 1) * args.ldc) + r, sizeof(raw_t));
             }
@@ -332,7 +339,7 @@ gemm_wave_kernel(const GemmArgs args)
 #pragma unroll
             for (int a = 0; a < AHEAD; ++a) {
                 const uint32_t g = first + a * threads, r = (g % GPC) * GROUP, c = min(g / GPC, n_here - 1);
-                if (__builtin_amdgcn_readfirstlane(g) >= GROUPS) continue;
+                if (__builtin_amdgcn_readfirstlane(g) >= n_here * GPC) continue;
                 rows_t o;
 #pragma unroll
                 for (int e = 0; e < GROUP; ++e) o.e[e] = C[(size_t)c * args.ldc + min(r + e, m_here - 1)];
@@ -341,7 +348,8 @@ gemm_wave_kernel(const GemmArgs args)
         }
     };
     auto old_rows = [&](const raw_t &x, uint32_t r) {
-        const int past = args.m >= (uint32_t)GROUP ? (int)r - min((int)r, (int)m_here - GROUP) : 0;          // < GROUP where r is a row
+        if (m_here % GROUP == 0 || args.m < (uint32_t)GROUP) return __builtin_bit_cast(rows_t, x);
+        const int past = (int)r - min((int)r, (int)m_here - GROUP);                                          // < GROUP where r is a row
         if constexpr (sizeof(raw_t) == 8) {
             const uint64_t v = __builtin_bit_cast(uint64_t, x) >> ((past & 3) * 16);
             return __builtin_bit_cast(rows_t, v);
@@ -444,7 +452,7 @@ gemm_wave_kernel(const GemmArgs args)
         const char *p = lds + (c * LDR + r) * sizeof(elem);
         auto of = [&](int w) { return *reinterpret_cast<const sums_t *>(p + w * Cfg::PARTIAL_BYTES); };
         // All reads ahead of the additions, whose order stays: a loop over `waves` is one LDS round trip per wavefront (the
-        // compiler unrolls it by eight and takes these seven in what is left over).  fp16 16 x 4096 x 4096: 8.45 -> 8.20 us.  fp16 16 x 4096 x 4096: 8.45 -> 8.20 us.
+        // compiler unrolls it by eight and takes these seven in what is left over).  fp16 16 x 4096 x 4096: 8.45 -> 8.20 us.
         sums_t s = of(0);
         if (waves > 1) {                                         // 4 or 8
             const sums_t s1 = of(1), s2 = of(2), s3 = of(3);
