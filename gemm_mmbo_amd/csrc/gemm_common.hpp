@@ -56,7 +56,7 @@ struct GemmArgs {
     uint32_t quartered;     // dgemm.hpp: this many last tiles of the walk are shared by four work-groups each, a quarter of the tile to each
     uint32_t ws_narrow;     // 1: a tile's span of the split-K workspace (tile columns x m floats) fits 32-bit offsets
     uint32_t c_narrow;      // 1: a tile's span of C (tile columns x ldc) fits 32-bit offsets
-    uint32_t c_odd;         // fp16: C starts on a dword, but some of its columns on an odd element
+    uint32_t c_odd;         // fp16: some of C's columns start on an odd element
 };
 
 // fp64 tiles that may go out as quarters (GemmArgs::quartered)

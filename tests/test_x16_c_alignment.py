@@ -40,3 +40,31 @@ def test_columns_of_c_at_any_element(dtype, ta, tb):
             got, guard = U.run_gpu(p, cid, (0, 0, offset))
             U.check(p, got, f"{d['name']} {'NT'[ta]}{'NT'[tb]} {m}x{n}x{bk * slices} beta {beta} ldc {m + more} offset {offset}")
             assert np.all(guard == 0), "wrote past the end of C"
+
+
+def test_every_column_of_c_on_an_odd_element():
+    """fp16, C on an odd element and an even leading dimension: every length of the group that an edge cuts, whole tiles, a batch, beta on and
+    off; the element in front of C, whose dword the first column shares, stays as it is."""
+    import torch
+
+    import gemm_mmbo_amd as G
+    for i, cid in enumerate(_ids(F16)):
+        d = G.config_info(F16, cid)
+        bm, bn = d["macro_tile_m"], d["macro_tile_n"]
+        shapes = [(bm // 2 + 16 + r, bn - 2 + r % 3, 1) for r in range(8)] + [(2 * bm, bn, 1), (9, 10, 1), (5, bn, 1), (bm + 3, bn + 1, 3)]
+        for q, (m, n, batch) in enumerate(shapes):
+            ta, tb, beta = 1 if m < 8 else (i + q) % 2, (q // 2) % 2, (0.5, 0.0, 1.0)[(i + q) % 3]     # (no row-contiguous A of fewer than 8 rows)
+            p = U.Problem(F16, ta, tb, m, n, 64 + 8 * (q % 2), 1.0, beta, ldc=m + m % 2, batch=batch, seed=30 * i + q, dist="normal",
+                          c_fill="uniform" if beta else "nan")
+            got, guard = U.run_gpu(p, cid, (0, 0, 1))
+            U.check(p, got, f"{d['name']} {'NT'[ta]}{'NT'[tb]} {m}x{n} batch {batch} beta {beta}")
+            assert np.all(guard == 0), "wrote past the end of C"
+        m, n, k = bm + 5, bn, 64
+        A, B = (torch.ones(count, device="cuda", dtype=torch.float16) for count in (m * k, k * n))
+        C = torch.full(((m + m % 2) * n + 2,), -7.0, device="cuda", dtype=torch.float16)
+        G.gemm(F16, 0, 0, m, n, k, 1.0, A, m, B, k, 0.5, C.data_ptr() + 2, m + m % 2, cid)
+        torch.cuda.synchronize()
+        assert float(C[0]) == -7.0 and float(C[-1]) == -7.0
+        want = torch.full((n, m + m % 2), k - 3.5, device="cuda", dtype=torch.float16)
+        want[:, m:] = -7.0
+        assert torch.equal(C[1:-1].view(n, m + m % 2), want)
