@@ -1213,8 +1213,10 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     a.c_prefetch = cref.x16 && dtype == MMBO_F16 && beta_f != 0.0f && split == 1 && a.c_narrow && !a.c_odd;
     // C with the non-temporal hint: only where resident work-groups walk at least four rounds of tiles (256 CUs) with a long
     // slice loop -- there the operand panels the next tiles share are worth more in the L2 than a fast epilogue (8192^3:
-    // +0.3 %); with fewer rounds or a short k plain stores win (fp16 6144^3 +1.6 %, 44160 x 2048 x 384 +2.7 %, 64 x 512^3 +14 %)
-    a.c_stream = cref.x16 && rr.depth * (rr.bm + rr.bn) * 64 > 80 * 1024 && (size_t)nwg0 * nwg1 >= 4 * 256 && k >= 4096;
+    // +0.3 %); with fewer rounds or a short k plain stores win (fp16 6144^3 +1.6 %, 44160 x 2048 x 384 +2.7 %, 64 x 512^3 +14 %).
+    // Columns off 16 bytes never: their pieces of lines have to meet in the L2 (NN 8192 x 8192 x 4096, C off by 4 bytes, us: fp16
+    // 463 -> 411, fp32 off by 8 bytes 3,917 -> 3,799).
+    a.c_stream = cref.x16 && a.vec_c && rr.depth * (rr.bm + rr.bn) * 64 > 80 * 1024 && (size_t)nwg0 * nwg1 >= 4 * 256 && k >= 4096;
 
     if (cref.ring && !cref.x16 && (!a.vec_a || !a.vec_b)) return MMBO_ERR_INVALID_CONFIG;
     // Split-K: the partial sums go to the stream's own workspace (or the static one), and both launches that use it (the

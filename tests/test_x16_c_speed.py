@@ -35,3 +35,9 @@ def test_odd_columns_cost_the_same_whatever_element_c_starts_on(beta):
     """16-byte accesses off a dword boundary took 1.25 to 1.5 times as long as the epilogue for odd columns."""
     known, all_odd, half_odd = _times(8192, 2048, 256, 0, 1, beta, [(8193, 0), (8192, 1), (8193, 1)], 100)
     assert all_odd <= 1.15 * known and half_odd <= 1.15 * known, (known, all_odd, half_odd)
+
+
+def test_large_product_into_columns_off_16_bytes():
+    """With the streaming hint, whose stores of partial lines nothing merges: 1.13 times the time of whole lines."""
+    aligned, off = _times(8192, 8192, 4096, 0, 0, 0.0, [(8192, 0), (8192, 2)], 6)
+    assert off <= 1.07 * aligned, (aligned, off)
