@@ -71,7 +71,7 @@ struct Tile {
     // memory round trips one behind the other, each waited for before the next (fp16 halves share registers).  fp16 TN, us: 33 x
     // 4096 x 4093 17.7 -> 15.1, 40 x 2048 x 1001 with beta 6.1 -> 5.8.  What does not exist is not requested, and nothing is
     // shifted where no group is cut (every line repeated and every group shifted, us: fp32 NT 480 x 1280 x 111 6.74 -> 6.41, 640 x 414 x
-    // 1009 12.67 -> 12.53, fp16 NN 2269 x 25 x 744 4.80 -> 4.63, with beta 4.99 -> 4.86).
+    // 1009 12.67 -> 12.53, fp16 NN 2269 x 25 x 744 4.80 -> 4.63, with beta 4.99 -> 4.83).
     __device__ static inline void fetch(u32x4 (&x)[LOADS], const char *g, uint32_t ld, uint32_t valid, uint32_t k_here, uint32_t before, int lane)
     {
         const uint32_t here = KC ? k_here : valid;                    // elements of the contiguous dimension from this slice's origin on
@@ -101,14 +101,6 @@ struct Tile {
             const uint32_t at = 16 + (KC ? min(line, valid - 1) : line) * ld * ESZ + min((int)first, (int)here - (int)EPC) * ESZ;
             x[i] = __builtin_amdgcn_raw_buffer_load_b128(slice, (KC ? first : line) >= k_here ? 0x80000000u : at, 0, 0);   // (element alignment is enough)
         }
-        if (__builtin_amdgcn_readfirstlane(here) % EPC != 0) {
-#pragma unroll
-            for (int i = 0; i < LOADS; ++i) {
-                uint32_t line, first;
-                slot(lane, i, line, first);
-                x[i] = ring::drop_elements<ESZ>(x[i], (int)first - min((int)first, (int)here - (int)EPC));
-            }
-        }
     }
     // line (row of a k-contiguous tile, else k) and first element of LDS slot i * 64 + lane
     __device__ static inline void slot(int lane, int i, uint32_t &line, uint32_t &first)
@@ -121,8 +113,18 @@ struct Tile {
             first = ((lane % CPR) ^ rc_mask(line)) * EPC;
         }
     }
-    __device__ static inline void put(const u32x4 (&x)[LOADS], char *dst, int lane)
+    // What fetch requested, to LDS.  (The shift is here, behind both operands' requests: it is the first to wait for them.)
+    __device__ static inline void put(u32x4 (&x)[LOADS], uint32_t valid, uint32_t k_here, uint32_t before, char *dst, int lane)
     {
+        const uint32_t here = __builtin_amdgcn_readfirstlane(KC ? k_here : valid);
+        if (here % EPC != 0 && __builtin_amdgcn_readfirstlane(before) + here >= EPC) {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) {
+                uint32_t line, first;
+                slot(lane, i, line, first);
+                x[i] = ring::drop_elements<ESZ>(x[i], (int)first - min((int)first, (int)here - (int)EPC));
+            }
+        }
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) *reinterpret_cast<u32x4 *>(dst + i * 1024 + lane * 16) = x[i];
     }
@@ -348,12 +350,12 @@ gemm_wave_kernel(const GemmArgs args)
         }
     };
     auto old_rows = [&](const raw_t &x, uint32_t r) {
-        if (m_here % GROUP == 0 || args.m < (uint32_t)GROUP) return __builtin_bit_cast(rows_t, x);
-        const int past = (int)r - min((int)r, (int)m_here - GROUP);                                          // < GROUP where r is a row
+        const int past = args.m >= (uint32_t)GROUP ? (int)r - min((int)r, (int)m_here - GROUP) : 0;          // < GROUP where r is a row
         if constexpr (sizeof(raw_t) == 8) {
             const uint64_t v = __builtin_bit_cast(uint64_t, x) >> ((past & 3) * 16);
             return __builtin_bit_cast(rows_t, v);
         } else {
+            if (m_here % GROUP == 0) return __builtin_bit_cast(rows_t, x);                                   // (no group is cut)
             return __builtin_bit_cast(rows_t, ring::drop_elements<ESZ>(x, past));
         }
     };
@@ -421,8 +423,8 @@ gemm_wave_kernel(const GemmArgs args)
         u32x4 xa[TileA::LOADS], xb[TileB::LOADS];
         TileA::fetch(xa, gA + slices * stepA, lda, m_here, k_here, TA ? k0 : row0, lane);
         TileB::fetch(xb, gB + slices * stepB, ldb, n_here, k_here, TB ? col0 : k0, lane);
-        TileA::put(xa, my_ring, lane);
-        TileB::put(xb, my_ring + TileA::BYTES, lane);
+        TileA::put(xa, m_here, k_here, TA ? k0 : row0, my_ring, lane);
+        TileB::put(xb, n_here, k_here, TB ? col0 : k0, my_ring + TileA::BYTES, lane);
         // (what a lane reads is what others of its wavefront wrote: in order for the hardware, but not something the compiler
         // can tell, which sees one thread's addresses)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
