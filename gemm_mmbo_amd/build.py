@@ -72,6 +72,8 @@ def _units():
     for dtype in (0, 1):
         for tile in range(NUM_X16_TILES):
             units.append(("inst_x16.hip", f"inst_x16_{dtype}_{tile}.o", [f"-DMMBO_DTYPE={dtype}", f"-DMMBO_TILE={tile}"]))
+    for tile in range(NUM_X16_TILES):
+        units.append(("inst_x16.hip", f"inst_x16_odd_c_{tile}.o", ["-DMMBO_DTYPE=1", f"-DMMBO_TILE={tile}", "-DMMBO_ODD_C"]))
     for dtype in (0, 1, 2):
         for tile in range(NUM_WAVE_TILES[dtype]):
             units.append(("inst_wave.hip", f"inst_wave_{dtype}_{tile}.o", [f"-DMMBO_DTYPE={dtype}", f"-DMMBO_TILE={tile}"]))

@@ -360,19 +360,32 @@ struct X16Cfg {
 // lines only when the first of them is even -- s even for a ring of five buffers, s odd for a ring of six.  The launcher
 // therefore gives the k-contiguous operand the even iterations on five buffers and the odd ones on six (six buffers, fp16:
 // 3072^3 NN on the 192 x 192 tile 52.2 -> 50.3 us, 1024 x 1024 x 4096 on 64 x 64 21.1 -> 18.9, 2048 x 1024 x 4096 on 128 x 64 27.2 -> 25.3).
-// OLD_C_AHEAD: the variant for beta != 0 that fetches a tile's old C into LDS under the tile's last four slices (see c_ahead
-// below; both load schedules).  A kernel of its own, chosen by the host: with the code in the one kernel, calls that have no C to read paid
-// 1.5-3 % on short-k and mid-size shapes for tails that had grown.
+// ROLE: what of C the host sends this variant.  Kernels of their own, each without the others' code: in one kernel, calls that
+// have no C to read paid 1.5-3 % on short-k and mid-size shapes for tails that had grown.
+//   GENERAL    everything else: any GlobalSplitU, C of any span.  Where the tile has an OLD_C variant (Cfg::C_PREFETCH) it
+//              updates C only where a tile's span of C does not fit 32-bit offsets: every other call with beta != 0 goes to that one.
+//   OLD_C      beta != 0, one split, narrow C (args.c_prefetch): a tile's old C is fetched into LDS under the tile's last four
+//              slices (see c_ahead below; both load schedules).
+//   ODD_C      fp16 columns of C on odd elements, one split, narrow C (args.c_odd): every tile leaves through the edge epilogue,
+//              which moves its accesses to the dwords.
+// Code of fp16 256 x 256 TN on lines, its beta variant: 221 KB with all of it and 86 spilled scalars, 85 KB and 52 without; us,
+// on the same box: 64 x 512^3 beta = 1 TN 22.9 -> 22.2, NN 23.6 -> 22.8, NT 8192 x 2048 x 256 15.0 -> 14.7, NN 4088 x 4096 x 2052 beta = 1
+// 67.4 -> 66.5, TT 1500 x 1400 x 999 14.4 -> 13.9.
 // BOTH_EVEN: the variant for two k-contiguous operands (TN) whose rows start on memory lines: both operands' pairs on the
 // even iterations (see BOTH below).  A kernel of its own, chosen by the host.
+enum class CRole { GENERAL, OLD_C, ODD_C };
+
 template <typename T, bool TA, bool TB, int BM, int BN, int WM, int WN, int DEPTH, bool PAIR = (TA || !TB),
-          int EVEN_OP = (TA ? 0 : 1), bool OLD_C_AHEAD = false, bool BOTH_EVEN = false>
+          int EVEN_OP = (TA ? 0 : 1), CRole ROLE = CRole::GENERAL, bool BOTH_EVEN = false>
 __global__ void __launch_bounds__(WM * WN * 64)
 gemm_x16_kernel(const GemmArgs args)
 {
-    static_assert(!OLD_C_AHEAD || X16Cfg<T, TA, TB, BM, BN, WM, WN, DEPTH>::C_PREFETCH, "no old-C variant of this kernel");
     using namespace x16;
     using Cfg = X16Cfg<T, TA, TB, BM, BN, WM, WN, DEPTH>;
+    constexpr bool GENERAL = ROLE == CRole::GENERAL, OLD_C_AHEAD = ROLE == CRole::OLD_C, ODD_C = ROLE == CRole::ODD_C;
+    static_assert(!OLD_C_AHEAD || Cfg::C_PREFETCH, "no old-C variant of this kernel");
+    static_assert(!ODD_C || sizeof(T) == 2, "only fp16 columns start off a dword");
+    constexpr bool UPDATES_C = !GENERAL || !Cfg::C_PREFETCH;        // beta != 0 and a narrow C may meet here
     using TileA = typename Cfg::TileA;
     using TileB = typename Cfg::TileB;
     using FragA = typename Cfg::FragA;
@@ -412,7 +425,14 @@ gemm_x16_kernel(const GemmArgs args)
     zb = __builtin_amdgcn_readfirstlane(zb);
     // (the division runs on the vector unit: back to scalar registers, so that what follows from it -- the k range, the
     // slice count, the loop test -- stays scalar as well)
-    const uint32_t split = __builtin_amdgcn_readfirstlane(zb / args.batch), batch = __builtin_amdgcn_readfirstlane(zb % args.batch);
+    uint32_t split = 0, batch = zb;
+    if constexpr (GENERAL) {
+        split = __builtin_amdgcn_readfirstlane(zb / args.batch);
+        batch = __builtin_amdgcn_readfirstlane(zb % args.batch);
+    } else {
+        // (opaque: known to be zero, all that follows from it would be worked out ahead of the tile loop and kept, in spilled registers)
+        asm volatile("" : "+s"(split));
+    }
     const uint32_t row0 = wg0 * BM, col0 = wg1 * BN;
     const uint32_t lda = args.lda, ldb = args.ldb;
     const uint32_t k_begin = split * args.k_per_split;
@@ -490,7 +510,7 @@ gemm_x16_kernel(const GemmArgs args)
     // start at  C_tile + (lane's column * ldc + lane's row of the pair) + (j * 16 * ldc + i * 16)  elements -- the part in
     // front is the lane's constant offset, the part behind a scalar offset of the load.  Group q goes to the ring buffer of
     // slice n_slice - 4 + q / C_PER_SLICE (free from that slice's iteration on), at wave * C_PER_SLICE KB + (q % C_PER_SLICE) KB.
-    const bool c_ahead = OLD_C_AHEAD && args.c_prefetch != 0 && m_here == (uint32_t)BM && n_here == (uint32_t)BN &&
+    const bool c_ahead = OLD_C_AHEAD && m_here == (uint32_t)BM && n_here == (uint32_t)BN &&
                          k_tail == 0 && n_slice >= DEPTH + 1;
     // (set up whether used or not: a descriptor that is assigned under a branch ends up in vector registers, where a
     // buffer load cannot take it)
@@ -870,7 +890,7 @@ gemm_x16_kernel(const GemmArgs args)
     // workspace [split][batch][n][m] and the reduction kernel applies alpha and beta.
     const uint32_t wrow0 = row0 + wm * Cfg::TM + 4 * (lane >> 4), wcol0 = col0 + wn * Cfg::TN + (lane & 15);
     const bool edge = m_here < (uint32_t)BM || n_here < (uint32_t)BN;
-    if (edge || (args.splits == 1 && (!args.c_narrow || (ESZ == 2 && args.c_odd)))) {
+    if (ODD_C || edge || (GENERAL && args.splits == 1 && !args.c_narrow)) {
         // Edge tile (reference: the un-shift and the guarded store, src/gemm/ref/Kernels.cpp:1007-1121).  Tile row r is
         // row r of C, except in the last 16-byte group of a row-contiguous A (Tile::rc_group_off): there tile rows
         // gsm+shm .. gsm+EPC-1 are rows gsm .. m_here-1, and tile rows gsm .. gsm+shm-1 repeat rows that the group
@@ -884,13 +904,12 @@ gemm_x16_kernel(const GemmArgs args)
         const uint32_t gsm = TA ? e_m : (e_m - 1) / EPC * EPC, shm = TA ? 0u : gsm + EPC - e_m;
         const uint32_t gsn = !TB ? e_n : (e_n - 1) / EPC * EPC, shn = !TB ? 0u : gsn + EPC - e_n;
         const float alpha = args.alpha, beta = args.beta;
-        const bool to_ws = args.splits > 1;
         T *C = static_cast<T *>(args.C) + (int64_t)batch * args.strideC;
         const uint32_t lcol0 = wn * Cfg::TN + (e_lane & 15);
         // the column of C a lane's tile column stands for, relative to the tile's first, if any
         auto column_exists = [&](uint32_t lc) { return lc < gsn || (lc >= gsn + shn && lc - shn < e_n); };
         auto column = [&](uint32_t lc) { return lc < gsn ? lc : lc - shn; };
-        if (to_ws || !args.c_narrow) {
+        if (const bool to_ws = GENERAL && args.splits > 1; GENERAL && (to_ws || !args.c_narrow)) {
             // Partial sums, or a C whose tiles span more than the 32-bit offsets of a buffer access: four rows of sums as one
             // vector where all four exist unshifted, everything else element by element.
             const uint32_t vec_rows = shm == 0 ? e_m : gsm, lrow0 = wm * Cfg::TM + 4 * (e_lane >> 4);
@@ -948,7 +967,9 @@ gemm_x16_kernel(const GemmArgs args)
         const uint32_t g4 = e_lane >> 4;
         const uint32_t lrow0 = wm * Cfg::TM + (PAIRS && (g4 & 1) ? 4 * g4 + 12 : 4 * g4);
         const uint32_t whole_end = e_m / EPC * EPC, cut = e_m % EPC;                // rows in whole groups, rows of the cut one
-        const bool any_odd = PAIRS && args.c_odd != 0, read_c = beta != 0.0f;
+        // (a test also in the variant for which the host has made it: known to be true, the compiler takes every request of old C
+        // apart as it arrives, each waited for before the next goes out; NN 4088 x 4096 x 2052 66.5 -> 73.5 us)
+        const bool read_c = UPDATES_C && beta != 0.0f;
         const T *const c_tile = C + (size_t)col0 * args.ldc + row0;
         // (the buffer starts eight elements before the tile: the reads above reach back one row, and up to EPC - 1)
         constexpr uint32_t BEFORE = 8;
@@ -978,10 +999,6 @@ gemm_x16_kernel(const GemmArgs args)
         union group_t { T e[EPC]; u32x4 v; };
         // (up to 16 units, 64 registers, at a time: with 32 on the 128 x 128 wave tile the compiler ran out of registers)
         constexpr int UNITS = FR * FN, COLS = PAIRS ? (UNITS > 16 ? FN / 2 : FN) : (FN % 4 == 0 && 4 * FR <= 16) ? 4 : (FN % 2 == 0 && 2 * FR <= 16) ? 2 : 1, CHUNK = COLS * FR;
-        // (a copy of the walk for each: its instructions come cold, once per tile; in one, 1792 x 1405 x 1600 NT beta = 0.5 took 18.6 us
-        // instead of 16.5)
-        auto walk = [&](auto ODD_COLUMNS) {
-        constexpr bool ODD = decltype(ODD_COLUMNS)::value;
         static_for<UNITS / CHUNK>([&](auto CC) {
         constexpr int j0 = decltype(CC)::value * COLS;
         group_t old_c[CHUNK];
@@ -990,7 +1007,7 @@ gemm_x16_kernel(const GemmArgs args)
             static_for<COLS>([&](auto J) {
                 constexpr int jj = decltype(J)::value, j = j0 + jj;
                 const uint32_t lc = lcol0 + j * 16, col_off = column(lc) * args.ldc + BEFORE;
-                [[maybe_unused]] const uint32_t odd = ODD ? (tile_odd + column(lc) * args.ldc) & 1 : 0u;
+                [[maybe_unused]] const uint32_t odd = ODD_C ? (tile_odd + column(lc) * args.ldc) & 1 : 0u;
                 static_for<FR>([&](auto I) {
                     constexpr int i = decltype(I)::value, q = jj * FR + i;
                     const uint32_t lr = lrow0 + i * UNIT_ROWS;
@@ -1009,7 +1026,7 @@ gemm_x16_kernel(const GemmArgs args)
                         }
                     }
                 });
-                if constexpr (ODD) {
+                if constexpr (ODD_C) {
                     old_last[jj] = 0;
                     if (odd && column_exists(lc) && whole_end != 0 && bottom >= lrow0 && ((bottom - lrow0) & (UNIT_ROWS - 1)) == 0)
                         old_last[jj] = __builtin_amdgcn_raw_buffer_load_b16(tile_c, (col_off + bottom + EPC - 1) * ESZ, 0, 0);
@@ -1020,7 +1037,7 @@ gemm_x16_kernel(const GemmArgs args)
         constexpr int jj = decltype(J)::value, j = j0 + jj;
         const uint32_t lc = lcol0 + j * 16, col_off = column(lc) * args.ldc + BEFORE;
         const bool col_ok = column_exists(lc);
-        [[maybe_unused]] const uint32_t odd = ODD ? (tile_odd + column(lc) * args.ldc) & 1 : 0u;
+        [[maybe_unused]] const uint32_t odd = ODD_C ? (tile_odd + column(lc) * args.ldc) & 1 : 0u;
         [[maybe_unused]] uint32_t old_saved = 0, new_saved = 0;
         static_for<FR>([&](auto I) {
             constexpr int i = FR - 1 - decltype(I)::value, q = jj * FR + i;
@@ -1034,7 +1051,7 @@ gemm_x16_kernel(const GemmArgs args)
                 float y[4] = {alpha * acc_read<b1>(), alpha * acc_read<b1 + 1>(), alpha * acc_read<b1 + 2>(), alpha * acc_read<b1 + 3>()};
                 if (read_c) {
                     u32x4 c = old_c[q].v;
-                    if constexpr (ODD) {
+                    if constexpr (ODD_C) {
                         uint32_t first_below = below(c[0], old_saved);
                         if (last) first_below = old_last[jj];
                         const u32x4 d = one_row_on(c, first_below);
@@ -1070,13 +1087,13 @@ gemm_x16_kernel(const GemmArgs args)
                 for (int r = 0; r < 4; ++r) out.e[r] = read_c ? (T)__builtin_fmaf(beta, (float)c.e[r], v[r]) : (T)v[r];
             }
             u32x4 rows = out.v;                                      // what this lane writes, from row lr (lr + 1 in an odd column) on
-            if constexpr (ODD) {
+            if constexpr (ODD_C) {
                 const u32x4 d = one_row_on(rows, below(rows[0], new_saved));
                 if (odd && whole) rows = d;
             }
             if (col_ok) {
                 const uint32_t at = (col_off + lr + odd) * ESZ;
-                if (whole && !(ODD && odd && last)) {
+                if (whole && !(ODD_C && odd && last)) {
                     __builtin_amdgcn_raw_buffer_store_b128(rows, tile_c, at, 0, 0);
                 } else if (is_cut) {
                     // (dword-sized pieces at any element: the sizes are the cut's binary digits)
@@ -1098,7 +1115,7 @@ gemm_x16_kernel(const GemmArgs args)
                         else __builtin_amdgcn_raw_buffer_store_b32(v[0], tile_c, p, 0, 0);
                     }
                 }
-                if constexpr (ODD) {
+                if constexpr (ODD_C) {
                     if (odd && whole && last) {
                         __builtin_amdgcn_raw_buffer_store_b96(u32x3{rows[0], rows[1], rows[2]}, tile_c, at, 0, 0);
                         __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(out.v[3] >> 16), tile_c, at + 12, 0, 0);
@@ -1110,16 +1127,9 @@ gemm_x16_kernel(const GemmArgs args)
         });
         });
         });
-        };
-        if constexpr (PAIRS) {
-            if (any_odd) walk(std::true_type{});
-            else walk(std::false_type{});
-        } else {
-            walk(std::false_type{});
-        }
         continue;
     }
-    if (args.splits > 1) {
+    if (GENERAL && args.splits > 1) {
         float *ws = args.ws + ((size_t)split * args.batch + batch) * (size_t)args.m * args.n;
         if (BM * BN < 256 * 256 && args.ws_narrow) {
             // The partial sums as device-scope buffer stores (the tile's part of the workspace as a buffer; args.ws_narrow:
@@ -1191,17 +1201,21 @@ gemm_x16_kernel(const GemmArgs args)
     auto c_buffer = [&]() {
         return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(uniform_address(c_origin)), 0, 0x7fffffff, 0x00020000);
     };
-    const uint32_t c_block_col = 16 * ldc * ESZ;                          // bytes from a block's column to the next block's
+    uint32_t c_block_col = 16 * ldc * ESZ;                                // bytes from a block's column to the next block's
     // this lane's first element of the wave tile: four rows of one column per block, or, fp16 pairs, eight rows of two blocks
-    const uint32_t c_lane = ((wn * Cfg::TN + (lane & 15)) * ldc + wm * Cfg::TM + 4 * (lane >> 4)) * ESZ;
-    const uint32_t c_lane_pair = ((wn * Cfg::TN + (lane & 15)) * ldc + (pair_row0 - row0)) * ESZ;
+    uint32_t c_lane = ((wn * Cfg::TN + (lane & 15)) * ldc + wm * Cfg::TM + 4 * (lane >> 4)) * ESZ;
+    uint32_t c_lane_pair = ((wn * Cfg::TN + (lane & 15)) * ldc + (pair_row0 - row0)) * ESZ;
+    // (the blocks' addresses do not depend on the tile, and the compiler works them out ahead of the tile loop where nothing else in the
+    // epilogue takes their registers: with more block columns than rows that spilled 50 registers of the 192 x 256 tile.  There
+    // they are derived here, behind the slice loop; on the other tiles that costs 0.5-1 % of a short-k call)
+    if constexpr (GENERAL && FN > FM) asm volatile("" : "+s"(c_block_col), "+v"(c_lane), "+v"(c_lane_pair));
     auto store_c = [](auto STREAM, auto value, __amdgpu_buffer_rsrc_t tile_c, uint32_t lane_and_row, uint32_t column) {
         constexpr int policy = decltype(STREAM)::value;
         if constexpr (sizeof(value) == 16) __builtin_amdgcn_raw_buffer_store_b128(value, tile_c, lane_and_row, column, policy);
         else __builtin_amdgcn_raw_buffer_store_b64(value, tile_c, lane_and_row, column, policy);
     };
     auto per_policy = [&](auto &&body) {
-        if (args.c_stream) body(std::integral_constant<int, 2>{});                  // nt
+        if (Cfg::LDS_BYTES > 80 * 1024 && args.c_stream) body(std::integral_constant<int, 2>{});                  // nt (resident tiles only)
         else if (args.vec_c) body(std::integral_constant<int, 16>{});                // sc1
         else body(std::integral_constant<int, 0>{});                                 // plain
     };
@@ -1210,7 +1224,7 @@ gemm_x16_kernel(const GemmArgs args)
         typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
         return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), f16x2));
     };
-    if (beta != 0.0f) {
+    if (OLD_C_AHEAD || (UPDATES_C && beta != 0.0f)) {
         if constexpr (PAIRED_C) {
             // the whole wave tile of old C is requested before its first value is used (see below) -- or was requested
             // under the last four slices and is waiting in the ring buffers those slices left (c_ahead)

@@ -32,6 +32,10 @@ hipError_t launch_ring(int transA, int transB, const GemmArgs &args, hipStream_t
 template <int DTYPE, int TILE>
 hipError_t launch_x16(int transA, int transB, const GemmArgs &args, hipStream_t stream);
 
+// Its fp16 variant for columns of C on odd elements (args.c_odd; launch_x16 hands such calls on).
+template <int TILE>
+hipError_t launch_x16_odd_c(int transA, int transB, const GemmArgs &args, hipStream_t stream);
+
 // DGEMM kernel of fp64 tile row TILE; grid = (nwg0*nwg1, 1, batch).
 template <int TILE>
 hipError_t launch_dgemm(int transA, int transB, const GemmArgs &args, hipStream_t stream);

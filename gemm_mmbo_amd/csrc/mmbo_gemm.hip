@@ -1207,7 +1207,8 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     // fp16: columns on odd elements, some or all of them, leave by the epilogue that keeps its accesses to whole groups of rows on
     // dwords (a group that the edge cuts is read and written where it lies).  NT 8192 x 2048 x 256, us: C on an odd element, ldc 8192,
     // 27.6 -> 21.6, with beta 39.1 -> 29.3; ldc 8193 29.6 -> 20.9 and 39.2 -> 30.2; from a dword 20.9 and 30.1.
-    a.c_odd = dtype == MMBO_F16 && ((uintptr_t)C % 4 != 0 || ldc % 2 != 0 || (batch > 1 && strideC % 2 != 0));
+    // (one split and a narrow C: the x16 kernel's variants for odd columns and for a prefetched old C take nothing else)
+    a.c_odd = cref.x16 && dtype == MMBO_F16 && split == 1 && a.c_narrow && ((uintptr_t)C % 4 != 0 || ldc % 2 != 0 || (batch > 1 && strideC % 2 != 0));
     // beta != 0 on the x16 kernel's fp16 path: the old C of a tile is fetched into LDS under the tile's last slices (through
     // buffer loads, at any alignment)
     a.c_prefetch = cref.x16 && dtype == MMBO_F16 && beta_f != 0.0f && split == 1 && a.c_narrow && !a.c_odd;
