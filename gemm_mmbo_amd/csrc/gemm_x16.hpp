@@ -177,8 +177,8 @@ struct Tile {
     // src/gemm/ref/Kernels.cpp:921-1005, zero-fills k >= remainder): the same slots as the direct loads fill, written
     // through registers, with zeros from k_tail on.  g = operand origin of this tile at the tail slice, k_before = the k in front of
     // it.  Only elements that exist are read: a 16-byte chunk along k that straddles the end comes as the 16 bytes that end there, shifted
-    // (element by element, halves that share a register, it was a memory round trip for each).  Nothing branches, so all requests of
-    // both operands are out before the first is waited for.  fp16, us: TN 16 x (640 x 640 x 135) 12.1 -> 10.1, NN 6007 x 5003 x 703
+    // (element by element, halves that share a register, it was a memory round trip for each).  No lane branches, only the whole
+    // wavefront, on a k shorter than one chunk, so all requests of both operands are out before the first is waited for.  fp16, us: TN 16 x (640 x 640 x 135) 12.1 -> 10.1, NN 6007 x 5003 x 703
     // 72.5 -> 64.6, TN 1023 x 777 x 1022 10.3 -> 9.4.
     __device__ static inline void slot(int wave, int lane, int i, uint32_t &line, uint32_t &chunk)
     {
@@ -960,7 +960,7 @@ gemm_x16_kernel(const GemmArgs args)
         // beta = 0 15.5 / 17.9 / 15.3, beta = 0.5 15.0 / 20.9 / 15.9).  In such a column a lane reads the eight rows from one before
         // its own, writes the eight from one after, and the row that is missing comes from, or belongs to, the next group down
         // the column: another lane of the same unit or the next unit's, so units are walked upwards.  At the end of the wave tile
-        // the odd rows travel alone.  ldc 1793 of the same calls: 16.3 and 18.8; 8192 x 2048 x 256, ldc 8193, 27.6 -> 20.6 and 37.5 -> 29.8.
+        // the odd rows travel alone; the cut group is read and written where it lies, on or off a dword.  ldc 1793 of the same calls: 16.3 and 18.8; 8192 x 2048 x 256, ldc 8193, 27.6 -> 20.6 and 37.5 -> 29.8.
         constexpr bool PAIRS = ESZ == 2;
         static_assert(!PAIRS || FM % 2 == 0, "fp16 blocks go out in vertical pairs");
         constexpr int FR = PAIRS ? FM / 2 : FM, UNIT_ROWS = PAIRS ? 32 : 16;          // units down a wave tile, rows of each
@@ -999,6 +999,7 @@ gemm_x16_kernel(const GemmArgs args)
         union group_t { T e[EPC]; u32x4 v; };
         // (up to 16 units, 64 registers, at a time: with 32 on the 128 x 128 wave tile the compiler ran out of registers)
         constexpr int UNITS = FR * FN, COLS = PAIRS ? (UNITS > 16 ? FN / 2 : FN) : (FN % 4 == 0 && 4 * FR <= 16) ? 4 : (FN % 2 == 0 && 2 * FR <= 16) ? 2 : 1, CHUNK = COLS * FR;
+        static_assert(FN % COLS == 0 && UNITS % CHUNK == 0 && CHUNK <= 16, "every unit belongs to one whole chunk");
         static_for<UNITS / CHUNK>([&](auto CC) {
         constexpr int j0 = decltype(CC)::value * COLS;
         group_t old_c[CHUNK];
@@ -1308,9 +1309,9 @@ gemm_x16_kernel(const GemmArgs args)
         });
         continue;
     }
-    // beta == 0: C is never read.  The aligned and the element-wise variant are separate straight-line sequences: with
-    // the choice made per block the epilogue was bound by instruction issue (64 blocks x ~20 instructions with two
-    // branches each took 7 us of a 220 us tile at 8192^3, whatever the number of work-groups writing at the time).
+    // beta == 0: C is never read.  One straight-line sequence per cache policy: with choices made per block the epilogue was
+    // bound by instruction issue (64 blocks x ~20 instructions with two branches each took 7 us of a 220 us tile at 8192^3,
+    // whatever the number of work-groups writing at the time).
     if constexpr (PAIRED_C) {
         // alpha == 1 gets a copy of the sequence without the multiplications: with the packed conversions that makes 4 (12)
         // instructions per eight results where scalar casts took 16.

@@ -1194,8 +1194,6 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     a.chip_block = cref.x16 && rr.depth * (rr.bm + rr.bn) * 64 > 80 * 1024 && nwg0 >= 16 && nwg1 >= 16;
     // batches of problems of at most 32 tiles (an XCD's CUs hold them at one time): each problem on one XCD
     a.batch_xcd = split == 1 && batch >= a.nxcd && batch % a.nxcd == 0 && nwg0 * nwg1 <= 32;
-    // (the x16 kernel's whole-tile epilogue addresses C as a buffer with 32-bit offsets: where a tile's span of C, its columns x
-    // ldc, does not fit them, C goes out element by element instead)
     auto on_lines = [&](const void *p, size_t ld, long long stride) {
         return ((uintptr_t)p % 128 == 0) && ((ld * esz) % 128 == 0) && (batch == 1 || ((size_t)stride * esz) % 128 == 0);
     };
@@ -1203,6 +1201,8 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     a.quartered = f64 ? (uint32_t)quartered_tiles(cref.tile, nwg0 * nwg1, batch, k) : 0;
     a.ws_narrow = (size_t)r.bn * m * 4 < 0x7FFFFF00ull;
     a.vec_c = aligned16(C, ldc, strideC);
+    // (the x16 kernel addresses C as a buffer with 32-bit offsets: where a tile's span of C, its columns x ldc, does not fit them, C goes
+    // out element by element instead)
     a.c_narrow = (size_t)r.bn * ldc * esz < 0x7FFFFF00ull;
     // fp16: columns on odd elements, some or all of them, leave by the epilogue that keeps its accesses to whole groups of rows on
     // dwords (a group that the edge cuts is read and written where it lies).  NT 8192 x 2048 x 256, us: C on an odd element, ldc 8192,
