@@ -369,8 +369,8 @@ struct X16Cfg {
 //   ODD_C      fp16 columns of C on odd elements, one split, narrow C (args.c_odd): every tile leaves through the edge epilogue,
 //              which moves its accesses to the dwords.
 // Code of fp16 256 x 256 TN on lines, its beta variant: 221 KB with all of it and 86 spilled scalars, 85 KB and 52 without; us,
-// on the same box: 64 x 512^3 beta = 1 TN 22.9 -> 22.2, NN 23.6 -> 22.8, NT 8192 x 2048 x 256 15.0 -> 14.7, NN 4088 x 4096 x 2052 beta = 1
-// 67.4 -> 66.5, TT 1500 x 1400 x 999 14.4 -> 13.9.
+// on the same box: 64 x 512^3 beta = 1 TN 24.1 -> 23.6, NN 24.9 -> 24.4, NT 8192 x 2048 x 256 15.1 -> 14.9, NN 4088 x 4096 x 2052 beta = 1
+// 67.2 -> 66.4, TT 1500 x 1400 x 999 14.3 -> 13.8.
 // BOTH_EVEN: the variant for two k-contiguous operands (TN) whose rows start on memory lines: both operands' pairs on the
 // even iterations (see BOTH below).  A kernel of its own, chosen by the host.
 enum class CRole { GENERAL, OLD_C, ODD_C };
