@@ -79,6 +79,24 @@ constexpr RingRow kX16Tiles[NUM_X16_TILES] = {
     {192, 256, 2, 2, 5},     // four wavefronts of 96 x 128
 };
 
+// Tiles of the kernel that multiplies fp32 operands as three bf16 planes (gemm_planes.hpp); depthU is 32.  The first two have config ids, fp32
+// only, which continue after the x16 ones:  planes_tile + kPlanesIdTiles * split_index.  The automatic pick takes all four by a rule of its own.
+constexpr int NUM_PLANES_TILES = 4;
+struct PlanesRow {
+    int bm, bn;
+    int wm, wn;       // wavefronts along M and N
+    int kg;           // groups of such wavefronts that share k
+    int sets;         // slices of fp32 elements in flight to registers
+};
+constexpr PlanesRow kPlanesTiles[NUM_PLANES_TILES] = {
+    {256, 128, 4, 2, 1, 1},     // eight wavefronts of 64 x 64, 144 KB of LDS
+    {128, 128, 2, 4, 1, 2},     // of 64 x 32, 96 KB
+    {128, 64, 2, 2, 2, 2},      // two groups of 64 x 32, 144 KB
+    {64, 64, 2, 2, 2, 4},       // two groups of 32 x 32, 96 KB
+};
+constexpr int kPlanesBk = 32;
+constexpr int kPlanesIdTiles = 2;
+
 // Tiles of the split-by-wavefront kernel (gemm_wave.hpp), all element types.  They have no config ids: the automatic pick takes
 // them by a rule of its own (mmbo_gemm.hip).
 constexpr int NUM_WAVE_TILES = 8;
@@ -102,12 +120,14 @@ constexpr int wave_tiles(int dtype) { return dtype == 2 ? 6 : NUM_WAVE_TILES; }
 constexpr int wave_max_waves(const WaveRow &r) { return 8 * r.depth * (r.bm + r.bn) * 64 <= 160 * 1024 ? 8 : 4; }
 
 // Config ids (fp32 and fp16 share them): [0, kStagedConfigs) the staged kernel's (tile, split) pairs, then the ring
-// kernel's (ring tile, split) pairs, then the x16 kernel's.  split_index indexes kSplits.
+// kernel's (ring tile, split) pairs, then the x16 kernel's; fp32 has those of the kernel on bf16 planes behind them.  split_index indexes kSplits.
 constexpr int kStagedConfigs = NUM_TILES * NUM_SPLITS;
 constexpr int kRingConfigs = NUM_RING_TILES * NUM_SPLITS;
 constexpr int kX16Base = kStagedConfigs + kRingConfigs;
 constexpr int kX16Configs = NUM_X16_TILES * NUM_SPLITS;
-constexpr int kNumConfigs = kX16Base + kX16Configs;
+constexpr int kPlanesBase = kX16Base + kX16Configs;
+constexpr int kPlanesConfigs = kPlanesIdTiles * NUM_SPLITS;
+constexpr int num_configs(int dtype) { return dtype == 0 ? kPlanesBase + kPlanesConfigs : kPlanesBase; }
 constexpr int split_index(int split)
 {
     for (int i = 0; i < NUM_SPLITS; ++i)
@@ -117,5 +137,6 @@ constexpr int split_index(int split)
 constexpr int staged_config_id(int tile, int split_idx) { return tile + NUM_TILES * split_idx; }
 constexpr int ring_config_id(int tile, int split_idx) { return kStagedConfigs + tile + NUM_RING_TILES * split_idx; }
 constexpr int x16_config_id(int tile, int split_idx) { return kX16Base + tile + NUM_X16_TILES * split_idx; }
+constexpr int planes_config_id(int tile, int split_idx) { return kPlanesBase + tile + kPlanesIdTiles * split_idx; }
 
 }  // namespace mmbo

@@ -47,6 +47,10 @@ int dgemm_lds_bytes();
 template <int DTYPE, int TILE>
 hipError_t launch_wave(int transA, int transB, const GemmArgs &args, int waves, hipStream_t stream);
 
+// fp32 kernel on three bf16 planes (gemm_planes.hpp) of planes tile row TILE; grid = (nwg0*nwg1, 1, batch*splits).
+template <int TILE>
+hipError_t launch_planes(int transA, int transB, const GemmArgs &args, hipStream_t stream);
+
 hipError_t launch_splitk_reduce(int dtype, const GemmArgs &args, hipStream_t stream);
 
 }  // namespace mmbo

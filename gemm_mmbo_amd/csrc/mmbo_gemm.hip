@@ -23,20 +23,22 @@ namespace mmbo {
 namespace {
 
 // Config ids (configs.hpp): [0, kStagedConfigs) are the staged kernel's (tile, split) pairs, then the ring kernel's
-// (ring tile, split) pairs, then the x16 kernel's.  A ring config applies when m, n are multiples of its tile, k splits
+// (ring tile, split) pairs, then the x16 kernel's, then (fp32) the bf16 planes kernel's.  A ring config applies when m, n are multiples of its tile, k splits
 // into whole slices and A, B are 16-byte aligned; otherwise the call is refused with MMBO_ERR_INVALID_CONFIG.
 struct ConfigRef {
     bool ring;      // a direct-to-LDS kernel (ring or x16)
     int tile;
     int split;
     bool x16;
+    bool planes;    // (neither ring nor x16)
 };
 inline ConfigRef config_ref(int id)
 {
-    if (id >= kX16Base) return {true, (id - kX16Base) % NUM_X16_TILES, kSplits[(id - kX16Base) / NUM_X16_TILES], true};
-    if (id < kStagedConfigs) return {false, id % NUM_TILES, kSplits[id / NUM_TILES], false};
+    if (id >= kPlanesBase) return {false, (id - kPlanesBase) % kPlanesIdTiles, kSplits[(id - kPlanesBase) / kPlanesIdTiles], false, true};
+    if (id >= kX16Base) return {true, (id - kX16Base) % NUM_X16_TILES, kSplits[(id - kX16Base) / NUM_X16_TILES], true, false};
+    if (id < kStagedConfigs) return {false, id % NUM_TILES, kSplits[id / NUM_TILES], false, false};
     id -= kStagedConfigs;
-    return {true, id % NUM_RING_TILES, kSplits[id / NUM_RING_TILES], false};
+    return {true, id % NUM_RING_TILES, kSplits[id / NUM_RING_TILES], false, false};
 }
 inline bool valid_dtype(int dtype) { return dtype == MMBO_F32 || dtype == MMBO_F16 || dtype == MMBO_F64; }
 
@@ -57,6 +59,9 @@ inline bool ring_shape_ok(int dtype, int tile, int split, int transA, int transB
     if (m % r.bm || n % r.bn || k % bk) return false;
     return (k / bk) % (size_t)split == 0;
 }
+
+// ... the kernel on bf16 planes?  Any, except a memory-contiguous dimension shorter than one 16-byte load.
+inline bool planes_shape_ok(int transA, int transB, size_t m, size_t n, size_t k) { return k >= 4 && (transA || m >= 4) && (!transB || n >= 4); }
 
 thread_local int g_last_hip_error = 0;
 
@@ -291,6 +296,14 @@ hipError_t dispatch_wave(int tile, int ta, int tb, const GemmArgs &a, int waves,
 }
 
 template <int TILE>
+hipError_t dispatch_planes(int tile, int ta, int tb, const GemmArgs &a, hipStream_t s)
+{
+    if (tile == TILE) return launch_planes<TILE>(ta, tb, a, s);
+    if constexpr (TILE + 1 < NUM_PLANES_TILES) return dispatch_planes<TILE + 1>(tile, ta, tb, a, s);
+    return hipErrorInvalidValue;
+}
+
+template <int TILE>
 hipError_t dispatch_dgemm(int tile, int ta, int tb, const GemmArgs &a, hipStream_t s)
 {
     if (tile == TILE) return launch_dgemm<TILE>(ta, tb, a, s);
@@ -470,7 +483,23 @@ const char *mmbo_status_string(int status)
 int mmbo_num_configs(int dtype)
 {
     if (!valid_dtype(dtype)) return -MMBO_ERR_INVALID_DTYPE;
-    return dtype == MMBO_F64 ? NUM_F64_TILES : kNumConfigs;
+    return dtype == MMBO_F64 ? NUM_F64_TILES : num_configs(dtype);
+}
+
+static void describe_planes(int tile, int split, mmbo_config_desc *out)
+{
+    const PlanesRow &r = kPlanesTiles[tile];
+    std::memset(out, 0, sizeof(*out));
+    std::snprintf(out->name, sizeof(out->name), "MT%03dx%03dx%02d_WT%03dx%03d_W%d_GSU%02d_LSU%02d_BF16X3", r.bm, r.bn, kPlanesBk, r.bm / r.wm,
+                  r.bn / r.wn, r.wm * r.wn * r.kg, split, r.kg);
+    out->macro_tile_m = r.bm;
+    out->macro_tile_n = r.bn;
+    out->depth_u = kPlanesBk;
+    out->threads = r.wm * r.wn * r.kg * 64;
+    out->wave_tile_m = r.bm / r.wm;
+    out->wave_tile_n = r.bn / r.wn;
+    out->split_k = split;
+    out->lds_bytes = r.kg * 2 * 3 * (r.bm + r.bn) * 64;
 }
 
 int mmbo_config_info(int dtype, int config_id, mmbo_config_desc *out)
@@ -489,6 +518,10 @@ int mmbo_config_info(int dtype, int config_id, mmbo_config_desc *out)
         return MMBO_OK;
     }
     const ConfigRef c = config_ref(config_id);
+    if (c.planes) {
+        describe_planes(c.tile, c.split, out);
+        return MMBO_OK;
+    }
     if (c.ring) {
         const RingRow &r = c.x16 ? kX16Tiles[c.tile] : kRingTiles[c.tile];
         std::snprintf(out->name, sizeof(out->name), "MT%03dx%03dx%02d_WT%03dx%03d_W%d_GSU%02d_DTL1_RING%d%s", r.bm, r.bn,
@@ -519,11 +552,14 @@ int mmbo_config_info(int dtype, int config_id, mmbo_config_desc *out)
     return MMBO_OK;
 }
 
+static TileRow planes_tile(int tile) { return TileRow{kPlanesTiles[tile].bm, kPlanesTiles[tile].bn, kPlanesBk, 0, 0}; }
+
 // Macro tile (and depthU) of a config id.
 static TileRow config_tile(int dtype, int id)
 {
     if (dtype == MMBO_F64) return kTilesF64[id];
     const ConfigRef c = config_ref(id);
+    if (c.planes) return planes_tile(c.tile);
     if (!c.ring) return tile_row(dtype, c.tile);
     const RingRow &rr = c.x16 ? kX16Tiles[c.tile] : kRingTiles[c.tile];
     return TileRow{rr.bm, rr.bn, ring_bk(dtype), 0, 0};
@@ -909,6 +945,84 @@ WavePick pick_wave(const WaveShape &p, bool may_split, double limit = 1e300)
     return best;
 }
 
+// By 8 % at least: nearer than that the models do not tell the two apart (110 drawn shapes, against the tables' configs alone:
+// 1.367 times faster in the geometric mean, two slower by over 2 %; without the margin 1.361 and seven).  Updates of a C inside a
+// much larger matrix: by 17 %.  Neither model knows where the columns of C lie; of 13 such shapes modelled up to 1.2 times faster seven
+// were slower (fp16 NT 512 x 797 x 96, ldc 44160, 5.1 -> 6.4 us), of 15 beyond that none.
+// The ring kernel's 64 x 64 tile without a split, picked for a few microseconds of work, takes 2.65 us less than its model says (55 drawn
+// shapes, 2.1 - 3.0), which matters only here: by 2.0 us, as this kernel takes 0.6 less on its smallest calls and 5 % less on the others.  us
+// here / there: fp16 TT 1024 x 640 x 512 6.4 / 5.1, TT 4 x 576 x 320 x 512 8.4 / 5.7, TN 768 x 128 x 640 4.4 / 5.5, fp32 NN 448 x 768 x 304 7.0 / 8.1.
+WavePick pick_wave_over(const WaveShape &q, bool may_split, int config_id, double table_us)
+{
+    double bar = (q.wide_c ? 0.83 : 0.92) * table_us;
+    if (q.dtype != MMBO_F64 && config_id == ring_config_id(3, 0)) bar = std::min(bar, table_us - 2.0);
+    return pick_wave(q, may_split, bar);             // (none at `bar` or beyond)
+}
+WaveShape packed_shape(int dtype, int transA, int transB, size_t m, size_t n, size_t k, int batch, bool read_c)
+{
+    return wave_shape(dtype, transA, transB, m, n, k, batch, transA ? k : m, transB ? n : k, m, read_c);
+}
+
+// ---- fp32 on the bf16 pipes (gemm_planes.hpp) -----------------------------------------------------------------------------
+
+// Modelled microseconds: work-groups run in rounds of 256, one to a CU; each costs a start and an epilogue (that reads C) and its slices
+// (a group's, where two share k), which take less where part of the chip is idle -- the clock rises --, beside that what the bytes take
+// from memory.  Constants: least squares over 12,600 times, 1,454 drawn shapes x every (tile, splits) that fits them: 5 - 7 % rms; the
+// pick is 0.4 % behind the fastest of them on average, 22 % at worst.
+double planes_model_us(int tile, int split, size_t m, size_t n, size_t k, int batch)
+{
+    static const double start[NUM_PLANES_TILES] = {5.25 + 2.52, 3.65 + 1.61, 3.96 + 0.94, 3.83 + 0.62}, slice[NUM_PLANES_TILES] = {1.803, 1.090, 1.312, 0.865},
+                        idle_chip[NUM_PLANES_TILES] = {0.848, 0.878, 0.886, 0.904};
+    const double launch = 1.67, bytes_per_us = 4.04e6, hidden = 0.126, reduce = 2.88, reduce_per_mb = 0.320;
+    const PlanesRow &r = kPlanesTiles[tile];
+    const size_t slices = ceil_div(k, (size_t)kPlanesBk), per_split = ceil_div(slices, (size_t)split), splits = ceil_div(slices, per_split);
+    const double wgs = (double)(ceil_div(m, (size_t)r.bm) * ceil_div(n, (size_t)r.bn) * splits) * batch;
+    const double c_mb = (double)m * n * batch * 4e-6;
+    auto round = [&](double busy) {
+        return start[tile] + (double)ceil_div(per_split, (size_t)r.kg) * slice[tile] * (idle_chip[tile] + (1.0 - idle_chip[tile]) * busy);
+    };
+    const double full = std::floor(wgs / 256), last = wgs - full * 256;
+    const double work = full * round(1.0) + (last > 0 ? round(last / 256) : 0.0);
+    const double memory = (((double)m * k + (double)k * n) * batch * 4.0 + c_mb * 1e6) / bytes_per_us;
+    return std::max(work, memory) + hidden * std::min(work, memory) + launch + (splits > 1 ? reduce + reduce_per_mb * c_mb * (double)splits : 0.0);
+}
+
+struct PlanesPick {
+    int tile;           // row of kPlanesTiles; < 0: none
+    int split;
+};
+
+// What the kernel is to run a shape with, where it beats what else would run it -- `us` microseconds modelled, k added up in `runs` runs -- by
+// a tenth (nearer than that the models do not tell them apart).  Partial sums (k split over work-groups) of at most max_bytes.
+// No result becomes less exact: a sum in planes has a third of the fp32 MFMAs' error, which grows with the root of a run's length, so a
+// run may be eight times as long as theirs.  k below 64 was not measured to be as exact on operands of widely different magnitudes.
+// Not for calls of a few microseconds, where a work-group has next to no slices to overlap anything with (us before / with it: TT 46 x 128 x
+// 128 x 384 10.9 / 13.0, NT 1280 x 512 x 144 6.8 / 8.2; with fewer than five slices up to 30: NT 4334 x 1152 x 128 19.9 / 26.2, but of 40 us
+// and more 1.13 - 1.2 times faster; NT 1735 x 652 x 160 11.2 / 13.2).
+PlanesPick pick_planes(int transA, int transB, size_t m, size_t n, size_t k, int batch, int runs, double us, double max_bytes)
+{
+    PlanesPick best{-1, 0};
+    double best_us = 0.90 * us;
+    if (k < 64 || us < (k < 160 ? 30.0 : k < 256 ? 16.0 : 12.0) || !planes_shape_ok(transA, transB, m, n, k)) return best;
+    for (int tile = 0; tile < NUM_PLANES_TILES; ++tile) {
+        const PlanesRow &r = kPlanesTiles[tile];
+        const size_t tiles = ceil_div(m, (size_t)r.bm) * ceil_div(n, (size_t)r.bn);
+        for (int split : kSplits) {
+            if ((size_t)batch * split > 65535) break;
+            if (split > 1 && ((double)split * batch * (double)m * (double)n * sizeof(float) > max_bytes || tiles * batch * split > 1100 ||
+                              k / kPlanesBk < (size_t)4 * r.kg * split))
+                break;
+            if (runs > 8 * split * r.kg) continue;
+            const double t = planes_model_us(tile, split, m, n, k, batch);
+            if (t < best_us) {
+                best_us = t;
+                best = PlanesPick{tile, split};
+            }
+        }
+    }
+    return best;
+}
+
 // What the automatic pick runs for a shape.  The models are walked once per shape and thread (a microsecond or two, a part of what a
 // small call takes); a small table of four ways keeps the answers, which are a function of the key alone.
 // Whether a call needs a workspace, and how large a one at most, follows from the shape alone, not from beta or leading dimensions:
@@ -916,6 +1030,7 @@ WavePick pick_wave(const WaveShape &p, bool may_split, double limit = 1e300)
 // shape whose pick of mmbo_select_config splits k is first planned with packed operands and without C.  Where that plan needs no
 // workspace, no call of the shape does; where it needs one, every call of the shape holds one as large.
 struct Plan {
+    PlanesPick planes;  // tile < 0: wave
     WavePick wave;      // tile < 0: config_id
     int config_id;
     bool workspace;     // may partial sums go through memory?
@@ -957,26 +1072,16 @@ Plan plan_for(const WaveShape &p)
     double table_us;
     plan.config_id = select_config(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, &table_us);
     const int table_split = p.dtype == MMBO_F64 ? 1 : config_ref(plan.config_id).split;
-    // By 8 % at least: nearer than that the models do not tell the two apart (110 drawn shapes, against the tables' configs alone:
-    // 1.367 times faster in the geometric mean, two slower by over 2 %; without the margin 1.361 and seven).  Updates of a C inside a
-    // much larger matrix: by 17 %.  Neither model knows where the columns of C lie; of 13 such shapes modelled up to 1.2 times faster seven
-    // were slower (fp16 NT 512 x 797 x 96, ldc 44160, 5.1 -> 6.4 us), of 15 beyond that none.
-    // The ring kernel's 64 x 64 tile without a split, picked for a few microseconds of work, takes 2.65 us less than its model says (55 drawn
-    // shapes, 2.1 - 3.0), which matters only here: by 2.0 us, as this kernel takes 0.6 less on its smallest calls and 5 % less on the others.  us
-    // here / there: fp16 TT 1024 x 640 x 512 6.4 / 5.1, TT 4 x 576 x 320 x 512 8.4 / 5.7, TN 768 x 128 x 640 4.4 / 5.5, fp32 NN 448 x 768 x 304 7.0 / 8.1.
-    auto choose = [&](const WaveShape &q, bool may_split) {
-        double bar = (q.wide_c ? 0.83 : 0.92) * table_us;
-        if (q.dtype != MMBO_F64 && plan.config_id == ring_config_id(3, 0)) bar = std::min(bar, table_us - 2.0);
-        return pick_wave(q, may_split, bar);             // (none at `bar` or beyond)
-    };
+    auto choose = [&](const WaveShape &q, bool may_split) { return pick_wave_over(q, may_split, plan.config_id, table_us); };
     plan.workspace = false;
     plan.reserve = 0;
+    const double table_bytes = (double)table_split * p.batch * p.m * p.n * sizeof(float);
+    const WaveShape packed_call = packed_shape(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, false);
+    WavePick packed{-1, 0, 0, 0};
+    if (table_split > 1) packed = choose(packed_call, true);
     if (table_split == 1) {
         plan.wave = choose(p, false);
     } else {
-        const WavePick packed = choose(wave_shape(p.dtype, p.transA, p.transB, p.m, p.n, p.k, p.batch, p.transA ? p.k : p.m,
-                                                  p.transB ? p.n : p.k, p.m, false), true);
-        const double table_bytes = (double)table_split * p.batch * p.m * p.n * sizeof(float);
         plan.workspace = packed.tile < 0 || packed.split > 1;
         if (!plan.workspace) {
             plan.wave = pick_wave(p, false);
@@ -986,13 +1091,31 @@ Plan plan_for(const WaveShape &p)
             plan.reserve = packed.tile < 0 ? (size_t)std::min(table_bytes, 1e18) : kWaveSumsBytes;
         }
     }
+    // fp32 in planes: a matter of the shape alone, as its workspace is -- against what would run the packed call without C.
+    plan.planes = PlanesPick{-1, 0};
+    if (p.dtype == MMBO_F32 && !config_ref(plan.config_id).planes) {
+        if (table_split == 1) packed = choose(packed_call, false);
+        // (the ring kernel's 64 x 64 tile takes some 2 us less than its model says: see pick_wave_over)
+        const double us = packed.tile >= 0 ? packed.us : plan.config_id == ring_config_id(3, 0) ? table_us - 2.0 : table_us;
+        WaveShape with_c = packed_call;
+        with_c.read_c = true;
+        int runs = table_split;
+        for (const WavePick &w : {packed, choose(with_c, table_split > 1)})
+            if (w.tile >= 0) runs = std::max(runs, w.waves * w.split);
+        plan.planes = pick_planes(p.transA, p.transB, p.m, p.n, p.k, p.batch, runs, us,
+                                  plan.workspace ? std::max(table_bytes, (double)kWaveSumsBytes) : 0.0);
+        if (plan.planes.tile >= 0 && plan.planes.split > 1)
+            plan.reserve = std::max(plan.reserve, (size_t)plan.planes.split * p.batch * p.m * p.n * sizeof(float));
+    }
     set.way[set.next] = Entry{true, key, plan};
     set.next = (set.next + 1) % kWays;
     return plan;
 }
 
-// What MMBO_CONFIG_AUTO runs: the split-by-wavefront kernel, which takes any shape and alignment, or a config.
+// What MMBO_CONFIG_AUTO runs: the kernel on bf16 planes or the split-by-wavefront kernel, which take any alignment, or a config.
 struct Route {
+    bool planes;
+    PlanesPick planes_pick;
     bool wave;
     WavePick pick;
     int config_id;
@@ -1008,12 +1131,17 @@ int route_for(const WaveShape &p, bool aligned16, WsSource ws_source, Route &r)
     const Plan plan = plan_for(p);
     r.pick = plan.wave;
     r.reserve = plan.reserve;
+    r.planes_pick = plan.planes;
+    if (ws_source == WsSource::kStatic)      // partial sums that fit the array of the entry point that allocates nothing
+        while (r.planes_pick.split > 1 && (double)r.planes_pick.split * p.batch * (double)p.m * (double)p.n * sizeof(float) > (double)kScratchPartialBytes)
+            r.planes_pick.split /= 2;
+    r.planes = plan.planes.tile >= 0 && tile_span_ok(planes_tile(plan.planes.tile), p.transA, p.transB, p.lda, p.ldb, esz);
     // (a pair of slices must span less than the 2 GiB of a buffer descriptor)
     r.wave = plan.wave.tile >= 0 &&
              tile_span_ok(TileRow{kWaveTiles[plan.wave.tile].bm, kWaveTiles[plan.wave.tile].bn, (int)(2 * 64 / esz), 0, 0}, p.transA, p.transB,
                           p.lda, p.ldb, esz);
     int id = r.config_id = plan.config_id;
-    if (r.wave) return MMBO_OK;
+    if (r.planes || r.wave) return MMBO_OK;
     const bool f64 = p.dtype == MMBO_F64;
     // The pick is made from the shape alone.  The ring kernels also need 16-byte aligned A and B, every
     // direct-to-LDS kernel a tile's span of an operand below 2 GiB: where the operands at hand do not qualify, the
@@ -1040,10 +1168,10 @@ int route_for(const WaveShape &p, bool aligned16, WsSource ws_source, Route &r)
             if (kSplits[sidx] == 1) return true;
             if (!plan.workspace) return false;
             if ((double)kSplits[sidx] * p.batch * (double)p.m * (double)p.n * sizeof(float) > (double)kScratchPartialBytes) return false;
-            return !c.ring || ring_shape_ok(p.dtype, c.tile, kSplits[sidx], p.transA, p.transB, p.m, p.n, p.k, c.x16);
+            return c.planes || !c.ring || ring_shape_ok(p.dtype, c.tile, kSplits[sidx], p.transA, p.transB, p.m, p.n, p.k, c.x16);
         };
         while (si > 0 && !fits(si)) --si;
-        id = c.x16 ? x16_config_id(c.tile, si) : c.ring ? ring_config_id(c.tile, si) : staged_config_id(c.tile, si);
+        id = c.planes ? planes_config_id(c.tile, si) : c.x16 ? x16_config_id(c.tile, si) : c.ring ? ring_config_id(c.tile, si) : staged_config_id(c.tile, si);
     }
     if (!tile_span_ok(config_tile(p.dtype, id), p.transA, p.transB, p.lda, p.ldb, esz)) {
         // enormous leading dimensions: the first staged tile (no split-K) whose span fits, large tiles first
@@ -1054,6 +1182,24 @@ int route_for(const WaveShape &p, bool aligned16, WsSource ws_source, Route &r)
         if (id < 0) return MMBO_ERR_INVALID_SIZE;
     }
     r.config_id = id;
+    return MMBO_OK;
+}
+
+// The partial sums' buffer of a call that needs `needed` bytes (0: none), in a.ws; a call of the library's own workspace sees to
+// `reserve` bytes as well.
+int hold_workspace(hipStream_t s, WsSource ws_source, size_t needed, size_t reserve, WsHold &hold, GemmArgs &a)
+{
+    size_t bytes = needed;
+    if (ws_source == WsSource::kLibrary && reserve > (needed > 0 ? std::max(needed, kWaveSumsBytes) : 0)) {
+        // (a call under capture takes what is there: it cannot allocate, nor must it where it needs nothing)
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) bytes = std::max(bytes, reserve);
+    }
+    if (bytes == 0) return MMBO_OK;
+    char *base = nullptr;
+    const int rc = ws_source == WsSource::kStatic ? static_scratch(&base) : workspace(s, bytes, hold, &base);
+    if (rc != MMBO_OK && needed > 0) return rc;
+    a.ws = reinterpret_cast<float *>(base);
     return MMBO_OK;
 }
 
@@ -1082,18 +1228,7 @@ int run_wave(const WaveShape &p, const WavePick &w, GemmArgs &a, hipStream_t s, 
     a.vec_c = ((uintptr_t)a.C % 16 == 0) && ((a.ldc * esz) % 16 == 0) && (((size_t)a.strideC * esz) % 16 == 0);
     WsHold ws_hold;
     const size_t needed = a.splits > 1 ? (size_t)a.splits * p.batch * p.m * p.n * sizeof(float) : 0;
-    size_t bytes = needed;
-    if (ws_source == WsSource::kLibrary && reserve > (needed > 0 ? kWaveSumsBytes : 0)) {
-        // (a call under capture takes what is there: it cannot allocate, nor must it where it needs nothing)
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) bytes = std::max(bytes, reserve);
-    }
-    if (bytes > 0) {
-        char *base = nullptr;
-        int rc = ws_source == WsSource::kStatic ? static_scratch(&base) : workspace(s, bytes, ws_hold, &base);
-        if (rc != MMBO_OK && needed > 0) return rc;
-        a.ws = reinterpret_cast<float *>(base);
-    }
+    if (int rc = hold_workspace(s, ws_source, needed, reserve, ws_hold, a)) return rc;
     hipError_t e = p.dtype == MMBO_F64 ? dispatch_wave<2, 0>(w.tile, p.transA, p.transB, a, w.waves, s)
                    : p.dtype == MMBO_F32 ? dispatch_wave<0, 0>(w.tile, p.transA, p.transB, a, w.waves, s)
                                          : dispatch_wave<1, 0>(w.tile, p.transA, p.transB, a, w.waves, s);
@@ -1124,7 +1259,7 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
               const void *alpha, const void *A, size_t lda, long long strideA,
               const void *B, size_t ldb, long long strideB, const void *beta, void *C,
               size_t ldc, long long strideC, int batch, int config_id, void *stream, WsSource ws_source,
-              const WavePick *named_wave = nullptr)
+              const WavePick *named_wave = nullptr, const PlanesPick *named_planes = nullptr)
 {
     if (!valid_dtype(dtype)) return MMBO_ERR_INVALID_DTYPE;
     if ((transA & ~1) || (transB & ~1)) return MMBO_ERR_INVALID_OP;
@@ -1159,18 +1294,26 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     a.vec_b = aligned16(B, ldb, strideB);
     hipStream_t s = static_cast<hipStream_t>(stream);
 
-    if (config_id == MMBO_CONFIG_AUTO) {
+    PlanesPick planes{-1, 0};
+    size_t reserve = 0;
+    if (named_planes) {
+        planes = *named_planes;
+    } else if (config_id == MMBO_CONFIG_AUTO) {
         const WaveShape p = wave_shape(dtype, transA, transB, m, n, k, batch, lda, ldb, ldc, f64 ? beta_d != 0.0 : beta_f != 0.0f);
         if (named_wave) return run_wave(p, *named_wave, a, s, ws_source, 0);
         Route r;
         if (int rc = route_for(p, a.vec_a && a.vec_b, ws_source, r)) return rc;
-        if (r.wave) return run_wave(p, r.pick, a, s, ws_source, r.reserve);
+        if (r.planes) planes = r.planes_pick;
+        else if (r.wave) return run_wave(p, r.pick, a, s, ws_source, r.reserve);
         config_id = r.config_id;
+        if (dtype == MMBO_F32) reserve = r.reserve;
     }
-    const ConfigRef cref = f64 ? ConfigRef{false, config_id, 1, false} : config_ref(config_id);
+    const ConfigRef cref = planes.tile >= 0 ? ConfigRef{false, planes.tile, planes.split, false, true}
+                           : f64 ? ConfigRef{false, config_id, 1, false, false} : config_ref(config_id);
     int split = cref.split;
     const RingRow &rr = cref.x16 ? kX16Tiles[cref.tile] : kRingTiles[cref.ring ? cref.tile : 0];
-    TileRow r = f64 ? kTilesF64[config_id] : cref.ring ? TileRow{rr.bm, rr.bn, ring_bk(dtype), 0, 0} : tile_row(dtype, cref.tile);
+    const TileRow r = cref.planes ? planes_tile(cref.tile) : config_tile(dtype, config_id);
+    if (cref.planes && !planes_shape_ok(transA, transB, m, n, k)) return MMBO_ERR_INVALID_CONFIG;
     if (cref.ring && !ring_shape_ok(dtype, cref.tile, split, transA, transB, m, n, k, cref.x16)) return MMBO_ERR_INVALID_CONFIG;
 
     if (!tile_span_ok(r, transA, transB, lda, ldb, esz)) return MMBO_ERR_INVALID_CONFIG;
@@ -1223,22 +1366,13 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     // Split-K: the partial sums go to the stream's own workspace (or the static one), and both launches that use it (the
     // GEMM and the reduction, which adds the splits in a fixed order) are queued before the hold on that workspace
     // is given up.
+    const size_t needed = split > 1 ? (size_t)split * batch * m * n * sizeof(float) : 0;
+    if (ws_source == WsSource::kStatic && needed > kScratchPartialBytes) return MMBO_ERR_WORKSPACE;
     WsHold ws_hold;
-    if (split > 1) {
-        const size_t bytes = (size_t)split * batch * m * n * sizeof(float);
-        char *base = nullptr;
-        if (ws_source == WsSource::kStatic) {
-            if (bytes > kScratchPartialBytes) return MMBO_ERR_WORKSPACE;
-            int rc = static_scratch(&base);
-            if (rc != MMBO_OK) return rc;
-        } else {
-            int rc = workspace(s, bytes, ws_hold, &base);
-            if (rc != MMBO_OK) return rc;
-        }
-        a.ws = reinterpret_cast<float *>(base);
-    }
+    if (int rc = hold_workspace(s, ws_source, needed, reserve, ws_hold, a)) return rc;
     hipError_t e;
     if (f64) e = dispatch_dgemm<0>(cref.tile, transA, transB, a, s);
+    else if (cref.planes) e = dispatch_planes<0>(cref.tile, transA, transB, a, s);
     else if (cref.x16) e = dtype == MMBO_F32 ? dispatch_x16<0, 0>(cref.tile, transA, transB, a, s)
                                         : dispatch_x16<1, 0>(cref.tile, transA, transB, a, s);
     else if (cref.ring) e = dtype == MMBO_F32 ? dispatch_ring<0, 0>(cref.tile, transA, transB, a, s)
@@ -1262,11 +1396,17 @@ int mmbo_auto_info(int dtype, int transA, int transB, size_t m, size_t n, size_t
 {
     if (!config_id || !out) return MMBO_ERR_NULL_POINTER;
     if (int rc = check_problem(dtype, transA, transB, m, n, k, lda, ldb, ldc, batch)) return rc;
-    Route r{false, {}, 0, 0};
+    Route r{};
     if (m != 0 && n != 0 && batch != 0) {
         const size_t esz = element_size(dtype);
         const bool aligned16 = (lda * esz) % 16 == 0 && (ldb * esz) % 16 == 0;
         if (int rc = route_for(wave_shape(dtype, transA, transB, m, n, k, batch, lda, ldb, ldc, reads_c != 0), aligned16, WsSource::kLibrary, r)) return rc;
+    }
+    if (r.planes) {
+        const bool has_id = r.planes_pick.tile < kPlanesIdTiles;
+        *config_id = has_id ? planes_config_id(r.planes_pick.tile, split_index(r.planes_pick.split)) : MMBO_CONFIG_AUTO;
+        describe_planes(r.planes_pick.tile, r.planes_pick.split, out);
+        return MMBO_OK;
     }
     if (!r.wave) {
         *config_id = r.config_id;
@@ -1311,6 +1451,17 @@ int mmbo_internal_wave_gemm(int dtype, int transA, int transB, size_t m, size_t 
     const WavePick pick{tile, waves, split, 0.0};
     return gemm_impl(dtype, transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch,
                      MMBO_CONFIG_AUTO, stream, WsSource::kLibrary, &pick);
+}
+
+// Not part of the interface: mmbo_gemm_strided_batched (fp32) on a given row of kPlanesTiles with a given GlobalSplitU.
+int mmbo_internal_planes_gemm(int transA, int transB, size_t m, size_t n, size_t k, const void *alpha, const void *A, size_t lda,
+                              long long strideA, const void *B, size_t ldb, long long strideB, const void *beta, void *C, size_t ldc,
+                              long long strideC, int batch, int tile, int split, void *stream)
+{
+    if (tile < 0 || tile >= NUM_PLANES_TILES || split < 1 || split > 16) return MMBO_ERR_INVALID_CONFIG;
+    const PlanesPick pick{tile, split};
+    return gemm_impl(MMBO_F32, transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch,
+                     MMBO_CONFIG_AUTO, stream, WsSource::kLibrary, nullptr, &pick);
 }
 
 int mmbo_gemm_strided_batched(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
