@@ -43,6 +43,10 @@ class ConfigDesc(ctypes.Structure):
 
 
 _lib = None
+try:
+    from . import _frontend             # the GEMM front-ends without ctypes (csrc/frontend.cc); without it they are the functions below
+except ImportError:
+    _frontend = None
 
 
 def lib():
@@ -98,6 +102,9 @@ def lib():
         L.mmbo_status_string.restype = ctypes.c_char_p
         L.mmbo_last_hip_error.restype = ci
         L.mmbo_version.restype = ctypes.c_char_p
+        if _frontend is not None:
+            _frontend.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in
+                             (L.mmbo_gemm, L.mmbo_gemm_strided_batched, L.mmbo_gemm_strided_batched_static_workspace)))
         _lib = L
     return _lib
 
@@ -157,6 +164,14 @@ def gemm_strided_batched_static_workspace(dtype, transA, transB, m, n, k, alpha,
                                                             lda, strideA, _devptr(B), ldb, strideB, ctypes.byref(be),
                                                             _devptr(C), ldc, strideC, batch, config_id,
                                                             _stream_handle(stream)))
+
+
+_PYTHON_FRONT_ENDS = (gemm, gemm_strided_batched, gemm_strided_batched_static_workspace)
+if _frontend is not None:
+    # plain calls go straight to the C ABI, all others to the functions above
+    _frontend.setup(*_PYTHON_FRONT_ENDS, _check)
+    gemm, gemm_strided_batched = _frontend.gemm, _frontend.gemm_strided_batched
+    gemm_strided_batched_static_workspace = _frontend.gemm_strided_batched_static_workspace
 
 
 def static_workspace_bytes():

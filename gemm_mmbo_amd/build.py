@@ -3,17 +3,20 @@
     python -m gemm_mmbo_amd.build [--force]
 
 Each (element type, tile row) pair is its own translation unit so the kernels compile in
-parallel; objects go to gemm_mmbo_amd/csrc/build/, the library to gemm_mmbo_amd/csrc/.
+parallel; objects go to gemm_mmbo_amd/csrc/build/, the library to gemm_mmbo_amd/csrc/.  The CPython module of the Python front-ends
+(csrc/frontend.cc, host code) is built beside this file.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(CSRC, "libmmbo_gemm.so")
+FRONTEND = os.path.join(HERE, "_frontend" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 NUM_TILES = 6  # keep in step with csrc/configs.hpp
 NUM_RING_TILES = 4
@@ -111,6 +114,18 @@ def _compile(unit, force, newest_dep):
     return obj, "compiled"
 
 
+def _build_frontend(force, newest_dep):
+    src = os.path.join(CSRC, "frontend.cc")
+    if not force and os.path.exists(FRONTEND) and os.path.getmtime(FRONTEND) >= max(newest_dep, os.path.getmtime(src)):
+        return "up to date"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-I" + sysconfig.get_paths()["include"], src,
+           "-o", FRONTEND]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"building {FRONTEND} failed:\n{' '.join(cmd)}\n{r.stderr[-4000:]}")
+    return "compiled"
+
+
 def build(force=False, verbose=True, jobs=None):
     os.makedirs(OBJ, exist_ok=True)
     _check_toolchain(verbose)
@@ -119,6 +134,7 @@ def build(force=False, verbose=True, jobs=None):
     jobs = jobs or min(8, os.cpu_count() or 1)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         results = list(ex.map(lambda u: _compile(u, force, newest), units))
+    results.append((os.path.basename(FRONTEND), _build_frontend(force, newest)))
     if verbose:
         for obj, what in results:
             print(f"  {obj}: {what}")
