@@ -23,6 +23,7 @@ NUM_RING_TILES = 4
 NUM_F64_TILES = 6
 NUM_X16_TILES = 8
 NUM_PLANES_TILES = 4
+NUM_DOTS_TILES = 6
 NUM_WAVE_TILES = {0: 8, 1: 8, 2: 6}  # by element type (fp32, fp16, fp64)
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -83,6 +84,8 @@ def _units():
             units.append(("inst_wave.hip", f"inst_wave_{dtype}_{tile}.o", [f"-DMMBO_DTYPE={dtype}", f"-DMMBO_TILE={tile}"]))
     for tile in range(NUM_PLANES_TILES):
         units.append(("inst_planes.hip", f"inst_planes_{tile}.o", [f"-DMMBO_TILE={tile}"]))
+    for tile in range(NUM_DOTS_TILES):
+        units.append(("inst_dots.hip", f"inst_dots_{tile}.o", [f"-DMMBO_TILE={tile}"]))
     for tile in range(NUM_F64_TILES):
         units.append(("inst_dgemm.hip", f"inst_dgemm_{tile}.o", [f"-DMMBO_TILE={tile}"]))
     return units

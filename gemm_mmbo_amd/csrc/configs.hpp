@@ -119,6 +119,16 @@ constexpr int wave_tiles(int dtype) { return dtype == 2 ? 6 : NUM_WAVE_TILES; }
 // wavefronts of a work-group that share k, at most: eight where their rings fit the 160 KB of LDS
 constexpr int wave_max_waves(const WaveRow &r) { return 8 * r.depth * (r.bm + r.bn) * 64 <= 160 * 1024 ? 8 : 4; }
 
+// Tiles of the fp64 kernel for small results of long sums (gemm_dots.hpp); no config ids either.
+constexpr int NUM_DOTS_TILES = 6;
+struct DotsRow {
+    int fm, fn;       // blocks of four rows, of four columns
+    int depth;        // steps in a wavefront's LDS ring
+};
+constexpr DotsRow kDotsTiles[NUM_DOTS_TILES] = {{1, 1, 8}, {1, 2, 6}, {2, 1, 6}, {2, 2, 4}, {2, 4, 3}, {4, 2, 3}};
+constexpr int kDotsWaves = 8;
+constexpr int kDotsStep = 32;
+
 // Config ids (fp32 and fp16 share them): [0, kStagedConfigs) the staged kernel's (tile, split) pairs, then the ring
 // kernel's (ring tile, split) pairs, then the x16 kernel's; fp32 has those of the kernel on bf16 planes behind them.  split_index indexes kSplits.
 constexpr int kStagedConfigs = NUM_TILES * NUM_SPLITS;

@@ -51,6 +51,10 @@ hipError_t launch_wave(int transA, int transB, const GemmArgs &args, int waves, 
 template <int TILE>
 hipError_t launch_planes(int transA, int transB, const GemmArgs &args, hipStream_t stream);
 
+// fp64 kernel for small results of long sums (gemm_dots.hpp) of dots tile row TILE; grid = (batch, nwg0*nwg1).
+template <int TILE>
+hipError_t launch_dots(int transA, int transB, const GemmArgs &args, hipStream_t stream);
+
 hipError_t launch_splitk_reduce(int dtype, const GemmArgs &args, hipStream_t stream);
 
 }  // namespace mmbo

@@ -296,6 +296,14 @@ hipError_t dispatch_wave(int tile, int ta, int tb, const GemmArgs &a, int waves,
 }
 
 template <int TILE>
+hipError_t dispatch_dots(int tile, int ta, int tb, const GemmArgs &a, hipStream_t s)
+{
+    if (tile == TILE) return launch_dots<TILE>(ta, tb, a, s);
+    if constexpr (TILE + 1 < NUM_DOTS_TILES) return dispatch_dots<TILE + 1>(tile, ta, tb, a, s);
+    return hipErrorInvalidValue;
+}
+
+template <int TILE>
 hipError_t dispatch_planes(int tile, int ta, int tb, const GemmArgs &a, hipStream_t s)
 {
     if (tile == TILE) return launch_planes<TILE>(ta, tb, a, s);
@@ -1023,6 +1031,66 @@ PlanesPick pick_planes(int transA, int transB, size_t m, size_t n, size_t k, int
     return best;
 }
 
+// ---- fp64 sums without a split over work-groups (gemm_dots.hpp) -------------------------------------------------------
+
+// (a pair of rows that the edge cuts is the two that end there, so a row-contiguous operand has two at least)
+bool dots_shape_ok(int tile, int transA, int transB, size_t m, size_t n, size_t k)
+{
+    const DotsRow &r = kDotsTiles[tile];
+    return k > 0 && (transA || m >= 2) && (!transB || n >= 2) &&
+           ceil_div(m, 4 * (size_t)r.fm) * ceil_div(n, 4 * (size_t)r.fn) <= 65535;
+}
+// (its tiles' own spans are smaller, but a call that no config of the tables may take is refused: what the smallest of them, 32 x 32, takes)
+bool dots_span_ok(int transA, int transB, size_t lda, size_t ldb)
+{
+    return tile_span_ok(TileRow{32, 32, kDotsStep, 0, 0}, transA, transB, lda, ldb, sizeof(double));
+}
+
+// Modelled microseconds: work-groups run in rounds of 256, one to a CU; each costs a start and its steps, a step as long as the slowest of the
+// lines its CU pulls, the lines all CUs pull, and its products; a wavefront's steps share round trips.  Beside that what the bytes take from
+// memory, and C, which goes element by element.  Constants: least squares over 7,100 times, 1,192 drawn shapes x every tile: 12 % rms.
+double dots_model_us(const WaveShape &p, int tile)
+{
+    const double launch = 1.62, start = 0.705, cu_bytes = 110.6e3, chip_bytes = 24.5e6, block = 0.0033, load = 0.0104, round_trips = 1.92 / 8,
+                 memory_bytes = 7.64e6, hidden = 0.72, c_us = 37.7e-6;
+    const DotsRow &r = kDotsTiles[tile];
+    auto lines = [&](int rows, size_t dim, bool k_contiguous, size_t ld) {
+        const double here = (double)std::min((size_t)rows, ceil_div(dim, (size_t)4) * 4);
+        const bool on_lines = ld % 16 == 0;
+        if (k_contiguous) return here * kDotsStep * 8 * (on_lines ? 1.0 : 1.25);
+        return kDotsStep * (on_lines ? 128.0 : here * 8 + 112);
+    };
+    const double line_bytes = lines(4 * r.fm, p.m, p.transA, p.lda) + lines(4 * r.fn, p.n, !p.transB, p.ldb);
+    const double steps = (double)p.k / kDotsStep, wgs = (double)(ceil_div(p.m, 4 * (size_t)r.fm) * ceil_div(p.n, 4 * (size_t)r.fn)) * p.batch;
+    auto round = [&](double busy) {
+        const double step = std::max(std::max(line_bytes / cu_bytes, line_bytes * busy / chip_bytes), r.fm * r.fn * block + (r.fm + r.fn) * load);
+        return start + std::max(steps * step, round_trips * std::ceil(steps / kDotsWaves));
+    };
+    const double full = std::floor(wgs / 256), last = wgs - 256 * full, c = (double)p.m * p.n * p.batch;
+    const double work = full * round(256) + (last > 0 ? round(last) : 0.0);
+    const double memory = ((double)p.m * p.k + (double)p.k * p.n) * p.batch * 8 / memory_bytes + c * (p.read_c ? 16 : 8) / memory_bytes;
+    return std::max(launch + std::max(work, memory) + hidden * std::min(work, memory) + c * c_us, 5.1);
+}
+
+// The row of kDotsTiles to run a shape on, where it beats the `us` microseconds modelled of what else would by a tenth, below 7 us and with two
+// row-contiguous operands -- each line that their narrow tiles touch is partly others' -- by a sixth; -1: none.  (6,518 drawn fp64 shapes, with
+// a tenth for all: taken for 645, which went 1.62 times faster in the geometric mean -- 2.1 - 2.6 with two k-contiguous operands,
+// 1.1 - 1.4 with none --, 14 slower by over 3 %, eight of them with none and four more below 7 us.)
+int pick_dots(const WaveShape &p, double us)
+{
+    int best = -1;
+    double best_us = (us < 7.0 || (!p.transA && p.transB) ? 0.84 : 0.90) * us;
+    for (int tile = 0; tile < NUM_DOTS_TILES; ++tile) {
+        if (!dots_shape_ok(tile, p.transA, p.transB, p.m, p.n, p.k)) continue;
+        const double t = dots_model_us(p, tile);
+        if (t < best_us) {
+            best_us = t;
+            best = tile;
+        }
+    }
+    return best;
+}
+
 // What the automatic pick runs for a shape.  The models are walked once per shape and thread (a microsecond or two, a part of what a
 // small call takes); a small table of four ways keeps the answers, which are a function of the key alone.
 // Whether a call needs a workspace, and how large a one at most, follows from the shape alone, not from beta or leading dimensions:
@@ -1030,7 +1098,8 @@ PlanesPick pick_planes(int transA, int transB, size_t m, size_t n, size_t k, int
 // shape whose pick of mmbo_select_config splits k is first planned with packed operands and without C.  Where that plan needs no
 // workspace, no call of the shape does; where it needs one, every call of the shape holds one as large.
 struct Plan {
-    PlanesPick planes;  // tile < 0: wave
+    PlanesPick planes;  // tile < 0: dots
+    int dots;           // row of kDotsTiles; < 0: wave
     WavePick wave;      // tile < 0: config_id
     int config_id;
     bool workspace;     // may partial sums go through memory?
@@ -1107,15 +1176,19 @@ Plan plan_for(const WaveShape &p)
         if (plan.planes.tile >= 0 && plan.planes.split > 1)
             plan.reserve = std::max(plan.reserve, (size_t)plan.planes.split * p.batch * p.m * p.n * sizeof(float));
     }
+    plan.dots = p.dtype == MMBO_F64 ? pick_dots(p, plan.wave.tile >= 0 ? plan.wave.us : table_us) : -1;
     set.way[set.next] = Entry{true, key, plan};
     set.next = (set.next + 1) % kWays;
     return plan;
 }
 
-// What MMBO_CONFIG_AUTO runs: the kernel on bf16 planes or the split-by-wavefront kernel, which take any alignment, or a config.
+// What MMBO_CONFIG_AUTO runs: the kernel on bf16 planes, that for small results of long sums or the split-by-wavefront kernel, which take any
+// alignment, or a config.
 struct Route {
     bool planes;
     PlanesPick planes_pick;
+    bool dots;
+    int dots_tile;
     bool wave;
     WavePick pick;
     int config_id;
@@ -1136,12 +1209,14 @@ int route_for(const WaveShape &p, bool aligned16, WsSource ws_source, Route &r)
         while (r.planes_pick.split > 1 && (double)r.planes_pick.split * p.batch * (double)p.m * (double)p.n * sizeof(float) > (double)kScratchPartialBytes)
             r.planes_pick.split /= 2;
     r.planes = plan.planes.tile >= 0 && tile_span_ok(planes_tile(plan.planes.tile), p.transA, p.transB, p.lda, p.ldb, esz);
+    r.dots_tile = plan.dots;
+    r.dots = plan.dots >= 0 && dots_span_ok(p.transA, p.transB, p.lda, p.ldb);
     // (a pair of slices must span less than the 2 GiB of a buffer descriptor)
     r.wave = plan.wave.tile >= 0 &&
              tile_span_ok(TileRow{kWaveTiles[plan.wave.tile].bm, kWaveTiles[plan.wave.tile].bn, (int)(2 * 64 / esz), 0, 0}, p.transA, p.transB,
                           p.lda, p.ldb, esz);
     int id = r.config_id = plan.config_id;
-    if (r.planes || r.wave) return MMBO_OK;
+    if (r.planes || r.dots || r.wave) return MMBO_OK;
     const bool f64 = p.dtype == MMBO_F64;
     // The pick is made from the shape alone.  The ring kernels also need 16-byte aligned A and B, every
     // direct-to-LDS kernel a tile's span of an operand below 2 GiB: where the operands at hand do not qualify, the
@@ -1240,6 +1315,16 @@ int run_wave(const WaveShape &p, const WavePick &w, GemmArgs &a, hipStream_t s, 
     return MMBO_OK;
 }
 
+// The fp64 kernel for small results of long sums on row `tile` of kDotsTiles.
+int run_dots(const WaveShape &p, int tile, GemmArgs &a, hipStream_t s)
+{
+    const DotsRow &r = kDotsTiles[tile];
+    a.nwg0 = (uint32_t)ceil_div(p.m, 4 * r.fm); a.nwg1 = (uint32_t)ceil_div(p.n, 4 * r.fn);
+    a.columns_first = a.nwg1 > a.nwg0;
+    const hipError_t e = dispatch_dots<0>(tile, p.transA, p.transB, a, s);
+    return e == hipSuccess ? MMBO_OK : hip_fail(e);
+}
+
 // What both entry points and the queries check of a problem before anything else.
 int check_problem(int dtype, int transA, int transB, size_t m, size_t n, size_t k, size_t lda, size_t ldb, size_t ldc, int batch)
 {
@@ -1259,7 +1344,7 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
               const void *alpha, const void *A, size_t lda, long long strideA,
               const void *B, size_t ldb, long long strideB, const void *beta, void *C,
               size_t ldc, long long strideC, int batch, int config_id, void *stream, WsSource ws_source,
-              const WavePick *named_wave = nullptr, const PlanesPick *named_planes = nullptr)
+              const WavePick *named_wave = nullptr, const PlanesPick *named_planes = nullptr, const int *named_dots = nullptr)
 {
     if (!valid_dtype(dtype)) return MMBO_ERR_INVALID_DTYPE;
     if ((transA & ~1) || (transB & ~1)) return MMBO_ERR_INVALID_OP;
@@ -1301,9 +1386,11 @@ int gemm_impl(int dtype, int transA, int transB, size_t m, size_t n, size_t k,
     } else if (config_id == MMBO_CONFIG_AUTO) {
         const WaveShape p = wave_shape(dtype, transA, transB, m, n, k, batch, lda, ldb, ldc, f64 ? beta_d != 0.0 : beta_f != 0.0f);
         if (named_wave) return run_wave(p, *named_wave, a, s, ws_source, 0);
+        if (named_dots) return run_dots(p, *named_dots, a, s);
         Route r;
         if (int rc = route_for(p, a.vec_a && a.vec_b, ws_source, r)) return rc;
         if (r.planes) planes = r.planes_pick;
+        else if (r.dots) return run_dots(p, r.dots_tile, a, s);
         else if (r.wave) return run_wave(p, r.pick, a, s, ws_source, r.reserve);
         config_id = r.config_id;
         if (dtype == MMBO_F32) reserve = r.reserve;
@@ -1408,6 +1495,21 @@ int mmbo_auto_info(int dtype, int transA, int transB, size_t m, size_t n, size_t
         describe_planes(r.planes_pick.tile, r.planes_pick.split, out);
         return MMBO_OK;
     }
+    if (r.dots) {
+        const DotsRow &row = kDotsTiles[r.dots_tile];
+        std::memset(out, 0, sizeof(*out));
+        const int bm = 4 * row.fm, bn = 4 * row.fn;
+        std::snprintf(out->name, sizeof(out->name), "MT%03dx%03dx%02d_WT%03dx%03d_W%d_GSU01_LSU%02d_DTL1_DOTS%d", bm, bn, kDotsStep, bm, bn,
+                      kDotsWaves, kDotsWaves, row.depth);
+        out->macro_tile_m = out->wave_tile_m = bm;
+        out->macro_tile_n = out->wave_tile_n = bn;
+        out->depth_u = kDotsStep;
+        out->threads = kDotsWaves * 64;
+        out->split_k = 1;
+        out->lds_bytes = kDotsWaves * row.depth * (row.fm + row.fn) * 1024;
+        *config_id = MMBO_CONFIG_AUTO;
+        return MMBO_OK;
+    }
     if (!r.wave) {
         *config_id = r.config_id;
         return mmbo_config_info(dtype, r.config_id, out);
@@ -1462,6 +1564,18 @@ int mmbo_internal_planes_gemm(int transA, int transB, size_t m, size_t n, size_t
     const PlanesPick pick{tile, split};
     return gemm_impl(MMBO_F32, transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch,
                      MMBO_CONFIG_AUTO, stream, WsSource::kLibrary, nullptr, &pick);
+}
+
+// Not part of the interface: mmbo_gemm_strided_batched (fp64) on a given row of kDotsTiles.
+int mmbo_internal_dots_gemm(int transA, int transB, size_t m, size_t n, size_t k, const void *alpha, const void *A, size_t lda,
+                            long long strideA, const void *B, size_t ldb, long long strideB, const void *beta, void *C, size_t ldc,
+                            long long strideC, int batch, int tile, void *stream)
+{
+    if (tile < 0 || tile >= NUM_DOTS_TILES) return MMBO_ERR_INVALID_CONFIG;
+    if (int rc = check_problem(MMBO_F64, transA, transB, m, n, k, lda, ldb, ldc, batch)) return rc;
+    if (!dots_shape_ok(tile, transA, transB, m, n, k) || !dots_span_ok(transA, transB, lda, ldb)) return MMBO_ERR_INVALID_SIZE;
+    return gemm_impl(MMBO_F64, transA, transB, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch,
+                     MMBO_CONFIG_AUTO, stream, WsSource::kLibrary, nullptr, nullptr, &tile);
 }
 
 int mmbo_gemm_strided_batched(int dtype, int transA, int transB, size_t m, size_t n, size_t k,

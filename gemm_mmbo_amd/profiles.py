@@ -44,7 +44,7 @@ import time
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PEAK_TFLOPS = {"h": 2500.0, "s": 157.3, "d": 78.6}
 ESZ = {"h": 2, "s": 4, "d": 8}
-LIB_KERNEL = re.compile(r"mmbo(::|\d+)?.*(gemm_x16_kernel|gemm_ring_kernel|gemm_staged_kernel|gemm_wave_kernel|gemm_planes_kernel|dgemm_kernel|splitk_reduce_kernel)")
+LIB_KERNEL = re.compile(r"mmbo(::|\d+)?.*(gemm_x16_kernel|gemm_ring_kernel|gemm_staged_kernel|gemm_wave_kernel|gemm_planes_kernel|gemm_dots_kernel|dgemm_kernel|splitk_reduce_kernel)")
 LONG_KERNEL_NS = 200e3          # below this GRBM_GUI_ACTIVE is not a clock measurement
 
 SQ_COUNTERS = ["SQ_VALU_MFMA_BUSY_CYCLES", "SQ_BUSY_CYCLES", "SQ_WAVE_CYCLES", "SQ_INSTS_VALU_MFMA_MOPS_F16",
