@@ -953,6 +953,25 @@ WavePick pick_wave(const WaveShape &p, bool may_split, double limit = 1e300)
     return best;
 }
 
+// What the staged kernel takes where mmbo_select_config picks it, in place of the `us` of that pick's model.  The model knows the tiles of a few
+// large problems; the calls that still come to this kernel are batches of narrow problems and operands with less than 16 bytes of m or
+// n in memory, whose rounds of short work-groups, and whose loads by elements where columns start off 16 bytes, take up to seven times as
+// long as it says.  Least squares over the times of 828 such drawn calls (fp16 574, fp32 254): 17 - 21 % rms, 24 - 45 % without.
+bool is_staged(int dtype, int config_id)
+{
+    if (dtype == MMBO_F64) return false;
+    const ConfigRef c = config_ref(config_id);
+    return !c.ring && !c.planes;
+}
+double staged_us(const WaveShape &p, int config_id, double us)
+{
+    const double small = 4.9;
+    if (!is_staged(p.dtype, config_id) || us <= small) return us;
+    const bool f32 = p.dtype == MMBO_F32, off_a = p.lda % (f32 ? 4 : 8) != 0, off_b = p.ldb % (f32 ? 4 : 8) != 0;
+    const double a = f32 ? (p.transA ? 1.13 : 1.32) : (p.transA ? 1.35 : 1.65), b = f32 ? 1.05 : (p.transB ? 1.55 : 1.25);
+    return small + (us - small) * (!f32 ? 2.15 : off_a || off_b ? 2.0 : 1.75) * (off_a ? a : 1.0) * (off_b ? b : 1.0);
+}
+
 // By 8 % at least: nearer than that the models do not tell the two apart (110 drawn shapes, against the tables' configs alone:
 // 1.367 times faster in the geometric mean, two slower by over 2 %; without the margin 1.361 and seven).  Updates of a C inside a
 // much larger matrix: by 17 %.  Neither model knows where the columns of C lie; of 13 such shapes modelled up to 1.2 times faster seven
@@ -960,11 +979,23 @@ WavePick pick_wave(const WaveShape &p, bool may_split, double limit = 1e300)
 // The ring kernel's 64 x 64 tile without a split, picked for a few microseconds of work, takes 2.65 us less than its model says (55 drawn
 // shapes, 2.1 - 3.0), which matters only here: by 2.0 us, as this kernel takes 0.6 less on its smallest calls and 5 % less on the others.  us
 // here / there: fp16 TT 1024 x 640 x 512 6.4 / 5.1, TT 4 x 576 x 320 x 512 8.4 / 5.7, TN 768 x 128 x 640 4.4 / 5.5, fp32 NN 448 x 768 x 304 7.0 / 8.1.
+// Against a staged config the model of this kernel, too, is at the end of what it was fitted to: from 8 us on by a quarter (fp32) or a
+// fifth, and by half where it says a wavefront per work-group on problems over 32 wide or, fp32, over 40 us (one wavefront to a work-group
+// reuses what the staged kernel's four share), unless the tables' own model says so, too.  Drawn calls that left the staged kernel: with a
+// margin of 8 % alone fp16 1.62 times faster in the geometric mean, 71 of 3,960 slower by over 3 %, fp32 1.30 and 168 of 2,120; with these
+// bars fp16 1.66 and 24 of 2,816, fp32 (a third of them in planes) 1.47 and 6 of 191.  us, staged / split by wavefront: fp16 NT 191 x 102 x
+// 32 x 512 43.0 / 12.6, 2 x 2267 x 7424 43.2 / 11.4, TT 12320 x 4 x 5569 91.7 / 22.8; the other way, fp32 TN 128 x 56 x 512 x 384 49.1 / 87.7.
 WavePick pick_wave_over(const WaveShape &q, bool may_split, int config_id, double table_us)
 {
-    double bar = (q.wide_c ? 0.83 : 0.92) * table_us;
-    if (q.dtype != MMBO_F64 && config_id == ring_config_id(3, 0)) bar = std::min(bar, table_us - 2.0);
-    return pick_wave(q, may_split, bar);             // (none at `bar` or beyond)
+    const double us = staged_us(q, config_id, table_us);
+    double bar = (q.wide_c ? 0.83 : 0.92) * us;
+    if (q.dtype != MMBO_F64 && config_id == ring_config_id(3, 0)) bar = std::min(bar, us - 2.0);
+    const WavePick w = pick_wave(q, may_split, bar);             // (none at `bar` or beyond)
+    if (w.tile >= 0 && w.us >= 8.0 && is_staged(q.dtype, config_id)) {
+        const bool half = (w.waves == 1 && std::min(q.m, q.n) > 32) || (q.dtype == MMBO_F32 && w.us > 40.0);
+        if (w.us >= (q.wide_c ? 0.83 : 0.92) * table_us && w.us >= (q.dtype == MMBO_F32 ? (half ? 0.45 : 0.75) : half ? 0.5 : 0.8) * us) return WavePick{-1, 0, 0, bar};
+    }
+    return w;
 }
 WaveShape packed_shape(int dtype, int transA, int transB, size_t m, size_t n, size_t k, int batch, bool read_c)
 {
@@ -1129,7 +1160,8 @@ Plan plan_for(const WaveShape &p)
     Key key;
     std::memset(&key, 0, sizeof(key));                   // (compared as bytes)
     key.dtype = p.dtype; key.transA = p.transA; key.transB = p.transB; key.batch = p.batch; key.read_c = p.read_c; key.wide_c = p.wide_c;
-    key.lines_a = p.lda % per_line == 0; key.lines_b = p.ldb % per_line == 0;
+    auto alignment = [&](size_t ld) { return ld % per_line == 0 ? 2 : ld % (per_line / 8) == 0; };
+    key.lines_a = alignment(p.lda); key.lines_b = alignment(p.ldb);
     key.m = p.m; key.n = p.n; key.k = p.k;
     size_t h = p.m * 0x9E3779B97F4A7C15ull ^ p.n * 0xC2B2AE3D27D4EB4Full ^ p.k * 0x165667B19E3779F9ull ^
                (size_t)(p.batch * 16 + p.dtype * 4 + p.transA * 2 + p.transB) * 0x27D4EB2F165667C5ull;
@@ -1165,7 +1197,7 @@ Plan plan_for(const WaveShape &p)
     if (p.dtype == MMBO_F32 && !config_ref(plan.config_id).planes) {
         if (table_split == 1) packed = choose(packed_call, false);
         // (the ring kernel's 64 x 64 tile takes some 2 us less than its model says: see pick_wave_over)
-        const double us = packed.tile >= 0 ? packed.us : plan.config_id == ring_config_id(3, 0) ? table_us - 2.0 : table_us;
+        const double us = packed.tile >= 0 ? packed.us : plan.config_id == ring_config_id(3, 0) ? table_us - 2.0 : staged_us(packed_call, plan.config_id, table_us);
         WaveShape with_c = packed_call;
         with_c.read_c = true;
         int runs = table_split;

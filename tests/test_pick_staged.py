@@ -1,0 +1,25 @@
+"""Where the automatic pick leaves the staged kernel for the split-by-wavefront one, and where it stays (no GPU needed)."""
+import pytest
+
+import util as U
+
+
+@pytest.mark.parametrize("dtype,ta,tb,m,n,k,batch,wave", [
+    (U.F16, 0, 1, 102, 32, 512, 191, True),        # a batch of narrow problems, columns off 16 bytes
+    (U.F16, 0, 1, 2, 2267, 7424, 1, True),         # less than 16 bytes of m in memory
+    (U.F16, 1, 1, 12320, 4, 5569, 1, True),
+    (U.F32, 0, 1, 3, 9000, 4096, 1, True),
+    (U.F16, 1, 1, 37, 384, 397, 229, False),       # over 32 wide, a wavefront per work-group
+    (U.F32, 1, 0, 56, 512, 384, 128, False),
+    (U.F16, 0, 0, 32, 32, 32, 1, None),            # a few microseconds: either
+])
+def test_where_the_pick_leaves_the_staged_kernel(dtype, ta, tb, m, n, k, batch, wave):
+    import gemm_mmbo_amd as G
+    a = G.auto_info(dtype, ta, tb, m, n, k, batch)
+    if wave is None:
+        assert a["config_id"] == G.CONFIG_AUTO or a["config_id"] == G.select_config(dtype, ta, tb, m, n, k, batch)
+        return
+    assert ("WAVE" in a["name"]) == wave, a["name"]
+    # whether a call needs a workspace still follows from the pick of the tables
+    if a["split_k"] > 1:
+        assert G.config_info(dtype, G.select_config(dtype, ta, tb, m, n, k, batch))["split_k"] > 1
