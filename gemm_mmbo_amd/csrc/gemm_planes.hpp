@@ -6,10 +6,10 @@
 // small products to another, and the two are added when the sum over k is whole.
 //
 // Why: an fp32 MFMA does 128 multiply-adds per clock and CU, a bf16 one 2,048, a sixth of that is 341.  us, before / with it (before: the fp32 MFMA
-// kernels), NT 4096^3 with alpha and beta 948 / 538, TN 640 x 384 x 10000 accumulated 48.9 / 36.9, NN 2048^3 127 / 84, 4096 x 128 x 4096 39 / 32, NT 44160
+// kernels), NT 4096^3 with alpha and beta 948 / 538, TN 640 x 384 x 10000 accumulated 48.8 / 36.7, NN 2048^3 127 / 84, 4096 x 128 x 4096 39 / 32, NT 44160
 // x 2048 x 384 accumulated 561 / 412.  What bounds it: at 4096^3 power -- 1.53 PFLOP/s of bf16 products at a 1.9 GHz clock, where a loop of nothing but
-// these MFMAs sustains 1.9 on such data --, on smaller tiles the vector instructions that take the elements apart (64 x 64 tile,
-// 1024^3, 21.0 us: without them and the LDS writes 15.1, without the MFMAs 16.3).
+// these MFMAs sustains 1.9 on such data --, on smaller tiles the vector instructions that take the elements apart (64 x 64 tile with two
+// groups of wavefronts, 1024^3, 21.0 us: without them and the LDS writes 15.1, without the MFMAs 16.3).
 // Precision: fewer roundings than the fp32 MFMAs' (one per eight k instead of one per k), and those of the small products
 // 2^-8 times smaller.  2-norm error against 64 bits, this form / v_mfma_f32_16x16x4_f32, uniform [-1, 1]: k = 64 4.5e-8 / 1.4e-7, 1024
 // 1.7e-7 / 5.7e-7, 32768 1.2e-6 / 3.3e-6; uniform [0, 1] at 32768 8.5e-7 / 2.4e-6; operands spread over 2^-20 .. 2^20 at 64 6.1e-8 / 7.2e-8, at
@@ -17,7 +17,7 @@
 //
 // What the planes cannot hold is found out and computed again, for the whole tile, with fp32 MFMAs: see `suspect`.
 //
-// Structure, one work-group of eight wavefronts per BM x BN tile of C, two to a SIMD (with one, the MFMAs' 16 clocks and the four of each other
+// Structure, one work-group of eight (64 x 64 tile: twelve) wavefronts per BM x BN tile of C, two (three) to a SIMD (with one, the MFMAs' 16 clocks and the four of each other
 // instruction add up: NN 4096^3 620 us instead of 557):
 //   - slices of 32 k go memory -> registers (fp32) -> three planes -> LDS -> MFMA fragments.  Each element is taken apart once
 //     per work-group (12 vector instructions per two elements), not once per wavefront that uses it.  The planes are written
@@ -29,7 +29,11 @@
 //     first fragment reads of the next slice.
 //   - every MFMA is followed by its share of the other instructions, in source order and fenced: left to the scheduler, MFMAs gather
 //     and the vector unit idles, then the other way round.
-//   - the small tiles' two groups of wavefronts take every second slice each: 64 x 32 wavefront tiles read less LDS per MFMA than 32 x 32.
+//   - the 128 x 64 tile's two groups of wavefronts take every second slice each: 64 x 32 wavefront tiles read less LDS per MFMA than 32 x 32.
+//     The 64 x 64 tile has three groups, three wavefronts to a SIMD: with two the barrier and the trips to LDS left the pipes idle for
+//     part of each slice (two groups with four slices in flight each / three with two, us: NN 1024^3 22.4 / 21.2, TN 1024^3 19.0 / 18.1, NN 768 x
+//     1024 x 2048 31.5 / 30.0, TN 640 x 384 x 10000 128.1 / 114.8, with k split four ways 45.3 / 42.4; over 2,142 drawn shapes 1.08 -
+//     1.13 times faster from 80 slices on, 1.02 - 1.05 from 12 on, below that 0.96 - 1.03).
 //   - rows of a tile lie in LDS in the order 0, 4, 8, .., 1, 5, 9, ..: a lane's four accumulators of blocks BM/4 rows apart are then four
 //     consecutive rows of C, sixteen lanes 256 contiguous bytes, and a lane's writes of four loaded rows fall on different banks.
 #pragma once
@@ -237,7 +241,7 @@ gemm_planes_kernel(const GemmArgs args)
     static_assert(JW == 4 || (BM == 64 && WM == 2), "row quads, or halves of them");
     constexpr int U = SETS > 2 ? SETS : 2;               // slices per turn of the loop: registers and LDS halves are then named at compile time
     static_assert(U % SETS == 0 && U % 2 == 0, "the roles repeat every U slices");
-    static_assert(KG == 1 || KG == 2, "one or two groups of wavefronts");
+    static_assert(KG >= 1 && KG <= 3, "one to three groups of wavefronts");
     constexpr int NP = NB / 2, GROUPS = MB * NP;         // pairs of blocks, twelve MFMAs each, per slice
     constexpr int CAP = 16 * (OpA::PAIRS + OpB::PAIRS);
     constexpr OpList<CAP> ops = list_ops<OpA, OpB, CAP>();
@@ -470,8 +474,9 @@ gemm_planes_kernel(const GemmArgs args)
     typedef f32x2 __attribute__((aligned(4))) f32x2_u;
     using Rows = typename std::conditional<JW == 4, f32x4, f32x2>::type;
     using Rows_u = typename std::conditional<JW == 4, f32x4_u, f32x2_u>::type;
-    constexpr int NE = NB / KG;
-    const int n0 = (int)((wn * NB + kg * NE) * 16);      // first physical column this wavefront stores (see below)
+    constexpr int NE = KG == 1 ? NB : NB / 2;            // columns of blocks a wavefront stores, from physical column n0 on (see below)
+    const bool stores = KG < 3 || kg < 2;
+    const int n0 = (int)((wn * NB + (KG < 3 || kg < 2 ? kg : 0) * NE) * 16);
     const int j0 = JW == 4 ? 0 : 2 * (int)wm;            // first member of its quads
     const bool to_ws = args.splits > 1;
     const uint32_t ldo = to_ws ? args.m : args.ldc;
@@ -482,7 +487,7 @@ gemm_planes_kernel(const GemmArgs args)
     auto column = [&](int nb, int i) { return row_b((n0 + nb * 16) % QB + 4 * (int)l4 + i, (n0 + nb * 16) / QB); };
     auto column_in = [&](int nb, int i) {
         const int q = (n0 + nb * 16) % QB + 4 * (int)l4 + i, j = (n0 + nb * 16) / QB;
-        return 4 * q < rows_b && (TB ? column(nb, i) >= 4 * q : 4 * q + j < rows_b);
+        return stores && 4 * q < rows_b && (TB ? column(nb, i) >= 4 * q : 4 * q + j < rows_b);
     };
     auto c_at = [&](int nb, int i, int qi) { return out + (size_t)(col0 + column(nb, i)) * ldo + row0 + 4 * quad(qi) + j0; };
     // the old C of whole quads, all of it requested before anything else is done (one round trip to memory; a block of columns at a time, four)
@@ -499,7 +504,8 @@ gemm_planes_kernel(const GemmArgs args)
 
     // ---- the sums ---------------------------------------------------------------------------------------------------
     // Two groups: each wavefront hands half of its columns of blocks to the wavefront of the same rows and columns in the other group and
-    // adds what it gets to the rest (the first group's sum first).  From here on a wavefront has NE columns of blocks, from n0 on.
+    // adds what it gets to the rest (the first group's sum first).  A third group hands one half to each of them, which add it behind their
+    // own, and goes on with zeros that it does not store.  From here on a wavefront has NE columns of blocks, from n0 on.
     f32x4 sum[MB][NE];
     if constexpr (KG == 1) {
 #pragma unroll
@@ -507,24 +513,37 @@ gemm_planes_kernel(const GemmArgs args)
 #pragma unroll
             for (int j = 0; j < NE; ++j) sum[i][j] = big[i][j] + small[i][j];
     } else {
-        f32x4 *mine = reinterpret_cast<f32x4 *>(lds) + (kg * WM * WN + wave) * (MB * NE * 64) + lane;     // (the last slice's barrier is behind its last read)
-        const f32x4 *other = reinterpret_cast<f32x4 *>(lds) + ((kg ^ 1) * WM * WN + wave) * (MB * NE * 64) + lane;
-        static_for<2>([&](auto K) {
+        // (the last slice's barrier is behind its last read)  half h of what group g hands on:
+        auto half = [&](uint32_t g, uint32_t h) {
+            return reinterpret_cast<f32x4 *>(lds) + ((g < 2 ? g : 2 + h) * WM * WN + wave) * (MB * NE * 64) + lane;
+        };
+        static_for<KG>([&](auto K) {
             constexpr int k = decltype(K)::value;
             if ((int)kg != k) return;
 #pragma unroll
             for (int i = 0; i < MB; ++i)
 #pragma unroll
                 for (int j = 0; j < NE; ++j) {
-                    mine[(i * NE + j) * 64] = big[i][(k ^ 1) * NE + j] + small[i][(k ^ 1) * NE + j];
-                    sum[i][j] = big[i][k * NE + j] + small[i][k * NE + j];
+                    if constexpr (k == 2) {
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) half(2, h)[(i * NE + j) * 64] = big[i][h * NE + j] + small[i][h * NE + j];
+                        sum[i][j] = f32x4{0, 0, 0, 0};
+                    } else {
+                        half(k, 0)[(i * NE + j) * 64] = big[i][(k ^ 1) * NE + j] + small[i][(k ^ 1) * NE + j];
+                        sum[i][j] = big[i][k * NE + j] + small[i][k * NE + j];
+                    }
                 }
         });
         barrier();
+        if (stores) {
 #pragma unroll
-        for (int i = 0; i < MB; ++i)
+            for (int i = 0; i < MB; ++i)
 #pragma unroll
-            for (int j = 0; j < NE; ++j) sum[i][j] += other[(i * NE + j) * 64];
+                for (int j = 0; j < NE; ++j) {
+                    sum[i][j] += half(kg ^ 1, 0)[(i * NE + j) * 64];
+                    if constexpr (KG == 3) sum[i][j] += half(2, kg)[(i * NE + j) * 64];
+                }
+        }
         barrier();
     }
 
