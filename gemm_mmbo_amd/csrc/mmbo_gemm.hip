@@ -1032,7 +1032,9 @@ struct PlanesPick {
 };
 
 // What the kernel is to run a shape with, where it beats what else would run it -- `us` microseconds modelled, k added up in `runs` runs -- by
-// a tenth (nearer than that the models do not tell them apart).  Partial sums (k split over work-groups) of at most max_bytes.
+// a tenth, from 16 us on by a twentieth (nearer than that the models do not tell them apart; the twentieth, and the ring kernel's model taken at
+// its word from there on, moved 2,694 drawn calls, 1.16 times faster in the geometric mean, 20 slower by over 3 %: updates of k = 256 up to a
+// fifth).  Partial sums (k split over work-groups) of at most max_bytes.
 // No result becomes less exact: a sum in planes has a third of the fp32 MFMAs' error, which grows with the root of a run's length, so a
 // run may be eight times as long as theirs.  k below 64 was not measured to be as exact on operands of widely different magnitudes.
 // Not for calls of a few microseconds, where a work-group has next to no slices to overlap anything with (us before / with it: TT 46 x 128 x
@@ -1041,7 +1043,7 @@ struct PlanesPick {
 PlanesPick pick_planes(int transA, int transB, size_t m, size_t n, size_t k, int batch, int runs, double us, double max_bytes)
 {
     PlanesPick best{-1, 0};
-    double best_us = 0.90 * us;
+    double best_us = (us < 16.0 ? 0.90 : 0.95) * us;
     if (k < 64 || us < (k < 160 ? 30.0 : k < 256 ? 16.0 : 12.0) || !planes_shape_ok(transA, transB, m, n, k)) return best;
     for (int tile = 0; tile < NUM_PLANES_TILES; ++tile) {
         const PlanesRow &r = kPlanesTiles[tile];
@@ -1196,8 +1198,9 @@ Plan plan_for(const WaveShape &p)
     plan.planes = PlanesPick{-1, 0};
     if (p.dtype == MMBO_F32 && !config_ref(plan.config_id).planes) {
         if (table_split == 1) packed = choose(packed_call, false);
-        // (the ring kernel's 64 x 64 tile takes some 2 us less than its model says: see pick_wave_over)
-        const double us = packed.tile >= 0 ? packed.us : plan.config_id == ring_config_id(3, 0) ? table_us - 2.0 : staged_us(packed_call, plan.config_id, table_us);
+        // (the ring kernel's 64 x 64 tile takes some 2 us less than its model says for a few microseconds of work: see pick_wave_over.  From 16
+        // on it takes what the model says or more: 1024^3 21.4 - 22.3, modelled 21.6 - 22.2; in planes 19.2 - 19.8.)
+        const double us = packed.tile >= 0 ? packed.us : plan.config_id == ring_config_id(3, 0) && table_us < 16.0 ? table_us - 2.0 : staged_us(packed_call, plan.config_id, table_us);
         WaveShape with_c = packed_call;
         with_c.read_c = true;
         int runs = table_split;
