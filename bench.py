@@ -23,11 +23,18 @@ sys.path.insert(0, ROOT)
 
 METRIC = "GEMM TFLOP/s + % of MFMA peak, fp16 & fp32 at 8192^3, 1 MI355X"
 PEAK_TFLOPS = {"f16": 2500.0, "f32": 157.3, "f64": 78.6}      # MI355X published dense matrix peaks
+
+
+def peak_tflops(head, config_name):
+    """The matrix peak a launch is priced against: fp32 in three bf16 planes does six bf16 products for each of its own."""
+    return PEAK_TFLOPS["f16"] / 6 if "BF16X3" in config_name else PEAK_TFLOPS[head]
+
+
 # Bytes per launch that crossed the L2 <-> fabric boundary come from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs of this
 # same command (each scaled by the counter's reading for a plain elementwise pass of known size).  They are not measured
 # by this run: they are read from the "traffic:" line of the profile summary below, which names the kernel they were
 # taken on, and are reported only while that is still the kernel this run launches.
-TRAFFIC_PROFILE = {"f16": "profiles/gemm_x16_f16_8192.txt", "f32": "profiles/gemm_x16_f32_8192.txt"}
+TRAFFIC_PROFILE = {"f16": "profiles/gemm_x16_f16_8192.txt", "f32": "profiles/gemm_planes_f32_8192.txt"}
 
 
 def profiled_traffic(head, tile_config):
@@ -225,9 +232,10 @@ def ragged_legs(G, torch, steps, warmup):
             G.gemm(dtype, ta, tb, m, n, k, 1.0, A, lda, B, ldb, 0.0, C, m, G.CONFIG_AUTO, stream)
         us = timed_launches(torch, stream, run, max(steps, 20), max(warmup, 5), groups=10, settle_min_ms=30.0, settle_max_ms=200.0)["median_ms"] * 1e3
         tf = 2.0 * m * n * k / us * 1e-6
+        name = G.auto_info(dtype, ta, tb, m, n, k)["name"]
         out[f"{dname}_{'NT'[ta]}{'NT'[tb]}_{m}x{n}x{k}"] = {"us": round(us, 1), "tflops": round(tf, 1),
-                                                            "frac_of_peak": round(tf / PEAK_TFLOPS["f16" if dtype == G.F16 else "f32"], 4),
-                                                            "tile_config": G.auto_info(dtype, ta, tb, m, n, k)["name"]}
+                                                            "frac_of_peak": round(tf / peak_tflops("f16" if dtype == G.F16 else "f32", name), 4),
+                                                            "tile_config": name}
         del A, B, C
     return out
 
@@ -260,9 +268,10 @@ def config_legs(G, torch, steps, warmup):
         tf = 2.0 * m * n * k * batch / us * 1e-6
         esz = 2 if dtype == G.F16 else 4
         gbps = batch * (m * k + k * n + m * n * (2 if beta != 0 else 1)) * esz / us * 1e-3
+        name = G.auto_info(dtype, ta, tb, m, n, k, batch, reads_c=beta != 0)["name"]
         out[key] = {"us": round(us, 1), "tflops": round(tf, 1),
-                    "frac_of_peak": round(tf / PEAK_TFLOPS["f16" if dtype == G.F16 else "f32"], 4),
-                    "algorithmic_GBps": round(gbps, 1), "tile_config": G.auto_info(dtype, ta, tb, m, n, k, batch, reads_c=beta != 0)["name"]}
+                    "frac_of_peak": round(tf / peak_tflops("f16" if dtype == G.F16 else "f32", name), 4),
+                    "algorithmic_GBps": round(gbps, 1), "tile_config": name}
         if batch > 1:
             # the memory-bound one: a plain streaming kernel with the same bytes read (A, B, old C) and written, on this box
             out[key]["stream_kernel_same_bytes_us"] = round(
@@ -366,8 +375,8 @@ def main():
         "config": {"workload": f"{'H' if head == 'f16' else 'S'}GEMM NN M=N=K=8192 lda=ldb=ldc=8192 alpha=1 beta=0, "
                                + ("A,B ~ N(0,1)*0.1 rounded to fp16, fp32 accumulate" if head == "f16" else "A,B ~ U[-1,1]"),
                    "tile_config": r["cfg"]["name"]},
-        "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_TFLOPS[head], "unit": "TFLOP/s",
-                     "frac": round(achieved / PEAK_TFLOPS[head], 4), "traffic": traffic, "traffic_source": traffic_source,
+        "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": round(peak_tflops(head, r["cfg"]["name"]), 1), "unit": "TFLOP/s",
+                     "frac": round(achieved / peak_tflops(head, r["cfg"]["name"]), 4), "traffic": traffic, "traffic_source": traffic_source,
                      "algorithmic_bytes": alg_bytes, "flops_per_launch": flops,
                      "kernel_ms": round(t["median_ms"], 4)},
         "timing": {"statistic": "median over the groups of the timed region; value and ms_per_step use it",
@@ -385,13 +394,13 @@ def main():
         # what a register-only MFMA loop sustains on this box (the chip lowers its clock under power)
         out["mfma_issue_ceiling"] = ceilings
         c = ceilings.get(f"{head}_random_operands")
-        if c:
+        if c and "BF16X3" not in r["cfg"]["name"]:      # (the loop is of fp32 MFMAs)
             out["roofline"]["frac_of_measured_mfma_ceiling"] = round(achieved / c["tflops"], 4)
     if head == "f16" and "f32" in res:
         q = res["f32"]
         out["also"] = {"fp32_tflops": round(flops / q["ev_ms"] * 1e-9, 2), "fp32_ms_per_step": round(q["ev_ms"], 4),
-                       "fp32_frac_of_peak": round(flops / q["ev_ms"] * 1e-9 / PEAK_TFLOPS["f32"], 4),
-                       "fp32_peak": PEAK_TFLOPS["f32"], "fp32_tile_config": q["cfg"]["name"], "fp32_steps": q["steps"],
+                       "fp32_frac_of_peak": round(flops / q["ev_ms"] * 1e-9 / peak_tflops("f32", q["cfg"]["name"]), 4),
+                       "fp32_peak": round(peak_tflops("f32", q["cfg"]["name"]), 1), "fp32_tile_config": q["cfg"]["name"], "fp32_steps": q["steps"],
                        "fp32_groups": q["t"]["groups"],
                        "fp32_max_rel_err": float(f"{q['rel']:.3e}"), "fp32_rel_err_limit": float(f"{q['limit']:.3e}")}
     if ones_tflops is not None:

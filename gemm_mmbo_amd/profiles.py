@@ -44,6 +44,13 @@ import time
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PEAK_TFLOPS = {"h": 2500.0, "s": 157.3, "d": 78.6}
 ESZ = {"h": 2, "s": 4, "d": 8}
+
+
+def peak_tflops(d, kernel):
+    # (fp32 in three bf16 planes does six bf16 products for each of its own; kernel: its name or its config's)
+    return round(PEAK_TFLOPS["h"] / 6, 1) if "BF16X3" in kernel or "gemm_planes_kernel" in kernel else PEAK_TFLOPS[d]
+
+
 LIB_KERNEL = re.compile(r"mmbo(::|\d+)?.*(gemm_x16_kernel|gemm_ring_kernel|gemm_staged_kernel|gemm_wave_kernel|gemm_planes_kernel|gemm_dots_kernel|dgemm_kernel|splitk_reduce_kernel)")
 LONG_KERNEL_NS = 200e3          # below this GRBM_GUI_ACTIVE is not a clock measurement
 
@@ -63,7 +70,8 @@ SKINNY = ["h,N,N,4096,128,4096", "s,N,N,4096,128,4096", "h,N,N,128,4096,8192", "
 CONFIGS = ["s,N,N,1024,1024,1024", "s,N,T,4096,4096,4096,1,1.5,0.5", "s,T,N,4096,4096,4096,1,1.5,0.5",
            "h,T,N,512,512,512,64,1,1", "d,N,T,44160,2048,384,1,-1,1,44160"]
 MIDSIZE = ["h,N,N,2048,2048,2048", "h,N,N,3000,3000,3000", "h,N,N,4096,4096,4096"]
-SMALL_THIN = ["h,N,N,16,4096,4096", "s,N,N,96,72,150,5", "d,N,N,64,489,4640", "h,N,T,32,59,55680"]
+SMALL_THIN = ["h,N,N,16,4096,4096", "s,N,N,96,72,150,5", "d,N,N,64,489,4640", "h,N,T,32,59,55680",
+              "d,T,N,49,45,57216", "h,N,T,102,32,512,191"]
 FP64_UPDATES = ["d,N,T,2304,2048,384,1,-1,1,44160", "d,N,T,1152,2048,384,1,-1,1,44160", "d,N,T,1121,1088,1692"]
 
 CASES = {
@@ -71,8 +79,8 @@ CASES = {
         "title": "HGEMM NN 8192^3 (fp16 in/out, fp32 accumulate), the benchmark's headline leg",
         "program": ["bench.py", "--no-cpu", "--only", "f16"], "short": ["--steps", "5", "--warmup", "2"],
         "passes": ["trace", "sq", "tcc", "fetch", "write"], "dtype": "h", "shape": (8192, 8192, 8192, 1, 0.0)},
-    "gemm_x16_f32_8192": {
-        "title": "SGEMM NN 8192^3, the benchmark's fp32 leg",
+    "gemm_planes_f32_8192": {
+        "title": "SGEMM NN 8192^3 in three bf16 planes, the benchmark's fp32 leg",
         "program": ["bench.py", "--no-cpu", "--only", "f32"], "short": ["--steps", "10", "--warmup", "2"],
         "passes": ["trace", "sq", "tcc", "fetch", "write"], "dtype": "s", "shape": (8192, 8192, 8192, 1, 0.0)},
     "skinny_cfg4": {
@@ -84,7 +92,7 @@ CASES = {
         "program": ["-m", "gemm_mmbo_amd.report", "shapes"] + CONFIGS + ["--no-check", "--reps", "10", "--ceilings"],
         "passes": ["trace", "sq"], "specs": CONFIGS},
     "small_thin": {
-        "title": "Small, thin and long-k GEMMs that the split-by-wavefront kernel takes, automatic pick",
+        "title": "Small, thin and long-k GEMMs that the split-by-wavefront kernel and the fp64 one on 4 x 4 blocks take, automatic pick",
         "program": ["-m", "gemm_mmbo_amd.report", "shapes"] + SMALL_THIN + ["--no-check", "--reps", "10"],
         "passes": ["trace", "sq", "fetch", "write"], "specs": SMALL_THIN},
     "fp64_updates": {
@@ -260,7 +268,6 @@ def summarise_bench(case, outdir):
     d = c["dtype"]
     flops = 2.0 * m * n * k * batch
     alg_read, alg_write = (m * k + k * n) * ESZ[d] * batch, m * n * ESZ[d] * batch
-    peak = PEAK_TFLOPS[d]
     L = [c["title"] + "; MI355X", "=" * 120]
     tr = read_trace(os.path.join(outdir, "trace"))
     recs = read_json_lines(os.path.join(outdir, "trace.stdout"))
@@ -268,6 +275,7 @@ def summarise_bench(case, outdir):
     mine = [x for x in tr if LIB_KERNEL.search(x["name"]) and "splitk" not in x["name"]]
     if not mine:
         raise ValueError(f"{outdir}/trace holds no dispatch of this library's kernels")
+    peak = peak_tflops(d, mine[0]["name"])
     by = per_kernel(mine)
     kernel = max(by, key=lambda kname: sum(by[kname]))
     runs = [x for x in mine if x["name"] == kernel]
@@ -380,8 +388,9 @@ def summarise_shapes(case, outdir):
             tot += median(durs)
             L.append(f"   {short_name(name):112s} timed dispatches {len(durs):4d}  median {median(durs) / 1e3:8.1f} us  min {min(durs) / 1e3:8.1f}")
         tf = flops / tot * 1e-3
-        bound_tf = min(PEAK_TFLOPS[d], flops / alg * 8.0)
-        L.append(f"   per GEMM {tot / 1e3:.1f} us -> {tf:.1f} TFLOP/s = {tf / PEAK_TFLOPS[d]:.4f} of the {PEAK_TFLOPS[d]} TFLOP/s matrix peak; "
+        peak = peak_tflops(d, r["config"])
+        bound_tf = min(peak, flops / alg * 8.0)
+        L.append(f"   per GEMM {tot / 1e3:.1f} us -> {tf:.1f} TFLOP/s = {tf / peak:.4f} of the {peak} TFLOP/s matrix peak; "
                  f"{alg / tot:.0f} GB/s algorithmic = {alg / tot / 8000:.3f} of 8 TB/s; {tf / bound_tf:.3f} of the roofline bound min(peak, intensity x 8 TB/s)")
         L.append(f"   gap between consecutive dispatches: median {median(gaps(timed)) / 1e3:.1f} us;  the driver's HIP-event time per call in this run: "
                  f"{r['gpu_ms_median'] * 1e3:.1f} us ({r['tflops']} TFLOP/s, {r['frac_of_peak']} of peak)")

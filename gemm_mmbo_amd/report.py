@@ -70,12 +70,17 @@ def spec_of(shape):
     return s + (f",{ldc}" if ldc else "")
 
 
-def roofline(d, m, n, k, batch, beta):
+def peak_tflops(d, config_name):
+    # (fp32 in three bf16 planes does six bf16 products for each of its own)
+    return PEAK_TFLOPS["h"] / 6 if "BF16X3" in config_name else PEAK_TFLOPS[d]
+
+
+def roofline(d, m, n, k, batch, beta, peak):
     flops = 2.0 * m * n * k * batch
     nbytes = batch * (m * k + k * n + m * n * (2 if beta != 0 else 1)) * ESZ[d]
     hbm_tflops = flops / nbytes * HBM_TBPS if nbytes else float("inf")      # arithmetic intensity x 8 TB/s, in TFLOP/s
-    bound = "mfma" if PEAK_TFLOPS[d] <= hbm_tflops else "hbm"
-    return flops, nbytes, bound, min(PEAK_TFLOPS[d], hbm_tflops)
+    bound = "mfma" if peak <= hbm_tflops else "hbm"
+    return flops, nbytes, bound, min(peak, hbm_tflops)
 
 
 def run_shape(G, torch, shape, reps, inner, config, check, seed=1):
@@ -135,14 +140,14 @@ def run_shape(G, torch, shape, reps, inner, config, check, seed=1):
     torch.cuda.synchronize()
     per = sorted(ev[g].elapsed_time(ev[g + 1]) / inner for g in range(reps))
     med = per[len(per) // 2] if len(per) % 2 else 0.5 * (per[len(per) // 2 - 1] + per[len(per) // 2])
-    flops, nbytes, bound, bound_tf = roofline(d, m, n, k, batch, beta)
+    flops, nbytes, bound, bound_tf = roofline(d, m, n, k, batch, beta, peak_tflops(d, name))
     tf = flops / med * 1e-9
     gbps = nbytes / med * 1e-6
     return {"spec": spec_of(shape), "calls_total": calls[0], "calls_timed": reps * inner,
             "dtype": d, "transA": ta, "transB": tb, "m": m, "n": n, "k": k, "batch": batch, "lda": lda, "ldb": ldb, "ldc": ldc,
             "alpha": alpha, "beta": beta, "config_id": cid, "config": name, "gpu_ms_median": round(med, 5),
             "gpu_ms_min": round(per[0], 5), "gpu_ms_max": round(per[-1], 5), "groups": reps, "launches_per_group": inner,
-            "tflops": round(tf, 2), "frac_of_peak": round(tf / PEAK_TFLOPS[d], 4), "bound": bound,
+            "tflops": round(tf, 2), "frac_of_peak": round(tf / peak_tflops(d, name), 4), "bound": bound,
             "bound_tflops": round(bound_tf, 1), "frac_of_bound": round(tf / bound_tf, 4), "algorithmic_bytes": nbytes,
             "algorithmic_GBps": round(gbps, 1), "frac_of_hbm_peak": round(gbps / (HBM_TBPS * 1e3), 4),
             "max_rel_err": None if rel is None else float(f"{rel:.3e}"), "checked_against": against}

@@ -29,7 +29,10 @@
  *   - config_id selects a row of the tile-config table, like the reference's kernelId
  *     (src/gemm/constants.h:34-47,106-135); MMBO_CONFIG_AUTO lets the library pick: a config of the table, or, for problems
  *     too small to fill the chip with the table's tiles, a kernel without a config id whose wavefronts split k among
- *     themselves.  Every shape runs under MMBO_CONFIG_AUTO.  Named configs: the general kernel's (no "DTL1" in the name) take any shape and
+ *     themselves (fp64 results of a few rows and columns: another such kernel, on 4 x 4 blocks).  fp32 products that pay for it are
+ *     formed on the bf16 matrix pipes from three bf16 planes per operand ("BF16X3" in the name; ids behind the other types' table for
+ *     two of its tiles): no bit of an operand is dropped, the error against exact arithmetic is below that of the fp32 matrix
+ *     instructions, and tiles with values that planes cannot hold are computed with those.  Every shape runs under MMBO_CONFIG_AUTO.  Named configs: the general kernel's (no "DTL1" in the name) take any shape and
  *     alignment; of the direct-to-LDS ones ("DTL1") the "MFMA16x16" family takes m, n that end inside a tile, k that
  *     ends inside a slice and A, B at any element alignment (the reference's kernels take whole tiles only: its
  *     launcher floors the grid, src/gemm/driver.h:49-50), and reads no byte outside the operands: it fetches 16
@@ -112,11 +115,11 @@ int mmbo_config_info(int dtype, int config_id, mmbo_config_desc *out);
 /* The per-shape pick among the configs of the table (reference: the exact-size -> solution table of
  * src/gemm/ref/vega20_Cijk_Ailk_Bjlk_DB.yaml:929-1177).  Returns a config id >= 0, or a
  * negative mmbo_status on bad arguments.  Pure host logic: needs no device.  (MMBO_CONFIG_AUTO runs this config unless
- * the kernel without a config id is faster on the shape.) */
+ * a kernel without a config id, or fp32 in bf16 planes, is faster on the shape.) */
 int mmbo_select_config(int dtype, int transA, int transB, size_t m, size_t n, size_t k, int batch);
 
 /* What a call with MMBO_CONFIG_AUTO runs, for reports and tests: *config_id is a config of the table, described in *out as
- * mmbo_config_info does, or MMBO_CONFIG_AUTO for the kernel without a config id, whose tile, threads, GlobalSplitU and
+ * mmbo_config_info does, or MMBO_CONFIG_AUTO for a kernel without a config id, whose tile, threads, GlobalSplitU and
  * wavefronts that share k ("LSU" in the name, as in the reference's solution names) *out then describes.  reads_c: beta is
  * not zero.  A, B, C and the batch strides count as 16-byte aligned and the workspace as the library's own.  Pure host logic: needs
  * no device. */
