@@ -953,7 +953,7 @@ WavePick pick_wave(const WaveShape &p, bool may_split, double limit = 1e300)
     return best;
 }
 
-// What the staged kernel takes where mmbo_select_config picks it, in place of the `us` of that pick's model.  The model knows the tiles of a few
+// What the pick of mmbo_select_config takes, in place of the `us` of that pick's model.  The staged kernel's: the model knows the tiles of a few
 // large problems; the calls that still come to this kernel are batches of narrow problems and operands with less than 16 bytes of m or
 // n in memory, whose rounds of short work-groups, and whose loads by elements where columns start off 16 bytes, take up to seven times as
 // long as it says.  Least squares over the times of 828 such drawn calls (fp16 574, fp32 254): 17 - 21 % rms, 24 - 45 % without.
@@ -963,8 +963,17 @@ bool is_staged(int dtype, int config_id)
     const ConfigRef c = config_ref(config_id);
     return !c.ring && !c.planes;
 }
-double staged_us(const WaveShape &p, int config_id, double us)
+// fp64's, for its 32 x 32 and 64 x 64 tiles: the model shares the MFMAs' time out, but a slice of 16 k takes a work-group a round trip however idle
+// its CU is.  us per slice, 2,600 drawn calls: 32 x 32 with up to three work-groups per CU 0.35 - 0.39 (128 slices and more, whose operands the L2
+// does not hold, 0.57 - 0.60), where the model says 0.16 for one; 64 x 64 with one 0.70 - 0.75 (0.78).
+double config_us(const WaveShape &p, int config_id, double us)
 {
+    if (p.dtype == MMBO_F64) {
+        const int bm = kTilesF64[config_id].bm, bn = kTilesF64[config_id].bn;
+        const size_t slices = ceil_div(p.k, (size_t)16);
+        if (bm != bn || bm > 64) return us;
+        return std::max(us, 4.0 + (double)slices * (bm == 32 ? (slices < 128 ? 0.37 : 0.55) : slices < 128 ? 0.68 : 0.76));
+    }
     const double small = 4.9;
     if (!is_staged(p.dtype, config_id) || us <= small) return us;
     const bool f32 = p.dtype == MMBO_F32, off_a = p.lda % (f32 ? 4 : 8) != 0, off_b = p.ldb % (f32 ? 4 : 8) != 0;
@@ -987,10 +996,14 @@ double staged_us(const WaveShape &p, int config_id, double us)
 // 32 x 512 43.0 / 12.6, 2 x 2267 x 7424 43.2 / 11.4, TT 12320 x 4 x 5569 91.7 / 22.8; the other way, fp32 TN 128 x 56 x 512 x 384 49.1 / 87.7.
 WavePick pick_wave_over(const WaveShape &q, bool may_split, int config_id, double table_us)
 {
-    const double us = staged_us(q, config_id, table_us);
+    const double us = config_us(q, config_id, table_us);
     double bar = (q.wide_c ? 0.83 : 0.92) * us;
     if (q.dtype != MMBO_F64 && config_id == ring_config_id(3, 0)) bar = std::min(bar, us - 2.0);
     const WavePick w = pick_wave(q, may_split, bar);             // (none at `bar` or beyond)
+    // fp64 against a slice's round trip (config_us): from 50 us on by a quarter.  Drawn calls that left the tables' kernel for it: 1.77 times faster in
+    // the geometric mean and 93 of 3,675 slower by over 3 % with 8 % throughout, 1.90 and 3 of 1,381 so.  us: NT 409 x 456 x 18536 652.6 / 164.3.
+    if (w.tile >= 0 && q.dtype == MMBO_F64 && w.us >= 50.0 && w.us >= (q.wide_c ? 0.83 : 0.92) * table_us && w.us >= 0.75 * us)
+        return WavePick{-1, 0, 0, bar};
     if (w.tile >= 0 && w.us >= 8.0 && is_staged(q.dtype, config_id)) {
         const bool half = (w.waves == 1 && std::min(q.m, q.n) > 32) || (q.dtype == MMBO_F32 && w.us > 40.0);
         if (w.us >= (q.wide_c ? 0.83 : 0.92) * table_us && w.us >= (q.dtype == MMBO_F32 ? (half ? 0.45 : 0.75) : half ? 0.5 : 0.8) * us) return WavePick{-1, 0, 0, bar};
@@ -1200,7 +1213,7 @@ Plan plan_for(const WaveShape &p)
         if (table_split == 1) packed = choose(packed_call, false);
         // (the ring kernel's 64 x 64 tile takes some 2 us less than its model says for a few microseconds of work: see pick_wave_over.  From 16
         // on it takes what the model says or more: 1024^3 21.4 - 22.3, modelled 21.6 - 22.2; in planes 19.2 - 19.8.)
-        const double us = packed.tile >= 0 ? packed.us : plan.config_id == ring_config_id(3, 0) && table_us < 16.0 ? table_us - 2.0 : staged_us(packed_call, plan.config_id, table_us);
+        const double us = packed.tile >= 0 ? packed.us : plan.config_id == ring_config_id(3, 0) && table_us < 16.0 ? table_us - 2.0 : config_us(packed_call, plan.config_id, table_us);
         WaveShape with_c = packed_call;
         with_c.read_c = true;
         int runs = table_split;
@@ -1211,7 +1224,7 @@ Plan plan_for(const WaveShape &p)
         if (plan.planes.tile >= 0 && plan.planes.split > 1)
             plan.reserve = std::max(plan.reserve, (size_t)plan.planes.split * p.batch * p.m * p.n * sizeof(float));
     }
-    plan.dots = p.dtype == MMBO_F64 ? pick_dots(p, plan.wave.tile >= 0 ? plan.wave.us : table_us) : -1;
+    plan.dots = p.dtype == MMBO_F64 ? pick_dots(p, plan.wave.tile >= 0 ? plan.wave.us : config_us(p, plan.config_id, table_us)) : -1;
     set.way[set.next] = Entry{true, key, plan};
     set.next = (set.next + 1) % kWays;
     return plan;

@@ -1,4 +1,4 @@
-"""Where the automatic pick leaves the staged kernel for the split-by-wavefront one, and where it stays (no GPU needed)."""
+"""Where the automatic pick leaves the kernels of the tables for the split-by-wavefront one, and where it stays (no GPU needed)."""
 import pytest
 
 import util as U
@@ -11,9 +11,12 @@ import util as U
     (U.F32, 0, 1, 3, 9000, 4096, 1, True),
     (U.F16, 1, 1, 37, 384, 397, 229, False),       # over 32 wide, a wavefront per work-group
     (U.F32, 1, 0, 56, 512, 384, 128, False),
+    (U.F64, 0, 0, 736, 256, 17856, 1, True),       # a work-group's slices at a round trip each
+    (U.F64, 0, 1, 44160, 2048, 384, 1, False),
+    (U.F64, 0, 0, 2048, 2048, 2048, 1, False),
     (U.F16, 0, 0, 32, 32, 32, 1, None),            # a few microseconds: either
 ])
-def test_where_the_pick_leaves_the_staged_kernel(dtype, ta, tb, m, n, k, batch, wave):
+def test_where_the_pick_leaves_the_tables(dtype, ta, tb, m, n, k, batch, wave):
     import gemm_mmbo_amd as G
     a = G.auto_info(dtype, ta, tb, m, n, k, batch)
     if wave is None:
