@@ -86,13 +86,12 @@ struct PlanesRow {
     int bm, bn;
     int wm, wn;       // wavefronts along M and N
     int kg;           // groups of such wavefronts that share k
-    int sets;         // slices of fp32 elements in flight to registers
 };
 constexpr PlanesRow kPlanesTiles[NUM_PLANES_TILES] = {
-    {256, 128, 4, 2, 1, 1},     // eight wavefronts of 64 x 64, 144 KB of LDS
-    {128, 128, 2, 4, 1, 2},     // of 64 x 32, 96 KB
-    {128, 64, 2, 2, 2, 2},      // two groups of 64 x 32, 144 KB
-    {64, 64, 2, 2, 3, 2},       // three groups of 32 x 32, 144 KB
+    {256, 128, 4, 2, 1},     // eight wavefronts of 64 x 64, 144 KB of LDS
+    {128, 128, 2, 4, 1},     // of 64 x 32, 96 KB
+    {128, 64, 2, 2, 2},      // two groups of 64 x 32, 144 KB
+    {64, 64, 2, 2, 3},       // three groups of 32 x 32, 144 KB
 };
 constexpr int kPlanesBk = 32;
 constexpr int kPlanesIdTiles = 2;

@@ -24,14 +24,15 @@
 //     k-contiguous whatever the operand's layout in memory (a lane that loaded rows instead of k holds them transposed in its registers),
 //     so all four transposes run one loop of 128-bit fragment reads.  (The remainder below a plane by v_dot2_f32_bf16, which needs no
 //     unpacking: fewer instructions, but they run in the matrix pipe, an MFMA and one of them 32 clocks.)
-//   - LDS holds two slices: while slice s is multiplied, slice s + 1 is taken apart and written, and slice s + 1 + SETS is
-//     requested from memory.  One barrier per slice.  The MFMAs of a slice's last row of blocks are issued behind the barrier, over the
+//   - LDS holds two slices: while slice s is multiplied, slice s + 1 is taken apart and written, and slice s + 2 is requested into the
+//     registers that this frees, a slice's MFMAs ahead of its use.  (Two slices ahead, in a second set of registers: 1.2 % slower in the
+//     128 x 128 tile, 2.9 in the 128 x 64, 2.5 in the 64 x 64, 4,243 drawn calls, most on short k; four: 2 - 5 % more.)  One barrier per slice.  The MFMAs of a slice's last row of blocks are issued behind the barrier, over the
 //     first fragment reads of the next slice.
 //   - every MFMA is followed by its share of the other instructions, in source order and fenced: left to the scheduler, MFMAs gather
 //     and the vector unit idles, then the other way round.
 //   - the 128 x 64 tile's two groups of wavefronts take every second slice each: 64 x 32 wavefront tiles read less LDS per MFMA than 32 x 32.
 //     The 64 x 64 tile has three groups, three wavefronts to a SIMD: with two the barrier and the trips to LDS left the pipes idle for
-//     part of each slice (two groups with four slices in flight each / three with two, us: NN 1024^3 22.4 / 21.2, TN 1024^3 19.0 / 18.1, NN 768 x
+//     part of each slice (two groups with four slices in flight each / three with two, before it was one, us: NN 1024^3 22.4 / 21.2, TN 1024^3 19.0 / 18.1, NN 768 x
 //     1024 x 2048 31.5 / 30.0, TN 640 x 384 x 10000 128.1 / 114.8, with k split four ways 45.3 / 42.4; over 2,142 drawn shapes 1.08 -
 //     1.13 times faster from 80 slices on, 1.02 - 1.05 from 12 on, below that 0.96 - 1.03).
 //   - rows of a tile lie in LDS in the order 0, 4, 8, .., 1, 5, 9, ..: a lane's four accumulators of blocks BM/4 rows apart are then four
@@ -226,8 +227,7 @@ struct PlanesCfg {
     static constexpr int LDS_BYTES = 2 * BUF * KG;
 };
 
-// SETS: slices in flight from memory (register sets of the fp32 elements).
-template <bool TA, bool TB, int BM, int BN, int WM, int WN, int KG, int SETS>
+template <bool TA, bool TB, int BM, int BN, int WM, int WN, int KG>
 __global__ void __launch_bounds__(WM * WN * KG * 64, WM * WN * KG / 4)
 gemm_planes_kernel(const GemmArgs args)
 {
@@ -239,8 +239,7 @@ gemm_planes_kernel(const GemmArgs args)
     constexpr int MB = BM / WM / 16, NB = BN / WN / 16;  // 16 x 16 blocks of a wavefront along m and n
     constexpr int JW = BM / WM >= 64 ? 4 : 2, QW = MB / JW;
     static_assert(JW == 4 || (BM == 64 && WM == 2), "row quads, or halves of them");
-    constexpr int U = SETS > 2 ? SETS : 2;               // slices per turn of the loop: registers and LDS halves are then named at compile time
-    static_assert(U % SETS == 0 && U % 2 == 0, "the roles repeat every U slices");
+    constexpr int U = 2;                                 // slices per turn of the loop: registers and LDS halves are then named at compile time
     static_assert(KG >= 1 && KG <= 3, "one to three groups of wavefronts");
     constexpr int NP = NB / 2, GROUPS = MB * NP;         // pairs of blocks, twelve MFMAs each, per slice
     constexpr int CAP = 16 * (OpA::PAIRS + OpB::PAIRS);
@@ -285,7 +284,7 @@ gemm_planes_kernel(const GemmArgs args)
     opA.wbase += group_lds;
     opB.wbase += group_lds + 3 * OpA::PLANE;
 
-    u32x4 rawA[SETS][OpA::NV], rawB[SETS][OpB::NV];      // see `phase`
+    u32x4 rawA[OpA::NV], rawB[OpB::NV];                  // the slice that is taken apart next
     float maxA = 0.0f, maxB = 0.0f;                      // largest element seen
 
     // One entry of `ops`.
@@ -380,20 +379,20 @@ gemm_planes_kernel(const GemmArgs args)
         c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, n_side), __builtin_bit_cast(bf16x8, m_side), c, 0, 0, 0);
     };
 
-    const char *ahead_a = gA + (int64_t)(1 + SETS) * stepA, *ahead_b = gB + (int64_t)(1 + SETS) * stepB;     // of the slice requested next
+    const char *ahead_a = gA + 2 * stepA, *ahead_b = gB + 2 * stepB;     // of the slice requested next
     // One slice.  Its phase PH says which registers and which half of LDS hold what; phases count so that the last slice has phase 0.
     auto slice = [&](auto PH, auto LAST, int s) {
-        constexpr int ph = decltype(PH)::value, par = ph & 1, set = (ph + 1) % SETS;
+        constexpr int ph = decltype(PH)::value, par = ph & 1;
         constexpr bool last = decltype(LAST)::value;
         constexpr uint32_t here = par ? Cfg::BUF : 0, next = par ? 0 : Cfg::BUF;
         if constexpr (!last) {
             if (s + 2 == ns && has_partial) {
-                opA.fix_partial(rawA[set], left);
-                opB.fix_partial(rawB[set], left);
+                opA.fix_partial(rawA, left);
+                opB.fix_partial(rawB, left);
             }
-            aim_at(s + 1 + SETS);
+            aim_at(s + 2);
         }
-        const int bytes = bytes_of(s + 1 + SETS);
+        const int bytes = bytes_of(s + 2);
         // A group: two neighbouring blocks, six MFMAs each, with its share of what else there is to do spread over
         // them: first the fragment reads that the next groups need, then entries of `ops`.
         static_for<GROUPS + (last ? NP : 0)>([&](auto G) {
@@ -422,7 +421,7 @@ gemm_planes_kernel(const GemmArgs args)
                         constexpr int e = d - a_reads, nbr = (FB == 1 ? 2 * (g - 1) : 2 * h) + e % 2;
                         read_b(fb[FB == 1 ? 0 : par][nbr][e / 2], nbr, e / 2, here);
                     } else {
-                        act_on(std::integral_constant<int, from + d - reads>{}, rawA[set], rawB[set], next, ahead_a, ahead_b, bytes);
+                        act_on(std::integral_constant<int, from + d - reads>{}, rawA, rawB, next, ahead_a, ahead_b, bytes);
                     }
                 });
                 __builtin_amdgcn_sched_barrier(0);
@@ -436,21 +435,18 @@ gemm_planes_kernel(const GemmArgs args)
     // slice 0, of phase `first`, is taken apart ahead of the loop
     const int first = (U - (ns - 1) % U) % U;
     static_for<U>([&](auto PH) {
-        constexpr int ph = decltype(PH)::value, set = ph % SETS;
+        constexpr int ph = decltype(PH)::value;
         constexpr uint32_t here = ph & 1 ? Cfg::BUF : 0;
         if (first != ph) return;
-        static_for<SETS>([&](auto X) {
-            constexpr int x = decltype(X)::value;
-            aim_at(x);
-            load_slice(rawA[(ph + x) % SETS], rawB[(ph + x) % SETS], x);
-        });
+        aim_at(0);
+        load_slice(rawA, rawB, 0);
         if (ns == 1 && has_partial) {
-            opA.fix_partial(rawA[set], left);
-            opB.fix_partial(rawB[set], left);
+            opA.fix_partial(rawA, left);
+            opB.fix_partial(rawB, left);
         }
-        aim_at(SETS);
+        aim_at(1);
         static_for<ops.n>([&](auto U) {
-            act_on(U, rawA[set], rawB[set], here, gA + (int64_t)SETS * stepA, gB + (int64_t)SETS * stepB, bytes_of(SETS));
+            act_on(U, rawA, rawB, here, gA + stepA, gB + stepB, bytes_of(1));
         });
     });
     barrier();

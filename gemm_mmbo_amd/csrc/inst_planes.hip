@@ -18,7 +18,7 @@ template <bool TA, bool TB>
 hipError_t launch_one(const GemmArgs &args, hipStream_t stream)
 {
     using Cfg = PlanesCfg<TA, TB, R.bm, R.bn, R.wm, R.wn, R.kg>;
-    auto kernel = gemm_planes_kernel<TA, TB, R.bm, R.bn, R.wm, R.wn, R.kg, R.sets>;
+    auto kernel = gemm_planes_kernel<TA, TB, R.bm, R.bn, R.wm, R.wn, R.kg>;
     static_assert(Cfg::LDS_BYTES <= 160 * 1024, "two slices of planes do not fit the 160 KB of LDS");
     static std::atomic<bool> attr_set[64];           // zero-initialised; several host threads may race to set it: harmless
     int dev = 0;
