@@ -74,3 +74,21 @@ def test_where_the_automatic_pick_takes_it(ta, tb, m, n, k, lda, taken):
     assert ("DOTS" in info["name"]) == taken, info["name"]
     if taken:
         assert info["split_k"] == 1 and info["threads"] == 512 and info["lds_bytes"] <= 160 * 1024
+
+
+def test_nothing_else_reads_the_direct_loads_register(tmp_path):
+    """The direct loads are asm statements that change M0 without saying so: only they, and the s_mov in front of each, may name it; and
+    scratch memory would put loads of the compiler's own between them."""
+    import os
+
+    import test_kernel_asm as K
+    if not os.path.exists(K.HIPCC):
+        pytest.skip("hipcc not installed")
+    path = K._compile(("inst_dots.hip", ["-DMMBO_TILE=3"]), str(tmp_path))
+    kernels = {name: body for name, body in K._kernels(path).items() if any(t.startswith("v_mfma") for t in body)}
+    assert len(kernels) == 4
+    for name, body in kernels.items():
+        loads = [t for t in body if t.startswith("buffer_load_dwordx4") and "lds" in t]
+        assert loads and len([t for t in body if t.startswith("s_mov_b32 m0")]) == len(loads), name
+        assert not [t for t in body if " m0" in t and not t.startswith("s_mov_b32 m0")], name
+        assert not [t for t in body if t.startswith("scratch_")], name
