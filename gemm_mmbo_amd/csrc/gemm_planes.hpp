@@ -559,8 +559,9 @@ gemm_planes_kernel(const GemmArgs args)
         for (int j = 0; j < NE; ++j) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                poison = __builtin_fmaf(sum[i][j][e], 0.0f, poison);
-                least = min(least, (__builtin_bit_cast(uint32_t, sum[i][j][e]) << 1) - 1);
+                const float x = sum[i][j][e];             // (the bits of sum[i][j][e] would be those of element 0: __builtin_bit_cast takes the whole vector)
+                poison = __builtin_fmaf(x, 0.0f, poison);
+                least = min(least, (__builtin_bit_cast(uint32_t, x) << 1) - 1);
             }
         }
     const float k_f = (float)k_len;

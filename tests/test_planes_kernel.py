@@ -128,6 +128,26 @@ def test_values_that_three_planes_cannot_hold(ta, tb):
             assert np.all(np.abs(got[ok] - want[ok]) <= k * (2.0 ** -24 * terms[ok] + 2.0 ** -150)), label
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+def test_one_small_column(ta, tb):
+    """A column of B whose lower planes fall below bf16's smallest number, beside ordinary ones: each place that a column can have among the four that a
+    lane holds."""
+    m, n, k = 150, 140, 70
+    for col in (0, 1, 2, 3, 77, 138):
+        p = U.Problem(F32, ta, tb, m, n, k, seed=col)
+        a = p.A.reshape((k, m) if ta else (m, k), order="F").T if ta else p.A.reshape((m, k), order="F")
+        b = p.B.reshape((n, k), order="F").T.copy() if tb else p.B.reshape((k, n), order="F").copy()
+        b[:, col] *= np.float32(2.0) ** -122
+        p.B = np.asfortranarray(b.T if tb else b).reshape(-1, order="F").copy()
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        # k roundings, each of at most half an ulp: 2^-24 of the terms' sum, or 2^-150 where the sum is below the smallest normal number
+        bound = k * (2.0 ** -24 * (np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64))) + 2.0 ** -150)
+        for tile, split in [(t, s) for t in range(4) for s in (1, 2)]:
+            got = _run(p, tile, split)[0].reshape((m, n), order="F").astype(np.float64)
+            off = np.abs(got - want) > bound
+            assert not off.any(), f"column {col}: {TILES[tile]} split {split}: {np.argwhere(off)[:3].tolist()}, {got[off][:3]} not {want[off][:3]}"
+
+
 def test_not_less_exact_than_the_fp32_matrix_instructions():
     """2-norm of the error against 64 bits, on the same operands: one run of k in planes beside one run of fp32 matrix instructions.  Uniform,
     positive and widely spread operands."""
