@@ -15,7 +15,7 @@
 // 1.7e-7 / 5.7e-7, 32768 1.2e-6 / 3.3e-6; uniform [0, 1] at 32768 8.5e-7 / 2.4e-6; operands spread over 2^-20 .. 2^20 at 64 6.1e-8 / 7.2e-8, at
 // 32768 1.1e-6 / 1.4e-6.  (Six products into one accumulator: equal to the fp32 MFMAs', and behind them on spread operands.)
 //
-// What the planes cannot hold is found out and computed again, for the whole tile, with fp32 MFMAs: see `suspect`.
+// What the planes cannot hold is found out and computed again, for the whole tile, with fp32 MFMAs: see `again`.
 //
 // Structure, one work-group of eight (64 x 64 tile: twelve) wavefronts per BM x BN tile of C, two (three) to a SIMD (with one, the MFMAs' 16 clocks and the four of each other
 // instruction add up: NN 4096^3 620 us instead of 557):
@@ -546,13 +546,16 @@ gemm_planes_kernel(const GemmArgs args)
     // ---- what the planes cannot hold -----------------------------------------------------------------------------
     // (a) An infinity, a NaN or an element that rounds to a bf16 infinity leaves no finite accumulator in its row or column of the tile
     //     (inf - inf and inf * 0 are NaN), and so does a sum that overflows.
-    // (b) bf16 is granular to 2^-133, so planes of elements below 2^-109 lose bits: of a sum, at most k * 2^-133 * the largest element
-    //     of the tile's operands.  Only a sum that is not 2^25 times that may show it.
-    // (c) Elements below 2^-134 vanish altogether: only zeros in the whole tile although both operands hold something else.
-    // In any of these cases the work-group computes its tile again with fp32 MFMAs.  Ordinary data has none of them: at k = 4096 (b)
-    // starts with sums below 2^-126 where no element reaches 2^-30, 2^-76 where none reaches 2^20, 2^-36 up to 2^60.
+    // (b) bf16 is granular to 2^-133: planes of elements below 2^-109 lose bits, and elements below 2^-134 vanish.  Of a sum that is, at
+    //     most, k * 2^-133 * the largest element of the tile's operands, so only a sum that is not 2^25 times that may show it, an exact zero
+    //     among them.  Ordinary data has such sums too -- rows of zeros, of zeros and small integers, at k = 4096 anything below 2^-126 where no
+    //     element reaches 2^-30, 2^-76 where none reaches 2^20, 2^-36 up to 2^60 --, so then the work-group looks through its rows and columns
+    //     for elements below 2^-109: one more pass over the operands, bound by what a CU pulls from the L2 (a row of zeros in every tile, us
+    //     without it / with it: NN 1024^3 21.6 / 26.9, 2048^3 88 / 106, 4096^3 539 / 688, TN 640 x 384 x 10000 41 / 64).
+    // (c) A sum below k * 2^-138 is within reach of fp32's own smallest numbers, where the small products end.
+    // With (a), (c), or an element that (b) finds, the work-group computes its tile again with fp32 MFMAs.
     float poison = 0.0f;
-    uint32_t least = 0xffffffffu;                         // of 2 |sum| - 1 as bits: zeros last
+    uint32_t least = 0xffffffffu, most = 0;               // of 2 |sum| - 1 as bits: zeros last
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -561,7 +564,9 @@ gemm_planes_kernel(const GemmArgs args)
             for (int e = 0; e < 4; ++e) {
                 const float x = sum[i][j][e];             // (the bits of sum[i][j][e] would be those of element 0: __builtin_bit_cast takes the whole vector)
                 poison = __builtin_fmaf(x, 0.0f, poison);
-                least = min(least, (__builtin_bit_cast(uint32_t, x) << 1) - 1);
+                const uint32_t bits = (__builtin_bit_cast(uint32_t, x) << 1) - 1;
+                least = min(least, bits);
+                most = max(most, bits);
             }
         }
     const float k_f = (float)k_len;
@@ -575,20 +580,48 @@ gemm_planes_kernel(const GemmArgs args)
     flags |= any(largest >= 0x1p-30f) ? 16 : 0;
     flags |= any(largest >= 0x1p+20f) ? 32 : 0;
     flags |= any(largest >= 0x1p+60f) ? 64 : 0;
-    flags |= any(least != 0xffffffffu) ? 128 : 0;
+    flags |= stores && any(most == 0xffffffffu) ? 128 : 0;
     flags |= any(maxA != 0.0f) ? 256 : 0;
     flags |= any(maxB != 0.0f) ? 512 : 0;
     uint32_t *shared_flags = reinterpret_cast<uint32_t *>(lds);
-    if (lane == 0) shared_flags[wave_of_all] = flags;
-    barrier();
-    flags = 0;
+    auto of_all = [&](uint32_t x) {                       // x of all wavefronts, or-ed
+        if (lane == 0) shared_flags[wave_of_all] = x;
+        barrier();
+        x = 0;
 #pragma unroll
-    for (int w = 0; w < WM * WN * KG; ++w) flags |= shared_flags[w];
-    flags = __builtin_amdgcn_readfirstlane(flags);
+        for (int w = 0; w < WM * WN * KG; ++w) x |= shared_flags[w];
+        shared_flags += WM * WN * KG;
+        return (uint32_t)__builtin_amdgcn_readfirstlane(x);
+    };
+    flags = of_all(flags);
     // (bits 1-3: a sum below the limit; bits 4-6: an element that the limit holds for)
-    const bool suspect = (flags & 1) || (flags >> 4 & flags >> 1 & 7) || (flags & (128 | 256 | 512)) == (256 | 512);
+    bool again = flags & 1;
+    if (!again && ((flags >> 4 & flags >> 1 & 7) || (flags & (128 | 256 | 512)) == (128 | 256 | 512))) {
+        // the requests of the loop once more (their offsets anew: kept, they would cost the loop registers)
+        uint32_t t = tid;
+        asm volatile("" : "+v"(t));
+        opA.init(t, lda, rows_a);
+        opB.init(t, ldb, rows_b);
+        uint32_t smallest = 0xffffffffu;                  // of 2 |element| - 1 as bits
+        auto look = [&](int x) {
+            load_slice(rawA, rawB, x);
+#pragma unroll
+            for (int v = 0; v < OpA::NV; ++v)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) smallest = min(smallest, (rawA[v][e] << 1) - 1);
+#pragma unroll
+            for (int v = 0; v < OpB::NV; ++v)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) smallest = min(smallest, (rawB[v][e] << 1) - 1);
+        };
+#pragma unroll 4
+        for (int x = 0; x < ns - 1; ++x) look(x);
+        aim_at(ns - 1);
+        look(ns - 1);
+        again = of_all(any(smallest < __builtin_bit_cast(uint32_t, 0x1p-109f) << 1));
+    }
 
-    if (suspect) {
+    if (again) {
         const float *a0 = reinterpret_cast<const float *>(gA - kg * one_a) + (TA ? 4 : 0), *b0 = reinterpret_cast<const float *>(gB - kg * one_b) + (TB ? 0 : 4);
         int64_t at_a[MB], at_b[NE];
 #pragma unroll

@@ -148,6 +148,45 @@ def test_one_small_column(ta, tb):
             assert not off.any(), f"column {col}: {TILES[tile]} split {split}: {np.argwhere(off)[:3].tolist()}, {got[off][:3]} not {want[off][:3]}"
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_elements_that_planes_lose_beside_ordinary_ones(ta, tb):
+    """Elements that vanish in three planes, or leave nothing of a sum, in some rows or columns of tiles whose other sums are ordinary: such a sum
+    is an exact zero.  (Below 2^-134 an element vanishes, below 2^-109 it loses bits.)"""
+    m, n, k = 150, 140, 70
+    two = np.float32(2.0)
+
+    def pair(a, b):                       # 2^-120 (1 + 2^-20) - 2^-120, the first one's tail below the planes
+        a[33] = 0
+        a[33, 1], a[33, 40] = two ** -120 * (1 + two ** -20), -(two ** -120)
+        b[1], b[40] = two ** 100, two ** 100
+    cases = {                             # what is done to op(A) and op(B)
+        "vanishing row": lambda a, b: (a.__setitem__(7, np.sign(a[7]) * two ** -136), b.__imul__(two ** 100)),
+        "vanishing column": lambda a, b: (b.__setitem__((slice(None), 77), np.sign(b[:, 77]) * two ** -138), a.__imul__(two ** 100)),
+        "vanishing row beside an ordinary operand": lambda a, b: a.__setitem__(149, np.float32(1e-41)),
+        "last column of a cut tile": lambda a, b: (b.__setitem__((slice(None), 139), np.float32(1e-42)), a.__imul__(two ** 90)),
+        "one element beside zeros": lambda a, b: (a.__setitem__(64, 0), a.__setitem__((64, 69), np.float32(1e-41)), b.__imul__(np.float32(1e30))),
+        "subnormal row": lambda a, b: (a.__setitem__(130, a[130] * two ** -127), b.__imul__(two ** 60)),
+        "zero rows and columns": lambda a, b: (a.__setitem__(slice(20, 90), 0), b.__setitem__((slice(None), slice(60, 140)), 0)),
+        "cancelling pair": pair,
+    }
+    for name, spoil in cases.items():
+        p = U.Problem(F32, ta, tb, m, n, k, seed=len(name))
+        a = p.A.reshape((k, m) if ta else (m, k), order="F").T.copy() if ta else p.A.reshape((m, k), order="F").copy()
+        b = p.B.reshape((n, k), order="F").T.copy() if tb else p.B.reshape((k, n), order="F").copy()
+        spoil(a, b)
+        p.A = np.asfortranarray(a.T if ta else a).reshape(-1, order="F").copy()
+        p.B = np.asfortranarray(b.T if tb else b).reshape(-1, order="F").copy()
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        # k roundings, each of at most half an ulp: 2^-24 of the terms' sum, or 2^-150 where the sum is below the smallest normal number
+        bound = k * (2.0 ** -24 * (np.abs(a.astype(np.float64)) @ np.abs(b.astype(np.float64))) + 2.0 ** -150)
+        if name == "cancelling pair":
+            bound[33] = 0                 # (two products and their sum, all of them fp32 numbers)
+        for tile, split in [(t, s) for t in range(4) for s in (1, 2)]:
+            got = _run(p, tile, split)[0].reshape((m, n), order="F").astype(np.float64)
+            off = np.abs(got - want) > bound
+            assert not off.any(), f"{name}: {TILES[tile]} split {split}: {np.argwhere(off)[:3].tolist()}, {got[off][:3]} not {want[off][:3]}"
+
+
 def test_not_less_exact_than_the_fp32_matrix_instructions():
     """2-norm of the error against 64 bits, on the same operands: one run of k in planes beside one run of fp32 matrix instructions.  Uniform,
     positive and widely spread operands."""
