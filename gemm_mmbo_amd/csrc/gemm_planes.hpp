@@ -621,35 +621,105 @@ gemm_planes_kernel(const GemmArgs args)
         again = of_all(any(smallest < __builtin_bit_cast(uint32_t, 0x1p-109f) << 1));
     }
 
-    if (again) {
-        const float *a0 = reinterpret_cast<const float *>(gA - kg * one_a) + (TA ? 4 : 0), *b0 = reinterpret_cast<const float *>(gB - kg * one_b) + (TB ? 0 : 4);
-        int64_t at_a[MB], at_b[NE];
+    // Steps of 16 k, four to a lane (in one load where the operand is contiguous along k), straight to registers and DEPTH steps ahead of their MFMAs.
+    // The time is that of the planes and then the fp32 MFMAs' own.  us, ordinary data / a NaN in every tile (there, element by element and four k
+    // at a time: in brackets) / the fp32 MFMA kernels: NN 4096^3 540 / 1402 (3110) / 925, TN 538 / 1413 (4012) / 914, NT with alpha and beta 620 / 1535
+    // (2610) / 940, NN 2048^3 88 / 226 (526) / 128, NN 1024^3 21.5 / 51 (184) / 25.6, TN 640 x 384 x 10000 41 / 133 (379) / 54.
+    if (again && stores) {
+        constexpr int DEPTH = MB * NE >= 16 ? 2 : 4;
+        const char *a0 = gA - kg * one_a + (TA ? 16 : 0), *b0 = gB - kg * one_b + (TB ? 0 : 16);
+        // byte offsets of a lane's first k (A contiguous along the rows: of the JW rows that it has of a quad, for the blocks of all of them)
+        constexpr int LA = TA ? MB : QW;
+        uint32_t at_a[LA], at_b[NE];
 #pragma unroll
-        for (int i = 0; i < MB; ++i) {
-            const int p = (block_a(i) + (JW == 4 ? wm * QW : 2 * wm)) * 16 + l16;
-            const int r = row_a(p % (BM / 4), p / (BM / 4)) + OpA::lead(rows_a);
-            at_a[i] = TA ? (int64_t)r * lda : r;
-#pragma unroll
-            for (int j = 0; j < NE; ++j) sum[i][j] = f32x4{0, 0, 0, 0};
+        for (int i = 0; i < LA; ++i) {
+            const uint32_t r = row_a(quad(i % QW), j0 + i / QW) + OpA::lead(rows_a);
+            at_a[i] = (TA ? r * lda + 4 * l4 : 4 * l4 * lda + r) * 4;
         }
 #pragma unroll
         for (int j = 0; j < NE; ++j) {
             const int p = n0 + j * 16 + l16;
-            const int r = row_b(p % QB, p / QB) + OpB::lead(rows_b);
-            at_b[j] = TB ? r : (int64_t)r * ldb;
+            const uint32_t r = row_b(p % QB, p / QB) + OpB::lead(rows_b);
+            at_b[j] = (TB ? 4 * l4 * ldb + r : r * ldb + 4 * l4) * 4;
+#pragma unroll
+            for (int i = 0; i < MB; ++i) sum[i][j] = f32x4{0, 0, 0, 0};
         }
-        for (int kk = 0; kk < k_len; kk += 4) {
-            const int k = min(kk + (int)l4, k_len - 1);
-            const bool in = kk + (int)l4 < k_len;
-            float a[MB], b[NE];
+        const int steps = k_len / 16, rest = k_len % 16;
+        const int64_t step_a = (TA ? (int64_t)16 : (int64_t)16 * lda) * 4, step_b = (TB ? (int64_t)16 * ldb : (int64_t)16) * 4;
+        struct Step {
+            float a[MB][4], b[NE][4];
+        } x[DEPTH];
+        // N elements in a row
+        auto load = [](auto N, auto &&put, const char *origin, uint32_t off, uint32_t more) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(origin), 0, 0x7fffffff, 0x00020000);
+            auto number = [](uint32_t w) { return __builtin_bit_cast(float, w); };
+            if constexpr (decltype(N)::value == 4) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, more, 0);
+                static_for<4>([&](auto E) { put(E) = number(v[decltype(E)::value]); });
+            } else if constexpr (decltype(N)::value == 2) {
+                const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, more, 0);
+                static_for<2>([&](auto E) { put(E) = number(v[decltype(E)::value]); });
+            } else {
+                put(std::integral_constant<int, 0>{}) = number(__builtin_amdgcn_raw_buffer_load_b32(r, off, more, 0));
+            }
+        };
+        constexpr std::integral_constant<int, 1> one;
+        constexpr std::integral_constant<int, 4> four;
+        constexpr std::integral_constant<int, JW> rows;
+        auto fetch = [&](Step &to, int s) {
+            const char *oa = a0 + s * step_a, *ob = b0 + s * step_b;
+            static_for<LA>([&](auto I) {
+                constexpr int i = decltype(I)::value;
+                if constexpr (TA) load(four, [&](auto T) -> float & { return to.a[i][decltype(T)::value]; }, oa, at_a[i], 0);
+                else static_for<4>([&](auto T) {
+                    load(rows, [&](auto J) -> float & { return to.a[decltype(J)::value * QW + i][decltype(T)::value]; }, oa, at_a[i], decltype(T)::value * lda * 4);
+                });
+            });
+            static_for<NE>([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                if constexpr (!TB) load(four, [&](auto T) -> float & { return to.b[j][decltype(T)::value]; }, ob, at_b[j], 0);
+                else static_for<4>([&](auto T) { load(one, [&](auto) -> float & { return to.b[j][decltype(T)::value]; }, ob, at_b[j], decltype(T)::value * ldb * 4); });
+            });
+        };
+        auto multiply = [&](const Step &of) {
 #pragma unroll
-            for (int i = 0; i < MB; ++i) a[i] = in ? a0[at_a[i] + (TA ? (int64_t)k : (int64_t)k * lda)] : 0.0f;
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int j = 0; j < NE; ++j) b[j] = in ? b0[at_b[j] + (TB ? (int64_t)k * ldb : (int64_t)k)] : 0.0f;
+                for (int i = 0; i < MB; ++i)
 #pragma unroll
-            for (int i = 0; i < MB; ++i)
+                    for (int j = 0; j < NE; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(of.b[j][t], of.a[i][t], sum[i][j], 0, 0, 0);
+        };
+        if (steps >= DEPTH) {
 #pragma unroll
-                for (int j = 0; j < NE; ++j) sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[j], a[i], sum[i][j], 0, 0, 0);
+            for (int d = 0; d < DEPTH; ++d) fetch(x[d], d);
+        }
+        int s = 0;
+        for (; s + DEPTH <= steps; s += DEPTH)
+            static_for<DEPTH>([&](auto D) {
+                constexpr int d = decltype(D)::value;
+                multiply(x[d]);
+                fetch(x[d], min(s + d + DEPTH, steps - 1));
+            });
+        for (; s < steps; ++s) {
+            fetch(x[0], s);
+            multiply(x[0]);
+        }
+        if (rest > 0) {
+            // element by element; an offset outside the buffer brings zero
+            const char *oa = a0 + steps * step_a, *ob = b0 + steps * step_b;
+            static_for<4>([&](auto T) {
+                constexpr int t = decltype(T)::value;
+                const bool in = (int)(4 * l4) + t < rest;
+                static_for<MB>([&](auto I) {
+                    constexpr int i = decltype(I)::value;
+                    load(one, [&](auto) -> float & { return x[0].a[i][t]; }, oa, in ? at_a[TA ? i : i % QW] + (TA ? 0 : i / QW * 4) : 0x80000000u, (TA ? t : t * lda) * 4);
+                });
+                static_for<NE>([&](auto J) {
+                    constexpr int j = decltype(J)::value;
+                    load(one, [&](auto) -> float & { return x[0].b[j][t]; }, ob, in ? at_b[j] : 0x80000000u, (TB ? t * ldb : t) * 4);
+                });
+            });
+            multiply(x[0]);
         }
     }
 

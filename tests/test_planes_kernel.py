@@ -187,6 +187,55 @@ def test_elements_that_planes_lose_beside_ordinary_ones(ta, tb):
             assert not off.any(), f"{name}: {TILES[tile]} split {split}: {np.argwhere(off)[:3].tolist()}, {got[off][:3]} not {want[off][:3]}"
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_tiles_that_are_computed_again(ta, tb):
+    """A NaN in every tile: the other rows come from the fp32 MFMAs, in steps of 16 k whole and cut, tiles cut by the edge, NaN in the padding."""
+    for tile, (bm, bn) in enumerate(TILES):
+        for i, k in enumerate((4, 15, 16, 17, 31, 33, 64, 79, 130, 208)):
+            m, n, split, pad = bm + (5, 3, 62)[i % 3], (bn + 3, bn - 1)[i % 2], (1, 2)[i // 5 % 2], (0, 1, 4)[i % 3]
+            p = U.Problem(F32, ta, tb, m, n, k, lda=(k if ta else m) + pad, ldb=(n if tb else k) + pad, seed=10 * tile + i)
+            for operand, ld, rows in ((p.A, p.lda, k if ta else m), (p.B, p.ldb, n if tb else k)):
+                operand.reshape(-1, ld)[:, rows:] = np.nan
+            stored_a, stored_b = p.A.reshape(-1, p.lda)[:, :k if ta else m], p.B.reshape(-1, p.ldb)[:, :n if tb else k]     # (column by column)
+            a, b = stored_a if ta else stored_a.T, stored_b.T if not tb else stored_b
+            spoiled = (3, bm + 1)
+            for row in spoiled:
+                for q in range(0, k, 32 * ((k + 63) // 64)):          # (in every split)
+                    a[row, q] = np.nan
+            others = [r for r in range(m) if r not in spoiled]
+            got, guard = _run(p, tile, split, (i % 2, i // 2 % 2, i % 3))
+            got = got.reshape((m, n), order="F").astype(np.float64)
+            label = f"{bm}x{bn} split {split} {'NT'[ta]}{'NT'[tb]} {m}x{n}x{k} pad {pad}"
+            assert np.isnan(got[list(spoiled)]).all() and np.all(guard == 0), label
+            x, y = a[others].astype(np.float64), b.astype(np.float64)
+            # k roundings, each of at most half an ulp of the terms' sum
+            assert np.all(np.abs(got[others] - x @ y) <= k * 2.0 ** -24 * (np.abs(x) @ np.abs(y))), label
+
+
+def test_what_a_tile_that_is_computed_again_costs():
+    """NN 1024^3 with a NaN in every tile, beside the same call without: 2.4 times the time, 8.5 where elements are fetched one by one."""
+    import torch
+
+    import gemm_mmbo_amd as G
+    n = 1024
+    assert "_BF16X3" in G.auto_info(F32, 0, 0, n, n, n)["name"]
+    A = [torch.rand(n * n, device="cuda") * 2 - 1 for _ in range(2)]
+    A[1].view(n, n)[0, ::64] = float("nan")
+    B, C = torch.rand(n * n, device="cuda") * 2 - 1, torch.empty(n * n, device="cuda")
+    best = [float("inf")] * 2
+    for _ in range(8):
+        for q in range(2):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            G.gemm(F32, 0, 0, n, n, n, 1.0, A[q], n, B, n, 0.0, C, n)
+            start.record()
+            for _ in range(20):
+                G.gemm(F32, 0, 0, n, n, n, 1.0, A[q], n, B, n, 0.0, C, n)
+            end.record()
+            end.synchronize()
+            best[q] = min(best[q], start.elapsed_time(end))
+    assert best[1] < 4 * best[0], best
+
+
 def test_not_less_exact_than_the_fp32_matrix_instructions():
     """2-norm of the error against 64 bits, on the same operands: one run of k in planes beside one run of fp32 matrix instructions.  Uniform,
     positive and widely spread operands."""
