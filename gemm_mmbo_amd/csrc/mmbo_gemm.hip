@@ -1044,12 +1044,18 @@ struct PlanesPick {
     int split;
 };
 
+// Are sums in planes, k added up in `runs` runs, as exact as those of the fp32 MFMAs in `others`?  The error of a sum grows with its runs' length, and how
+// much longer a run in planes may be depends on the operands.  Equal 2-norm errors against 64 bits at k = 512 .. 32768: uniform [-1, 1] and normal
+// operands eight times as long, uniform [0, 1] 2.8 times, operands spread over 2^-10 .. 2^10 four times, over 2^-20 .. 2^20 twice (k = 512, 2048; 8192 1.9
+// times, 32768 1.5 times).  Beyond 32 runs, those of the split-by-wavefront kernel, no number of runs in planes is as exact on the latter (2048: 64
+// runs of fp32 MFMAs 9.3e-8, planes 9.8e-8 at best).
+bool planes_as_exact(size_t k, int runs, int others) { return others <= 32 && (k <= 4096 ? others <= 2 * runs : 2 * others <= 3 * runs); }
+
 // What the kernel is to run a shape with, where it beats what else would run it -- `us` microseconds modelled, k added up in `runs` runs -- by
 // a tenth, from 16 us on by a twentieth (nearer than that the models do not tell them apart; the twentieth, and the ring kernel's model taken at
 // its word from there on, moved 2,694 drawn calls, 1.16 times faster in the geometric mean, 20 slower by over 3 %: updates of k = 256 up to a
 // fifth).  Partial sums (k split over work-groups) of at most max_bytes.
-// No result becomes less exact: a sum in planes has a third of the fp32 MFMAs' error, which grows with the root of a run's length, so a
-// run may be eight times as long as theirs.  k below 64 was not measured to be as exact on operands of widely different magnitudes.
+// Only where sums stay as exact (planes_as_exact); k below 64 was not measured to be on operands of widely different magnitudes.
 // Not for calls of a few microseconds, where a work-group has next to no slices to overlap anything with (us before / with it: TT 46 x 128 x
 // 128 x 384 10.9 / 13.0, NT 1280 x 512 x 144 6.8 / 8.2; with fewer than five slices up to 30: NT 4334 x 1152 x 128 19.9 / 26.2, but of 40 us
 // and more 1.13 - 1.2 times faster; NT 1735 x 652 x 160 11.2 / 13.2).
@@ -1066,7 +1072,7 @@ PlanesPick pick_planes(int transA, int transB, size_t m, size_t n, size_t k, int
             if (split > 1 && ((double)split * batch * (double)m * (double)n * sizeof(float) > max_bytes || tiles * batch * split > 1100 ||
                               k / kPlanesBk < (size_t)4 * r.kg * split))
                 break;
-            if (runs > 8 * split * r.kg) continue;
+            if (!planes_as_exact(k, split * r.kg, runs)) continue;
             const double t = planes_model_us(tile, split, m, n, k, batch);
             if (t < best_us) {
                 best_us = t;
@@ -1223,6 +1229,10 @@ Plan plan_for(const WaveShape &p)
                                   plan.workspace ? std::max(table_bytes, (double)kWaveSumsBytes) : 0.0);
         if (plan.planes.tile >= 0 && plan.planes.split > 1)
             plan.reserve = std::max(plan.reserve, (size_t)plan.planes.split * p.batch * p.m * p.n * sizeof(float));
+        // (but a call whose leading dimensions would have it run in more runs than the packed one keeps those)
+        if (plan.planes.tile >= 0 && plan.wave.tile >= 0 &&
+            !planes_as_exact(p.k, plan.planes.split * kPlanesTiles[plan.planes.tile].kg, plan.wave.waves * plan.wave.split))
+            plan.planes.tile = -1;
     }
     plan.dots = p.dtype == MMBO_F64 ? pick_dots(p, plan.wave.tile >= 0 ? plan.wave.us : config_us(p, plan.config_id, table_us)) : -1;
     set.way[set.next] = Entry{true, key, plan};
@@ -1253,10 +1263,18 @@ int route_for(const WaveShape &p, bool aligned16, WsSource ws_source, Route &r)
     r.pick = plan.wave;
     r.reserve = plan.reserve;
     r.planes_pick = plan.planes;
-    if (ws_source == WsSource::kStatic)      // partial sums that fit the array of the entry point that allocates nothing
-        while (r.planes_pick.split > 1 && (double)r.planes_pick.split * p.batch * (double)p.m * (double)p.n * sizeof(float) > (double)kScratchPartialBytes)
-            r.planes_pick.split /= 2;
     r.planes = plan.planes.tile >= 0 && tile_span_ok(planes_tile(plan.planes.tile), p.transA, p.transB, p.lda, p.ldb, esz);
+    if (ws_source == WsSource::kStatic && r.planes) {
+        // partial sums that fit the array of the entry point that allocates nothing -- unless what else would run the call is more exact then
+        auto fitting = [&](int split) {
+            while (split > 1 && (double)split * p.batch * (double)p.m * (double)p.n * sizeof(float) > (double)kScratchPartialBytes) split /= 2;
+            return split;
+        };
+        r.planes_pick.split = fitting(plan.planes.split);
+        if (r.planes_pick.split < plan.planes.split)
+            r.planes = planes_as_exact(p.k, r.planes_pick.split * kPlanesTiles[plan.planes.tile].kg,
+                                       plan.wave.tile >= 0 ? plan.wave.waves * plan.wave.split : fitting(config_ref(plan.config_id).split));
+    }
     r.dots_tile = plan.dots;
     r.dots = plan.dots >= 0 && dots_span_ok(p.transA, p.transB, p.lda, p.ldb);
     // (a pair of slices must span less than the 2 GiB of a buffer descriptor)

@@ -1,0 +1,54 @@
+"""Where the automatic pick takes fp32 products in bf16 planes (gemm_planes.hpp): never in sums of so much longer runs of k that they are less exact
+than those of the fp32 matrix instructions, whose runs the cases name."""
+import re
+
+import numpy as np
+import pytest
+
+import util as U
+
+F32 = U.F32
+
+
+def _runs(info):
+    lsu = re.search(r"LSU(\d+)", info["name"])
+    return info["split_k"] * (int(lsu.group(1)) if lsu else 1)
+
+
+@pytest.mark.parametrize("ta,tb,m,n,k,batch,others", [
+    (1, 1, 384, 384, 2048, 16, 4), (1, 0, 96, 384, 32768, 64, 8), (0, 1, 640, 512, 16384, 4, 4), (1, 0, 300, 300, 20000, 1, 32), (0, 0, 128, 5120, 8192, 1, 8),
+    (1, 1, 704, 719, 25984, 1, 16), (0, 1, 568, 62, 49646, 1, 64), (1, 1, 288, 288, 26240, 1, 64), (1, 0, 2080, 1024, 2176, 1, 4),
+])
+def test_runs_in_planes_are_not_too_long(ta, tb, m, n, k, batch, others):
+    import gemm_mmbo_amd as G
+    info = G.auto_info(F32, ta, tb, m, n, k, batch)
+    if "_BF16X3" in info["name"]:
+        assert others <= 32 and _runs(info) * (2 if k <= 4096 else 1.5) >= others, info["name"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb,m,n,k,batch,others", [
+    (1, 1, 384, 384, 2048, 16, ("MT192x192", "_MFMA16x16x4_ACC", 4)), (0, 0, 128, 5120, 8192, 1, ("MT064x064", "_RING6", 8)),
+    (0, 1, 640, 512, 16384, 4, ("MT064x064", "_RING6", 4)),
+])
+def test_the_pick_is_as_exact_as_the_fp32_matrix_instructions_it_replaces(ta, tb, m, n, k, batch, others):
+    """2-norm of the error against 64 bits on the same operands.  By 3 %: where runs in planes may be twice as long, the two are equal on the widest
+    spread of operands, and two sets of a million roundings give it to about 1 %."""
+    import gemm_mmbo_amd as G
+    tile, family, split = others
+    native = next(c for c in range(G.num_configs(F32)) if (d := G.config_info(F32, c))["name"].startswith(tile) and d["name"].endswith(family) and d["split_k"] == split)
+    for dist in ("uniform", "positive", "spread"):
+        p = U.Problem(F32, ta, tb, m, n, k, batch=batch, seed=k)
+        if dist == "positive":
+            p.A, p.B = np.abs(p.A), np.abs(p.B)
+        if dist == "spread":
+            rng = np.random.default_rng(k)
+            p.A = (p.A * np.exp2(rng.uniform(-20, 20, p.A.size))).astype(np.float32)
+            p.B = (p.B * np.exp2(rng.uniform(-20, 20, p.B.size))).astype(np.float32)
+        a, b = (x.reshape((batch, -1, ld)).astype(np.float64) for x, ld in ((p.A, p.lda), (p.B, p.ldb)))
+        want = ((b if not tb else b.transpose(0, 2, 1)) @ (a if not ta else a.transpose(0, 2, 1))).reshape(-1)      # (C's columns, one after the other)
+
+        def error(got):
+            return float(np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want))
+        here, limit = error(U.run_gpu(p)[0]), error(U.run_gpu(p, native)[0])
+        assert here <= 1.03 * limit, (dist, here, limit)
