@@ -1044,12 +1044,19 @@ struct PlanesPick {
     int split;
 };
 
-// Are sums in planes, k added up in `runs` runs, as exact as those of the fp32 MFMAs in `others`?  The error of a sum grows with its runs' length, and how
-// much longer a run in planes may be depends on the operands.  Equal 2-norm errors against 64 bits at k = 512 .. 32768: uniform [-1, 1] and normal
-// operands eight times as long, uniform [0, 1] 2.8 times, operands spread over 2^-10 .. 2^10 four times, over 2^-20 .. 2^20 twice (k = 512, 2048; 8192 1.9
-// times, 32768 1.5 times).  Beyond 32 runs, those of the split-by-wavefront kernel, no number of runs in planes is as exact on the latter (2048: 64
-// runs of fp32 MFMAs 9.3e-8, planes 9.8e-8 at best).
-bool planes_as_exact(size_t k, int runs, int others) { return others <= 32 && (k <= 4096 ? others <= 2 * runs : 2 * others <= 3 * runs); }
+// Are sums in planes, k added up in `runs` runs, as exact as those of the fp32 MFMAs in `others`?  The error of a sum grows with its runs' length; how
+// much longer a run in planes may be depends on the operands.  Equal 2-norm errors against 64 bits, k = 512 .. 32768: uniform [-1, 1] and normal
+// operands eight times as long, uniform [0, 1] 2.8 times, operands spread over 2^-10 .. 2^10 four times, over 2^-20 .. 2^20 of either sign twice (k = 512,
+// 2048; 8192 1.9 times, 32768 1.5 times), positive ones twice from 256 k to a run on.  Shorter runs of the fp32 MFMAs leave planes less to gain -- the
+// 32 products that one MFMA adds are cut to its largest one's bits --: k = 512 of positive operands over 2^-10 .. 2^10, fp32 MFMAs / planes, four runs of
+// 128 1.4e-7 / 0.86e-7, eight of 64 0.89 / 0.85, sixteen of 32 0.78 / 0.91.  Of 300 drawn calls that come to planes, on four kinds of operands, none is
+// less exact by over 0.1 %.  (Eight times throughout took 25 more of 3,000 drawn calls to planes and 16 into fewer splits: 1.18 times faster.)
+bool planes_as_exact(size_t k, int runs, int others)
+{
+    if (others <= 1) return true;
+    const size_t length = k / (size_t)others;
+    return length >= 256 ? (k <= 4096 ? others <= 2 * runs : 2 * others <= 3 * runs) : length >= 128 && others <= runs;
+}
 
 // What the kernel is to run a shape with, where it beats what else would run it -- `us` microseconds modelled, k added up in `runs` runs -- by
 // a tenth, from 16 us on by a twentieth (nearer than that the models do not tell them apart; the twentieth, and the ring kernel's model taken at
@@ -1220,19 +1227,13 @@ Plan plan_for(const WaveShape &p)
         // (the ring kernel's 64 x 64 tile takes some 2 us less than its model says for a few microseconds of work: see pick_wave_over.  From 16
         // on it takes what the model says or more: 1024^3 21.4 - 22.3, modelled 21.6 - 22.2; in planes 19.2 - 19.8.)
         const double us = packed.tile >= 0 ? packed.us : plan.config_id == ring_config_id(3, 0) && table_us < 16.0 ? table_us - 2.0 : config_us(packed_call, plan.config_id, table_us);
-        WaveShape with_c = packed_call;
-        with_c.read_c = true;
-        int runs = table_split;
-        for (const WavePick &w : {packed, choose(with_c, table_split > 1)})
-            if (w.tile >= 0) runs = std::max(runs, w.waves * w.split);
-        plan.planes = pick_planes(p.transA, p.transB, p.m, p.n, p.k, p.batch, runs, us,
+        auto runs = [&](const WavePick &w) { return w.tile >= 0 ? w.waves * w.split : table_split; };
+        plan.planes = pick_planes(p.transA, p.transB, p.m, p.n, p.k, p.batch, runs(packed), us,
                                   plan.workspace ? std::max(table_bytes, (double)kWaveSumsBytes) : 0.0);
         if (plan.planes.tile >= 0 && plan.planes.split > 1)
             plan.reserve = std::max(plan.reserve, (size_t)plan.planes.split * p.batch * p.m * p.n * sizeof(float));
-        // (but a call whose leading dimensions would have it run in more runs than the packed one keeps those)
-        if (plan.planes.tile >= 0 && plan.wave.tile >= 0 &&
-            !planes_as_exact(p.k, plan.planes.split * kPlanesTiles[plan.planes.tile].kg, plan.wave.waves * plan.wave.split))
-            plan.planes.tile = -1;
+        // (but a call whose beta or leading dimensions would have it run in more runs than the packed one without C keeps to those)
+        if (plan.planes.tile >= 0 && !planes_as_exact(p.k, plan.planes.split * kPlanesTiles[plan.planes.tile].kg, runs(plan.wave))) plan.planes.tile = -1;
     }
     plan.dots = p.dtype == MMBO_F64 ? pick_dots(p, plan.wave.tile >= 0 ? plan.wave.us : config_us(p, plan.config_id, table_us)) : -1;
     set.way[set.next] = Entry{true, key, plan};

@@ -18,12 +18,13 @@ def _runs(info):
 @pytest.mark.parametrize("ta,tb,m,n,k,batch,others", [
     (1, 1, 384, 384, 2048, 16, 4), (1, 0, 96, 384, 32768, 64, 8), (0, 1, 640, 512, 16384, 4, 4), (1, 0, 300, 300, 20000, 1, 32), (0, 0, 128, 5120, 8192, 1, 8),
     (1, 1, 704, 719, 25984, 1, 16), (0, 1, 568, 62, 49646, 1, 64), (1, 1, 288, 288, 26240, 1, 64), (1, 0, 2080, 1024, 2176, 1, 4),
+    (0, 1, 4264, 256, 256, 1, 4), (0, 0, 858, 1408, 768, 1, 4),
 ])
 def test_runs_in_planes_are_not_too_long(ta, tb, m, n, k, batch, others):
     import gemm_mmbo_amd as G
     info = G.auto_info(F32, ta, tb, m, n, k, batch)
     if "_BF16X3" in info["name"]:
-        assert others <= 32 and _runs(info) * (2 if k <= 4096 else 1.5) >= others, info["name"]
+        assert k // others >= 128 and _runs(info) * (1 if k // others < 256 else 2 if k <= 4096 else 1.5) >= others, info["name"]
 
 
 @pytest.mark.gpu
