@@ -31,8 +31,14 @@
  *     too small to fill the chip with the table's tiles, a kernel without a config id whose wavefronts split k among
  *     themselves (fp64 results of a few rows and columns: another such kernel, on 4 x 4 blocks).  fp32 products that pay for it are
  *     formed on the bf16 matrix pipes from three bf16 planes per operand ("BF16X3" in the name; ids behind the other types' table for
- *     two of its tiles): no bit of an operand is dropped, the error against exact arithmetic is below that of the fp32 matrix
- *     instructions, and tiles with values that planes cannot hold are computed with those.  Every shape runs under MMBO_CONFIG_AUTO.  Named configs: the general kernel's (no "DTL1" in the name) take any shape and
+ *     two of its tiles).  No bit of an operand is dropped; of the nine products of planes three, together below 2^-23 of a
+ *     product, are left out.  The 2-norm error against exact arithmetic is that of the fp32 matrix instructions or below, a third of it
+ *     on long sums of terms of like size -- but 1.7 % above, at most 1.61 half units in the last place instead of 1.00, for sums with a
+ *     single term that is not zero (a diagonal, a one-hot operand).  Tiles with values that planes cannot hold -- infinities, NaN, the
+ *     far ends of the range -- are computed again with those instructions, in up to 1.6 times the time of a call that uses nothing else
+ *     (small calls 2.0, with k split 2.5 times); exact zeros among a tile's sums cost a pass over its operands, up to 1.3 times the time
+ *     (with k split 1.6).  A named config without "BF16X3" has neither.
+ *     Every shape runs under MMBO_CONFIG_AUTO.  Named configs: the general kernel's (no "DTL1" in the name) take any shape and
  *     alignment; of the direct-to-LDS ones ("DTL1") the "MFMA16x16" family takes m, n that end inside a tile, k that
  *     ends inside a slice and A, B at any element alignment (the reference's kernels take whole tiles only: its
  *     launcher floors the grid, src/gemm/driver.h:49-50), and reads no byte outside the operands: it fetches 16

@@ -259,3 +259,23 @@ def test_not_less_exact_than_the_fp32_matrix_instructions():
             for tile in range(4):
                 here = error(_run(p, tile, 1)[0])
                 assert here <= limit, (dist, k, TILES[tile], here, limit)
+
+
+def test_sums_of_few_terms():
+    """A weighted gather and its like: op(A) with one, two or sixteen elements that are not zero in a row.  From two terms on not less exact than the fp32 matrix
+    instructions; a single product lacks x2*y3 + x3*y2 + x3*y3, at most (2 * 2^-8 * 2^-16 + 2^-32) of it, beside one rounding of half a unit, 2^-24 of it."""
+    import gemm_mmbo_amd as G
+    native = next(c for c in range(G.num_configs(F32)) if "_ACC" in (d := G.config_info(F32, c))["name"] and d["macro_tile_m"] == d["macro_tile_n"] == 128)
+    m, n, k = 512, 384, 256
+    for terms in (1, 2, 16):
+        p = U.Problem(F32, 1, 0, m, n, k, seed=terms)
+        a = p.A.reshape(m, k)
+        np.put_along_axis(a, np.argsort(np.random.default_rng(terms).random((m, k)), axis=1)[:, terms:], 0, axis=1)
+        want = p.exact().reshape(-1, order="F")
+        native_off, off = (x[0].astype(np.float64) - want for x in (U.run_gpu(p, native), _run(p, 1, 1)))
+        if terms > 1:
+            assert np.linalg.norm(off) <= np.linalg.norm(native_off), terms
+        else:
+            assert np.all(np.abs(off) <= (2.0 ** -23 + 2.0 ** -32 + 2.0 ** -24) * np.abs(want))
+            # (1.017 is measured on a million products; these are 200,000)
+            assert np.linalg.norm(off) <= 1.03 * np.linalg.norm(native_off)
