@@ -1060,17 +1060,21 @@ bool planes_as_exact(size_t k, int runs, int others)
 
 // What the kernel is to run a shape with, where it beats what else would run it -- `us` microseconds modelled, k added up in `runs` runs -- by
 // a tenth, from 16 us on by a twentieth (nearer than that the models do not tell them apart; the twentieth, and the ring kernel's model taken at
-// its word from there on, moved 2,694 drawn calls, 1.16 times faster in the geometric mean, 20 slower by over 3 %: updates of k = 256 up to a
-// fifth).  Partial sums (k split over work-groups) of at most max_bytes.
+// its word from there on, moved 2,694 drawn calls, 1.16 times faster in the geometric mean; of 420 of that kind on the present kernel none is
+// slower by over 2 %).  Partial sums (k split over work-groups) of at most max_bytes.
 // Only where sums stay as exact (planes_as_exact); k below 64 was not measured to be on operands of widely different magnitudes.
-// Not for calls of a few microseconds, where a work-group has next to no slices to overlap anything with (us before / with it: TT 46 x 128 x
+// Not (planes_may_pay) for calls of a few microseconds, where a work-group has next to no slices to overlap anything with (us before / with it: TT 46 x 128 x
 // 128 x 384 10.9 / 13.0, NT 1280 x 512 x 144 6.8 / 8.2; with fewer than five slices up to 30: NT 4334 x 1152 x 128 19.9 / 26.2, but of 40 us
 // and more 1.13 - 1.2 times faster; NT 1735 x 652 x 160 11.2 / 13.2).
+bool planes_may_pay(int transA, int transB, size_t m, size_t n, size_t k, double us)
+{
+    return k >= 64 && us >= (k < 160 ? 30.0 : k < 256 ? 16.0 : 12.0) && planes_shape_ok(transA, transB, m, n, k);
+}
 PlanesPick pick_planes(int transA, int transB, size_t m, size_t n, size_t k, int batch, int runs, double us, double max_bytes)
 {
     PlanesPick best{-1, 0};
     double best_us = (us < 16.0 ? 0.90 : 0.95) * us;
-    if (k < 64 || us < (k < 160 ? 30.0 : k < 256 ? 16.0 : 12.0) || !planes_shape_ok(transA, transB, m, n, k)) return best;
+    if (!planes_may_pay(transA, transB, m, n, k, us)) return best;
     for (int tile = 0; tile < NUM_PLANES_TILES; ++tile) {
         const PlanesRow &r = kPlanesTiles[tile];
         const size_t tiles = ceil_div(m, (size_t)r.bm) * ceil_div(n, (size_t)r.bn);
@@ -1150,7 +1154,7 @@ int pick_dots(const WaveShape &p, double us)
     return best;
 }
 
-// What the automatic pick runs for a shape.  The models are walked once per shape and thread (a microsecond or two, a part of what a
+// What the automatic pick runs for a shape.  The models are walked once per shape and thread (2 - 4 us, a part of what a
 // small call takes); a small table of four ways keeps the answers, which are a function of the key alone.
 // Whether a call needs a workspace, and how large a one at most, follows from the shape alone, not from beta or leading dimensions:
 // a program runs a shape once and then captures a call of that shape that may differ in those, which cannot allocate.  So a
@@ -1222,7 +1226,9 @@ Plan plan_for(const WaveShape &p)
     }
     // fp32 in planes: a matter of the shape alone, as its workspace is -- against what would run the packed call without C.
     plan.planes = PlanesPick{-1, 0};
-    if (p.dtype == MMBO_F32 && !config_ref(plan.config_id).planes) {
+    // (What would run it takes what the table's config does at most: small calls need not walk the models for that.)
+    if (p.dtype == MMBO_F32 && !config_ref(plan.config_id).planes &&
+        planes_may_pay(p.transA, p.transB, p.m, p.n, p.k, config_us(packed_call, plan.config_id, table_us))) {
         if (table_split == 1) packed = choose(packed_call, false);
         // (the ring kernel's 64 x 64 tile takes some 2 us less than its model says for a few microseconds of work: see pick_wave_over.  From 16
         // on it takes what the model says or more: 1024^3 21.4 - 22.3, modelled 21.6 - 22.2; in planes 19.2 - 19.8.)
