@@ -53,3 +53,47 @@ def test_the_pick_is_as_exact_as_the_fp32_matrix_instructions_it_replaces(ta, tb
             return float(np.linalg.norm(got.astype(np.float64) - want) / np.linalg.norm(want))
         here, limit = error(U.run_gpu(p)[0]), error(U.run_gpu(p, native)[0])
         assert here <= 1.03 * limit, (dist, here, limit)
+
+
+@pytest.mark.parametrize("ta,tb,m,n,k,batch,name,split", [
+    (0, 1, 5120, 5120, 1024, 1, "MT256x128x32", 1), (0, 1, 44160, 2048, 256, 1, "MT256x128x32", 1), (1, 0, 2500, 1500, 700, 1, "MT128x128x32", 1),
+    (0, 0, 256, 256, 256, 64, "MT128x128x32", 1), (1, 0, 640, 384, 10000, 1, "MT128x064x32", 8), (0, 1, 768, 768, 2048, 3, "MT128x064x32", 1),
+    (0, 0, 1024, 1024, 1024, 1, "MT064x064x32", 1), (1, 1, 800, 900, 1300, 1, "MT064x064x32", 1),
+])
+def test_the_pick_reaches_every_tile(ta, tb, m, n, k, batch, name, split):
+    import gemm_mmbo_amd as G
+    info = G.auto_info(F32, ta, tb, m, n, k, batch)
+    assert info["name"].startswith(name) and "_BF16X3" in info["name"] and info["split_k"] == split, info["name"]
+    # k is split over work-groups only where the tables' pick needs a workspace, too
+    assert split == 1 or G.config_info(F32, G.select_config(F32, ta, tb, m, n, k, batch))["split_k"] > 1
+
+
+@pytest.mark.parametrize("dtype,ta,tb,m,n,k,batch,ld", [
+    (U.F32, 0, 0, 512, 512, 512, 1, {}),                        # a few microseconds
+    (U.F32, 0, 0, 3, 9000, 8192, 1, {}), (U.F32, 1, 1, 9000, 3, 8192, 1, {}),       # less than 16 bytes of a contiguous dimension
+    (U.F32, 0, 0, 4096, 4096, 63, 1, {}), (U.F32, 0, 0, 4096, 4096, 0, 1, {}),
+    (U.F32, 1, 0, 5000, 5000, 5000, 1, {"lda": 1 << 23}),       # 128 rows and more span 2 GiB
+    (U.F16, 0, 0, 4096, 4096, 4096, 1, {}), (U.F64, 0, 0, 4096, 4096, 4096, 1, {}),
+])
+def test_where_the_pick_does_not_take_planes(dtype, ta, tb, m, n, k, batch, ld):
+    import gemm_mmbo_amd as G
+    assert "BF16X3" not in G.auto_info(dtype, ta, tb, m, n, k, batch, **ld)["name"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb,m,n,k,batch,split,tile", [(1, 1, 3000, 1500, 6144, 1, 1, 1), (0, 0, 256, 1500, 16384, 2, 8, 1), (1, 0, 2304, 768, 6144, 3, 1, 0)])
+def test_partial_sums_that_the_static_workspace_does_not_hold(ta, tb, m, n, k, batch, split, tile):
+    """The entry point that allocates nothing runs the same tile with the largest split whose partial sums fit: bit for bit what that split gives."""
+    import torch
+
+    import gemm_mmbo_amd as G
+    import test_planes_kernel as P
+    info = G.auto_info(F32, ta, tb, m, n, k, batch)
+    assert info["name"].startswith("MT%03dx%03dx32" % P.TILES[tile]) and "_BF16X3" in info["name"]
+    sums = m * n * batch * 4
+    assert info["split_k"] * sums > G.static_workspace_bytes() >= split * sums * (split > 1) and 2 * split * sums > G.static_workspace_bytes()
+    p = U.Problem(F32, ta, tb, m, n, k, batch=batch, seed=split)
+    A, B, C = (torch.from_numpy(x).cuda() for x in (p.A, p.B, p.C))
+    G.gemm_strided_batched_static_workspace(F32, ta, tb, m, n, k, 1.0, A, p.lda, p.sa, B, p.ldb, p.sb, 0.0, C, p.ldc, p.sc, batch)
+    torch.cuda.synchronize()
+    assert np.array_equal(C.cpu().numpy(), P._run(p, tile, split)[0])
