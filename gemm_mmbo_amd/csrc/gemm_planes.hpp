@@ -43,9 +43,8 @@
 #pragma once
 
 #include <type_traits>
-#include <utility>
 
-#include "gemm_common.hpp"
+#include "gemm_ring.hpp"
 
 namespace mmbo {
 namespace planes {
@@ -53,10 +52,7 @@ namespace planes {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F &&f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F &&f) { static_for_impl(f, std::make_integer_sequence<int, N>{}); }
+using ring::static_for;
 
 constexpr int BK = 32;      // k per slice: one MFMA's, 64 bytes of a row in each plane
 
