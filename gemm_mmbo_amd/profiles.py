@@ -61,6 +61,7 @@ PASSES = {
     "trace": ["--kernel-trace", "--stats"],
     "sq": ["--pmc"] + SQ_COUNTERS + ["--kernel-trace"],
     "tcc": ["--pmc"] + TCC_COUNTERS + ["--kernel-trace"],
+    "bf16": ["--pmc", "SQ_INSTS_VALU_MFMA_MOPS_BF16", "--kernel-trace"],        # (the pass above is full)
     "fetch": ["--pmc", "FETCH_SIZE", "--kernel-trace"],
     "write": ["--pmc", "WRITE_SIZE", "--kernel-trace"],
 }
@@ -82,7 +83,7 @@ CASES = {
     "gemm_planes_f32_8192": {
         "title": "SGEMM NN 8192^3 in three bf16 planes, the benchmark's fp32 leg",
         "program": ["bench.py", "--no-cpu", "--only", "f32"], "short": ["--steps", "10", "--warmup", "2"],
-        "passes": ["trace", "sq", "tcc", "fetch", "write"], "dtype": "s", "shape": (8192, 8192, 8192, 1, 0.0)},
+        "passes": ["trace", "sq", "bf16", "tcc", "fetch", "write"], "dtype": "s", "shape": (8192, 8192, 8192, 1, 0.0)},
     "skinny_cfg4": {
         "title": "Skinny and irregular GEMMs (benchmark configuration 4), NN, alpha = 1, beta = 0, automatic pick",
         "program": ["-m", "gemm_mmbo_amd.report", "shapes"] + SKINNY + ["--no-check", "--reps", "10", "--ceilings"],
@@ -223,9 +224,9 @@ def derived_lines(c, dur_ns, flops=None):
         else:
             busy = c["SQ_VALU_MFMA_BUSY_CYCLES"] / 1024 / (dur_ns * 2.4)
             L.append(f"MFMA busy cycles = {busy * 100:.1f} % of the kernel's duration at 2.4 GHz (too short a kernel for a clock figure)")
-    for key, per in (("SQ_INSTS_VALU_MFMA_MOPS_F16", 512), ("SQ_INSTS_VALU_MFMA_MOPS_F32", 512)):
+    for key, per in (("SQ_INSTS_VALU_MFMA_MOPS_F16", 512), ("SQ_INSTS_VALU_MFMA_MOPS_F32", 512), ("SQ_INSTS_VALU_MFMA_MOPS_BF16", 512)):
         if flops and c.get(key, 0) > 0:
-            L.append(f"{key} * {per} = {c[key] * per:.4e} flop (algorithmic {flops:.4e})")
+            L.append(f"{key} * {per} = {c[key] * per:.4e} flop (algorithmic {flops:.4e}{'; six products of planes for each' if key.endswith('BF16') else ''})")
     if c.get("SQ_LDS_IDX_ACTIVE", 0) > 0:
         L.append(f"LDS bank-conflict cycles / LDS active cycles = {c.get('SQ_LDS_BANK_CONFLICT', 0.0) / c['SQ_LDS_IDX_ACTIVE'] * 100:.1f} %")
     if c.get("TCC_HIT_sum", 0) + c.get("TCC_MISS_sum", 0) > 0:
@@ -295,15 +296,17 @@ def summarise_bench(case, outdir):
         ev = bench.get("ms_per_step") if "ms_per_step" in bench else None
         L.append(f"   bench.py's own HIP-event timing of the same launches inside this profiled run: median {ev * 1e3:.1f} us per launch "
                  f"({bench.get('value')} TFLOP/s, frac {bench.get('roofline', {}).get('frac')})" if ev else "   (no bench.py record in trace.stdout)")
-        ceil = bench.get("mfma_issue_ceiling", {})
+        # (the loop of an fp32 leg is of fp32 MFMAs: no ceiling of a kernel of bf16 ones)
+        ceil = bench.get("mfma_issue_ceiling", {}) if "gemm_planes_kernel" not in kernel else {}
         key = {"h": "f16", "s": "f32", "d": "f64"}[d]
         for kind in ("random", "ones"):
             cc = ceil.get(f"{key}_{kind}_operands")
             if cc:
                 L.append(f"   register-only MFMA loop in the same session, {kind} operands (mmbo_probe_mfma_ceiling): {cc['tflops']} TFLOP/s at "
                          f"{cc['shader_mhz']} MHz = {cc['tflops'] / peak:.3f} of peak;  kernel / ceiling = {tf / cc['tflops']:.4f}")
-        L.append("   To compare with a benchmark line from another box: frac differs by the boxes' sustained clocks (a few percent on the"
-                 " power-limited fp16 kernel); kernel / ceiling (random operands) = roofline.frac_of_measured_mfma_ceiling does not.")
+        if ceil:
+            L.append("   To compare with a benchmark line from another box: frac differs by the boxes' sustained clocks (a few percent on the"
+                     " power-limited fp16 kernel); kernel / ceiling (random operands) = roofline.frac_of_measured_mfma_ceiling does not.")
     L.append("")
     num = 2
     for pname in c["passes"][1:]:
@@ -395,7 +398,7 @@ def summarise_shapes(case, outdir):
         L.append(f"   gap between consecutive dispatches: median {median(gaps(timed)) / 1e3:.1f} us;  the driver's HIP-event time per call in this run: "
                  f"{r['gpu_ms_median'] * 1e3:.1f} us ({r['tflops']} TFLOP/s, {r['frac_of_peak']} of peak)")
         key = {"h": "f16", "s": "f32", "d": "f64"}[d] + "_random_operands"
-        if key in ceil and r["bound"] == "mfma":
+        if key in ceil and r["bound"] == "mfma" and "BF16X3" not in r["config"]:       # (the loop is of fp32 MFMAs)
             L.append(f"   kernel / ceiling (random operands) = {tf / ceil[key]['tflops']:.4f}")
         if "sq" in extra:
             sparts, cnt = extra["sq"]

@@ -114,3 +114,30 @@ def test_every_kernel_of_the_library_counts_as_one_of_its_own():
     for k in kernels:
         assert P.LIB_KERNEL.search(f"void mmbo::{k}<float, false, false>(mmbo::GemmArgs)"), k
         assert P.LIB_KERNEL.search(f"_ZN4mmbo{len(k)}{k}IDF16_Lb0EEEvNS_8GemmArgsE"), k
+
+
+def test_a_kernel_of_bf16_mfmas_has_no_ceiling_of_fp32_ones(tmp_path):
+    """The benchmark's fp32 leg measures a loop of fp32 MFMAs; three bf16 planes run beyond it."""
+    import shutil
+    tree = tmp_path / "bench_f32"
+    shutil.copytree(os.path.join(FIX, "bench_f16"), tree)
+    for d, _, files in os.walk(tree):
+        for f in files:
+            path = os.path.join(d, f)
+            text = open(path).read()
+            with open(path, "w") as out:
+                out.write(text.replace("gemm_x16_kernel", "gemm_planes_kernel").replace("f16_random_operands", "f32_random_operands"))
+    text = P.summarise("gemm_planes_f32_8192", str(tree))
+    assert "gemm_planes_kernel" in text and "ceiling" not in text and "of the 416.7 TFLOP/s matrix peak" in text
+    assert P.derived_lines({"SQ_INSTS_VALU_MFMA_MOPS_BF16": 6e9}, 1e6, 5e11) == [
+        "SQ_INSTS_VALU_MFMA_MOPS_BF16 * 512 = 3.0720e+12 flop (algorithmic 5.0000e+11; six products of planes for each)"]
+    assert sum(c.startswith("SQ_") for c in P.SQ_COUNTERS) <= 8              # what one pass holds
+
+
+def test_the_tuner_names_ids_as_the_table_does():
+    import gemm_mmbo_amd as G
+    from gemm_mmbo_amd import tune
+    ids = [tune.table_id(G, G.F32, c) for c in range(G.num_configs(G.F32))]
+    assert len(set(ids)) == len(ids) and ids[:30] == [str(c) for c in range(30)]
+    assert ids[33] == "ring_id(3, 1)" and ids[50] == "x16_id(0, 1)" and ids[89] == "x16_id(7, 16)"
+    assert ids[90:] == [f"planes_id({t}, {s})" for s in (1, 2, 4, 8, 16) for t in (0, 1)]
