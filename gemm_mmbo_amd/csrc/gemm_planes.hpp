@@ -569,7 +569,7 @@ gemm_planes_kernel(const GemmArgs args)
     //     among them.  Ordinary data has such sums too -- rows of zeros, of zeros and small integers, at k = 4096 anything below 2^-126 where no
     //     element reaches 2^-30, 2^-76 where none reaches 2^20, 2^-36 up to 2^60 --, so then the work-group looks through its rows and columns
     //     for elements below 2^-109: one more pass over the operands, bound by what a CU pulls from the L2 (a row of zeros in every tile, us
-    //     without it / with it: NN 1024^3 21.6 / 26.9, 2048^3 88 / 106, 4096^3 539 / 688, TN 640 x 384 x 10000 41 / 64).
+    //     without it / with it: NN 1024^3 21.8 / 26.6, 2048^3 92 / 113, 4096^3 556 / 649, TN 640 x 384 x 10000 40.5 / 64).
     // (c) A sum below k * 2^-138 is within reach of fp32's own smallest numbers, where the small products end.
     // With (a), (c), or an element that (b) finds, the work-group computes its tile again with fp32 MFMAs.
     float poison = 0.0f;
@@ -640,14 +640,17 @@ gemm_planes_kernel(const GemmArgs args)
     }
 
     // Steps of 16 k, four to a lane (in one load where the operand is contiguous along k), straight to registers and DEPTH steps ahead of their MFMAs.
+    // Runs of 128 k, so that no sum is less exact than those of the kernels that planes replace, whose runs are as long or longer.
     // The time is that of the planes and then the fp32 MFMAs' own.  us, ordinary data / a NaN in every tile (there, element by element and four k
-    // at a time: in brackets) / the fp32 MFMA kernels: NN 4096^3 540 / 1402 (3110) / 925, TN 538 / 1413 (4012) / 914, NT with alpha and beta 620 / 1535
-    // (2610) / 940, NN 2048^3 88 / 226 (526) / 128, NN 1024^3 21.5 / 51 (184) / 25.6, TN 640 x 384 x 10000 41 / 133 (379) / 54.
+    // at a time: in brackets) / the fp32 MFMA kernels: NN 4096^3 556 / 1479 (3110) / 927, TN 567 / 1502 (4012) / 914, NT with alpha and beta 635 / 1598
+    // (2610) / 941, NN 2048^3 92 / 235 (526) / 136, NN 1024^3 21.8 / 51.6 (184) / 25.2, TN 640 x 384 x 10000 40.5 / 130 (379) / 54.  (One run of all k: 5 %
+    // less at 4096^3.)
     if (again && stores) {
         constexpr int DEPTH = MB * NE >= 16 ? 2 : 4;
         const char *a0 = gA - kg * one_a + (TA ? 16 : 0), *b0 = gB - kg * one_b + (TB ? 0 : 16);
         // byte offsets of a lane's first k (A contiguous along the rows: of the JW rows that it has of a quad, for the blocks of all of them)
         constexpr int LA = TA ? MB : QW;
+        f32x4 total[MB][NE];                              // of whole runs
         uint32_t at_a[LA], at_b[NE];
 #pragma unroll
         for (int i = 0; i < LA; ++i) {
@@ -660,7 +663,7 @@ gemm_planes_kernel(const GemmArgs args)
             const uint32_t r = row_b(p % QB, p / QB) + OpB::lead(rows_b);
             at_b[j] = (TB ? 4 * l4 * ldb + r : r * ldb + 4 * l4) * 4;
 #pragma unroll
-            for (int i = 0; i < MB; ++i) sum[i][j] = f32x4{0, 0, 0, 0};
+            for (int i = 0; i < MB; ++i) sum[i][j] = total[i][j] = f32x4{0, 0, 0, 0};
         }
         const int steps = k_len / 16, rest = k_len % 16;
         const int64_t step_a = (TA ? (int64_t)16 : (int64_t)16 * lda) * 4, step_b = (TB ? (int64_t)16 * ldb : (int64_t)16) * 4;
@@ -711,13 +714,24 @@ gemm_planes_kernel(const GemmArgs args)
 #pragma unroll
             for (int d = 0; d < DEPTH; ++d) fetch(x[d], d);
         }
+        auto end_run = [&] {
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int j = 0; j < NE; ++j) {
+                    total[i][j] += sum[i][j];
+                    sum[i][j] = f32x4{0, 0, 0, 0};
+                }
+        };
         int s = 0;
-        for (; s + DEPTH <= steps; s += DEPTH)
+        for (; s + DEPTH <= steps; s += DEPTH) {
             static_for<DEPTH>([&](auto D) {
                 constexpr int d = decltype(D)::value;
                 multiply(x[d]);
                 fetch(x[d], min(s + d + DEPTH, steps - 1));
             });
+            if ((s + DEPTH) % 8 == 0) end_run();
+        }
         for (; s < steps; ++s) {
             fetch(x[0], s);
             multiply(x[0]);
@@ -739,6 +753,11 @@ gemm_planes_kernel(const GemmArgs args)
             });
             multiply(x[0]);
         }
+        end_run();
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NE; ++j) sum[i][j] = total[i][j];
     }
 
     // ---- and out ----------------------------------------------------------------------------------------------------

@@ -35,7 +35,7 @@
  *     product, are left out.  The 2-norm error against exact arithmetic is that of the fp32 matrix instructions or below, a third of it
  *     on long sums of terms of like size -- but 1.7 % above, at most 1.61 half units in the last place instead of 1.00, for sums with a
  *     single term that is not zero (a diagonal, a one-hot operand).  Tiles with values that planes cannot hold -- infinities, NaN, the
- *     far ends of the range -- are computed again with those instructions, in up to 1.6 times the time of a call that uses nothing else
+ *     far ends of the range -- are computed again with those instructions, in up to 1.7 times the time of a call that uses nothing else
  *     (small calls 2.0, with k split 2.5 times); exact zeros among a tile's sums cost a pass over its operands, up to 1.3 times the time
  *     (with k split 1.6).  A named config without "BF16X3" has neither.
  *     Every shape runs under MMBO_CONFIG_AUTO.  Named configs: the general kernel's (no "DTL1" in the name) take any shape and

@@ -302,3 +302,23 @@ def test_a_cut_group_of_rows_costs_no_round_trips_of_its_own():
             end.synchronize()
             best[m] = min(best[m], start.elapsed_time(end))
     assert best[1639] < 1.15 * best[1640], best
+
+
+def test_tiles_that_are_computed_again_are_as_exact():
+    """A NaN in every tile, the error of the other rows against 64 bits beside that of eight runs of fp32 matrix instructions (1,024 k each), on operands of one
+    sign, where it grows with a run's length."""
+    import gemm_mmbo_amd as G
+    native = next(c for c in range(G.num_configs(F32)) if "_ACC" in (d := G.config_info(F32, c))["name"] and d["macro_tile_m"] == d["macro_tile_n"] == 128 and d["split_k"] == 8)
+    m, n, k = 256, 128, 8192
+    p = U.Problem(F32, 1, 0, m, n, k, seed=5)
+    p.A, p.B = np.abs(p.A), np.abs(p.B)
+    p.A.reshape(m, k)[::64, 0] = np.nan
+    rows = np.arange(m) % 64 != 0
+    want = (p.B.reshape(n, k).astype(np.float64) @ p.A.reshape(m, k)[rows].astype(np.float64).T)
+
+    def error(got):
+        return float(np.linalg.norm(got.reshape(n, m)[:, rows] - want) / np.linalg.norm(want))
+    limit = error(U.run_gpu(p, native)[0])
+    for tile in range(4):
+        here = error(_run(p, tile, 1)[0])
+        assert here <= limit, (TILES[tile], here, limit)
