@@ -1004,6 +1004,11 @@ WavePick pick_wave_over(const WaveShape &q, bool may_split, int config_id, doubl
     // the geometric mean and 93 of 3,675 slower by over 3 % with 8 % throughout, 1.90 and 3 of 1,381 so.  us: NT 409 x 456 x 18536 652.6 / 164.3.
     if (w.tile >= 0 && q.dtype == MMBO_F64 && w.us >= 50.0 && w.us >= (q.wide_c ? 0.83 : 0.92) * table_us && w.us >= 0.75 * us)
         return WavePick{-1, 0, 0, bar};
+    // (fp32: nor for fewer runs of k than the config's, whose sums are the more exact -- 3 of 3,000 drawn calls, TT 55 x 4480 x 2298 eight runs, here four --
+    // unless, again, the tables' own model says so)
+    if (w.tile >= 0 && q.dtype == MMBO_F32 && is_staged(q.dtype, config_id) && w.us >= (q.wide_c ? 0.83 : 0.92) * table_us &&
+        w.waves * w.split < config_ref(config_id).split)
+        return WavePick{-1, 0, 0, bar};
     if (w.tile >= 0 && w.us >= 8.0 && is_staged(q.dtype, config_id)) {
         const bool half = (w.waves == 1 && std::min(q.m, q.n) > 32) || (q.dtype == MMBO_F32 && w.us > 40.0);
         if (w.us >= (q.wide_c ? 0.83 : 0.92) * table_us && w.us >= (q.dtype == MMBO_F32 ? (half ? 0.45 : 0.75) : half ? 0.5 : 0.8) * us) return WavePick{-1, 0, 0, bar};

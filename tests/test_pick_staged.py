@@ -26,3 +26,16 @@ def test_where_the_pick_leaves_the_tables(dtype, ta, tb, m, n, k, batch, wave):
     # whether a call needs a workspace still follows from the pick of the tables
     if a["split_k"] > 1:
         assert G.config_info(dtype, G.select_config(dtype, ta, tb, m, n, k, batch))["split_k"] > 1
+
+
+@pytest.mark.parametrize("ta,tb,m,n,k,runs", [(1, 1, 55, 4480, 2298, 8), (1, 0, 3232, 36, 3968, 8), (1, 0, 1456, 42, 8064, 16)])
+def test_fp32_sums_are_not_added_up_in_fewer_runs_than_the_staged_kernels(ta, tb, m, n, k, runs):
+    import re
+
+    import gemm_mmbo_amd as G
+    assert "DTL1" not in (staged := G.config_info(U.F32, G.select_config(U.F32, ta, tb, m, n, k)))["name"] and staged["split_k"] == runs
+    a = G.auto_info(U.F32, ta, tb, m, n, k)
+    lsu = re.search(r"LSU(\d+)", a["name"])
+    if "_BF16X3" in a["name"]:                   # (a rule of its own)
+        return
+    assert a["split_k"] * (int(lsu[1]) if lsu else 1) >= runs, a["name"]
