@@ -64,16 +64,18 @@ def time_config(G, torch, dtype, ta, tb, m, n, k, batch, alpha, beta, cfg, reps)
 
 def table_id(G, dtype, cfg):
     """A config id in the syntax of csrc/tuned_table.hpp: ring_id(tile, GlobalSplitU) / x16_id(tile, GlobalSplitU) for the
-    direct-to-LDS families and planes_id for fp32 in bf16 planes (tile = row of kRingTiles / kX16Tiles / kPlanesTiles), the plain number
-    otherwise (staged ids, fp64 rows)."""
-    def family(c):
-        name = G.config_info(dtype, c)["name"]
-        return "planes_id" if "_BF16X3" in name else None if "DTL1" not in name else "x16_id" if "_ACC" in name else "ring_id"
-    if dtype == G.F64 or family(cfg) is None:
+    direct-to-LDS families (tile = row of kRingTiles / kX16Tiles), the plain number otherwise (staged ids, fp64 rows)."""
+    if dtype == G.F64:
         return str(cfg)
-    split = G.config_info(dtype, cfg)["split_k"]
-    unsplit = [c for c in range(G.num_configs(dtype)) if family(c) == family(cfg) and G.config_info(dtype, c)["split_k"] == 1]
-    return f"{family(cfg)}({(cfg - unsplit[0]) % len(unsplit)}, {split})"
+    d = G.config_info(dtype, cfg)
+    if "DTL1" not in d["name"]:
+        return str(cfg)
+    fam = [c for c in range(G.num_configs(dtype))
+           if ("DTL1" in G.config_info(dtype, c)["name"]) and (("_ACC" in G.config_info(dtype, c)["name"]) == ("_ACC" in d["name"]))
+           and G.config_info(dtype, c)["split_k"] == 1]
+    ntiles = len(fam)
+    tile = (cfg - fam[0]) % ntiles
+    return f"{'x16_id' if '_ACC' in d['name'] else 'ring_id'}({tile}, {d['split_k']})"
 
 
 def passes_check(G, torch, dtype, ta, tb, m, n, k, batch, alpha, beta, cfg):

@@ -132,12 +132,3 @@ def test_a_kernel_of_bf16_mfmas_has_no_ceiling_of_fp32_ones(tmp_path):
     assert P.derived_lines({"SQ_INSTS_VALU_MFMA_MOPS_BF16": 6e9}, 1e6, 5e11) == [
         "SQ_INSTS_VALU_MFMA_MOPS_BF16 * 512 = 3.0720e+12 flop (algorithmic 5.0000e+11; six products of planes for each)"]
     assert sum(c.startswith("SQ_") for c in P.SQ_COUNTERS) <= 8              # what one pass holds
-
-
-def test_the_tuner_names_ids_as_the_table_does():
-    import gemm_mmbo_amd as G
-    from gemm_mmbo_amd import tune
-    ids = [tune.table_id(G, G.F32, c) for c in range(G.num_configs(G.F32))]
-    assert len(set(ids)) == len(ids) and ids[:30] == [str(c) for c in range(30)]
-    assert ids[33] == "ring_id(3, 1)" and ids[50] == "x16_id(0, 1)" and ids[89] == "x16_id(7, 16)"
-    assert ids[90:] == [f"planes_id({t}, {s})" for s in (1, 2, 4, 8, 16) for t in (0, 1)]
