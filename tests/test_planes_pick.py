@@ -97,3 +97,58 @@ def test_partial_sums_that_the_static_workspace_does_not_hold(ta, tb, m, n, k, b
     G.gemm_strided_batched_static_workspace(F32, ta, tb, m, n, k, 1.0, A, p.lda, p.sa, B, p.ldb, p.sb, 0.0, C, p.ldc, p.sc, batch)
     torch.cuda.synchronize()
     assert np.array_equal(C.cpu().numpy(), P._run(p, tile, split)[0])
+
+
+CHANGES = [(1, 1, 4373, 72, 15807), (0, 0, 7440, 41, 14752)]
+
+
+def _calls(ta, tb, m, n, k):
+    """(padding of the leading dimensions, beta): calls of one shape that go to planes, and to another kernel whose runs planes would lengthen."""
+    import gemm_mmbo_amd as G
+    calls = [(0, 0.0), (1, 0.5), (0, 0.5)]
+    return calls, [G.auto_info(F32, ta, tb, m, n, k, 1, (k if ta else m) + pad, (n if tb else k) + pad, m, beta != 0)["name"] for pad, beta in calls]
+
+
+@pytest.mark.parametrize("shape", CHANGES)
+def test_calls_of_one_shape_may_differ_in_the_kernel(shape):
+    names = _calls(*shape)[1]
+    assert "_BF16X3" in names[0] and "_BF16X3" not in names[1], names
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", CHANGES)
+def test_one_call_of_such_a_shape_leaves_the_workspace_of_all(shape):
+    """Either kind of call first, then each captured: nothing is allocated, and each replay gives the bits of the eager call."""
+    import torch
+
+    import gemm_mmbo_amd as G
+    ta, tb, m, n, k = shape
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        A, B, C0 = (torch.rand(x, device="cuda") for x in ((m + k + 1) + (m + 1) * (k + 1), (n + k + 1) + (n + 1) * (k + 1), m * n))
+        C = C0.clone()
+
+        def call(pad, beta):
+            G.gemm(F32, ta, tb, m, n, k, 1.0, A, (k if ta else m) + pad, B, (n if tb else k) + pad, beta, C, m, -1, stream)
+        calls = _calls(*shape)[0]
+        for first in calls[:2]:
+            torch.cuda.synchronize()
+            G.release_workspace()
+            call(*first)
+            torch.cuda.synchronize()
+            held = G.workspace_info()
+            for c in calls:
+                C.copy_(C0)
+                call(*c)
+                torch.cuda.synchronize()
+                want = C.clone()
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=stream):
+                    call(*c)
+                for _ in range(3):
+                    C.copy_(C0)
+                    graph.replay()
+                    torch.cuda.synchronize()
+                    assert torch.equal(C, want), (shape, c)
+                assert G.workspace_info() == held, (shape, c)
+    G.release_workspace()
