@@ -33,8 +33,8 @@
  *     formed on the bf16 matrix pipes from three bf16 planes per operand ("BF16X3" in the name; ids behind the other types' table for
  *     two of its tiles).  No bit of an operand is dropped; of the nine products of planes three, together below 2^-23 of a
  *     product, are left out.  The 2-norm error against exact arithmetic is that of the fp32 matrix instructions or below, a third of it
- *     on long sums of terms of like size -- but 1.7 % above, at most 1.61 half units in the last place instead of 1.00, for sums with a
- *     single term that is not zero (a diagonal, a one-hot operand).  Tiles with values that planes cannot hold -- infinities, NaN, the
+ *     on long sums of terms of like size -- but 1.7 % above, at most 1.61 half units in the last place instead of 1.00, for sums that
+ *     a single term makes up (a diagonal, a one-hot operand).  Tiles with values that planes cannot hold -- infinities, NaN, the
  *     far ends of the range -- are computed again with those instructions, in up to 1.7 times the time of a call that uses nothing else
  *     (small calls 2.0, with k split 2.5 times); exact zeros among a tile's sums cost a pass over its operands, up to 1.3 times the time
  *     (with k split 1.6).  A named config without "BF16X3" has neither.
